@@ -196,9 +196,17 @@ def work(case):
 
 
 def tolerance(case):
-    # About four times the largest error measured against the same computation in 64 bits, over head sizes, masks,
-    # dropout and lengths up to 4096: attention 1.2e-6 (fp32), 3.5e-4 (fp16), 2.8e-3 (bf16); rows 7.2e-7, 3.1e-4, 2.4e-3
-    # (dropout rounds a 16-bit result once more).
+    # About four times the largest error measured against the same computation in 64 bits, over head sizes, masks, dropout
+    # and lengths ("rel"; "max" in brackets):
+    #   attention  fp32 1.2e-6 (4.6e-5)   fp16 3.5e-4 (1.5e-2)   bf16 2.8e-3 (0.12)
+    #   rows       fp32 7.2e-7 (3.0e-5)   fp16 3.1e-4 (3.1e-2)   bf16 2.4e-3 (0.28); dropout rounds 16 bits once more
+    #   columns in fp32: a sum in plain order down the column is off in proportion to its length, 2.6e-6 at 4096 elements
+    #   and 7.5e-5 (2.0e-3) at 65536
+    dtype = case["dtype"]
     if case["op"] == "rows":
-        return {"rel": {"float32": 3e-6, "float16": 1.4e-3, "bfloat16": 1.1e-2}[case["dtype"]]}
-    return {"rel": {"float32": 5e-6, "float16": 1.4e-3, "bfloat16": 1.1e-2}[case["dtype"]]}
+        limits = {"float32": {"rel": 3e-6, "max": 1.2e-4}, "float16": {"rel": 1.4e-3, "max": 0.13}, "bfloat16": {"rel": 1.1e-2, "max": 0.95}}
+        if dtype == "float32" and case["dim"] == 0:
+            rel = max(3e-6, 4.8e-9 * case["rows"])
+            return {"rel": rel, "max": 40 * rel}
+        return limits[dtype]
+    return {"float32": {"rel": 5e-6, "max": 2e-4}, "float16": {"rel": 1.4e-3, "max": 6e-2}, "bfloat16": {"rel": 1.1e-2, "max": 0.5}}[dtype]
