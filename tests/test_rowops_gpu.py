@@ -80,10 +80,29 @@ def test_modules_keep_dtype(dtype, device):
                                        ((300, 33), 0), ((4, 6, 128), 2)])
 def test_softmax_shapes_and_dtypes(shape, dim, dtype, device):
     """Wave-per-row and workgroup-per-row kernels, rows that stay in registers and rows too long for that (two sweeps),
-    16-byte and per-element accesses (odd lengths), the thread-per-row kernel (dim 0), a contiguous 3-D input along
+    16-byte and per-element accesses (odd lengths), the column kernel (dim 0), a contiguous 3-D input along
     its last dimension."""
     x, g = _pair(shape, 10 + shape[-1], dtype)
     _softmax_case(device, x * 3, g, dim, dtype, tag=f"softmax {shape} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,mask_dtype", [((2, 40), None), ((129, 2056), torch.uint8), ((4101, 24), torch.int64), ((300, 777), torch.bfloat16),
+                                              ((20000, 8), None), ((35001, 3), torch.bool), ((1025, 4096), None)])
+def test_softmax_down_the_columns(shape, mask_dtype, dtype, device):
+    """The column kernels: columns that stay in registers and columns swept twice, whole vectors and single elements across
+    the columns (odd widths), panels of every width, fewer panels than XCDs, masks of every element size."""
+    x, g = _pair(shape, 70 + shape[1], dtype)
+    mask = None if mask_dtype is None else _build_mask(shape, 71).to(mask_dtype)
+    if mask_dtype is None:
+        _softmax_case(device, x * 3, g, 0, dtype, tag=f"columns {shape} {dtype}")
+        return
+    tx = (x * 3).to(device).requires_grad_(True)
+    out = trident.function.masked_softmax(tx, mask.to(device), 0)
+    out.backward(g.to(device))
+    want = rowops.softmax_forward(parity.to64((x * 3).to(dtype)), 0, mask.float().numpy())
+    parity.close(out, want, dtype, f"columns {shape} {dtype} {mask_dtype}")
+    parity.close(tx.grad, rowops.softmax_backward(parity.to64(out), parity.to64(g), 0), dtype, f"columns {shape} grad")
 
 
 @pytest.mark.parametrize("mask_dtype", [torch.int64, torch.int32, torch.bool, torch.uint8, torch.float32, torch.bfloat16])
