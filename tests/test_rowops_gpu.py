@@ -79,11 +79,29 @@ def test_modules_keep_dtype(dtype, device):
 @pytest.mark.parametrize("shape,dim", [((5, 7), 1), ((64, 2048), 1), ((9, 2056), 1), ((3, 5000), 1), ((17, 4097), 1), ((3, 20000), 1),
                                        ((300, 33), 0), ((4, 6, 128), 2)])
 def test_softmax_shapes_and_dtypes(shape, dim, dtype, device):
-    """Wave-per-row and workgroup-per-row kernels, rows that stay in registers and rows too long for that (two sweeps),
+    """16 lanes, a wave or a workgroup per row, rows that stay in registers and rows too long for that (two sweeps),
     16-byte and per-element accesses (odd lengths), the column kernel (dim 0), a contiguous 3-D input along
     its last dimension."""
     x, g = _pair(shape, 10 + shape[-1], dtype)
     _softmax_case(device, x * 3, g, dim, dtype, tag=f"softmax {shape} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("x_size", [1, 3, 9, 255, 505, 513, 1273, 2041, 2047, 2553, 5113, 5121, 10239, 10241])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_softmax_of_rows_off_the_16_byte_boundaries(x_size, offset, dtype, device):
+    """Odd row lengths: the last length that each thread group holds in registers and the first beyond it (a row shares up to
+    two 16-byte pieces with its neighbours), with a mask; and the same rows in tensors that are not aligned themselves."""
+    rows = 5
+    storage, g = _pair((rows * x_size + offset,), 90 + x_size, dtype)
+    mask = _build_mask((rows, x_size), 91).to(torch.uint8)
+    tx = (storage * 3).to(device)[offset:].view(rows, x_size).requires_grad_(True)
+    tg = g.to(device)[offset:].view(rows, x_size)
+    out = trident.function.masked_softmax(tx, mask.to(device), 1)
+    (grad,) = torch.autograd.grad(out, (tx,), tg)
+    want = rowops.softmax_forward(parity.to64(tx.detach()), 1, mask.numpy())
+    parity.close(out, want, dtype, f"rows {x_size} + {offset} {dtype}")
+    parity.close(grad, rowops.softmax_backward(parity.to64(out), parity.to64(tg), 1), dtype, f"rows {x_size} + {offset} grad")
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
