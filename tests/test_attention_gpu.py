@@ -504,6 +504,15 @@ def test_random_problems(dtype, S, D, variant, batches, heads, seed, device):
     _abi_case(device, dtype, S, D, variant, seed, batches=batches, heads=heads)
 
 
+@pytest.mark.parametrize("variant", ["plain", "causal", "dropout", "causal+dropout"])
+@pytest.mark.parametrize("dtype,S", [(torch.float16, 1), (torch.bfloat16, 33), (torch.float16, 224), (torch.bfloat16, 257),
+                                     (torch.bfloat16, 481), (torch.float16, 511), (torch.bfloat16, 640), (torch.bfloat16, 769)])
+def test_any_length_of_the_phased_kernels_at_head_size_128(dtype, S, variant, device):
+    """Boundary handling of the 8-wave forward, phased dQ (unphased with dropout) and phased dK/dV kernels: a single row, a
+    last workgroup with one row, with whole waves that have none, a length that ends with a 32-row block."""
+    _abi_case(device, dtype, S, 128, variant, 4600 + S, batches=1, heads=3, matrix_cores=True)
+
+
 # ------------------------------------------------------------------ tile counts of the phased kernels
 @pytest.mark.parametrize("variant", ["plain", "causal", "causal+dropout"])
 @pytest.mark.parametrize("S,D", [(256, 128), (768, 128), (1280, 128), (768, 64), (1024, 64), (256, 32), (1280, 32)])
@@ -561,6 +570,13 @@ def test_a_head_does_not_depend_on_its_company(B, H, S, D, causal, device):
     parity.close(dq[B - 1:, hs], dq_r, dtype, "company dQ", a_dq)
     parity.close(dk[B - 1:, hs], dk_r, dtype, "company dK", a_dk)
     parity.close(dv[B - 1:, hs], dv_r, dtype, "company dV", a_dv)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_a_head_does_not_depend_on_its_company_at_any_length(causal, device):
+    """The same at a length that ends inside a workgroup's rows: 300 items on 256 compute units, so that persistent forward
+    workgroups go from a partial row tile to a whole one and back."""
+    test_a_head_does_not_depend_on_its_company(10, 10, 600, 128, causal, device)
 
 
 # ------------------------------------------------------------------ the combined backward entry point

@@ -32,7 +32,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // tiles (plus their lse and delta) in a ring of 4 filled by LDS-direct loads three tiles ahead.
 // Per 32-row query block: S = Q K^T and dP = dO V^T from row fragments, P and dS on the vector
 // ALU, dV^T += dO^T P and dK^T += Q^T dS with the transposed LDS reads of the same tiles.
-// RAGGED (4 waves, no mask; also serves D = 128, one workgroup per CU): S is not a multiple of 128. Loads clamp their
+// RAGGED (4 waves, no mask): S is not a multiple of 128. Loads clamp their
 // row index to S - 1, query rows >= S get probability 0 (they would otherwise add the last row once more), keys >= S
 // are not stored.
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false>
@@ -781,7 +781,10 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
 // With KEYMASK (kMaskF32 / kMaskT; never with the causal mask): an additive mask that is the same for every query row
 // (row stride 0: a key-padding mask). Lanes own keys here, so the whole mask is one value per lane, read once, and goes
 // into the exponent for free (the multiply by the scale becomes a fused multiply-add).
-template <typename T, int D, bool CAUSAL, bool DROPOUT = false, int KEYMASK = kNoMask>
+// RAGGED: S is not a multiple of 128. Loads clamp their row index to S - 1, rows at or beyond S get probability 0 (the
+// number of blocks is rounded up to an even one, at least four, as the phases assume; blocks wholly beyond S hold the
+// last row again and again), keys at or beyond S are not stored.
+template <typename T, int D, bool CAUSAL, bool DROPOUT = false, int KEYMASK = kNoMask, bool RAGGED = false>
 __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams p) {
     static_assert(KEYMASK == kNoMask || !CAUSAL, "a mask excludes the causal variant");
     using Tile = SwzTile<D>;
@@ -799,7 +802,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     static_assert(kHalfBytes == NW * 1024, "two Q loads and two dO loads per requesting wave and block");
     constexpr int kAccSteps = 4 * DH;                        // MFMAs that add one block
     constexpr int kSteps = 2 * kAccSteps + 2 * KK;           // matrix phase
-    constexpr int kRing = 4;
+    // (one fragment fewer in flight where boundary handling leaves no registers for four)
+    constexpr int kRing = RAGGED && !CAUSAL && !DROPOUT && std::is_same<T, f16_t>::value ? 3 : 4;
     __shared__ __attribute__((aligned(1024))) char smem[kSlots * kSlotBytes + kXchBytes];
     char* xch = smem + kSlots * kSlotBytes;
 
@@ -808,7 +812,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     const int kb = wave & 3, member = wave >> 2;
     const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     int bh, kt;
-    map_block(blockIdx.x, p.B * p.H, p.S / kKeys, CAUSAL ? kHeavyFirst : kUniformTiles, &bh, &kt);
+    map_block(blockIdx.x, p.B * p.H, (p.S + kKeys - 1) / kKeys, CAUSAL ? kHeavyFirst : kUniformTiles, &bh, &kt);
     const int b = bh / p.H, hd = bh % p.H;
     const int k0 = kt * kKeys;
     const int wkey0 = k0 + 32 * kb;
@@ -834,7 +838,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     }
 
     const int row_first = CAUSAL ? k0 : 0;          // first streamed row (block 0)
-    const int n_blocks = (p.S - row_first) / kBR;   // >= 4, even
+    const int n_blocks = RAGGED ? max(4, (p.S - row_first + 2 * kBR - 1) / (2 * kBR) * 2) : (p.S - row_first) / kBR;   // >= 4, even
     // A block is requested by the four waves of ONE member, the one that is in its vector phase when the request is
     // due (member 0 the even blocks, member 1 the odd ones): a vector-memory instruction holds its wave until the
     // memory pipeline has taken it, which the matrix phase cannot afford. Wave kb of the member fetches the 1 KiB
@@ -851,11 +855,27 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     auto issue_block = [&]() {  // this wave's share of its member's next block, if it exists
         if (next_block < n_blocks) {
             char* slot = smem + next_slot * kSlotBytes;
+            const int row0 = row_first + next_block * kBR;
+            if (RAGGED && row0 + kBR > p.S) {  // the sequence ends inside this block or before it
+                const int from = min(row0, p.S - 1), last = p.S - 1 - from;
+                int lane = threadIdx.x & 63;  // (offsets made here, not kept in registers across the loop)
+                asm volatile("" : "+v"(lane));
+                const char* q_from = qbase + from * qrow_bytes;
+                const char* g_from = gbase + from * grow_bytes;
+                lds_direct_load16(q_from, Tile::src_off_clamped(kb, lane, qrow_bytes, last), slot + kb * 1024);
+                lds_direct_load16(g_from, Tile::src_off_clamped(kb, lane, grow_bytes, last), slot + kHalfBytes + kb * 1024);
+                lds_direct_load16(q_from, Tile::src_off_clamped(kb + 4, lane, qrow_bytes, last), slot + (kb + 4) * 1024);
+                lds_direct_load16(g_from, Tile::src_off_clamped(kb + 4, lane, grow_bytes, last), slot + kHalfBytes + (kb + 4) * 1024);
+                lds_direct_load4(((kb & 1) ? delta_base : lse_base) + from, min(lane & 31, last) * 4, slot + aux_lds);
+            } else {
             lds_direct_load16(next_q, qoff, slot + kb * 1024);
             lds_direct_load16(next_g, goff, slot + kHalfBytes + kb * 1024);
             lds_direct_load16(next_q + 16 * qrow_bytes, qoff, slot + (kb + 4) * 1024);
             lds_direct_load16(next_g + 16 * grow_bytes, goff, slot + kHalfBytes + (kb + 4) * 1024);
-            lds_direct_load4(next_aux, (lane & 31) * 4, slot + aux_lds);
+            int aux = threadIdx.x & 31;
+            if constexpr (RAGGED) asm volatile("" : "+v"(aux));
+            lds_direct_load4(next_aux, aux * 4, slot + aux_lds);
+            }
         }
         next_block += 2;
         next_slot = next_slot >= kSlots - 2 ? next_slot + 2 - kSlots : next_slot + 2;
@@ -883,8 +903,10 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
             const int tile = blk / Tile::kBlocks, b16 = blk % Tile::kBlocks;
             const bool is_v = tile >= 2;
             const int64_t rb = is_v ? vrow_bytes : krow_bytes;
-            const char* src = (is_v ? vbase : kbase) + (k0 + 64 * (tile & 1)) * rb;
-            lds_direct_load16(src, static_cast<uint32_t>(Tile::src_off(b16, lane, rb)), kv_lds + blk * 1024);
+            const int row0 = k0 + 64 * (tile & 1), from = RAGGED ? min(row0, p.S - 1) : row0;
+            const char* src = (is_v ? vbase : kbase) + from * rb;
+            lds_direct_load16(src, RAGGED ? Tile::src_off_clamped(b16, lane, rb, p.S - 1 - from) : static_cast<uint32_t>(Tile::src_off(b16, lane, rb)),
+                              kv_lds + blk * 1024);
         }
     }
     issue_block();  // blocks 0 and 2 (member 0), 1 and 3 (member 1)
@@ -1007,6 +1029,12 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
             asm volatile("" : "+s"(rbo));
 #pragma unroll
             for (int i = 0; i < 16; ++i) sc_s[i] = key <= rbo + c_row(i, h) ? sc_s[i] : -INFINITY;
+        }
+        if (RAGGED && rb + kBR > p.S) {  // rows that do not exist (taken for the last blocks only, as above)
+            int left = p.S - rb - 4 * h;
+            asm volatile("" : "+v"(left));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc_s[i] = c_row(i, 0) < left ? sc_s[i] : -INFINITY;
         }
         const f32x16 s = sc_s, dp = sc_dp;
         const float* sDelta = reinterpret_cast<const float*>(smem + so + 2 * kHalfBytes) + 64;
@@ -1161,9 +1189,9 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
         // (the lane index taken afresh: the epilogue's per-lane offsets are computed here, not kept across the loop)
         int elane = threadIdx.x & 63;
         asm volatile("" : "+v"(elane));
-        Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, elane);
+        Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, elane, RAGGED ? p.S - wkey0 : 32);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
-        Store::run(dv, [](float x) { return x; }, patch, dv0, p.dvs[2] * 2, elane);
+        Store::run(dv, [](float x) { return x; }, patch, dv0, p.dvs[2] * 2, elane, RAGGED ? p.S - wkey0 : 32);
     }
 }
 
@@ -1178,13 +1206,20 @@ int launch_dkdv_waves(const KParams& p, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
     if (p.S % 128 != 0) {
-        // any length (no mask): 128-key workgroups of the 32-keys-per-wave kernel with boundary handling, for both
-        // head sizes (at D = 128 with the whole register file, one workgroup per CU)
+        // any length (no mask): 128-key workgroups with boundary handling
         if constexpr (MASK == kNoMask) {
-            const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
-            return static_cast<int>(hipGetLastError());
+            if constexpr (D == 128) {
+                const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(512);
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, CAUSAL, true, kNoMask, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, CAUSAL, false, kNoMask, true>), grid, block, 0, stream, p);
+                return static_cast<int>(hipGetLastError());
+            }
+            if constexpr (D < 128) {
+                const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+                return static_cast<int>(hipGetLastError());
+            }
         }
         return TRI_ATTN_ESHAPE;  // (mfma_supported keeps masked problems of such lengths away)
     }

@@ -32,7 +32,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // staging registers, no ds_write). Per 32-key block: S^T = K Q^T and dP^T = V dO^T from row
 // fragments, dS^T = P^T (dP^T - delta) on the vector ALU, dQ^T += K^T dS^T with K^T read through
 // transposed LDS reads of the same K tile.
-// RAGGED (4 waves, no mask): S is not a multiple of 128. Rows and keys at or beyond S do not exist: loads clamp
+// RAGGED (no mask): S is not a multiple of 32 NW. Rows and keys at or beyond S do not exist: loads clamp
 // their row index to S - 1, keys >= S get probability 0, rows >= S are not stored.
 // DMASK (with a mask): the kernel also writes the mask gradient dS (trident/kernel/attention.py:332-335), each lane four
 // consecutive keys of its row at a time; where the mask is broadcast over a dimension (dmask stride 0) the values are
@@ -41,7 +41,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // of reading it, and stores it for the dK/dV pass, which then runs after this one (tri_attn_bwd_dq_delta).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool DMASK = false, bool DELTA = false>
 __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
-    static_assert(!RAGGED || (NW == 4 && MASK == 0), "ragged lengths: 4 waves, no mask");
+    static_assert(!RAGGED || MASK == 0, "ragged lengths: no mask");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
     static_assert(!DELTA || MASK == 0, "delta on the way: the variants without a mask");
     using Tile = SwzTile<D>;
@@ -110,6 +110,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
     const int num_key_tiles = (p.S + kBN - 1) / kBN;
     int n_tiles = CAUSAL ? min((q0 + kRows) / kBN, num_key_tiles) : num_key_tiles;  // tiles the workgroup streams
     int my_tiles = CAUSAL ? min((wrow0 + 31) / kBN + 1, n_tiles) : n_tiles;         // tiles with keys visible to this wave
+    if (RAGGED && wrow0 >= p.S) my_tiles = 0;                                       // (a wave without a single row)
     // With the classes of the mask's blocks at hand: key tiles behind the last one that is not masked out altogether
     // are not streamed, and tiles whose mask is all zero over the workgroup's rows are not read.
     uint64_t zero_tiles = 0;
@@ -143,9 +144,13 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
             const bool is_v = blk >= Tile::kBlocks;
             const char* tile_src = is_v ? vbase + static_cast<int64_t>(t) * kBN * vrow_bytes
                                         : kbase + static_cast<int64_t>(t) * kBN * krow_bytes;
-            if (RAGGED && (t + 1) * kBN > p.S)  // the sequence ends inside this tile
-                lds_direct_load16(tile_src, Tile::src_off_clamped(is_v ? blk - Tile::kBlocks : blk, lane, is_v ? vrow_bytes : krow_bytes,
+            // the sequence ends inside this tile (at D = 128 every tile takes the clamped form: no registers for kept offsets)
+            if (RAGGED && (D == 128 || (t + 1) * kBN > p.S)) {
+                int l = lane;
+                asm volatile("" : "+v"(l));
+                lds_direct_load16(tile_src, Tile::src_off_clamped(is_v ? blk - Tile::kBlocks : blk, l, is_v ? vrow_bytes : krow_bytes,
                                                                   p.S - 1 - t * kBN), stage + blk * 1024);
+            }
             else
                 lds_direct_load16(tile_src, src_off[i], stage + blk * 1024);
         }
@@ -364,7 +369,9 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
 // With DELTA the kernel also computes delta = rowsum(dO * O) of its rows (instead of reading it) and stores
 // it for the dK/dV pass, which then has to run after this one: the separate pre-pass over O and dO
 // (trident/kernel/softmax.py:180-238) disappears into the prologue that loads the dO rows anyway.
-template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA>
+// RAGGED: S is not a multiple of 256; rows and keys at or beyond S as in the kernel above (clamped loads, probability 0,
+// not stored), a wave without a single row of its own only fetches and meets the barriers.
+template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false>
 __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p) {
     using Tile = SwzTile<D>;
     constexpr int NW = 8;
@@ -397,29 +404,34 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, l32 = lane & 31, h = lane >> 5;
     int bh, qt;
-    map_block(blockIdx.x, p.B * p.H, p.S / kRows, CAUSAL ? kHeavyLast : kUniformTiles, &bh, &qt);
+    map_block(blockIdx.x, p.B * p.H, (p.S + kRows - 1) / kRows, CAUSAL ? kHeavyLast : kUniformTiles, &bh, &qt);
     const int b = bh / p.H, hd = bh % p.H;
     const int q0 = qt * kRows;
     const int wrow0 = q0 + 32 * wave;
     const int qrow = wrow0 + l32;
+    const int wrow_ld = RAGGED ? min(wrow0, p.S - 1) : wrow0;  // (rows that do not exist read the last one)
+    const int qrow_ld = RAGGED ? min(qrow, p.S - 1) : qrow;
+    auto row_off = [&](int blk, int64_t stride_bytes) {  // of piece blk of this wave's rows, from row wrow_ld
+        return RAGGED ? Tile::src_off_clamped(blk, lane, stride_bytes, p.S - 1 - wrow_ld) : static_cast<uint32_t>(Tile::src_off(blk, lane, stride_bytes));
+    };
 
-    const char* qrows = static_cast<const char*>(p.q) + (b * p.qs[0] + hd * p.qs[1] + static_cast<int64_t>(wrow0) * p.qs[2]) * 2;
-    const char* gorows = static_cast<const char*>(p.d_o) + (b * p.dos[0] + hd * p.dos[1] + static_cast<int64_t>(wrow0) * p.dos[2]) * 2;
+    const char* qrows = static_cast<const char*>(p.q) + (b * p.qs[0] + hd * p.qs[1] + static_cast<int64_t>(wrow_ld) * p.qs[2]) * 2;
+    const char* gorows = static_cast<const char*>(p.d_o) + (b * p.dos[0] + hd * p.dos[1] + static_cast<int64_t>(wrow_ld) * p.dos[2]) * 2;
     const char* kbase = static_cast<const char*>(p.k) + (b * p.ks[0] + hd * p.ks[1]) * 2;
     const char* vbase = static_cast<const char*>(p.v) + (b * p.vs[0] + hd * p.vs[1]) * 2;
     const int64_t krow_bytes = p.ks[2] * 2, vrow_bytes = p.vs[2] * 2;
 
-    float lse = p.lse[static_cast<int64_t>(bh) * p.S + qrow];
+    float lse = p.lse[static_cast<int64_t>(bh) * p.S + qrow_ld];
     float dlt = 0.f;
-    if constexpr (!DELTA) dlt = p.delta[static_cast<int64_t>(bh) * p.S + qrow];
+    if constexpr (!DELTA) dlt = p.delta[static_cast<int64_t>(bh) * p.S + qrow_ld];
     char* q_stage = smem + kStageBytes + wave * kWaveRowBytes;
     char* g_stage = q_stage + NW * kWaveRowBytes;
 #pragma unroll
     for (int blk = 0; blk < kRowLoads; ++blk)
-        lds_direct_load16(qrows, static_cast<uint32_t>(Tile::src_off(blk, lane, p.qs[2] * 2)), q_stage + blk * 1024);
+        lds_direct_load16(qrows, row_off(blk, p.qs[2] * 2), q_stage + blk * 1024);
 #pragma unroll
     for (int blk = 0; blk < kRowLoads; ++blk)
-        lds_direct_load16(gorows, static_cast<uint32_t>(Tile::src_off(blk, lane, p.dos[2] * 2)), g_stage + blk * 1024);
+        lds_direct_load16(gorows, row_off(blk, p.dos[2] * 2), g_stage + blk * 1024);
     const float c = p.scale_log2;
     [[maybe_unused]] const float inv_scale = p.inv_scale;  // (a mask value joins its score before the scale: s + mask / scale)
 
@@ -427,8 +439,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = zero16();
 
-    const int n_tiles = CAUSAL ? (q0 + kRows) / kBN : p.S / kBN;     // tiles the workgroup streams
-    const int my_tiles = CAUSAL ? (wrow0 + 31) / kBN + 1 : n_tiles;  // tiles with keys visible to this wave
+    int n_tiles = CAUSAL ? (q0 + kRows) / kBN : p.S / kBN;     // tiles the workgroup streams
+    int my_tiles = CAUSAL ? (wrow0 + 31) / kBN + 1 : n_tiles;  // tiles with keys visible to this wave
+    if constexpr (RAGGED) {
+        const int num_key_tiles = (p.S + kBN - 1) / kBN;
+        n_tiles = CAUSAL ? min(n_tiles, num_key_tiles) : num_key_tiles;
+        my_tiles = wrow0 >= p.S ? 0 : (CAUSAL ? min(my_tiles, n_tiles) : n_tiles);
+    }
 
     // A wave fetches blocks wave, wave + NW, ... of the K tile and of the V tile: their rows are a
     // multiple of 16 apart, so one per-lane source offset serves all of them.
@@ -436,6 +453,18 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     const uint32_t voff = static_cast<uint32_t>(Tile::src_off(wave, lane, vrow_bytes));
     auto issue_tile = [&](int t) {
         char* stage = smem + (t % kStages) * kStageBytes + wave * 1024;
+        if (RAGGED && (t + 1) * kBN > p.S) {  // the sequence ends inside this tile
+            const int last = p.S - 1 - t * kBN;
+#pragma unroll
+            for (int i = 0; i < kPerOperand; ++i)
+                lds_direct_load16(kbase + static_cast<int64_t>(t) * kBN * krow_bytes,
+                                  Tile::src_off_clamped(wave + i * NW, lane, krow_bytes, last), stage + i * NW * 1024);
+#pragma unroll
+            for (int i = 0; i < kPerOperand; ++i)
+                lds_direct_load16(vbase + static_cast<int64_t>(t) * kBN * vrow_bytes,
+                                  Tile::src_off_clamped(wave + i * NW, lane, vrow_bytes, last), stage + Tile::kBytes + i * NW * 1024);
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < kPerOperand; ++i)
             lds_direct_load16(kbase + (static_cast<int64_t>(t) * kBN + i * kRowStep) * krow_bytes, koff, stage + i * NW * 1024);
@@ -461,11 +490,11 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     if constexpr (DELTA) {
         // the O rows follow into the place of the Q rows; this lane holds half of its row (the other half is
         // in lane ^ 32)
-        const char* orows = static_cast<const char*>(p.o) + (b * p.os[0] + hd * p.os[1] + static_cast<int64_t>(wrow0) * p.os[2]) * 2;
+        const char* orows = static_cast<const char*>(p.o) + (b * p.os[0] + hd * p.os[1] + static_cast<int64_t>(wrow_ld) * p.os[2]) * 2;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the Q rows are in registers
 #pragma unroll
         for (int blk = 0; blk < kRowLoads; ++blk)
-            lds_direct_load16(orows, static_cast<uint32_t>(Tile::src_off(blk, lane, p.os[2] * 2)), q_stage + blk * 1024);
+            lds_direct_load16(orows, row_off(blk, p.os[2] * 2), q_stage + blk * 1024);
         TRI_WAIT_VMCNT(0);
         asm volatile("" ::: "memory");
         float part = 0.f;
@@ -479,13 +508,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
             }
         }
         dlt = sum_xor32(part);
-        if (h == 0) p.delta[static_cast<int64_t>(bh) * p.S + qrow] = dlt;
+        if (h == 0 && (!RAGGED || qrow < p.S)) p.delta[static_cast<int64_t>(bh) * p.S + qrow] = dlt;
     }
 
     // Without dropout the subtraction in dS = P (dP - delta) is left to the matrix pipe: the dP^T accumulators start from
     // delta and take the product with the dO rows negated (delta - dP^T); dS^T comes out negated and the sign goes into
     // the scale of the final store.
-    constexpr bool kDeltaInAcc = !DROPOUT;
+    constexpr bool kDeltaInAcc = !DROPOUT && !(RAGGED && D == 128);  // (boundary handling leaves no registers for it at D = 128)
     f32x16 dlt16;
     if constexpr (kDeltaInAcc) {
 #pragma unroll
@@ -568,6 +597,11 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         // causal comparison)
         auto softmax_backward = [&](auto on_diagonal, int kb) {
             const int key0 = t * kBN + 32 * kb;
+            if (RAGGED && !CAUSAL && key0 + 32 > p.S) {  // keys that do not exist (under the causal mask no existing row sees them)
+                asm volatile("");                        // (a real branch)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) st[kb][i] = key0 + c_row(i, h) < p.S ? st[kb][i] : -INFINITY;
+            }
             float ds[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -638,7 +672,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         // kept (or, with every register in use, spilled) across the loop
         int elane = threadIdx.x & 63;
         asm volatile("" : "+v"(elane));
-        Store::run(acc, [sc](float x) { return x * sc; }, smem + wave * Store::kPatchBytes, out0, p.dqs[2] * 2, elane);
+        Store::run(acc, [sc](float x) { return x * sc; }, smem + wave * Store::kPatchBytes, out0, p.dqs[2] * 2, elane, RAGGED ? p.S - wrow0 : 32);
     }
 }
 
@@ -674,45 +708,60 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
 }
 
 // whether the phased dQ kernel serves this problem (no mask, 256-row workgroups, D >= 64; with dropout at D = 128 it
-// fits its registers only under the causal mask and with a fragment ring of 4). At D = 32 the kernel above needs 96
-// registers, two of its workgroups share a CU, and that measured 27 % faster than the phased pairs.
+// fits its registers only under the causal mask, without boundary handling and with a fragment ring of 4). At D = 32 the
+// kernel above needs 96 registers, two of its workgroups share a CU, and that measured 27 % faster than the phased pairs.
+// Lengths that are no multiple of 256: at D = 128 the phased kernel with boundary handling (against 4 unphased waves, bf16
+// causal, heads x S: 768 x 130 0.071 -> 0.044 ms, 768 x 450 0.216 -> 0.152, 136 x 1531 0.216 -> 0.145; 768 x 65 equal); at
+// D = 64 two 128-row workgroups share a CU, which is 5-30 % faster than the phased kernel up to S = 3000.
 template <int D, int MASK>
 bool dq_is_phased(const KParams& p) {
-    return MASK == kNoMask && D >= 64 && p.S % 256 == 0 && (D == 64 || p.thr8 <= 0 || p.causal);
+    if (MASK != kNoMask) return false;
+    return D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : D == 64 && p.S % 256 == 0;
+}
+
+// any length (no mask), with boundary handling
+template <typename T, int D, int NW, bool CAUSAL>
+int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
+    const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
+    if (with_delta) {
+        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
+        else if constexpr (D < 128) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
+        else return TRI_ATTN_ESHAPE;  // (without dropout: the phased kernel)
+    } else if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+    else if constexpr (D < 128) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+    else return TRI_ATTN_ESHAPE;
+    return static_cast<int>(hipGetLastError());
+}
+
+template <typename T, int D, bool CAUSAL, bool RAGGED>
+int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
+    const dim3 grid(p.B * p.H * ((p.S + 255) / 256)), block(512);
+    if constexpr (D == 64 || (CAUSAL && !RAGGED)) {
+        if (p.thr8 > 0) {
+            if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true, RAGGED>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, false, RAGGED>), grid, block, 0, stream, p);
+            return static_cast<int>(hipGetLastError());
+        }
+    }
+    if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, RAGGED>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false, RAGGED>), grid, block, 0, stream, p);
+    return static_cast<int>(hipGetLastError());
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     if constexpr (MASK == kNoMask && D >= 64) {
-        if (dq_is_phased<D, MASK>(p)) {
-            const dim3 grid(p.B * p.H * (p.S / 256)), block(512);
-            if constexpr (D == 64 || CAUSAL) {
-                if (p.thr8 > 0) {
-                    if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true>), grid, block, 0, stream, p);
-                    else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, false>), grid, block, 0, stream, p);
-                    return static_cast<int>(hipGetLastError());
-                }
-            }
-            if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false>), grid, block, 0, stream, p);
-            return static_cast<int>(hipGetLastError());
-        }
+        if (dq_is_phased<D, MASK>(p)) return p.S % 256 == 0 ? launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta)
+                                                           : launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);
     }
     if (with_delta && MASK != kNoMask) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
     // 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows)
     if constexpr (D > 16) {  // (a D = 16 tile has four blocks in all: four waves)
         if (p.S % 256 == 0) return launch_dq_waves<T, D, 8, CAUSAL, MASK>(p, stream, with_delta);
     }
+    if constexpr (D == 128 && MASK == kNoMask) return launch_dq_ragged<T, D, 8, CAUSAL>(p, stream, with_delta);  // (dropout)
     if (p.S % 128 == 0) return launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
-    if constexpr (MASK == kNoMask) {  // any other length: 128-row workgroups with boundary handling
-        const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-        if (with_delta) {
-            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, 4, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((mfma_dq_kernel<T, D, 4, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
-        } else if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((mfma_dq_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
-        return static_cast<int>(hipGetLastError());
-    }
+    if constexpr (MASK == kNoMask && D < 128) return launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);  // any other length
     return TRI_ATTN_ESHAPE;  // (mfma_supported keeps masked problems of such lengths away)
 }
 

@@ -32,11 +32,12 @@ constexpr float kTau = 8.f;  // lazy-rescale threshold, log2 domain
 
 enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
 
-// RAGGED (4 waves, no mask): S is not a multiple of 128. Query rows and keys at or beyond S do not exist: row and
-// tile loads clamp their row index to S - 1, the scores of keys >= S are set to -inf, and rows >= S are not stored.
+// RAGGED (no mask): S is not a multiple of 128. Query rows and keys at or beyond S do not exist: row and tile loads clamp
+// their row index to S - 1, the scores of keys >= S are set to -inf, and rows >= S are not stored. A wave without a
+// single row of its own only fetches its share of the tiles and meets the barriers.
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false>
 __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
-    static_assert(!RAGGED || (NW == 4 && MASK == 0), "ragged lengths: 4 waves, no mask");
+    static_assert(!RAGGED || MASK == 0, "ragged lengths: no mask");
     using Tile = SwzTile<D>;
     // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions. The ring then has
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
@@ -58,10 +59,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     constexpr int DB = D >= 32 ? D / 32 : 1;  // 32-row blocks of O^T (D = 16: one block whose upper 16 rows are not stored)
     constexpr int kSteps = 2 * KK;    // MFMAs of S^T per tile
     constexpr int kPvSteps = 4 * DB;  // MFMAs of O^T per tile
-    // operand fragments in flight (a mask and dropout together at D = 128 leave room for four only)
+    // operand fragments in flight (dropout together with a mask or boundary handling leaves room for four only at D = 128)
     // (at D = 32 the O^T product has four steps, and the softmax phase may request fragments of tile j only: tile j + 1
     // becomes visible with the barrier behind it)
-    constexpr int kRing = (D <= 32 || (D == 128 && MASK != kNoMask && DROPOUT)) ? 4 : 6;
+    constexpr int kRing = (D <= 32 || (D == 128 && (MASK != kNoMask || (RAGGED && NW == 8)) && DROPOUT)) ? 4 : 6;
     static_assert(kRing <= kPvSteps, "the softmax phase requests fragments of the O^T product only");
     // A mask block of a wave (32 rows x 64 keys) goes through a private LDS region (8 KiB for an fp32 mask, 4 KiB
     // for one of the operand type) when it fits (D = 64): lanes own rows, so direct loads would touch 32 cache
@@ -114,6 +115,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
             qf[kk] = *reinterpret_cast<const u32x4*>(qbase + qrow_ld * p.qs[2] * 2 + (2 * kk + h) * 16);
         n_tiles = CAUSAL ? min((q0 + kBM) / kBN, num_key_tiles) : num_key_tiles;  // tiles the workgroup streams
         my_tiles = CAUSAL ? min((wrow0 + 31) / kBN + 1, n_tiles) : n_tiles;       // tiles this wave has visible keys in
+        if (RAGGED && wrow0 >= p.S) my_tiles = 0;
     };
     set_item();
     // With the classes of the mask's blocks at hand (tri_attn_classify_mask): key tiles behind the last one that is not
@@ -583,9 +585,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     lds_barrier();
     char* o0 = static_cast<char*>(p.o) + (b * p.os[0] + hd * p.os[1] + static_cast<int64_t>(wrow0) * p.os[2]) * 2;
     float* lse_out = p.lse + static_cast<int64_t>(bh) * p.S + qrow;
+    const int rows_here = RAGGED ? p.S - wrow0 : 32;  // (of this item: the next one's are set below)
     bool more = false;
     if constexpr (kPersistent) {
-        more = map_item(blockIdx.x, gridDim.x, ++round, p.B * p.H, p.S / kBM, kOrder, &bh, &qt);
+        more = map_item(blockIdx.x, gridDim.x, ++round, p.B * p.H, num_row_tiles, kOrder, &bh, &qt);
         if (more) {
             set_item();
             request_first_tiles();
@@ -598,20 +601,21 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
         for (int cb = 0; cb < DB / kStoreBlocks; ++cb) {
             if (cb) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
             const f32x16(&part)[kStoreBlocks] = *reinterpret_cast<const f32x16(*)[kStoreBlocks]>(&oacc[kStoreBlocks * cb]);
-            Store::run(part, [inv](float x) { return x * inv; }, patch, o0 + cb * 128, p.os[2] * 2, lane,
-                       RAGGED ? p.S - wrow0 : 32);
+            Store::run(part, [inv](float x) { return x * inv; }, patch, o0 + cb * 128, p.os[2] * 2, lane, rows_here);
         }
     }
-    if (h == 0 && (!RAGGED || qrow < p.S)) *lse_out = m + fast_log2(l);
+    if (h == 0 && l32 < rows_here) *lse_out = m + fast_log2(l);
     if (!more) break;
     }
 }
 
-template <typename T, int D, bool CAUSAL>
+template <typename T, int D, int NW, bool CAUSAL>
 int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
-    const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+    const int items = p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW));
+    // (NW == 8: the kernel's kPersistent, one workgroup per CU walks the items)
+    const dim3 grid(NW == 8 ? persistent_grid(items) : items), block(64 * NW);
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -627,8 +631,10 @@ int launch_fwd_dropout(const KParams& p, hipStream_t stream) {
 
 template <typename T, int D, int NW>
 int launch_fwd_variant(int dtype, const KParams& p, hipStream_t stream) {
-    if (p.causal) return launch_fwd_dropout<T, D, NW, true, kNoMask>(p, stream);
-    if (p.mask == nullptr) return launch_fwd_dropout<T, D, NW, false, kNoMask>(p, stream);
+    if constexpr (!(D == 128 && NW == 4)) {  // (without a mask D = 128 never runs four waves: launch_fwd_waves)
+        if (p.causal) return launch_fwd_dropout<T, D, NW, true, kNoMask>(p, stream);
+        if (p.mask == nullptr) return launch_fwd_dropout<T, D, NW, false, kNoMask>(p, stream);
+    }
     if (p.mask_dtype == TRI_ATTN_F32) return launch_fwd_dropout<T, D, NW, false, kMaskF32>(p, stream);
     if (p.mask_dtype == dtype) return launch_fwd_dropout<T, D, NW, false, kMaskT>(p, stream);
     return TRI_ATTN_EDTYPE;
@@ -642,9 +648,17 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     if constexpr (D > 32) {
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
     }
+    // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
+    // one workgroup per CU, so that four waves are one per SIMD. bf16 causal, heads x S: 768 x 130 0.057 -> 0.034 ms,
+    // 768 x 450 0.168 -> 0.110, 136 x 1531 0.170 -> 0.109, 32 x 3000 0.141 -> 0.084; 768 x 65 0.026 -> 0.022.
+    if constexpr (D == 128) {
+        if (p.mask == nullptr) return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
+    }
     if (p.S % 128 == 0) return launch_fwd_variant<T, D, 4>(dtype, p, stream);
-    // any other length (no mask: mfma_supported): 128-row workgroups with boundary handling
-    return p.causal ? launch_fwd_ragged<T, D, true>(p, stream) : launch_fwd_ragged<T, D, false>(p, stream);
+    // any other length (no mask: mfma_supported) at D <= 64: 128-row workgroups with boundary handling, two of which share
+    // a CU (256-row ones measured 5-30 % slower at D = 64, S = 65 .. 6001)
+    if constexpr (D < 128) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
+    return TRI_ATTN_ESHAPE;
 }
 
 template <typename T>

@@ -146,7 +146,7 @@ bool mfma_supported(int which, int dtype, const KParams& p) {
 bool mfma_dq_fuses_delta(const KParams& p) {
     if (p.mask != nullptr) return false;
     if (!aligned16(p.o) || !strides8(p.os)) return false;
-    const bool phased = p.D >= 64 && p.S % 256 == 0 && (p.D == 64 || p.thr8 <= 0 || p.causal);  // (as the launcher decides)
+    const bool phased = p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0;  // (as the launcher decides)
     return !phased || tile_offsets_fit(p.os);
 }
 
