@@ -54,8 +54,14 @@ extern "C" {
 enum {
     TRI_ATTN_F32 = 0,
     TRI_ATTN_F16 = 1,
-    TRI_ATTN_BF16 = 2
+    TRI_ATTN_BF16 = 2,
+    TRI_ATTN_BOOL = 3          /* tri_attn_prepare_mask's source only: one byte per entry, nonzero = the key takes part */
 };
+
+/* Or-ed to mask_dtype: every row of the mask may be read up to the next multiple of 64 entries beyond S and holds finite
+ * values there (they are not used), and mask_classes, where given, also covers the blocks that S cuts. The 16-bit
+ * matrix-core kernels take masked lengths that are no multiple of 128 only so; tri_attn_prepare_mask makes such a mask. */
+#define TRI_ATTN_MASK_PADDED 0x100
 
 enum {
     TRI_ATTN_OK = 0,
@@ -76,7 +82,7 @@ typedef struct TriAttnArgs {
     int32_t dtype;             /* TRI_ATTN_F32 / F16 / BF16: element type of q,k,v,o,d_o,dq,dk,dv */
     int32_t B, H, S, D;        /* y_size = S, x_size = D in the reference's naming */
     int32_t is_causal;
-    int32_t mask_dtype;        /* element type of mask and dmask */
+    int32_t mask_dtype;        /* element type of mask and dmask, plus TRI_ATTN_MASK_PADDED where it holds */
     float softmax_scale;
     float dropout_p;
     uint64_t seed;             /* Philox key */
@@ -114,7 +120,7 @@ typedef struct TriAttnArgs {
                                   read by tri_attn_fwd / tri_attn_bwd*: dense [MB][MH][RB][S/64] bytes with MB = B (1 if
                                   mask_stride[0] == 0), MH = H (1 if mask_stride[1] == 0), RB = S/64 (1 if mask_stride[2] == 0);
                                   0 = every entry of the block is 0, 1 = every entry is -inf, 2 = anything else.
-                                  Only used where S is a multiple of 128. */
+                                  Only used where S is a multiple of 128, or with TRI_ATTN_MASK_PADDED (S/64 rounded up). */
 } TriAttnArgs;
 
 /* ABI version of the loaded library (TRI_ATTN_ABI_VERSION it was built with). */
@@ -181,12 +187,21 @@ int tri_attn_classify_mask(const TriAttnArgs* args);
  * negative TRI_ATTN_E* code. */
 int64_t tri_attn_mask_classes_size(const TriAttnArgs* args);
 
+/* Writes an additive padded mask for the kernels: args->mask is the destination (mask_dtype with TRI_ATTN_MASK_PADDED,
+ * 16-byte aligned, mask_stride[2] a multiple of 64 of at least S, or 0; a stride of 0 over a dimension of the destination
+ * keeps its entry 0 of the source), args->mask_classes receives the classes of its blocks
+ * (tri_attn_mask_classes_size bytes) unless it is NULL. `source` is logical [B,H,S,S] through source_stride (elements, any
+ * stride of at least 0): additive TRI_ATTN_F32 / F16 / BF16, or TRI_ATTN_BOOL (0 where nonzero, -inf elsewhere). One pass
+ * over the source; B, H, S and stream are read from args. The reference has no boolean masks and adds additive ones as
+ * they come (trident/kernel/attention.py:135-138). */
+int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t source_dtype, const int64_t* source_stride);
+
 /* Which kernel family a call would run, without launching anything (no counterpart in the reference): pass 0 =
  * tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq on these arguments. Returns 1 for the 16-bit matrix-core
- * (MFMA) kernels (fp16/bf16, D in {16,32,64,128}, 16-byte aligned rows; any S without a mask, S a multiple of 128 with
- * one); 2 for the 32-row-tile matrix-core kernels (everything else whose pointers and strides are multiples of
+ * (MFMA) kernels (fp16/bf16, D in {16,32,64,128}, 16-byte aligned rows; any S without a mask or with
+ * a padded one, S a multiple of 128 with any other); 2 for the 32-row-tile matrix-core kernels (everything else whose pointers and strides are multiples of
  * four elements: fp32 problems on the fp32 matrix instruction with fp32 products and sums; fp16/bf16 problems with
- * masked lengths that are no multiple of 128 on the 16-bit 32x32x8 instruction);
+ * unpadded masks at lengths that are no multiple of 128 on the 16-bit 32x32x8 instruction);
  * 0 for the general vector-ALU kernels (views that are not aligned so); or a negative TRI_ATTN_E* code. */
 int tri_attn_uses_matrix_cores(const TriAttnArgs* args, int pass);
 

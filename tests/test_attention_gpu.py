@@ -986,3 +986,64 @@ def test_config3_full_size_properties(device):
     o_p = trident.function.scaled_dot_product_attention(tq.detach()[:, perm], tk.detach()[:, perm],
                                                         tv.detach()[:, perm], is_causal=True)
     assert torch.equal(o_p, out.detach()[:, perm])
+
+
+# ------------------------------------------------------------------ padded masks
+@pytest.mark.parametrize("kind", ["bool keys", "bool", "f32", "16 bit", "16 bit+dropout", "bool keys+dropout"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 1, 64), (torch.float16, 65, 64), (torch.bfloat16, 129, 128),
+                                       (torch.float16, 255, 128), (torch.bfloat16, 321, 64), (torch.float16, 200, 32),
+                                       (torch.bfloat16, 333, 16), (torch.bfloat16, 384, 64), (torch.float16, 577, 128)])
+def test_masks_at_any_length(dtype, S, D, kind, device):
+    """Boolean masks and additive ones at lengths that are no multiple of 128 go through tri_attn_prepare_mask to the 16-bit
+    kernels with boundary handling: a single key, one key beyond a tile, beyond a workgroup's rows, whole waves without
+    rows, blocks of keys that are masked out behind the last active one (classes), dropout."""
+    from trident_amd.operation import Attention, _BooleanMask
+    q, k, v, d_o = _gen((2, 3, S, D), 5200 + S + D, dtype)
+    g = torch.Generator().manual_seed(S)
+    p = 0.2 if "dropout" in kind else 0.0
+    if "bool" in kind:
+        keep = torch.rand(2, 1, 1 if "keys" in kind else S, S, generator=g) > 0.3
+        keep[1, ..., (S + 1) // 2:] = False  # (the second sequence ends half way)
+        keep[..., 0] = True
+        mask = torch.zeros(keep.shape).masked_fill(~keep, float("-inf"))
+        given = _BooleanMask(keep.to(device))
+    else:
+        mask = torch.randn(1, 3, S, S, generator=g).to(torch.float32 if kind == "f32" else dtype)
+        given = mask.to(device)
+    scale, rng = 1.0 / math.sqrt(D), (31, 2) if p > 0 else (0, 0)
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    o, lse = Attention._forward(tq, tk, tv, given, p, False, scale, *rng)
+    dq, dk, dv, _ = Attention._backward(tdo, tq, tk, tv, o, lse, given, scale, p, False, *rng, False)
+    kw = dict(mask=mask, dropout_p=p, is_causal=False, scale=scale, seed=rng[0], offset=rng[1])
+    o_ref, _ = parity.oracle_forward(q, k, v, **kw)
+    parity.close(o, o_ref, dtype, f"{kind} O")
+    dq_r, dk_r, dv_r, _, _ = parity.oracle_backward(q, k, v, d_o, o=o, **kw)
+    _, a_dq, a_dk, a_dv = parity.oracle_abs_sums(q, k, v, d_o, o=o, **kw)
+    parity.close(dq, dq_r, dtype, f"{kind} dQ", a_dq)
+    parity.close(dk, dk_r, dtype, f"{kind} dK", a_dk)
+    parity.close(dv, dv_r, dtype, f"{kind} dV", a_dv)
+
+
+@pytest.mark.parametrize("source", [torch.bool, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("S", [1, 63, 128, 130])
+def test_prepared_masks_hold_the_source(source, S, device):
+    """tri_attn_prepare_mask: values, finite padding and classes for dense, broadcast and transposed sources."""
+    from trident_amd import operation
+    q = torch.zeros(2, 3, S, 16, dtype=torch.bfloat16, device=device)
+    for shape in ((2, 3, S, S), (2, 1, 1, S), (1, 3, S, S), (S, S), (2, 1, S, 1)):
+        dense = torch.randint(0, 2, shape, generator=torch.Generator().manual_seed(S)).to(source)
+        for m in (dense, dense.transpose(-1, -2).contiguous().transpose(-1, -2)):
+            prepared = operation._PreparedMask(m.to(device), q)
+            additive, classes = torch.as_strided(prepared.padded, (2, 3, S, S), prepared.strides), prepared.classes
+            want = torch.where(m, 0.0, float("-inf")) if source == torch.bool else m.float()
+            assert torch.equal(additive.cpu().float(), want.expand(2, 3, S, S))
+            rows = torch.as_strided(additive, (*additive.shape[:3], (S + 63) // 64 * 64), additive.stride())
+            assert torch.isfinite(rows[..., S:]).all()
+            blocks = torch.nn.functional.pad(want.expand(2, 3, S, S), (0, -S % 64, 0, -S % 64), value=float("nan"))
+            blocks = blocks.unfold(2, 64, 64).unfold(3, 64, 64).flatten(-2)
+            zero = ((blocks == 0) | blocks.isnan()).all(-1)
+            ninf = ((blocks == float("-inf")) | blocks.isnan()).all(-1)
+            expected = torch.full(zero.shape, 2).masked_fill(zero, 0).masked_fill(ninf, 1)
+            cb = (S + 63) // 64
+            dims = [1 if s == 0 else n for s, n in zip(additive.stride()[:2], additive.shape)] + [1 if additive.stride(2) == 0 else cb, cb]
+            assert torch.equal(classes.cpu().view(dims).expand(2, 3, cb, cb).long(), expected)

@@ -10,6 +10,8 @@ ENOFUSE = -9  # tri_attn_bwd_dq_delta: no fused kernel for this problem, nothing
 ABI_VERSION = 3
 ESCRATCH = -10  # tri_attn_bwd_noalloc: B*H*S above NOALLOC_MAX_ROWS, nothing launched
 NOALLOC_MAX_ROWS = 1 << 20
+BOOL = 3  # tri_attn_prepare_mask: the source is a boolean mask
+MASK_PADDED = 0x100  # in mask_dtype: rows may be read up to the next multiple of 64 entries
 
 _i64x4 = ctypes.c_int64 * 4
 
@@ -99,6 +101,7 @@ EXPORTS = (
     "tri_attn_uses_matrix_cores",
     "tri_attn_classify_mask",
     "tri_attn_mask_classes_size",
+    "tri_attn_prepare_mask",
 )
 
 _lib = None
@@ -126,6 +129,8 @@ def lib():
             fn.argtypes = [ctypes.POINTER(TriAttnArgs)]
         cdll.tri_attn_mask_classes_size.restype = ctypes.c_int64
         cdll.tri_attn_mask_classes_size.argtypes = [ctypes.POINTER(TriAttnArgs)]
+        cdll.tri_attn_prepare_mask.restype = ctypes.c_int
+        cdll.tri_attn_prepare_mask.argtypes = [ctypes.POINTER(TriAttnArgs), ctypes.c_void_p, ctypes.c_int32, ctypes.POINTER(ctypes.c_int64)]
         cdll.tri_attn_uses_matrix_cores.restype = ctypes.c_int
         cdll.tri_attn_uses_matrix_cores.argtypes = [ctypes.POINTER(TriAttnArgs), ctypes.c_int]
         cdll.tri_attn_dropout_mask.restype = ctypes.c_int

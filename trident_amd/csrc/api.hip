@@ -29,6 +29,14 @@ void copy3(int64_t* dst, const int64_t* src) {
     dst[2] = src[2];
 }
 
+// Layout of the classes of the mask's 64 x 64 blocks, broadcast like the mask itself.
+void set_class_strides(int64_t* mcs, const TriAttnArgs* a) {
+    const int64_t cb = (a->S + 63) / 64, rb = a->mask_stride[2] == 0 ? 1 : cb, mh = a->mask_stride[1] == 0 ? 1 : a->H;
+    mcs[2] = rb == 1 ? 0 : cb;
+    mcs[1] = mh == 1 ? 0 : rb * cb;
+    mcs[0] = a->mask_stride[0] == 0 ? 0 : mh * rb * cb;
+}
+
 // Common validation + translation. `need` bits: 1 = forward tensors, 2 = backward tensors.
 int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (a == nullptr) return TRI_ATTN_ENULL;
@@ -38,8 +46,10 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (static_cast<int64_t>(a->B) * a->H > 2147483647LL / 64) return TRI_ATTN_ESHAPE;
     if (!(a->dropout_p >= 0.f && a->dropout_p <= 1.f)) return TRI_ATTN_EDROPOUT;
     if (a->mask != nullptr && a->is_causal) return TRI_ATTN_EMASKCAUSAL;
+    const int mask_dtype = a->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    const bool padded = a->mask != nullptr && (a->mask_dtype & TRI_ATTN_MASK_PADDED) != 0;
     if (a->mask != nullptr || a->dmask != nullptr) {
-        if (a->mask_dtype < TRI_ATTN_F32 || a->mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
+        if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     }
     memset(p, 0, sizeof(*p));
     int rc;
@@ -99,14 +109,10 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
         // a stride of 0 over a dimension that has more than one entry: the gradient is summed over it
         p->dmask_acc = (a->B > 1 && a->dmask_stride[0] == 0) || (a->H > 1 && a->dmask_stride[1] == 0) ||
                        (a->S > 1 && a->dmask_stride[2] == 0);
-        if (p->dmask_acc && a->mask_dtype != TRI_ATTN_F32) return TRI_ATTN_EDTYPE;
+        if (p->dmask_acc && mask_dtype != TRI_ATTN_F32) return TRI_ATTN_EDTYPE;
     }
-    if (a->mask != nullptr && a->S % 128 == 0) {
-        // layout of the block classes (64 x 64 blocks), broadcast like the mask itself
-        const int64_t cb = a->S / 64, rb = a->mask_stride[2] == 0 ? 1 : cb, mh = a->mask_stride[1] == 0 ? 1 : a->H;
-        p->mcs[2] = rb == 1 ? 0 : cb;
-        p->mcs[1] = mh == 1 ? 0 : rb * cb;
-        p->mcs[0] = a->mask_stride[0] == 0 ? 0 : mh * rb * cb;
+    if (a->mask != nullptr && (a->S % 128 == 0 || padded)) {
+        set_class_strides(p->mcs, a);
         p->mcls = a->mask_classes;
     }
     p->B = a->B;
@@ -114,7 +120,8 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     p->S = a->S;
     p->D = a->D;
     p->causal = a->is_causal ? 1 : 0;
-    p->mask_dtype = a->mask_dtype;
+    p->mask_dtype = mask_dtype;
+    p->mask_padded = padded;
     p->scale = a->softmax_scale;
     p->scale_log2 = a->softmax_scale * kLog2e;
     p->inv_scale = a->softmax_scale != 0.f ? 1.f / a->softmax_scale : 0.f;
@@ -270,8 +277,8 @@ int64_t tri_attn_mask_classes_size(const TriAttnArgs* args) {
     if (args == nullptr) return TRI_ATTN_ENULL;
     if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
-    if (args->mask == nullptr || args->S % 128 != 0) return 0;
-    const int64_t cb = args->S / 64, rb = args->mask_stride[2] == 0 ? 1 : cb;
+    if (args->mask == nullptr || (args->S % 128 != 0 && !(args->mask_dtype & TRI_ATTN_MASK_PADDED))) return 0;
+    const int64_t cb = (args->S + 63) / 64, rb = args->mask_stride[2] == 0 ? 1 : cb;
     return (args->mask_stride[0] == 0 ? 1 : args->B) * (args->mask_stride[1] == 0 ? 1 : args->H) * rb * cb;
 }
 
@@ -280,23 +287,49 @@ int tri_attn_classify_mask(const TriAttnArgs* args) {
     if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr || args->mask_classes == nullptr) return TRI_ATTN_ENULL;
-    if (args->mask_dtype < TRI_ATTN_F32 || args->mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
+    const int mask_dtype = args->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     int rc = check_strides(args->mask_stride);
     if (rc) return rc;
     if (args->S % 128 != 0) return TRI_ATTN_ENOFUSE;
     KParams p;
     memset(&p, 0, sizeof(p));
     p.mask = args->mask;
-    p.mask_dtype = args->mask_dtype;
+    p.mask_dtype = mask_dtype;
     copy3(p.ms, args->mask_stride);
     p.B = args->B;
     p.H = args->H;
     p.S = args->S;
-    const int64_t cb = args->S / 64, rb = args->mask_stride[2] == 0 ? 1 : cb, mh = args->mask_stride[1] == 0 ? 1 : args->H;
-    p.mcs[2] = rb == 1 ? 0 : cb;
-    p.mcs[1] = mh == 1 ? 0 : rb * cb;
-    p.mcs[0] = args->mask_stride[0] == 0 ? 0 : mh * rb * cb;
+    set_class_strides(p.mcs, args);
     return launch_classify_mask(p, args->mask_classes, static_cast<hipStream_t>(args->stream));
+}
+
+int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t source_dtype, const int64_t* source_stride) {
+    if (args == nullptr || source == nullptr || source_stride == nullptr) return TRI_ATTN_ENULL;
+    if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
+    if (args->mask == nullptr) return TRI_ATTN_ENULL;
+    const int mask_dtype = args->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    if (!(args->mask_dtype & TRI_ATTN_MASK_PADDED) || mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
+    if (source_dtype < TRI_ATTN_F32 || source_dtype > TRI_ATTN_BOOL) return TRI_ATTN_EDTYPE;
+    int rc = check_strides(args->mask_stride);
+    if (rc) return rc;
+    for (int i = 0; i < 4; ++i)
+        if (source_stride[i] < 0) return TRI_ATTN_ESTRIDE;
+    const int64_t pitch = args->mask_stride[2];
+    if (pitch != 0 && (pitch % 64 != 0 || pitch < args->S)) return TRI_ATTN_ESTRIDE;
+    if (args->mask_stride[0] % 64 != 0 || args->mask_stride[1] % 64 != 0) return TRI_ATTN_ESTRIDE;
+    if (reinterpret_cast<uintptr_t>(args->mask) % 16 != 0) return TRI_ATTN_EALIGN;
+    KParams p;
+    memset(&p, 0, sizeof(p));
+    p.mask_dtype = mask_dtype;
+    copy3(p.ms, args->mask_stride);
+    p.B = args->B;
+    p.H = args->H;
+    p.S = args->S;
+    set_class_strides(p.mcs, args);
+    return launch_prepare_mask(p, const_cast<void*>(args->mask), args->mask_classes, source, source_dtype, source_stride,
+                               static_cast<hipStream_t>(args->stream));
 }
 
 int tri_attn_uses_matrix_cores(const TriAttnArgs* args, int pass) {

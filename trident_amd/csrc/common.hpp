@@ -33,6 +33,7 @@ struct KParams {
     int B, H, S, D;
     int causal;
     int mask_dtype;
+    int mask_padded;   // mask rows may be read up to the next multiple of 64 entries (finite values there)
     float scale;       // softmax_scale
     float scale_log2;  // softmax_scale * log2(e)
     float inv_scale;   // 1 / softmax_scale (0 where the scale is 0)

@@ -11,7 +11,8 @@ enum GenericKernel { kGenericFwd = 0, kGenericDelta = 1, kGenericDkdv = 2, kGene
 // generic.hip: any shape / dtype, vector-ALU fp32 arithmetic.
 int launch_generic_any(int which, int dtype, const KParams& p, hipStream_t stream);
 
-// mfma_*.hip: fp16/bf16, D in {64,128}, 16-byte aligned rows; any S without a mask, S a multiple of 128 with one.
+// mfma_*.hip: fp16/bf16, D in {16,32,64,128}, 16-byte aligned rows; any S without a mask or with a padded one, S a multiple
+// of 128 with any other.
 enum MfmaKernel { kMfmaFwd = 0, kMfmaDkdv = 1, kMfmaDq = 2 };
 bool mfma_supported(int which, int dtype, const KParams& p);
 int launch_mfma_fwd(int dtype, const KParams& p, hipStream_t stream);
@@ -28,6 +29,10 @@ bool mfma32_supported(int which, int dtype, const KParams& p);
 int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream);
 // Classes of the mask's 64 x 64 blocks (0 all zero, 1 all -inf, 2 mixed) into `out`, laid out as p.mcs says.
 int launch_classify_mask(const KParams& p, uint8_t* out, hipStream_t stream);
+// Source mask (additive, or bytes: TRI_ATTN_BOOL) -> padded additive mask `out` laid out as p.ms says, and its block classes
+// (unless nullptr) as p.mcs says.
+int launch_prepare_mask(const KParams& p, void* out, uint8_t* classes, const void* source, int source_dtype, const int64_t* source_stride,
+                        hipStream_t stream);
 enum MaskClass { kMaskZero = 0, kMaskNegInf = 1, kMaskMixed = 2 };
 // Number of workgroups for a kernel whose workgroups are persistent (one per CU, each walking several of
 // the `items`): min(items, CUs of the current device).

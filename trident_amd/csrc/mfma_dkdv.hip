@@ -32,12 +32,11 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // tiles (plus their lse and delta) in a ring of 4 filled by LDS-direct loads three tiles ahead.
 // Per 32-row query block: S = Q K^T and dP = dO V^T from row fragments, P and dS on the vector
 // ALU, dV^T += dO^T P and dK^T += Q^T dS with the transposed LDS reads of the same tiles.
-// RAGGED (4 waves, no mask): S is not a multiple of 128. Loads clamp their
+// RAGGED (no mask, or a padded one): S is not a multiple of 128. Loads clamp their
 // row index to S - 1, query rows >= S get probability 0 (they would otherwise add the last row once more), keys >= S
 // are not stored.
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false>
-__global__ __launch_bounds__(NW * 64, RAGGED ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
-    static_assert(!RAGGED || (NW == 4 && MASK == 0), "ragged lengths: 4 waves, no mask");
+__global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
     using Tile = SwzTile<D>;
     constexpr int kKeys = 32 * NW;
     constexpr int kStages = 4;
@@ -112,7 +111,8 @@ __global__ __launch_bounds__(NW * 64, RAGGED ? 1 : 2) void mfma_dkdv_wide_kernel
     uint64_t zero_tiles = 0;
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
-            const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + k0 / 64, p.mcs[2], n_tiles, kKeys / 64, 1, lane);
+            const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + k0 / 64, p.mcs[2], n_tiles,
+                                                RAGGED ? min(kKeys / 64, n_tiles - k0 / 64) : kKeys / 64, 1, lane);
             zero_tiles = tc.zero;
             if (tc.active) {
                 t_begin = __builtin_ctzll(tc.active);
@@ -150,13 +150,15 @@ __global__ __launch_bounds__(NW * 64, RAGGED ? 1 : 2) void mfma_dkdv_wide_kernel
     auto issue_mask = [&](int t) {  // rows of tile t x this wave's keys -> the wave's region, unless the tile is all zero
         if constexpr (kMaskViaLds) {
             if (mask_is_zero(t)) return;
+            const int col0 = RAGGED && wkey0 >= p.S ? 0 : wkey0;  // (a wave without a single key reads some row's first ones)
             const char* src = static_cast<const char*>(p.mask) +
-                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(t) * kBN * p.ms[2] + wkey0) * kMaskElt;
+                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(t) * kBN * p.ms[2] + col0) * kMaskElt;
             int l = lane;
             asm volatile("" : "+v"(l));  // offsets recomputed per tile rather than kept in registers
 #pragma unroll
             for (int blk = 0; blk < kMaskLoads; ++blk)
-                lds_direct_load16(src, static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
+                lds_direct_load16(src, RAGGED ? MaskTile::src_off_clamped(blk, l, p.ms[2] * kMaskElt, p.S - 1 - t * kBN)
+                                              : static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
         }
     };
     // issue order: mask block of the first tile, three tiles, then per tile j: mask j+1, tile j+3
@@ -229,10 +231,12 @@ __global__ __launch_bounds__(NW * 64, RAGGED ? 1 : 2) void mfma_dkdv_wide_kernel
                 }
             } else if constexpr (MASK != kNoMask) {
                 if (masked) {
-                    const int64_t mbase = b * p.ms[0] + hd * p.ms[1] + key;
+                    const int64_t mbase = b * p.ms[0] + hd * p.ms[1] + key_ld;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i)
-                        mk[i] = mask_at<T, MASK>(p.mask, mbase + static_cast<int64_t>(rb + c_row(i, h)) * p.ms[2]);
+                    for (int i = 0; i < 16; ++i) {
+                        const int row = RAGGED ? min(rb + c_row(i, h), p.S - 1) : rb + c_row(i, h);
+                        mk[i] = mask_at<T, MASK>(p.mask, mbase + static_cast<int64_t>(row) * p.ms[2]);
+                    }
                 }
             }
             const int qoff = 32 * qb * Tile::kRowBytes;
@@ -828,7 +832,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     const float c = p.scale_log2;
     [[maybe_unused]] const float inv_scale = p.inv_scale;  // (a mask value joins its score before the scale: s + mask / scale)
     float key_bias = 0.f;  // mask value of this lane's key, log2 domain
-    if constexpr (KEYMASK != kNoMask) key_bias = mask_at<T, KEYMASK>(p.mask, b * p.ms[0] + hd * p.ms[1] + key) * kLog2e;
+    if constexpr (KEYMASK != kNoMask) key_bias = mask_at<T, KEYMASK>(p.mask, b * p.ms[0] + hd * p.ms[1] + (RAGGED ? min(key, p.S - 1) : key)) * kLog2e;
 
     f32x16 dk[DH], dv[DH];
 #pragma unroll
@@ -1221,7 +1225,25 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
                 return static_cast<int>(hipGetLastError());
             }
         }
-        return TRI_ATTN_ESHAPE;  // (mfma_supported keeps masked problems of such lengths away)
+        if constexpr (MASK != kNoMask && D == 128) {
+            if (p.ms[2] == 0) {  // (a key-padding mask: as below)
+                const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(512);
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, false, true, MASK, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, false, false, MASK, true>), grid, block, 0, stream, p);
+                return static_cast<int>(hipGetLastError());
+            }
+        }
+        // a padded mask: one workgroup of 8 waves per CU at D = 64 (LDS), 4 waves with the whole register file at D = 128
+        if constexpr (MASK != kNoMask) {
+            // (dropout beside mask and boundary handling does not fit 256 registers: four waves)
+            constexpr int NW = D == 64 ? 8 : 4;
+            const int nw = p.thr8 > 0 ? 4 : NW;
+            const dim3 grid(p.B * p.H * ((p.S + 32 * nw - 1) / (32 * nw))), block(64 * nw);
+            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, false, MASK, true, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, NW, false, MASK, false, true>), grid, block, 0, stream, p);
+            return static_cast<int>(hipGetLastError());
+        }
+        return TRI_ATTN_ESHAPE;
     }
     if constexpr (D <= 64) {
         // the two-waves-per-SIMD kernel fits its registers: 8 waves (256 keys) when the sequence

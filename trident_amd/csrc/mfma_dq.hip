@@ -32,7 +32,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // staging registers, no ds_write). Per 32-key block: S^T = K Q^T and dP^T = V dO^T from row
 // fragments, dS^T = P^T (dP^T - delta) on the vector ALU, dQ^T += K^T dS^T with K^T read through
 // transposed LDS reads of the same K tile.
-// RAGGED (no mask): S is not a multiple of 32 NW. Rows and keys at or beyond S do not exist: loads clamp
+// RAGGED (no mask, or a padded one; no mask gradient): S is not a multiple of 32 NW. Rows and keys at or beyond S do not exist: loads clamp
 // their row index to S - 1, keys >= S get probability 0, rows >= S are not stored.
 // DMASK (with a mask): the kernel also writes the mask gradient dS (trident/kernel/attention.py:332-335), each lane four
 // consecutive keys of its row at a time; where the mask is broadcast over a dimension (dmask stride 0) the values are
@@ -40,8 +40,8 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // DELTA (no mask): the kernel also computes delta = rowsum(dO * O) of its rows from the dO rows it loads anyway, instead
 // of reading it, and stores it for the dK/dV pass, which then runs after this one (tri_attn_bwd_dq_delta).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool DMASK = false, bool DELTA = false>
-__global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
-    static_assert(!RAGGED || MASK == 0, "ragged lengths: no mask");
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) void mfma_dq_kernel(const KParams p) {
+    static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
     static_assert(!DELTA || MASK == 0, "delta on the way: the variants without a mask");
     using Tile = SwzTile<D>;
@@ -117,13 +117,13 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
             const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (q0 / 64) * p.mcs[2], 1, n_tiles,
-                                                kRows / 64, p.mcs[2], lane);
+                                                RAGGED ? min(kRows / 64, num_key_tiles - q0 / 64) : kRows / 64, p.mcs[2], lane);
             zero_tiles = tc.zero;
             // (a mask gradient written in place covers every tile: the tiles behind the last active one get their
             // zeros from the loop; an accumulated one adds into a buffer the caller has zero-filled)
             if (!DMASK || p.dmask_acc) {
                 n_tiles = tc.active ? 64 - __builtin_clzll(tc.active) : 1;
-                my_tiles = n_tiles;
+                my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
             }
         }
     }
@@ -159,13 +159,15 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
     auto issue_mask = [&](int t) {  // mask block of tile t -> this wave's region, unless it is all zero
         if constexpr (kMaskViaLds) {
             if (mask_is_zero(t)) return;
+            const int row0 = RAGGED ? min(wrow0, p.S - 1) : wrow0;
             const char* src = static_cast<const char*>(p.mask) +
-                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(wrow0) * p.ms[2] + t * kBN) * kMaskElt;
+                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(row0) * p.ms[2] + t * kBN) * kMaskElt;
             int l = lane;
             asm volatile("" : "+v"(l));  // offsets recomputed per tile rather than kept in registers
 #pragma unroll
             for (int blk = 0; blk < kMaskLoads; ++blk)
-                lds_direct_load16(src, static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
+                lds_direct_load16(src, RAGGED ? MaskTile::src_off_clamped(blk, l, p.ms[2] * kMaskElt, p.S - 1 - row0)
+                                              : static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
         }
     };
     // issue order: mask 0, tiles 0 1 2, then per tile j: mask j+1, tile j+3
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) mk[i] = 0.f;
                 } else {
-                    const int64_t mrow = b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(qrow) * p.ms[2] + t0 + 32 * kb;
+                    const int64_t mrow = b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(qrow_ld) * p.ms[2] + t0 + 32 * kb;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) mk[i] = mask_at<T, MASK>(p.mask, mrow + c_row(i, h));
                 }
@@ -295,8 +297,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_dq_kernel(const KParams p) {
                 for (int i = 0; i < 16; ++i) st[i] = t0 + 32 * kb + c_row(i, h) <= qrow ? st[i] : -INFINITY;
             }
             if (RAGGED && !CAUSAL && t0 + 32 * kb + 32 > p.S) {  // keys that do not exist
+                int left = p.S - t0 - 32 * kb - 4 * h;
+                asm volatile("" : "+v"(left));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) st[i] = t0 + 32 * kb + c_row(i, h) < p.S ? st[i] : -INFINITY;
+                for (int i = 0; i < 16; ++i) st[i] = c_row(i, 0) < left ? st[i] : -INFINITY;
             }
             float ds[16];
             if (masked) {
@@ -719,10 +723,15 @@ bool dq_is_phased(const KParams& p) {
     return D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : D == 64 && p.S % 256 == 0;
 }
 
-// any length (no mask), with boundary handling
-template <typename T, int D, int NW, bool CAUSAL>
+// any length (no mask, or a padded one), with boundary handling
+template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
     const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
+    if constexpr (MASK != kNoMask) {
+        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
+        return static_cast<int>(hipGetLastError());
+    }
     if (with_delta) {
         if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
         else if constexpr (D < 128) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
@@ -762,7 +771,10 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     if constexpr (D == 128 && MASK == kNoMask) return launch_dq_ragged<T, D, 8, CAUSAL>(p, stream, with_delta);  // (dropout)
     if (p.S % 128 == 0) return launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
     if constexpr (MASK == kNoMask && D < 128) return launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);  // any other length
-    return TRI_ATTN_ESHAPE;  // (mfma_supported keeps masked problems of such lengths away)
+    // a padded mask: at D = 64 one workgroup of 8 waves per CU beside an fp32 mask's staging regions, two of 4 beside a 16-bit
+    // one's (as the forward); at D = 128 four waves with the whole register file (in 256 registers the kernel spills)
+    if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, D == 64 && MASK == kMaskF32 ? 8 : 4, CAUSAL, MASK>(p, stream, false);
+    return TRI_ATTN_ESHAPE;
 }
 
 template <typename T, int D>

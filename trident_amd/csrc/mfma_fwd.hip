@@ -32,12 +32,11 @@ constexpr float kTau = 8.f;  // lazy-rescale threshold, log2 domain
 
 enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
 
-// RAGGED (no mask): S is not a multiple of 128. Query rows and keys at or beyond S do not exist: row and tile loads clamp
+// RAGGED (no mask, or a padded one): S is not a multiple of 32 NW. Query rows and keys at or beyond S do not exist: row and tile loads clamp
 // their row index to S - 1, the scores of keys >= S are set to -inf, and rows >= S are not stored. A wave without a
 // single row of its own only fetches its share of the tiles and meets the barriers.
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false>
-__global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
-    static_assert(!RAGGED || MASK == 0, "ragged lengths: no mask");
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) void mfma_fwd_kernel(const KParams p) {
     using Tile = SwzTile<D>;
     // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions. The ring then has
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
@@ -59,10 +58,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     constexpr int DB = D >= 32 ? D / 32 : 1;  // 32-row blocks of O^T (D = 16: one block whose upper 16 rows are not stored)
     constexpr int kSteps = 2 * KK;    // MFMAs of S^T per tile
     constexpr int kPvSteps = 4 * DB;  // MFMAs of O^T per tile
-    // operand fragments in flight (dropout together with a mask or boundary handling leaves room for four only at D = 128)
+    // operand fragments in flight (two of mask, dropout and boundary handling leave room for four only at D = 128)
     // (at D = 32 the O^T product has four steps, and the softmax phase may request fragments of tile j only: tile j + 1
     // becomes visible with the barrier behind it)
-    constexpr int kRing = (D <= 32 || (D == 128 && (MASK != kNoMask || (RAGGED && NW == 8)) && DROPOUT)) ? 4 : 6;
+    constexpr int kRing = (D <= 32 || (D == 128 && (MASK != kNoMask) + (RAGGED && NW == 8) + DROPOUT >= 2)) ? 4 : 6;
     static_assert(kRing <= kPvSteps, "the softmax phase requests fragments of the O^T product only");
     // A mask block of a wave (32 rows x 64 keys) goes through a private LDS region (8 KiB for an fp32 mask, 4 KiB
     // for one of the operand type) when it fits (D = 64): lanes own rows, so direct loads would touch 32 cache
@@ -125,10 +124,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
             const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (qt * kBM / 64) * p.mcs[2], 1, n_tiles,
-                                                kBM / 64, p.mcs[2], lane);
+                                                RAGGED ? min(kBM / 64, num_key_tiles - qt * kBM / 64) : kBM / 64, p.mcs[2], lane);
             zero_tiles = tc.zero;
             n_tiles = tc.active ? 64 - __builtin_clzll(tc.active) : 1;  // (fully masked rows still run one tile: NaN like softmax)
-            my_tiles = n_tiles;
+            my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
         }
     }
     auto mask_is_zero = [&](int t) { return MASK != kNoMask && ((zero_tiles >> t) & 1) != 0; };
@@ -143,13 +142,15 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     auto issue_mask = [&](int t) {  // mask block of tile t -> this wave's region (8 LDS-direct loads), unless it is all zero
         if constexpr (kMaskViaLds) {
             if (mask_is_zero(t)) return;
+            const int row0 = RAGGED ? min(wrow0, p.S - 1) : wrow0;
             const char* src = static_cast<const char*>(p.mask) +
-                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(wrow0) * p.ms[2] + t * kBN) * kMaskElt;
+                              (b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(row0) * p.ms[2] + t * kBN) * kMaskElt;
             int l = lane;
             asm volatile("" : "+v"(l));  // offsets recomputed per tile rather than kept in registers
 #pragma unroll
             for (int blk = 0; blk < kMaskBytes / 1024; ++blk)
-                lds_direct_load16(src, static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
+                lds_direct_load16(src, RAGGED ? MaskTile::src_off_clamped(blk, l, p.ms[2] * kMaskElt, p.S - 1 - row0)
+                                              : static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
         }
     };
     issue_mask(0);
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     auto load_mask = [&](int t) {
         if constexpr (MASK != kNoMask && !kMaskViaLds) {
             if (mask_is_zero(t)) return;  // (the tile then takes the arithmetic of a tile without a mask: mk is not read)
-            const int64_t mrow = b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(qrow) * p.ms[2] + t * kBN;
+            const int64_t mrow = b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(RAGGED ? min(qrow, p.S - 1) : qrow) * p.ms[2] + t * kBN;
 #pragma unroll
             for (int g = 0; g < 8; ++g) {
                 const int key0 = 32 * (g >> 2) + 8 * (g & 3) + 4 * h;
@@ -609,13 +610,21 @@ __global__ __launch_bounds__(NW * 64, 2) void mfma_fwd_kernel(const KParams p) {
     }
 }
 
-template <typename T, int D, int NW, bool CAUSAL>
+template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
+    if constexpr (D == 128 && NW == 8 && MASK != kNoMask) {
+        // (mask, dropout and boundary handling together need the whole register file: four waves)
+        if (p.thr8 > 0) return launch_fwd_ragged<T, D, 4, CAUSAL, MASK>(p, stream);
+    }
     const int items = p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW));
     // (NW == 8: the kernel's kPersistent, one workgroup per CU walks the items)
-    const dim3 grid(NW == 8 ? persistent_grid(items) : items), block(64 * NW);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+    const dim3 grid(NW == 8 && MASK == kNoMask ? persistent_grid(items) : items), block(64 * NW);
+    if (p.thr8 > 0) {
+        if constexpr (!(D == 128 && NW == 8 && MASK != kNoMask))
+            hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true, true>), grid, block, 0, stream, p);
+    } else if constexpr (!(D == 128 && NW == 4)) {
+        hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
+    }
     return static_cast<int>(hipGetLastError());
 }
 
@@ -655,6 +664,13 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
         if (p.mask == nullptr) return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
     }
     if (p.S % 128 == 0) return launch_fwd_variant<T, D, 4>(dtype, p, stream);
+    if (p.mask != nullptr) {
+        // A padded mask: as many waves as share a CU's LDS with the mask's staging regions. At D = 64 an fp32 mask leaves room
+        // for one workgroup per CU (8 waves), a 16-bit one for two of 4 waves.
+        if (p.mask_dtype == TRI_ATTN_F32) return launch_fwd_ragged<T, D, D >= 64 ? 8 : 4, false, kMaskF32>(p, stream);
+        if (p.mask_dtype == dtype) return launch_fwd_ragged<T, D, D == 128 ? 8 : 4, false, kMaskT>(p, stream);
+        return TRI_ATTN_EDTYPE;
+    }
     // any other length (no mask: mfma_supported) at D <= 64: 128-row workgroups with boundary handling, two of which share
     // a CU (256-row ones measured 5-30 % slower at D = 64, S = 65 .. 6001)
     if constexpr (D < 128) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);

@@ -19,7 +19,7 @@ __global__ __launch_bounds__(256) void delta_kernel(const KParams p) {
     const int sub = threadIdx.x % kLanes;
     const int64_t row_lin = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / kLanes;
     const int64_t total = static_cast<int64_t>(p.B) * p.H * p.S;
-    if (row_lin >= total) return;  // whole lane groups leave together: total is a multiple of 128
+    if (row_lin >= total) return;  // (the lanes of a row leave together)
     const int row = static_cast<int>(row_lin % p.S);
     const int bh = static_cast<int>(row_lin / p.S);
     const int b = bh / p.H, h = bh % p.H;
@@ -86,7 +86,71 @@ __global__ __launch_bounds__(256) void classify_mask_kernel(const KParams p, uin
     }
 }
 
+// Padded additive mask from a source mask, and the classes of its 64 x 64 blocks: one workgroup per block, lane = column,
+// a wave takes every fourth row (row-segment reads of 64 entries, coalesced for unit stride; writes of 128 or 256 bytes).
+// Replaces three elementwise passes over a boolean mask (fill, not, masked fill) and the classification pass.
+template <typename Src, typename Dst>
+__global__ __launch_bounds__(256) void prepare_mask_kernel(const KParams p, Dst* out, uint8_t* classes, const Src* src, int64_t s0, int64_t s1,
+                                                           int64_t s2, int64_t s3) {
+    __shared__ int wave_flags[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int cbn = (p.S + 63) / 64;
+    const int rbn = p.ms[2] == 0 ? 1 : cbn, mhn = p.ms[1] == 0 ? 1 : p.H;
+    int64_t w = blockIdx.x;
+    const int cb = static_cast<int>(w % cbn);
+    w /= cbn;
+    const int rb = static_cast<int>(w % rbn);
+    w /= rbn;
+    const int mh = static_cast<int>(w % mhn), mb = static_cast<int>(w / mhn);
+    const int key = cb * 64 + lane;
+    const bool live = key < p.S;
+    const int rows = p.ms[2] == 0 ? 1 : min(64, p.S - rb * 64);
+    const Src* from = src + mb * s0 + mh * s1 + static_cast<int64_t>(rb) * 64 * s2 + (live ? key : 0) * s3;
+    Dst* to = out + mb * p.ms[0] + mh * p.ms[1] + static_cast<int64_t>(rb) * 64 * p.ms[2] + key;
+    bool nonzero = false, finite = false;
+#pragma unroll 4
+    for (int r = wave; r < rows; r += 4) {
+        Dst v;
+        if constexpr (sizeof(Src) == 1) v = static_cast<Dst>(from[r * s2] != 0 ? 0.f : -INFINITY);
+        else v = static_cast<Dst>(from[r * s2]);  // (the types are equal)
+        const float x = static_cast<float>(v);
+        nonzero |= live && !(x == 0.f);
+        finite |= live && !(x == -INFINITY);
+        to[r * p.ms[2]] = live ? v : static_cast<Dst>(0.f);
+    }
+    if (classes == nullptr) return;
+    const int flags = (__builtin_amdgcn_ballot_w64(nonzero) != 0 ? 1 : 0) | (__builtin_amdgcn_ballot_w64(finite) != 0 ? 2 : 0);
+    if (lane == 0) wave_flags[wave] = flags;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int f = wave_flags[0] | wave_flags[1] | wave_flags[2] | wave_flags[3];
+        classes[mb * p.mcs[0] + mh * p.mcs[1] + rb * p.mcs[2] + cb] = static_cast<uint8_t>(f == 2 ? kMaskZero : (f == 1 ? kMaskNegInf : kMaskMixed));
+    }
+}
+
+template <typename Src, typename Dst>
+int launch_prepare_t(const KParams& p, void* out, uint8_t* classes, const void* source, const int64_t* s, hipStream_t stream) {
+    const int64_t cbn = (p.S + 63) / 64, rbn = p.ms[2] == 0 ? 1 : cbn, mhn = p.ms[1] == 0 ? 1 : p.H, mbn = p.ms[0] == 0 ? 1 : p.B;
+    const int64_t groups = cbn * rbn * mhn * mbn;
+    if (groups > 2147483647LL) return TRI_ATTN_ESHAPE;
+    hipLaunchKernelGGL((prepare_mask_kernel<Src, Dst>), dim3(static_cast<unsigned>(groups)), dim3(256), 0, stream, p, static_cast<Dst*>(out),
+                       classes, static_cast<const Src*>(source), s[0], s[1], s[2], s[3]);
+    return static_cast<int>(hipGetLastError());
+}
+
 }  // namespace
+
+int launch_prepare_mask(const KParams& p, void* out, uint8_t* classes, const void* source, int source_dtype, const int64_t* s, hipStream_t stream) {
+    const int to = p.mask_dtype;
+    if (source_dtype == TRI_ATTN_BOOL)
+        return to == TRI_ATTN_F32 ? launch_prepare_t<uint8_t, float>(p, out, classes, source, s, stream)
+             : to == TRI_ATTN_F16 ? launch_prepare_t<uint8_t, f16_t>(p, out, classes, source, s, stream)
+                                  : launch_prepare_t<uint8_t, bf16_t>(p, out, classes, source, s, stream);
+    if (source_dtype != to) return TRI_ATTN_EDTYPE;
+    return to == TRI_ATTN_F32 ? launch_prepare_t<float, float>(p, out, classes, source, s, stream)
+         : to == TRI_ATTN_F16 ? launch_prepare_t<f16_t, f16_t>(p, out, classes, source, s, stream)
+                              : launch_prepare_t<bf16_t, bf16_t>(p, out, classes, source, s, stream);
+}
 
 int launch_classify_mask(const KParams& p, uint8_t* out, hipStream_t stream) {
     const int per_lane = p.mask_dtype == TRI_ATTN_F32 ? 4 : 8;
@@ -107,8 +171,9 @@ static bool tile_offsets_fit(const int64_t* strides) { return strides[2] >= 0 &&
 bool mfma_supported(int which, int dtype, const KParams& p) {
     if (dtype != TRI_ATTN_F16 && dtype != TRI_ATTN_BF16) return false;
     if (p.D != 16 && p.D != 32 && p.D != 64 && p.D != 128) return false;
-    // lengths that are not multiples of 128 run the 4-wave kernels with boundary handling; those read no mask
-    if (p.S % 128 != 0 && p.mask != nullptr) return false;
+    // lengths that are not multiples of 128 run with boundary handling, which reads whole pieces of padded masks only and
+    // does not write a mask gradient
+    if (p.S % 128 != 0 && p.mask != nullptr && (!p.mask_padded || p.dmask != nullptr)) return false;
     if (!(p.scale > 0.f)) return false;  // the kernels take row maxima before scaling
     if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v)) return false;
     if (!strides8(p.qs) || !strides8(p.ks) || !strides8(p.vs)) return false;
@@ -164,8 +229,7 @@ int persistent_grid(int items) {
 
 int launch_delta(int dtype, const KParams& p, hipStream_t stream) {
     const bool vec = (dtype == TRI_ATTN_F16 || dtype == TRI_ATTN_BF16) && (p.D == 16 || p.D == 32 || p.D == 64 || p.D == 128) &&
-                     aligned16(p.o) && aligned16(p.d_o) && strides8(p.os) && strides8(p.dos) &&
-                     (static_cast<int64_t>(p.B) * p.H * p.S) % 128 == 0;
+                     aligned16(p.o) && aligned16(p.d_o) && strides8(p.os) && strides8(p.dos);
     if (!vec) return launch_generic_any(kGenericDelta, dtype, p, stream);
     if (dtype == TRI_ATTN_BF16)
         return p.D == 128 ? launch_delta_t<bf16_t, 128>(p, stream) : p.D == 64 ? launch_delta_t<bf16_t, 64>(p, stream)

@@ -130,6 +130,97 @@ def _mask_classes(mask: torch.Tensor, args):
     return classes
 
 
+class _BooleanMask:
+    """A boolean attn_mask (True = the key takes part) on its way through forward and backward: the additive mask the
+    kernels read is made by the forward call and kept for the backward."""
+
+    __slots__ = ("source", "device", "prepared")
+    requires_grad = False
+
+    def __init__(self, source):
+        self.source = source
+        self.device = source.device
+        self.prepared = None
+
+
+class _PreparedMask:
+    """Additive mask for ``query``'s kernels, its rows padded to whole pieces of 64 keys (tri_attn_prepare_mask), broadcast
+    like ``source`` (additive or boolean), and the classes of its blocks for the kernels that look at them. (Plain numbers
+    and two allocations: views of the buffer would cost a small call as much as its kernels.)"""
+
+    __slots__ = ("padded", "classes", "strides", "dtype")
+
+    def __init__(self, source, query):
+        num_batches, num_heads, y_size, _ = query.shape
+        full = (num_batches, num_heads, y_size, y_size)
+        missing = 4 - source.dim()
+        if missing < 0 or any(n != 1 and n != m for n, m in zip(source.shape, full[missing:])):
+            source.expand(full)  # (raises)
+        # (a dimension the source broadcasts is kept once)
+        shape = (1,) * missing + tuple(source.shape)
+        given = (0,) * missing + source.stride()
+        from_strides = [0 if n == 1 else t for n, t in zip(shape, given)]
+        batches, heads, rows = [1 if t == 0 else n for n, t in zip(shape[:3], from_strides)]
+        pitch = (y_size + 63) // 64 * 64
+        boolean = source.dtype == torch.bool
+        dtype = query.dtype if boolean else source.dtype
+        self.padded = torch.empty(batches * heads * rows * pitch, device=query.device, dtype=dtype)
+        self.strides = (heads * rows * pitch if batches > 1 else 0, rows * pitch if heads > 1 else 0, pitch if rows > 1 else 0, 1)
+        self.dtype = util.dtype(dtype) | _lib.MASK_PADDED
+        self.classes = None
+        args = _lib.TriAttnArgs()
+        args.struct_size = _lib.ARGS_PACKER.size
+        args.B, args.H, args.S = num_batches, num_heads, y_size
+        args.stream = torch._C._cuda_getCurrentRawStream(query.device.index)
+        if query.dtype != torch.float32:
+            blocks = pitch // 64
+            self.classes = torch.empty(batches * heads * (blocks if rows > 1 else 1) * blocks, dtype=torch.uint8, device=query.device)
+        self.describe(args)
+        _lib.check(_lib.lib().tri_attn_prepare_mask(ctypes.byref(args), source.data_ptr(), _lib.BOOL if boolean else util.dtype(dtype),
+                                                    (ctypes.c_int64 * 4)(*from_strides)))
+
+    def describe(self, args):
+        """The mask's fields of a call's arguments."""
+        args.mask = self.padded.data_ptr()
+        args.mask_dtype = self.dtype
+        args.mask_stride[:] = self.strides
+        if self.classes is not None:
+            args.mask_classes = self.classes.data_ptr()
+
+
+def _prepared_mask(mask, query):
+    """The _PreparedMask of a call, or None where the mask is handed over as it is. Boolean masks always have one. Additive
+    ones are copied into padded rows for 16-bit problems at lengths that are no multiple of 128, whose kernels fetch mask rows
+    in 16-byte pieces up to the end of a 64-key tile: one more pass over the mask (at the copy rate) in each direction against
+    kernels that read masks element by element (bf16, dense fp32 mask, forward + backward: B=16 H=12 S=777 D=64 2.22 -> 0.39 ms,
+    S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below 2^29 scores times head size the launches and their arguments cost a call more than
+    the kernels save (S=100 0.15 -> 0.21 ms). A mask that wants a gradient stays as it is: its gradient is laid out like it."""
+    if isinstance(mask, _BooleanMask):
+        if mask.prepared is None:
+            mask.prepared = _PreparedMask(mask.source, query)
+            mask.source = None
+        return mask.prepared
+    if query.dtype == torch.float32 or query.shape[2] % 128 == 0 or mask.dtype not in (torch.float32, query.dtype) or mask.requires_grad:
+        return None
+    num_batches, num_heads, y_size, x_size = query.shape
+    if num_batches * num_heads * y_size * y_size * max(x_size, 32) < 1 << 29:
+        return None
+    return _PreparedMask(mask.detach(), query)
+
+
+def _set_mask(args, mask, query):
+    """Describes ``mask`` (a tensor or a _BooleanMask) in a call's arguments; returns what to keep alive until it is enqueued."""
+    prepared = _prepared_mask(mask, query)
+    if prepared is not None:
+        prepared.describe(args)
+        return prepared
+    view = _expand_mask(mask.detach(), (*query.shape[:3], query.shape[2]))
+    args.mask = view.data_ptr()
+    args.mask_dtype = util.dtype(view.dtype)
+    args.mask_stride[:] = _strides_or_zero(view)
+    return view, _mask_classes(mask, args)
+
+
 def _expand_mask(mask: torch.Tensor, shape):
     """View of the additive mask broadcast to [B,H,S,S] (stride 0 on broadcast dims)."""
     view = mask
@@ -189,7 +280,7 @@ class Attention(torch.autograd.Function):
                     raise ValueError("Boolean mask is not supported yet.")
                 # torch's meaning of a boolean attn_mask: True = the key takes part in the attention (the additive
                 # mask is made in the operand type: half the bytes of an fp32 one for the 16-bit kernels to stream)
-                mask = torch.zeros(mask.shape, dtype=query.dtype, device=mask.device).masked_fill_(~mask, float("-inf"))
+                mask = _BooleanMask(mask)
 
         seed, offset = _next_seed() if dropout_p > 0.0 else (0, 0)
 
@@ -250,10 +341,8 @@ class Attention(torch.autograd.Function):
         num_batches, num_heads, y_size, x_size = query.shape
         output = torch.empty(query.shape, device=query.device, dtype=query.dtype)
         log2sum = torch.empty(num_batches, num_heads, y_size, device=query.device, dtype=torch.float32)
-        mask_view = _expand_mask(mask.detach(), (num_batches, num_heads, y_size, y_size)) if mask is not None else None
-
-        args = _make_args(query, key, value, output, log2sum, mask_view, dropout_p, is_causal, softmax_scale, seed, offset)
-        classes = _mask_classes(mask, args) if mask is not None else None  # (kept alive until the call is enqueued)
+        args = _make_args(query, key, value, output, log2sum, None, dropout_p, is_causal, softmax_scale, seed, offset)
+        _alive = _set_mask(args, mask, query) if mask is not None else None
 
         util.push_trace("kernel.Attention.forward")
         _lib.check(lib.tri_attn_fwd(ctypes.byref(args)))
@@ -277,12 +366,13 @@ class Attention(torch.autograd.Function):
         grad_value = torch.empty(value.shape, device=value.device, dtype=value.dtype)
         delta = torch.empty_like(log2sum) if delta_out is None else delta_out
         full = (num_batches, num_heads, y_size, y_size)
-        mask_view = _expand_mask(mask.detach(), full) if mask is not None else None
         # The mask gradient (trident/kernel/attention.py:332-335) in the mask's own shape: a full [B,H,S,S] mask gets
         # dS written in place; a broadcast mask gets a zero-filled fp32 buffer of its shape that the kernels add to
         # through strides of 0 (autograd's sum over the broadcast dimensions, without a [B,H,S,S] intermediate).
         grad_mask_buf = grad_mask_view = None
+        mask_view = None
         if want_grad_mask:
+            mask_view = _expand_mask(mask.detach(), full)
             shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
             if shape4 == full:
                 grad_mask_buf = torch.empty(full, device=mask.device, dtype=mask.dtype)
@@ -295,8 +385,12 @@ class Attention(torch.autograd.Function):
 
         args = _make_args(query, key, value, output, log2sum, mask_view, dropout_p, is_causal, softmax_scale, seed, offset,
                           grad_output, grad_query, grad_key, grad_value, grad_mask_view, delta)
-        # (the classes describe the mask tensor as the kernels see it: not when it was converted to fp32 above)
-        classes = _mask_classes(mask, args) if mask is not None and mask_view.dtype == mask.dtype else None
+        _alive = None
+        if mask is not None and not want_grad_mask:
+            _alive = _set_mask(args, mask, query)
+        elif mask is not None and mask_view.dtype == mask.dtype:
+            # (the classes describe the mask tensor as the kernels see it: not when it was converted to fp32 above)
+            _alive = _mask_classes(mask, args)
 
         # one call for the three backward launches (trident/operation/attention.py:161-199 launches the
         # delta pre-pass and the backward kernel): the library orders them, and where the dQ kernel can
