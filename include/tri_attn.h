@@ -156,6 +156,14 @@ int tri_attn_bwd_dq(const TriAttnArgs* args);
  * (trident/operation/attention.py:161-199); tri_attn_bwd picks between the two sequences itself. */
 int tri_attn_bwd_dq_delta(const TriAttnArgs* args);
 
+/* The gradient of a mask that batches or heads share (dmask_stride 0 over one or both; the mask broadcast the same way),
+ * summed over them: written, not added, to args->dmask in mask_dtype, with a fixed order of summation. For the 16-bit types,
+ * any S, 16-byte aligned rows of q, k, v, d_o, and a row stride of dmask that is not 0. Reads q,k,v,d_o,lse,delta,mask: it
+ * follows a tri_attn_bwd (with dmask NULL) or whatever computed delta. Returns TRI_ATTN_ENOFUSE without launching anything
+ * where it does not apply: tri_attn_bwd / tri_attn_bwd_dq with dmask set then adds the gradient up atomically. The reference
+ * stores dS per batch and head (trident/kernel/attention.py:332-335). */
+int tri_attn_bwd_dmask(const TriAttnArgs* args);
+
 /* The whole backward (trident/operation/attention.py:137-202): the results of bwd_delta, bwd_dkdv and
  * bwd_dq called in that order, written to delta, dk, dv, dq[, dmask]. The library may launch fewer
  * kernels and in another order: without a mask, for sequence lengths that are multiples of 256 (and
@@ -197,7 +205,7 @@ int64_t tri_attn_mask_classes_size(const TriAttnArgs* args);
 int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t source_dtype, const int64_t* source_stride);
 
 /* Which kernel family a call would run, without launching anything (no counterpart in the reference): pass 0 =
- * tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq on these arguments. Returns 1 for the 16-bit matrix-core
+ * tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq, 3 = tri_attn_bwd_dmask (1 or 0: applies or not) on these arguments. Returns 1 for the 16-bit matrix-core
  * (MFMA) kernels (fp16/bf16, D in {16,32,64,128}, 16-byte aligned rows; any S without a mask or with
  * a padded one, S a multiple of 128 with any other); 2 for the 32-row-tile matrix-core kernels (everything else whose pointers and strides are multiples of
  * four elements: fp32 problems on the fp32 matrix instruction with fp32 products and sums; fp16/bf16 problems with

@@ -1047,3 +1047,39 @@ def test_prepared_masks_hold_the_source(source, S, device):
             cb = (S + 63) // 64
             dims = [1 if s == 0 else n for s, n in zip(additive.stride()[:2], additive.shape)] + [1 if additive.stride(2) == 0 else cb, cb]
             assert torch.equal(classes.cpu().view(dims).expand(2, 3, cb, cb).long(), expected)
+
+
+# ------------------------------------------------------------------ mask gradients summed over batches and heads
+@pytest.mark.parametrize("shape", ["1HSS", "B1SS", "11SS"])
+@pytest.mark.parametrize("dtype,mask_dtype,B,H,S,D", [(torch.bfloat16, torch.bfloat16, 3, 2, 1, 64), (torch.float16, torch.float32, 2, 3, 31, 16),
+                                                      (torch.bfloat16, torch.float32, 5, 2, 65, 32), (torch.bfloat16, torch.bfloat16, 2, 2, 130, 128),
+                                                      (torch.float16, torch.float16, 2, 2, 256, 64), (torch.bfloat16, torch.float16, 2, 20, 260, 64)])
+def test_mask_gradient_of_a_shared_mask(dtype, mask_dtype, B, H, S, D, shape, device):
+    """tri_attn_bwd_dmask: one row, lengths that end inside a key block, a key tile and a row block, store pieces that are not
+    aligned, more and fewer pairs than waves, enough tiles for one row block per wave (the last case with 1HSS: 20 x 5 x 3
+    workgroups) and too few; the same bits twice."""
+    q, k, v, d_o = _gen((B, H, S, D), 6100 + S + D, dtype)
+    mshape = {"1HSS": (1, H, S, S), "B1SS": (B, 1, S, S), "11SS": (1, 1, S, S)}[shape]
+    mask = (0.5 * torch.randn(mshape, generator=torch.Generator().manual_seed(S))).to(mask_dtype)
+    trident.config.reference_limits = False
+    try:
+        _check(device, dtype, q, k, v, d_o, mask=mask, mask_grad=True, tag=f"shared dmask {shape}")
+        first, second = [_run(device, q, k, v, d_o, mask=mask, mask_grad=True)[4] for _ in range(2)]
+    finally:
+        trident.config.reference_limits = True
+    assert torch.equal(first, second)
+
+
+def test_mask_gradient_of_a_shared_mask_with_dropout(device):
+    B, H, S, D = 3, 2, 200, 64
+    q, k, v, d_o = _gen((B, H, S, D), 6200, torch.bfloat16)
+    mask = 0.5 * torch.randn(1, H, S, S, generator=torch.Generator().manual_seed(1))
+    from trident_amd.operation import Attention
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    tm = mask.to(device).requires_grad_(True)
+    scale = 1.0 / math.sqrt(D)
+    o, lse = Attention._forward(tq, tk, tv, tm, 0.2, False, scale, 9, 4)
+    *_, dm = Attention._backward(tdo, tq, tk, tv, o, lse, tm, scale, 0.2, False, 9, 4, True)
+    kw = dict(mask=mask, dropout_p=0.2, is_causal=False, scale=scale, seed=9, offset=4)
+    _, _, _, dm_r, _ = parity.oracle_backward(q, k, v, d_o, want_dmask=True, o=o, **kw)
+    parity.close(dm, dm_r, torch.bfloat16, "dropout shared dMask")

@@ -96,6 +96,7 @@ EXPORTS = (
     "tri_attn_bwd_dq",
     "tri_attn_bwd_dq_delta",
     "tri_attn_bwd",
+    "tri_attn_bwd_dmask",
     "tri_attn_bwd_noalloc",
     "tri_attn_dropout_mask",
     "tri_attn_uses_matrix_cores",
@@ -123,7 +124,7 @@ def lib():
         cdll.tri_attn_strerror.restype = ctypes.c_char_p
         cdll.tri_attn_strerror.argtypes = [ctypes.c_int]
         for name in ("tri_attn_fwd", "tri_attn_bwd_delta", "tri_attn_bwd_dkdv", "tri_attn_bwd_dq",
-                     "tri_attn_bwd_dq_delta", "tri_attn_bwd", "tri_attn_bwd_noalloc", "tri_attn_classify_mask"):
+                     "tri_attn_bwd_dq_delta", "tri_attn_bwd", "tri_attn_bwd_dmask", "tri_attn_bwd_noalloc", "tri_attn_classify_mask"):
             fn = getattr(cdll, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(TriAttnArgs)]

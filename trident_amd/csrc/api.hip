@@ -37,7 +37,7 @@ void set_class_strides(int64_t* mcs, const TriAttnArgs* a) {
     mcs[0] = a->mask_stride[0] == 0 ? 0 : mh * rb * cb;
 }
 
-// Common validation + translation. `need` bits: 1 = forward tensors, 2 = backward tensors.
+// Common validation + translation. `need` bits: 1 = forward, 2 = delta, 4 = dK/dV, 8 = dQ (and dMask), 16 = summed dMask.
 int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (a == nullptr) return TRI_ATTN_ENULL;
     if (a->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
@@ -81,6 +81,12 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
             if ((rc = check_strides(a->dmask_stride))) return rc;
         }
     }
+    if (need & 16) {
+        if (!a->q || !a->k || !a->v || !a->lse || !a->d_o || !a->delta || !a->mask || !a->dmask) return TRI_ATTN_ENULL;
+        if ((rc = check_strides(a->q_stride)) || (rc = check_strides(a->k_stride)) || (rc = check_strides(a->v_stride)) ||
+            (rc = check_strides(a->do_stride)) || (rc = check_strides(a->dmask_stride)))
+            return rc;
+    }
     if (a->mask != nullptr && (rc = check_strides(a->mask_stride))) return rc;
 
     p->q = a->q;
@@ -93,7 +99,7 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     p->dq = a->dq;
     p->dk = a->dk;
     p->dv = a->dv;
-    p->dmask = (need & 8) ? a->dmask : nullptr;
+    p->dmask = (need & (8 | 16)) ? a->dmask : nullptr;
     p->delta = a->delta;
     copy3(p->qs, a->q_stride);
     copy3(p->ks, a->k_stride);
@@ -109,7 +115,7 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
         // a stride of 0 over a dimension that has more than one entry: the gradient is summed over it
         p->dmask_acc = (a->B > 1 && a->dmask_stride[0] == 0) || (a->H > 1 && a->dmask_stride[1] == 0) ||
                        (a->S > 1 && a->dmask_stride[2] == 0);
-        if (p->dmask_acc && mask_dtype != TRI_ATTN_F32) return TRI_ATTN_EDTYPE;
+        if (p->dmask_acc && mask_dtype != TRI_ATTN_F32 && (need & 8)) return TRI_ATTN_EDTYPE;
     }
     if (a->mask != nullptr && (a->S % 128 == 0 || padded)) {
         set_class_strides(p->mcs, a);
@@ -188,7 +194,7 @@ const char* tri_attn_strerror(int status) {
         case TRI_ATTN_EDROPOUT: return "dropout_p must lie in [0, 1]";
         case TRI_ATTN_ESIZE: return "TriAttnArgs.struct_size does not match this library";
         case TRI_ATTN_EALIGN: return "pointer or stride alignment not supported";
-        case TRI_ATTN_ENOFUSE: return "no fused dQ + delta kernel for this problem (nothing launched)";
+        case TRI_ATTN_ENOFUSE: return "no fused kernel for this problem (nothing launched)";
         case TRI_ATTN_ESCRATCH: return "tri_attn_bwd_noalloc: B*H*S exceeds TRI_ATTN_NOALLOC_MAX_ROWS (nothing launched)";
         default: break;
     }
@@ -258,6 +264,14 @@ int tri_attn_bwd(const TriAttnArgs* args) {
     rc = tri_attn_bwd_dkdv(args);
     if (rc) return rc;
     return tri_attn_bwd_dq(args);
+}
+
+int tri_attn_bwd_dmask(const TriAttnArgs* args) {
+    KParams p;
+    const int rc = make_params(args, 16, &p);
+    if (rc) return rc;
+    if (!mfma_dmask_supported(args->dtype, p)) return TRI_ATTN_ENOFUSE;
+    return launch_mfma_dmask(args->dtype, p, static_cast<hipStream_t>(args->stream));
 }
 
 int tri_attn_bwd_noalloc(const TriAttnArgs* args) {
@@ -333,8 +347,12 @@ int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t s
 }
 
 int tri_attn_uses_matrix_cores(const TriAttnArgs* args, int pass) {
-    if (pass < 0 || pass > 2) return TRI_ATTN_ESHAPE;
+    if (pass < 0 || pass > 3) return TRI_ATTN_ESHAPE;
     KParams p;
+    if (pass == 3) {
+        const int bad = make_params(args, 16, &p);
+        return bad ? bad : (mfma_dmask_supported(args->dtype, p) ? 1 : 0);
+    }
     const int rc = make_params(args, pass == 0 ? 1 : (pass == 1 ? 4 : 8), &p);
     if (rc) return rc;
     const int which = pass == 0 ? kMfmaFwd : (pass == 1 ? kMfmaDkdv : kMfmaDq);

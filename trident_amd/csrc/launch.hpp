@@ -23,6 +23,10 @@ bool mfma_dq_fuses_delta(const KParams& p);
 int launch_mfma_dkdv(int dtype, const KParams& p, hipStream_t stream);
 int launch_delta(int dtype, const KParams& p, hipStream_t stream);
 
+// mfma_dmask.hip: gradient of a mask shared by batches or heads, summed over them.
+bool mfma_dmask_supported(int dtype, const KParams& p);
+int launch_mfma_dmask(int dtype, const KParams& p, hipStream_t stream);
+
 // mfma32.hip: the fp32 matrix instruction. fp32 / fp16 / bf16 storage, D in {16,32,64,128}, any S, any mask, rows
 // aligned to four elements. `which` is a MfmaKernel.
 bool mfma32_supported(int which, int dtype, const KParams& p);

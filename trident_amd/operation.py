@@ -188,19 +188,28 @@ class _PreparedMask:
             args.mask_classes = self.classes.data_ptr()
 
 
+def _sums_mask_gradient(mask, query):
+    """Whether the gradient of ``mask`` is summed over batches or heads, with rows and keys of its own (16-bit problems)."""
+    shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
+    num_batches, num_heads, y_size, _ = query.shape
+    return query.dtype != torch.float32 and shape4[2:] == (y_size, y_size) and shape4[:2] != (num_batches, num_heads)
+
+
 def _prepared_mask(mask, query):
     """The _PreparedMask of a call, or None where the mask is handed over as it is. Boolean masks always have one. Additive
     ones are copied into padded rows for 16-bit problems at lengths that are no multiple of 128, whose kernels fetch mask rows
     in 16-byte pieces up to the end of a 64-key tile: one more pass over the mask (at the copy rate) in each direction against
     kernels that read masks element by element (bf16, dense fp32 mask, forward + backward: B=16 H=12 S=777 D=64 2.22 -> 0.39 ms,
     S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below 2^29 scores times head size the launches and their arguments cost a call more than
-    the kernels save (S=100 0.15 -> 0.21 ms). A mask that wants a gradient stays as it is: its gradient is laid out like it."""
+    the kernels save (S=100 0.15 -> 0.21 ms). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it."""
     if isinstance(mask, _BooleanMask):
         if mask.prepared is None:
             mask.prepared = _PreparedMask(mask.source, query)
             mask.source = None
         return mask.prepared
-    if query.dtype == torch.float32 or query.shape[2] % 128 == 0 or mask.dtype not in (torch.float32, query.dtype) or mask.requires_grad:
+    if query.dtype == torch.float32 or query.shape[2] % 128 == 0 or mask.dtype not in (torch.float32, query.dtype):
+        return None
+    if mask.requires_grad and not _sums_mask_gradient(mask, query):
         return None
     num_batches, num_heads, y_size, x_size = query.shape
     if num_batches * num_heads * y_size * y_size * max(x_size, 32) < 1 << 29:
@@ -208,16 +217,18 @@ def _prepared_mask(mask, query):
     return _PreparedMask(mask.detach(), query)
 
 
-def _set_mask(args, mask, query):
-    """Describes ``mask`` (a tensor or a _BooleanMask) in a call's arguments; returns what to keep alive until it is enqueued."""
+def _set_mask(args, mask, query, view=None):
+    """Describes ``mask`` (a tensor or a _BooleanMask) in a call's arguments; returns what to keep alive until it is enqueued.
+    ``view``: its [B,H,S,S] view, where the arguments hold that already."""
     prepared = _prepared_mask(mask, query)
     if prepared is not None:
         prepared.describe(args)
         return prepared
-    view = _expand_mask(mask.detach(), (*query.shape[:3], query.shape[2]))
-    args.mask = view.data_ptr()
-    args.mask_dtype = util.dtype(view.dtype)
-    args.mask_stride[:] = _strides_or_zero(view)
+    if view is None:
+        view = _expand_mask(mask.detach(), (*query.shape[:3], query.shape[2]))
+        args.mask = view.data_ptr()
+        args.mask_dtype = util.dtype(view.dtype)
+        args.mask_stride[:] = _strides_or_zero(view)
     return view, _mask_classes(mask, args)
 
 
@@ -367,36 +378,52 @@ class Attention(torch.autograd.Function):
         delta = torch.empty_like(log2sum) if delta_out is None else delta_out
         full = (num_batches, num_heads, y_size, y_size)
         # The mask gradient (trident/kernel/attention.py:332-335) in the mask's own shape: a full [B,H,S,S] mask gets
-        # dS written in place; a broadcast mask gets a zero-filled fp32 buffer of its shape that the kernels add to
-        # through strides of 0 (autograd's sum over the broadcast dimensions, without a [B,H,S,S] intermediate).
-        grad_mask_buf = grad_mask_view = None
-        mask_view = None
+        # dS written in place; one shared by batches or heads gets dS summed over them by a kernel of its own
+        # (tri_attn_bwd_dmask); what that does not take (fp32, a mask that is also shared by the rows) gets a zero-filled
+        # fp32 buffer of its shape that the kernels add to through strides of 0.
+        grad_mask_buf = grad_mask_view = mask_view = None
+        summed = want_grad_mask and _sums_mask_gradient(mask, query)
         if want_grad_mask:
             mask_view = _expand_mask(mask.detach(), full)
             shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
-            if shape4 == full:
-                grad_mask_buf = torch.empty(full, device=mask.device, dtype=mask.dtype)
-                grad_mask_view = grad_mask_buf
-            else:
-                grad_mask_buf = torch.zeros(shape4, device=mask.device, dtype=torch.float32)
-                grad_mask_view = grad_mask_buf.expand(*full)
-                if mask_view.dtype != torch.float32:  # (mask and dmask share one dtype field)
-                    mask_view = _expand_mask(mask.detach().float(), full)
+            if shape4 == full or summed:
+                grad_mask_buf = torch.empty(shape4, device=mask.device, dtype=mask.dtype)
+                grad_mask_view = grad_mask_buf if shape4 == full else grad_mask_buf.expand(*full)
 
         args = _make_args(query, key, value, output, log2sum, mask_view, dropout_p, is_causal, softmax_scale, seed, offset,
                           grad_output, grad_query, grad_key, grad_value, grad_mask_view, delta)
         _alive = None
-        if mask is not None and not want_grad_mask:
-            _alive = _set_mask(args, mask, query)
-        elif mask is not None and mask_view.dtype == mask.dtype:
+        if summed:
+            summed = lib.tri_attn_uses_matrix_cores(ctypes.byref(args), 3) == 1
+            args.dmask = None
+        if mask is not None and (summed or not want_grad_mask):
+            _alive = _set_mask(args, mask, query, mask_view)
+        elif want_grad_mask:
+            if shape4 != full:
+                grad_mask_buf = torch.zeros(shape4, device=mask.device, dtype=torch.float32)
+                grad_mask_view = grad_mask_buf.expand(*full)
+                args.dmask = grad_mask_view.data_ptr()
+                args.dmask_stride[:] = _strides_or_zero(grad_mask_view)
+                if mask_view.dtype != torch.float32:  # (mask and dmask share one dtype field)
+                    mask_view = _expand_mask(mask.detach().float(), full)
+                    args.mask = mask_view.data_ptr()
+                    args.mask_dtype = util.dtype(torch.float32)
+                    args.mask_stride[:] = _strides_or_zero(mask_view)
             # (the classes describe the mask tensor as the kernels see it: not when it was converted to fp32 above)
-            _alive = _mask_classes(mask, args)
+            if mask_view.dtype == mask.dtype:
+                _alive = _mask_classes(mask, args)
 
         # one call for the three backward launches (trident/operation/attention.py:161-199 launches the
         # delta pre-pass and the backward kernel): the library orders them, and where the dQ kernel can
         # compute delta on its way the pre-pass disappears into it
         util.push_trace("kernel.Attention.backward")
         _lib.check(lib.tri_attn_bwd(ctypes.byref(args)))
+        if summed:
+            args.mask = mask_view.data_ptr()
+            args.mask_dtype = util.dtype(mask_view.dtype)
+            args.mask_stride[:] = _strides_or_zero(mask_view)
+            args.dmask = grad_mask_buf.data_ptr()
+            _lib.check(lib.tri_attn_bwd_dmask(ctypes.byref(args)))
         util.pop_trace()
 
         grad_mask = None
