@@ -71,26 +71,20 @@ __device__ __forceinline__ void store_mask_elem(void* base, int dtype, int64_t o
 struct Philox4 {
     uint32_t w[4];
 };
+// One of the ten rounds (r = 0 .. 9), for callers that spread them over other work.
+__device__ __forceinline__ void philox_round(Philox4& s, int r, uint32_t k0, uint32_t k1) {
+    const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * s.w[0];
+    const uint64_t p1 = static_cast<uint64_t>(0xCD9E8D57u) * s.w[2];
+    s.w[0] = static_cast<uint32_t>(p1 >> 32) ^ s.w[1] ^ (k0 + r * 0x9E3779B9u);
+    s.w[2] = static_cast<uint32_t>(p0 >> 32) ^ s.w[3] ^ (k1 + r * 0xBB67AE85u);
+    s.w[1] = static_cast<uint32_t>(p1);
+    s.w[3] = static_cast<uint32_t>(p0);
+}
 __device__ __forceinline__ Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                                  uint32_t k0, uint32_t k1) {
+    Philox4 out = {{c0, c1, c2, c3}};
 #pragma unroll
-    for (int r = 0; r < 10; ++r) {
-        const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * c0;
-        const uint64_t p1 = static_cast<uint64_t>(0xCD9E8D57u) * c2;
-        const uint32_t n0 = static_cast<uint32_t>(p1 >> 32) ^ c1 ^ k0;
-        const uint32_t n2 = static_cast<uint32_t>(p0 >> 32) ^ c3 ^ k1;
-        c1 = static_cast<uint32_t>(p1);
-        c3 = static_cast<uint32_t>(p0);
-        c0 = n0;
-        c2 = n2;
-        k0 += 0x9E3779B9u;
-        k1 += 0xBB67AE85u;
-    }
-    Philox4 out;
-    out.w[0] = c0;
-    out.w[1] = c1;
-    out.w[2] = c2;
-    out.w[3] = c3;
+    for (int r = 0; r < 10; ++r) philox_round(out, r, k0, k1);
     return out;
 }
 

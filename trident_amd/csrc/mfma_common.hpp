@@ -13,6 +13,8 @@
 // 16g + 8*(t/4) + 4h + t%4, and the A operand of that MFMA must present its K dimension in
 // exactly that slot order, which is what the transposed LDS reads of SwzTile below deliver.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace tri {
@@ -384,13 +386,24 @@ __device__ __forceinline__ Philox4 quad_bcast_from(int g, const Philox4& r) {
 // Row-owner form: this lane owns row i (i % 4 == lane % 4) and wants, for groups g = 0..3, the word
 // (4 key bytes) of keys key0 + gstride*g .. +3. `mine` is the block this lane generated for group
 // lane % 4, i.e. dropout_block(p, bh, i >> 2, (key0 + gstride * (lane % 4)) >> 2).
+// A 4 x 4 transposition inside the quad (lane g's word q goes to lane q's word g) by two exchanges, with lane ^ 1 and with
+// lane ^ 2: 4 moves and 12 selections (broadcasting the four blocks and picking words took 16 and 12).
 __device__ __forceinline__ void quad_row_words(const Philox4& mine, int lane, uint32_t (&w)[4]) {
-    const int q = lane & 3;
-    const Philox4 b0 = quad_bcast<0>(mine), b1 = quad_bcast<1>(mine), b2 = quad_bcast<2>(mine), b3 = quad_bcast<3>(mine);
-    w[0] = q == 0 ? b0.w[0] : (q == 1 ? b0.w[1] : (q == 2 ? b0.w[2] : b0.w[3]));
-    w[1] = q == 0 ? b1.w[0] : (q == 1 ? b1.w[1] : (q == 2 ? b1.w[2] : b1.w[3]));
-    w[2] = q == 0 ? b2.w[0] : (q == 1 ? b2.w[1] : (q == 2 ? b2.w[2] : b2.w[3]));
-    w[3] = q == 0 ? b3.w[0] : (q == 1 ? b3.w[1] : (q == 2 ? b3.w[2] : b3.w[3]));
+    const bool odd = (lane & 1) != 0, high = (lane & 2) != 0;
+    auto exchange = [](uint32_t& a, uint32_t& b, bool second, auto ctrl) {  // a of the second lane <-> b of the first
+        const uint32_t out = second ? a : b;
+        const uint32_t in = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(out), decltype(ctrl)::value, 0xf, 0xf, true));
+        a = second ? in : a;
+        b = second ? b : in;
+    };
+    using Xor1 = std::integral_constant<int, 0xB1>;  // quad_perm [1, 0, 3, 2]
+    using Xor2 = std::integral_constant<int, 0x4E>;  // quad_perm [2, 3, 0, 1]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = mine.w[i];
+    exchange(w[0], w[1], odd, Xor1{});
+    exchange(w[2], w[3], odd, Xor1{});
+    exchange(w[0], w[2], high, Xor2{});
+    exchange(w[1], w[3], high, Xor2{});
 }
 
 }  // namespace tri
