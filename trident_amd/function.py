@@ -13,6 +13,8 @@ def dropout(input, p=0.5, training=True):
     See Dropout for details.
     """
     if training:
+        if input.dim() == 2 and input.numel() > 0:  # (a view of the same shape is two more nodes of the graph)
+            return operation.Dropout.apply(input, p)
         return operation.Dropout.apply(input.view(-1, input.shape[-1]), p).view(input.shape)
     else:
         return input.clone()

@@ -50,12 +50,18 @@ def _same_layout(t: torch.Tensor, like: torch.Tensor):
     return out
 
 
+def _stream(input):
+    """Handle of torch's current stream on the tensor's device (a Stream object around it costs more than the rest of a
+    call's arguments)."""
+    return torch._C._cuda_getCurrentRawStream(input.device.index)
+
+
 def _row_args(input, dim):
     args = _lib.TriRowArgs()
     args.struct_size = ctypes.sizeof(_lib.TriRowArgs)
     args.dtype = util.dtype(input.dtype)
     args.y_size, args.x_size, args.y_stride, args.x_stride = size_and_stride(input, dim)
-    args.stream = torch.cuda.current_stream(input.device).cuda_stream
+    args.stream = _stream(input)
     return args
 
 
@@ -193,7 +199,7 @@ class Dropout(torch.autograd.Function):
         args.y_size, args.x_size = 1, source.numel()
         args.p = float(p)
         args.seed, args.offset = seed, offset
-        args.stream = torch.cuda.current_stream(source.device).cuda_stream
+        args.stream = _stream(source)
         if source.numel() == 0:
             return result
         lib = _lib.lib()
