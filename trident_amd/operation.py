@@ -6,6 +6,7 @@ Triton launches of the reference (attention.py:109, 161, 170) become calls into
 libtrident_attn.so (include/tri_attn.h).
 """
 import ctypes
+import weakref
 from typing import Any
 
 import torch
@@ -102,8 +103,8 @@ def forget_mask_classes():
 def _mask_classes(mask: torch.Tensor, args):
     """Sets args.mask_classes for the mask already described in ``args``; returns the tensor to keep alive, or None
     where the library has no use for classes (nothing is launched then)."""
-    import weakref
-
+    if args.S % 128 != 0:  # (padded masks bring theirs along; the kernels use no other classes at such lengths)
+        return None
     lib = _lib.lib()
     size = lib.tri_attn_mask_classes_size(ctypes.byref(args))
     if size <= 0:
@@ -207,29 +208,14 @@ def _prepared_mask(mask, query):
             mask.prepared = _PreparedMask(mask.source, query)
             mask.source = None
         return mask.prepared
-    if query.dtype == torch.float32 or query.shape[2] % 128 == 0 or mask.dtype not in (torch.float32, query.dtype):
+    num_batches, num_heads, y_size, x_size = query.shape
+    if y_size % 128 == 0 or num_batches * num_heads * y_size * y_size * max(x_size, 32) < 1 << 29:
+        return None
+    if query.dtype == torch.float32 or mask.dtype not in (torch.float32, query.dtype):
         return None
     if mask.requires_grad and not _sums_mask_gradient(mask, query):
         return None
-    num_batches, num_heads, y_size, x_size = query.shape
-    if num_batches * num_heads * y_size * y_size * max(x_size, 32) < 1 << 29:
-        return None
     return _PreparedMask(mask.detach(), query)
-
-
-def _set_mask(args, mask, query, view=None):
-    """Describes ``mask`` (a tensor or a _BooleanMask) in a call's arguments; returns what to keep alive until it is enqueued.
-    ``view``: its [B,H,S,S] view, where the arguments hold that already."""
-    prepared = _prepared_mask(mask, query)
-    if prepared is not None:
-        prepared.describe(args)
-        return prepared
-    if view is None:
-        view = _expand_mask(mask.detach(), (*query.shape[:3], query.shape[2]))
-        args.mask = view.data_ptr()
-        args.mask_dtype = util.dtype(view.dtype)
-        args.mask_stride[:] = _strides_or_zero(view)
-    return view, _mask_classes(mask, args)
 
 
 def _expand_mask(mask: torch.Tensor, shape):
@@ -352,8 +338,16 @@ class Attention(torch.autograd.Function):
         num_batches, num_heads, y_size, x_size = query.shape
         output = torch.empty(query.shape, device=query.device, dtype=query.dtype)
         log2sum = torch.empty(num_batches, num_heads, y_size, device=query.device, dtype=torch.float32)
-        args = _make_args(query, key, value, output, log2sum, None, dropout_p, is_causal, softmax_scale, seed, offset)
-        _alive = _set_mask(args, mask, query) if mask is not None else None
+        # (a mask handed over as it is goes into the arguments with everything else: setting its fields one by one afterwards
+        # cost a small call 2 us of its 17)
+        prepared = _prepared_mask(mask, query) if mask is not None else None
+        mask_view = None
+        if mask is not None and prepared is None:
+            mask_view = _expand_mask(mask.detach(), (num_batches, num_heads, y_size, y_size))
+        args = _make_args(query, key, value, output, log2sum, mask_view, dropout_p, is_causal, softmax_scale, seed, offset)
+        if prepared is not None:
+            prepared.describe(args)
+        classes = _mask_classes(mask, args) if mask_view is not None else None  # (kept alive until the call is enqueued)
 
         util.push_trace("kernel.Attention.forward")
         _lib.check(lib.tri_attn_fwd(ctypes.byref(args)))
@@ -383,8 +377,10 @@ class Attention(torch.autograd.Function):
         # fp32 buffer of its shape that the kernels add to through strides of 0.
         grad_mask_buf = grad_mask_view = mask_view = None
         summed = want_grad_mask and _sums_mask_gradient(mask, query)
-        if want_grad_mask:
+        prepared = _prepared_mask(mask, query) if mask is not None and not want_grad_mask else None
+        if mask is not None and prepared is None:
             mask_view = _expand_mask(mask.detach(), full)
+        if want_grad_mask:
             shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
             if shape4 == full or summed:
                 grad_mask_buf = torch.empty(shape4, device=mask.device, dtype=mask.dtype)
@@ -392,12 +388,16 @@ class Attention(torch.autograd.Function):
 
         args = _make_args(query, key, value, output, log2sum, mask_view, dropout_p, is_causal, softmax_scale, seed, offset,
                           grad_output, grad_query, grad_key, grad_value, grad_mask_view, delta)
-        _alive = None
+        classes = None  # (kept alive until the call is enqueued, as ``prepared``)
         if summed:
             summed = lib.tri_attn_uses_matrix_cores(ctypes.byref(args), 3) == 1
             args.dmask = None
-        if mask is not None and (summed or not want_grad_mask):
-            _alive = _set_mask(args, mask, query, mask_view)
+            if summed:
+                prepared = _prepared_mask(mask, query)
+        if prepared is not None:
+            prepared.describe(args)
+        elif mask is not None and (summed or not want_grad_mask):
+            classes = _mask_classes(mask, args)
         elif want_grad_mask:
             if shape4 != full:
                 grad_mask_buf = torch.zeros(shape4, device=mask.device, dtype=torch.float32)
@@ -411,7 +411,7 @@ class Attention(torch.autograd.Function):
                     args.mask_stride[:] = _strides_or_zero(mask_view)
             # (the classes describe the mask tensor as the kernels see it: not when it was converted to fp32 above)
             if mask_view.dtype == mask.dtype:
-                _alive = _mask_classes(mask, args)
+                classes = _mask_classes(mask, args)
 
         # one call for the three backward launches (trident/operation/attention.py:161-199 launches the
         # delta pre-pass and the backward kernel): the library orders them, and where the dQ kernel can
