@@ -1070,8 +1070,9 @@ def test_mask_gradient_of_a_shared_mask(dtype, mask_dtype, B, H, S, D, shape, de
     assert torch.equal(first, second)
 
 
-def test_mask_gradient_of_a_shared_mask_with_dropout(device):
-    B, H, S, D = 3, 2, 200, 64
+@pytest.mark.parametrize("B,H,S,D", [(3, 2, 200, 64), (3, 20, 260, 64), (2, 20, 260, 32)])
+def test_mask_gradient_of_a_shared_mask_with_dropout(B, H, S, D, device):
+    """Pairs split over the waves; one row block per wave with staged rows (20 x 5 x 3 workgroups) and with direct loads."""
     q, k, v, d_o = _gen((B, H, S, D), 6200, torch.bfloat16)
     mask = 0.5 * torch.randn(1, H, S, S, generator=torch.Generator().manual_seed(1))
     from trident_amd.operation import Attention

@@ -5,11 +5,16 @@
 // no atomic, no zero fill, a fixed order of summation, and the tile of the mask itself is read once for all pairs. The price is
 // S and dP once more (2 of the pass's 7 products), where the dQ pass, which has them, would send every dS to memory by itself:
 // bf16 B=8 H=12 S=512 D=64, bias [1,H,S,S]: the dQ pass with atomic adds took 0.61 ms, bound by the 25 M adds; without them
-// it takes 0.023 ms and this kernel 0.062, bound by its loads (lanes own rows: a load touches 32 cache lines).
+// it takes 0.023 ms and this kernel 0.039.
 //
 // A wave takes 32 rows x 64 keys: the K and V rows are the A operands, the Q and dO rows the B operands, so that lane l32 owns
-// a row with its lse and delta, and the accumulators (8 keys groups of 4) leave in row pieces. Operands come straight from
-// memory, 16 bytes per lane; the rows of a (batch, head) are read by S / 32 workgroups of one XCD and sit in its L2.
+// a row with its lse and delta, and the accumulators (8 keys groups of 4) leave in row pieces. The rows of a (batch, head) are
+// read by S / 32 workgroups of one XCD and sit in its L2.
+// D = 64: a workgroup stages the rows of a pair in LDS, in whole lines and K and V once for its four waves, with the next pair's
+// on their way in registers. Straight from memory, 16 bytes per lane, a load touches 32 cache lines and bounds the kernel: the
+// case above 0.059 -> 0.039 ms, B=2 H=16 S=2048 0.346 -> 0.278 ms. The other head sizes keep the direct loads: at D = 128 the
+// staged rows leave one workgroup per CU (0.511 -> 0.645 ms staged), at D = 32 the exponentials weigh more and the barriers cost
+// what the loads save (0.203 -> 0.228 ms).
 // SPLIT: too few tiles to fill the chip. The four waves of a workgroup then share one tile, take every fourth pair each, and
 // their sums meet in LDS; otherwise they are four row blocks of one key tile.
 #include "launch.hpp"
@@ -23,7 +28,12 @@ constexpr int kKeys = 64;
 template <typename T, int D, bool DROPOUT, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void mfma_dmask_kernel(const KParams p, int units, int per_xcd, bool by_fours) {
     constexpr int KK = D / 16;
-    __shared__ __attribute__((aligned(16))) float sums[SPLIT ? 3 * 32 * 64 : 1];
+    // staged rows of a pair: 64 of K, 64 of V, 128 of Q, 128 of dO, each 16 bytes longer than its elements (a fragment read's
+    // lanes then fall on different banks at every head size)
+    constexpr int kPitch = 2 * D + 16, kStaged = 2 * kKeys + 2 * 128;
+    constexpr bool kStage = !SPLIT && D == 64;
+    __shared__ __attribute__((aligned(16))) char smem[SPLIT ? 3 * 32 * 64 * 4 : kStage ? kStaged * kPitch : 16];
+    float* const sums = reinterpret_cast<float*>(smem);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     // consecutive tiles of one mask on one XCD
@@ -41,7 +51,7 @@ __global__ __launch_bounds__(256, 2) void mfma_dmask_kernel(const KParams p, int
     const int qrow = wrow0 + l32;
     const bool row_ok = qrow < p.S;
     const int qrow_ld = min(qrow, p.S - 1);
-    if (!SPLIT && wrow0 >= p.S) return;  // (a wave without a single row; no barrier in this variant)
+    if (!SPLIT && !kStage && wrow0 >= p.S) return;  // (a wave without a single row; no barrier in this variant)
 
     // mask values of this lane's row (log2 domain), the same for every pair; -inf for keys that do not exist
     float mk[32];
@@ -58,50 +68,117 @@ __global__ __launch_bounds__(256, 2) void mfma_dmask_kernel(const KParams p, int
 #pragma unroll
     for (int i = 0; i < 32; ++i) acc[i] = 0.f;
 
-    for (int pair = SPLIT ? wave : 0; pair < sum_b * sum_h; pair += SPLIT ? 4 : 1) {
-        const int b = mask_b + pair / sum_h, hd = mask_h + pair % sum_h;
-        const int64_t bh = static_cast<int64_t>(b) * p.H + hd;
-        const T* qp = static_cast<const T*>(p.q) + b * p.qs[0] + hd * p.qs[1] + qrow_ld * p.qs[2] + 8 * h;
-        const T* gp = static_cast<const T*>(p.d_o) + b * p.dos[0] + hd * p.dos[1] + qrow_ld * p.dos[2] + 8 * h;
-        const T* kp = static_cast<const T*>(p.k) + b * p.ks[0] + hd * p.ks[1] + 8 * h;
-        const T* vp = static_cast<const T*>(p.v) + b * p.vs[0] + hd * p.vs[1] + 8 * h;
-        const float lse = p.lse[bh * p.S + qrow_ld];
-        const float dlt = p.delta[bh * p.S + qrow_ld];
-        u32x4 qf[KK], gf[KK];
+    // dS of 32 rows x 32 keys of one pair, added to the accumulators of key block kb
+    const auto add = [&](int kb, int64_t bh, float lse, float dlt, const u32x4(&kf)[KK], const u32x4(&vf)[KK], const u32x4(&qf)[KK],
+                         const u32x4(&gf)[KK]) {
+        f32x16 s = zero16(), dp = zero16();
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            qf[kk] = *reinterpret_cast<const u32x4*>(qp + 16 * kk);
-            gf[kk] = *reinterpret_cast<const u32x4*>(gp + 16 * kk);
+            s = Mma<T>::run(kf[kk], qf[kk], s);
+            dp = Mma<T>::run(vf[kk], gf[kk], dp);
+        }
+        if constexpr (DROPOUT) {
+            const Philox4 mine = dropout_block(p, static_cast<uint32_t>(bh), qrow >> 2, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
+            uint32_t w[4];
+            quad_row_words(mine, lane, w);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int bb = 0; bb < 4; ++bb) {
+                    const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
+                    dp[4 * g + bb] = keep ? dp[4 * g + bb] * p.zscale : 0.f;
+                }
         }
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            const int64_t key = kb ? key_ld1 : key_ld0;
-            u32x4 kf[KK], vf[KK];
+        for (int i = 0; i < 16; ++i) acc[16 * kb + i] += fast_exp2(fmaf(s[i], p.scale_log2, mk[16 * kb + i]) - lse) * (dp[i] - dlt);
+    };
+
+    const int pairs = sum_b * sum_h;
+    if constexpr (!kStage) {
+        for (int pair = SPLIT ? wave : 0; pair < pairs; pair += SPLIT ? 4 : 1) {
+            const int b = mask_b + pair / sum_h, hd = mask_h + pair % sum_h;
+            const int64_t bh = static_cast<int64_t>(b) * p.H + hd;
+            const T* qp = static_cast<const T*>(p.q) + b * p.qs[0] + hd * p.qs[1] + qrow_ld * p.qs[2] + 8 * h;
+            const T* gp = static_cast<const T*>(p.d_o) + b * p.dos[0] + hd * p.dos[1] + qrow_ld * p.dos[2] + 8 * h;
+            const T* kp = static_cast<const T*>(p.k) + b * p.ks[0] + hd * p.ks[1] + 8 * h;
+            const T* vp = static_cast<const T*>(p.v) + b * p.vs[0] + hd * p.vs[1] + 8 * h;
+            const float lse = p.lse[bh * p.S + qrow_ld];
+            const float dlt = p.delta[bh * p.S + qrow_ld];
+            u32x4 qf[KK], gf[KK];
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
-                kf[kk] = *reinterpret_cast<const u32x4*>(kp + key * p.ks[2] + 16 * kk);
-                vf[kk] = *reinterpret_cast<const u32x4*>(vp + key * p.vs[2] + 16 * kk);
+                qf[kk] = *reinterpret_cast<const u32x4*>(qp + 16 * kk);
+                gf[kk] = *reinterpret_cast<const u32x4*>(gp + 16 * kk);
             }
-            f32x16 s = zero16(), dp = zero16();
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                const int64_t key = kb ? key_ld1 : key_ld0;
+                u32x4 kf[KK], vf[KK];
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) {
+                    kf[kk] = *reinterpret_cast<const u32x4*>(kp + key * p.ks[2] + 16 * kk);
+                    vf[kk] = *reinterpret_cast<const u32x4*>(vp + key * p.vs[2] + 16 * kk);
+                }
+                add(kb, bh, lse, dlt, kf, vf, qf, gf);
+            }
+        }
+    } else {
+        // Thread t moves the 16-byte pieces t, t + 256, ... of the pair's rows: consecutive lanes, consecutive addresses. The
+        // next pair's pieces are on their way while this one is multiplied.
+        constexpr int kPerRow = D / 8, kStep = 256 / kPerRow, kPieces = kStaged / kStep;
+        const int piece_row = static_cast<int>(threadIdx.x) / kPerRow, piece_col = static_cast<int>(threadIdx.x) % kPerRow * 8;
+        u32x4 piece[kPieces];
+        float lse_next, dlt_next;
+        const auto fetch = [&](int pair) {
+            const int b = mask_b + pair / sum_h, hd = mask_h + pair % sum_h;
+            const int64_t bh = static_cast<int64_t>(b) * p.H + hd;
+            const T* qp = static_cast<const T*>(p.q) + b * p.qs[0] + hd * p.qs[1] + piece_col;
+            const T* gp = static_cast<const T*>(p.d_o) + b * p.dos[0] + hd * p.dos[1] + piece_col;
+            const T* kp = static_cast<const T*>(p.k) + b * p.ks[0] + hd * p.ks[1] + piece_col;
+            const T* vp = static_cast<const T*>(p.v) + b * p.vs[0] + hd * p.vs[1] + piece_col;
+            int row0 = piece_row;
+            asm volatile("" : "+v"(row0));  // (row offsets are computed again for each pair: kept, they spill at D = 64)
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                const int r = row0 + i * kStep;  // (rows beyond the sequence: its last one, masked or not stored)
+                const T* from = r < kKeys           ? kp + min(t0 + r, p.S - 1) * p.ks[2]
+                                : r < 2 * kKeys       ? vp + min(t0 + r - kKeys, p.S - 1) * p.vs[2]
+                                : r < 2 * kKeys + 128 ? qp + min(rt * 128 + r - 2 * kKeys, p.S - 1) * p.qs[2]
+                                                      : gp + min(rt * 128 + r - 2 * kKeys - 128, p.S - 1) * p.dos[2];
+                piece[i] = *reinterpret_cast<const u32x4*>(from);
+            }
+            lse_next = p.lse[bh * p.S + qrow_ld];
+            dlt_next = p.delta[bh * p.S + qrow_ld];
+        };
+        const auto fragment = [&](int row, int kk) {
+            return *reinterpret_cast<const u32x4*>(smem + (row + l32) * kPitch + 32 * kk + 16 * h);
+        };
+        fetch(0);
+        for (int pair = 0; pair < pairs; ++pair) {
+            const int64_t bh = static_cast<int64_t>(mask_b + pair / sum_h) * p.H + mask_h + pair % sum_h;
+            const float lse = lse_next, dlt = dlt_next;
+            lds_barrier();  // (the fragments of the pair before have been read)
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(smem + (piece_row + i * kStep) * kPitch + 2 * piece_col) = piece[i];
+            lds_barrier();
+            if (pair + 1 < pairs) fetch(pair + 1);
+            u32x4 qf[KK], gf[KK];
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
-                s = Mma<T>::run(kf[kk], qf[kk], s);
-                dp = Mma<T>::run(vf[kk], gf[kk], dp);
-            }
-            if constexpr (DROPOUT) {
-                const Philox4 mine = dropout_block(p, static_cast<uint32_t>(bh), qrow >> 2, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
-                uint32_t w[4];
-                quad_row_words(mine, lane, w);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-#pragma unroll
-                    for (int bb = 0; bb < 4; ++bb) {
-                        const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
-                        dp[4 * g + bb] = keep ? dp[4 * g + bb] * p.zscale : 0.f;
-                    }
+                qf[kk] = fragment(2 * kKeys + 32 * wave, kk);
+                gf[kk] = fragment(2 * kKeys + 128 + 32 * wave, kk);
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[16 * kb + i] += fast_exp2(fmaf(s[i], p.scale_log2, mk[16 * kb + i]) - lse) * (dp[i] - dlt);
+            for (int kb = 0; kb < 2; ++kb) {
+                u32x4 kf[KK], vf[KK];
+#pragma unroll
+                for (int kk = 0; kk < KK; ++kk) {
+                    kf[kk] = fragment(32 * kb, kk);
+                    vf[kk] = fragment(kKeys + 32 * kb, kk);
+                }
+                add(kb, bh, lse, dlt, kf, vf, qf, gf);
+                __builtin_amdgcn_sched_barrier(0);  // (one key block's fragments at a time)
+            }
         }
     }
     if constexpr (SPLIT) {
@@ -139,7 +216,7 @@ int launch_dmask_t(const KParams& p, hipStream_t stream) {
     const int64_t masks = (p.dms[0] == 0 ? int64_t{1} : p.B) * (p.dms[1] == 0 ? 1 : p.H);
     const int64_t key_tiles = (p.S + kKeys - 1) / kKeys;
     // one key tile x 128 rows per workgroup where that gives every compute unit one, else 32 rows with the pairs split (with
-    // 384 such workgroups, the case above, split ones took 0.065 ms against 0.062: the loads are the limit, not their latency)
+    // 384 such workgroups, the case above, split ones took 0.065 ms against 0.062 with direct loads in both, 0.039 staged)
     const bool split = splits_pairs(p, masks);
     const int64_t units = masks * key_tiles * (split ? (p.S + 31) / 32 : (p.S + 127) / 128);
     if (units > 2147483647LL / 8) return TRI_ATTN_ESHAPE;
