@@ -1084,3 +1084,38 @@ def test_mask_gradient_of_a_shared_mask_with_dropout(B, H, S, D, device):
     kw = dict(mask=mask, dropout_p=0.2, is_causal=False, scale=scale, seed=9, offset=4)
     _, _, _, dm_r, _ = parity.oracle_backward(q, k, v, d_o, want_dmask=True, o=o, **kw)
     parity.close(dm, dm_r, torch.bfloat16, "dropout shared dMask")
+
+
+# ------------------------------------------------------------------ small gradients
+@pytest.mark.parametrize("kind", ["plain", "causal", "keys"])
+@pytest.mark.parametrize("S", [160, 511, 512])
+@pytest.mark.parametrize("grad_size", [1e-3, 1e-4])
+def test_small_fp16_gradients_keep_their_precision(grad_size, S, kind, device):
+    """dK of the phased kernel at D = 128: delta reaches the matrix pipe in fp16 terms, which have to hold it to fp32 precision
+    also where it is as small as fp16's subnormal numbers (peaked rows: probabilities near 1 carry its error straight to dK).
+    Bound: the roundings of dS to fp16 (half a unit in the last place, 2^-25 in the subnormal range), added as independent
+    ones over the rows, and that of the stored dK."""
+    from trident_amd.operation import Attention, _BooleanMask
+    D, dtype = 128, torch.float16
+    q, k, v, d_o = _gen((1, 2, S, D), 7000 + S, torch.float32)
+    q, k, v, d_o = (3 * q).to(dtype), k.to(dtype), v.to(dtype), (grad_size * d_o).to(dtype)
+    scale = 1.0 / math.sqrt(D)
+    hidden = torch.zeros(1, 1, S, S, dtype=torch.bool)
+    given = None
+    if kind == "causal":
+        hidden = torch.ones(S, S, dtype=torch.bool).triu(1).view(1, 1, S, S)
+    elif kind == "keys":
+        hidden = (torch.arange(S) >= S - 37).view(1, 1, 1, S)
+        given = _BooleanMask(~hidden.to(device))
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    o, lse = Attention._forward(tq, tk, tv, given, 0.0, kind == "causal", scale, 0, 0)
+    _, dk, _, _ = Attention._backward(tdo, tq, tk, tv, o, lse, given, scale, 0.0, kind == "causal", 0, 0, False)
+    q64, k64, v64, do64, o64 = [x.double().cpu() for x in (q, k, v, d_o, o)]
+    p = torch.softmax((q64 @ k64.transpose(-1, -2) * scale).masked_fill(hidden, -math.inf), -1)
+    ds = p * (do64 @ v64.transpose(-1, -2) - (do64 * o64).sum(-1, keepdim=True))
+    want = scale * ds.transpose(-1, -2) @ q64
+    rounding = torch.clamp(ds.abs() * 2.0 ** -11, min=2.0 ** -25) * (ds != 0)
+    bound = (scale ** 2 * (rounding ** 2).transpose(-1, -2) @ q64 ** 2).sum().sqrt()
+    bound = bound + torch.clamp(want.abs() * 2.0 ** -11, min=2.0 ** -25).norm()
+    error = (dk.double().cpu() - want).norm()
+    assert error <= bound, f"{kind}: {error / want.norm():.2e} of dK's norm, rounding explains {bound / want.norm():.2e}"

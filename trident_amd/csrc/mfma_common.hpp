@@ -81,18 +81,28 @@ __device__ __forceinline__ u32x4 pack8(const float* x) {
     return r;
 }
 
-// x as three 16-bit terms (K-slots 0-2 of an operand, the rest zero): their sum restores x to fp32 precision.
+// x as three 16-bit terms (K-slots 0-2 of an operand, the rest zero) that restore it to fp32 precision as
+// t0 + t1 / kUp + t2 / kUp^2: what is left after each rounding is scaled up before the next one. bf16 has fp32's exponents
+// and needs no scaling; in fp16, whose smallest step is 6e-8 however small x is, it keeps x to 1.4e-14 (a half step of
+// t0 is at most 2^-11 of its range, so that scaled by 2^11 it fits again).
 template <typename T>
-__device__ __forceinline__ u32x4 split3(float x) {
-    const float a = static_cast<float>(static_cast<T>(x));
-    const float r1 = x - a;
-    const float b = static_cast<float>(static_cast<T>(r1));
-    u32x4 r;
-    r.x = Mma<T>::pack2(a, b);
-    r.y = Mma<T>::pack2(r1 - b, 0.f);
-    r.z = r.w = 0;
-    return r;
-}
+struct Split3 {
+    static constexpr float kUp = std::is_same<T, f16_t>::value ? 2048.f : 1.f;
+    static __device__ __forceinline__ u32x4 terms(float x) {
+        const float a = static_cast<float>(static_cast<T>(x));
+        const float r1 = (x - a) * kUp;
+        const float b = static_cast<float>(static_cast<T>(r1));
+        u32x4 r;
+        r.x = Mma<T>::pack2(a, b);
+        r.y = Mma<T>::pack2((r1 - b) * kUp, 0.f);
+        r.z = r.w = 0;
+        return r;
+    }
+    // the other operand's three K-slots: what the terms are multiplied by, `unit` for x as a whole
+    static __device__ __forceinline__ u32x4 units(float unit) {
+        return u32x4{Mma<T>::pack2(unit, unit / kUp), Mma<T>::pack2(unit / (kUp * kUp), 0.f), 0, 0};
+    }
+};
 
 __device__ __forceinline__ f32x16 zero16() {
     f32x16 z;

@@ -953,7 +953,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     // whether this pair has anything in block r (under the causal mask: rows at or below its first key)
     auto block_on = [&](int r) { return r >= 0 && r < n_blocks && (!CAUSAL || r >= kb); };
 
-    constexpr float kFoldUnit = 256.f;  // the constant the split terms multiply (keeps f16 terms in range)
+    constexpr float kFoldUnit = 256.f;  // the constant the first of the split terms multiplies (keeps f16 terms in range)
     const float neg_inv_c = -1.f / c;
     f32x16 sc_s, sc_dp;  // S - lse / c and dP - delta of this member's next block
     u32x4 ring[kRing];
@@ -995,10 +995,9 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
             }
             if (n == 2 * kAccSteps) {
                 const u32x4 zero4 = {0, 0, 0, 0};
-                const u32x4 al = split3<T>(row_lse * neg_inv_c * (1.f / kFoldUnit));
-                const u32x4 ad = split3<T>(row_delta * (-1.f / kFoldUnit));
-                const uint32_t u2 = Mma<T>::pack2(kFoldUnit, kFoldUnit), u1 = Mma<T>::pack2(kFoldUnit, 0.f);
-                const u32x4 units = h == 0 ? u32x4{u2, u1, 0, 0} : zero4;
+                const u32x4 al = Split3<T>::terms(row_lse * neg_inv_c * (1.f / kFoldUnit));
+                const u32x4 ad = Split3<T>::terms(row_delta * (-1.f / kFoldUnit));
+                const u32x4 units = h == 0 ? Split3<T>::units(kFoldUnit) : zero4;
                 s = Mma<T>::run(h == 0 ? al : zero4, units, s);
                 if constexpr (!DROPOUT) dp = Mma<T>::run(h == 0 ? ad : zero4, units, dp);
             }
