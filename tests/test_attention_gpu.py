@@ -1049,6 +1049,63 @@ def test_prepared_masks_hold_the_source(source, S, device):
             assert torch.equal(classes.cpu().view(dims).expand(2, 3, cb, cb).long(), expected)
 
 
+@pytest.mark.parametrize("kind", ["bool keys", "f32", "16 bit"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 65, 16), (torch.float16, 333, 32), (torch.float16, 100, 64), (torch.bfloat16, 333, 64),
+                                       (torch.bfloat16, 65, 128), (torch.float16, 333, 128)])
+def test_padded_masks_sum_unrounded_probabilities(dtype, S, D, kind, device, monkeypatch):
+    """The softmax denominator at padded lengths is an fp32 sum of fp32 probabilities, not of those rounded for the product with
+    V: one key has score t, the others 0, with t chosen so that exp(-t) is as far from a 16-bit number as can be; a sum of
+    the rounded ones would be off by half a unit of the 16-bit type. Bound: one fp32 rounding per summand and 16 for the
+    exponential and its argument, in the log2 domain."""
+    from trident_amd import operation
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    scale = 1.0 / math.sqrt(D)
+    a = (torch.linspace(0.25, 2.0, 400) / scale).to(dtype).double()
+    p = torch.exp(-a * scale)
+    off = (p.to(dtype).double() - p).abs() / p
+    a, t = a[off.argmax()].item(), a[off.argmax()].item() * scale
+    q, k = torch.zeros(1, 2, S, D, dtype=dtype), torch.zeros(1, 2, S, D, dtype=dtype)
+    q[..., 0], k[..., 0, 0] = 1, a
+    v = torch.ones(1, 2, S, D, dtype=dtype)
+    keep = torch.arange(S) < S - 5
+    if kind == "bool keys":
+        given = operation._BooleanMask(keep.view(1, 1, 1, S).to(device))
+    else:
+        given = torch.zeros(1, 1, S, S, dtype=torch.float32 if kind == "f32" else dtype).masked_fill(~keep, -math.inf).to(device)
+    _, lse = operation.Attention._forward(q.to(device), k.to(device), v.to(device), given, 0.0, False, scale, 0, 0)
+    want = math.log2(math.exp(t) + S - 6)
+    assert (lse.double() - want).abs().max() <= (S + 16) * 2.0 ** -24 / math.log(2.0)
+
+
+@pytest.mark.parametrize("kind", ["bool keys", "f32", "16 bit"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 65, 16), (torch.float16, 333, 32), (torch.float16, 100, 64), (torch.bfloat16, 333, 64),
+                                       (torch.bfloat16, 65, 128), (torch.float16, 333, 128)])
+def test_padded_masks_keep_the_largest_probability_exact(dtype, S, D, kind, device, monkeypatch):
+    """Two keys take part, the first of the sequence with score 0 and V = -1 and one of the second tile with score t and V = 1:
+    the result is (1 - exp(-t)) / (1 + exp(-t)) up to its own rounding where the second key's probability is held as exactly
+    1, and off by the rounding of exp(t) where it is held against the first tile's maximum (t is chosen where that shows most)."""
+    from trident_amd import operation
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    scale = 1.0 / math.sqrt(D)
+    a = (torch.linspace(0.05, 0.3, 1000) / scale).to(dtype).double()
+    e = torch.exp(a * scale)
+    rounded = e.to(dtype).double()
+    off = ((rounded - 1) / (rounded + 1) - (e - 1) / (e + 1)).abs()
+    a, e = a[off.argmax()].item(), e[off.argmax()].item()
+    exact = (e - 1) / (e + 1)
+    allowed = torch.finfo(dtype).eps / 2 * exact + 2.0 ** -20
+    assert off.max() > 2 * allowed
+    q, k, v = (torch.zeros(1, 2, S, D, dtype=dtype) for _ in range(3))
+    q[..., 0], k[..., 64, 0], v[..., 0, :], v[..., 64, :] = 1, a, -1, 1
+    keep = (torch.arange(S) == 0) | (torch.arange(S) == 64)
+    if kind == "bool keys":
+        given = operation._BooleanMask(keep.view(1, 1, 1, S).to(device))
+    else:
+        given = torch.zeros(1, 1, S, S, dtype=torch.float32 if kind == "f32" else dtype).masked_fill(~keep, -math.inf).to(device)
+    o, _ = operation.Attention._forward(q.to(device), k.to(device), v.to(device), given, 0.0, False, scale, 0, 0)
+    assert (o.double() - exact).abs().max() <= allowed
+
+
 # ------------------------------------------------------------------ mask gradients summed over batches and heads
 @pytest.mark.parametrize("shape", ["1HSS", "B1SS", "11SS"])
 @pytest.mark.parametrize("dtype,mask_dtype,B,H,S,D", [(torch.bfloat16, torch.bfloat16, 3, 2, 1, 64), (torch.float16, torch.float32, 2, 3, 31, 16),

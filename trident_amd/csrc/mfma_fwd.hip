@@ -185,13 +185,15 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
         }
         const int i = idx % kPerOperand;
         if (RAGGED && (t + 1) * kBN > p.S) {  // the sequence ends inside this tile: clamped rows, offsets from the tile's first row
+            int l = lane;
+            if constexpr (D == 128) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
             const int last = p.S - 1 - t * kBN;
             if (idx < kPerOperand)
                 lds_direct_load16(kbase + static_cast<int64_t>(t) * kBN * krow_bytes,
-                                  Tile::src_off_clamped(wave + i * NW, lane, krow_bytes, last), stage + i * NW * 1024);
+                                  Tile::src_off_clamped(wave + i * NW, l, krow_bytes, last), stage + i * NW * 1024);
             else
                 lds_direct_load16(vbase + static_cast<int64_t>(t) * kBN * vrow_bytes,
-                                  Tile::src_off_clamped(wave + i * NW, lane, vrow_bytes, last), stage + kVRing + i * NW * 1024);
+                                  Tile::src_off_clamped(wave + i * NW, l, vrow_bytes, last), stage + kVRing + i * NW * 1024);
         } else if (idx < kPerOperand)
             lds_direct_load16(kbase + (static_cast<int64_t>(t) * kBN + i * kRowStep) * krow_bytes, koff, stage + i * NW * 1024);
         else
@@ -276,6 +278,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             // (block 0 precedes tile 0, which has landed)
             if (!mask_is_zero(t)) {
                 if (!first) wait_loads(false, tile_in_flight, v_in_flight);
+                int l32 = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
+                if constexpr (RAGGED && D == 128) asm volatile("" : "+v"(l32), "+v"(h));  // (addresses made here, not kept across the loop)
 #pragma unroll
                 for (int g = 0; g < 8; ++g) {  // keys 32 (g / 4) + 8 (g % 4) + 4 h .. + 3 of this lane's row
                     if constexpr (MASK == kMaskF32) {
@@ -304,7 +308,10 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     // Without dropout the softmax denominator is accumulated by the matrix pipe as well: an all-ones
     // A operand makes every row of the product the column sums of P^T, i.e. each lane holds (16
     // times) the sum over ALL keys of its query row, taken from the same rounded P that multiplies
-    // V. With dropout the sum has to be taken before elements are dropped, on the vector ALU.
+    // V. With dropout the sum has to be taken before elements are dropped, on the vector ALU. Padded masks (RAGGED) take
+    // it there too, from the probabilities before they are rounded: those problems came from kernels that did, and the
+    // backward starts from this sum (fp16, S = 511, peaked rows: error of dV 3.06e-4 -> 2.89e-4 of its norm).
+    constexpr bool kVectorSum = DROPOUT || (RAGGED && MASK != kNoMask);
     // Without dropout the exponentials of the second key block (and their conversion) are deferred into
     // the matrix phase, one or two per MFMA of the first key block's P V steps: that phase has issue slots
     // to spare, the softmax phase is the one the partner waits for.
@@ -344,7 +351,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             if (s < pv) {
                 oacc[s % DB] = Mma<T>::run(ring[s % kRing], pb[s / DB], oacc[s % DB]);
                 // row sums of P (every accumulator row gets the same sum over the 16 keys)
-                if (!DROPOUT && s % DB == DB - 1) lacc = Mma<T>::run(ones, pb[s / DB], lacc);
+                if (!kVectorSum && s % DB == DB - 1) lacc = Mma<T>::run(ones, pb[s / DB], lacc);
             } else {
                 const int s2 = s - pv;
                 sc[s2 / KK] = Mma<T>::run(ring[s % kRing], qf[s2 % KK], sc[s2 / KK]);
@@ -367,6 +374,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                         if (e * ne / 8 == ls) {
                             float& v = xd[8 * (g - 2) + e];
                             v = fast_exp2(fmaf(v, c, -m_def));
+                            if constexpr (kVectorSum) l += v;
                         }
                     if (ls == pack_step) pb[g] = pack8<T>(&xd[8 * (g - 2)]);
                 }
@@ -454,11 +462,10 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 }
             }
             if (RAGGED && !CAUSAL && t0 + kBN > p.S) {  // keys that do not exist (under the causal mask no existing row sees them)
+                int left = p.S - t0 - 4 * h;
+                asm volatile("" : "+v"(left));  // (made here, not kept in registers across the loop)
 #pragma unroll
-                for (int e = 0; e < 32; ++e) {
-                    const int key = t0 + 32 * (e >> 4) + c_row(e & 15, h);
-                    x[e] = key < p.S ? x[e] : -INFINITY;
-                }
+                for (int e = 0; e < 32; ++e) x[e] = 32 * (e >> 4) + c_row(e & 15, 0) < left ? x[e] : -INFINITY;
             }
             // two chains (a dependent maximum waits out the ALU latency) of three-operand maxima, written out: through
             // fmaxf the compiler first canonicalises the operands of each chain (a maximum of a value with itself)
@@ -473,8 +480,11 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             // Lazy rescaling: m is the reference exponent of l and of the O accumulators, not
             // necessarily the running maximum. It is only moved (and O rescaled) when some row of
             // the wave outgrew it by more than 2^kTau; until then probabilities may exceed 1 by
-            // that factor, which fp32 sums and 16-bit P hold without loss.
-            if (__builtin_amdgcn_ballot_w64(mx > m + kTau) != 0) {
+            // that factor, which fp32 sums and 16-bit P hold without loss. Padded masks (RAGGED) follow the maximum itself, as
+            // the kernels they came from did: a row's largest probability is then exactly 1 and only the smaller ones are
+            // rounded (fp16, S = 511, peaked rows: error of O 2.78e-4 -> 2.19e-4 of its norm).
+            constexpr float kSlack = RAGGED && MASK != kNoMask ? 0.f : kTau;
+            if (__builtin_amdgcn_ballot_w64(mx > m + kSlack) != 0) {
                 const float m_new = fmaxf(m, mx);
                 m_use = m_new == -INFINITY ? 0.f : m_new;
                 const float alpha = fast_exp2(m - m_use);
@@ -484,7 +494,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 for (int db = 0; db < DB; ++db)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) oacc[db][i] *= alpha;
-                if constexpr (!DROPOUT) {
+                if constexpr (!kVectorSum) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) lacc[i] *= alpha;
                 }
@@ -499,6 +509,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
 #pragma unroll
                 for (int e = 8 * ks; e < 8 * ks + 8; ++e) {
                     x[e] = fast_exp2(fmaf(x[e], c, -m_use));
+                    if constexpr (kVectorSum && !DROPOUT) l += x[e];
                 }
                 if constexpr (!DROPOUT) pb[ks] = pack8<T>(&x[8 * ks]);
                 if (ks < 2 && issued_v) issue_slice(j + dist, 2 + ks, issued, issued_v);
@@ -604,7 +615,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     }
     if (kPingPong && group == 0) lds_barrier();  // group 1 is still in its last matrix phase
 
-    l = DROPOUT ? sum_xor32(l) : lacc[0];
+    l = kVectorSum ? sum_xor32(l) : lacc[0];
     const float inv = (DROPOUT ? p.zscale : 1.f) / l;
     // every wave is out of the loop: the ring is free (for the waves' private transposition patches, and for
     // the first tiles of the next item)

@@ -189,6 +189,10 @@ class _PreparedMask:
             args.mask_classes = self.classes.data_ptr()
 
 
+# Scores times head size from which an additive mask at a ragged length is copied into padded rows (_prepared_mask).
+_PADS_FROM = 1 << 29
+
+
 def _sums_mask_gradient(mask, query):
     """Whether the gradient of ``mask`` is summed over batches or heads, with rows and keys of its own (16-bit problems)."""
     shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
@@ -201,7 +205,7 @@ def _prepared_mask(mask, query):
     ones are copied into padded rows for 16-bit problems at lengths that are no multiple of 128, whose kernels fetch mask rows
     in 16-byte pieces up to the end of a 64-key tile: one more pass over the mask (at the copy rate) in each direction against
     kernels that read masks element by element (bf16, dense fp32 mask, forward + backward: B=16 H=12 S=777 D=64 2.22 -> 0.39 ms,
-    S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below 2^29 scores times head size the launches and their arguments cost a call more than
+    S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below _PADS_FROM scores times head size the launches and their arguments cost a call more than
     the kernels save (S=100 0.15 -> 0.21 ms). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it."""
     if isinstance(mask, _BooleanMask):
         if mask.prepared is None:
@@ -209,7 +213,7 @@ def _prepared_mask(mask, query):
             mask.source = None
         return mask.prepared
     num_batches, num_heads, y_size, x_size = query.shape
-    if y_size % 128 == 0 or num_batches * num_heads * y_size * y_size * max(x_size, 32) < 1 << 29:
+    if y_size % 128 == 0 or num_batches * num_heads * y_size * y_size * max(x_size, 32) < _PADS_FROM:
         return None
     if query.dtype == torch.float32 or mask.dtype not in (torch.float32, query.dtype):
         return None
