@@ -63,6 +63,10 @@ enum {
  * matrix-core kernels take masked lengths that are no multiple of 128 only so; tri_attn_prepare_mask makes such a mask. */
 #define TRI_ATTN_MASK_PADDED 0x100
 
+/* Or-ed to mask_dtype: every value of the mask is 0 or -inf (what tri_attn_prepare_mask makes of a boolean mask). Only a hint:
+ * kernels that work with differences of large terms are kept for such masks. */
+#define TRI_ATTN_MASK_BINARY 0x200
+
 enum {
     TRI_ATTN_OK = 0,
     TRI_ATTN_ENULL = -1,      /* a required pointer is NULL */
@@ -82,7 +86,7 @@ typedef struct TriAttnArgs {
     int32_t dtype;             /* TRI_ATTN_F32 / F16 / BF16: element type of q,k,v,o,d_o,dq,dk,dv */
     int32_t B, H, S, D;        /* y_size = S, x_size = D in the reference's naming */
     int32_t is_causal;
-    int32_t mask_dtype;        /* element type of mask and dmask, plus TRI_ATTN_MASK_PADDED where it holds */
+    int32_t mask_dtype;        /* element type of mask and dmask, plus TRI_ATTN_MASK_PADDED / _BINARY where they hold */
     float softmax_scale;
     float dropout_p;
     uint64_t seed;             /* Philox key */

@@ -1106,6 +1106,35 @@ def test_padded_masks_keep_the_largest_probability_exact(dtype, S, D, kind, devi
     assert (o.double() - exact).abs().max() <= allowed
 
 
+@pytest.mark.parametrize("dtype,mask_dtype,S,D,value", [(torch.bfloat16, torch.float32, 65, 16, -1e38), (torch.float16, torch.float32, 200, 64, -2e38),
+                                                        (torch.bfloat16, torch.bfloat16, 200, 64, -1.2e38), (torch.bfloat16, torch.float32, 333, 128, -5e37),
+                                                        (torch.bfloat16, torch.bfloat16, 300, 128, -2e38), (torch.float16, torch.float32, 300, 128, -1e9)])
+@pytest.mark.parametrize("shape", ["rows", "keys"])
+def test_padded_masks_of_large_finite_values(dtype, mask_dtype, S, D, value, shape, device, monkeypatch):
+    """Rows (and with a key-padding mask a whole sequence) whose keys all carry the same large finite value weigh them alike,
+    as softmax does; the gradients are those of the kernels that take unpadded masks. (Of a row like that they hold no more
+    than the lse's last digit does, but they are finite.)"""
+    from trident_amd import operation
+    q, k, v, d_o = [x.to(device) for x in _gen((2, 2, S, D), 5600 + S, dtype)]
+    mask = torch.zeros(2, 1, S if shape == "rows" else 1, S, dtype=mask_dtype, device=device)
+    if shape == "rows":
+        mask[1, :, 3:70] = value
+    else:
+        mask[1] = value
+    scale = 1.0 / math.sqrt(D)
+    results = []
+    for pads_from in (0, 1 << 62):
+        monkeypatch.setattr(operation, "_PADS_FROM", pads_from)
+        o, lse = operation.Attention._forward(q, k, v, mask, 0.0, False, scale, 0, 0)
+        results.append((o, *operation.Attention._backward(d_o, q, k, v, o, lse, mask, scale, 0.0, False, 0, 0, False)[:3]))
+    alike = results[0][0][1, :, 3:70].float()
+    assert (alike - v[1].float().mean(1, keepdim=True)).abs().max() <= 2e-2
+    for name, padded, given in zip(("O", "dQ", "dK", "dV"), *results):
+        assert torch.isfinite(padded).all(), name
+        # (two kernels round P and dS to 16 bits on the way: a share of the largest sums, not of every entry)
+        assert (padded.float() - given.float()).abs().max() <= 4 * torch.finfo(dtype).eps * given.float().abs().max(), name
+
+
 # ------------------------------------------------------------------ mask gradients summed over batches and heads
 @pytest.mark.parametrize("shape", ["1HSS", "B1SS", "11SS"])
 @pytest.mark.parametrize("dtype,mask_dtype,B,H,S,D", [(torch.bfloat16, torch.bfloat16, 3, 2, 1, 64), (torch.float16, torch.float32, 2, 3, 31, 16),

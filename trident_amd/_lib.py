@@ -12,6 +12,7 @@ ESCRATCH = -10  # tri_attn_bwd_noalloc: B*H*S above NOALLOC_MAX_ROWS, nothing la
 NOALLOC_MAX_ROWS = 1 << 20
 BOOL = 3  # tri_attn_prepare_mask: the source is a boolean mask
 MASK_PADDED = 0x100  # in mask_dtype: rows may be read up to the next multiple of 64 entries
+MASK_BINARY = 0x200  # in mask_dtype: every value is 0 or -inf
 
 _i64x4 = ctypes.c_int64 * 4
 

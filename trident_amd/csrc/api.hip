@@ -46,7 +46,7 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (static_cast<int64_t>(a->B) * a->H > 2147483647LL / 64) return TRI_ATTN_ESHAPE;
     if (!(a->dropout_p >= 0.f && a->dropout_p <= 1.f)) return TRI_ATTN_EDROPOUT;
     if (a->mask != nullptr && a->is_causal) return TRI_ATTN_EMASKCAUSAL;
-    const int mask_dtype = a->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    const int mask_dtype = a->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);
     const bool padded = a->mask != nullptr && (a->mask_dtype & TRI_ATTN_MASK_PADDED) != 0;
     if (a->mask != nullptr || a->dmask != nullptr) {
         if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
@@ -128,6 +128,7 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     p->causal = a->is_causal ? 1 : 0;
     p->mask_dtype = mask_dtype;
     p->mask_padded = padded;
+    p->mask_binary = a->mask != nullptr && (a->mask_dtype & TRI_ATTN_MASK_BINARY) != 0;
     p->scale = a->softmax_scale;
     p->scale_log2 = a->softmax_scale * kLog2e;
     p->inv_scale = a->softmax_scale != 0.f ? 1.f / a->softmax_scale : 0.f;
@@ -301,7 +302,7 @@ int tri_attn_classify_mask(const TriAttnArgs* args) {
     if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr || args->mask_classes == nullptr) return TRI_ATTN_ENULL;
-    const int mask_dtype = args->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    const int mask_dtype = args->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);
     if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     int rc = check_strides(args->mask_stride);
     if (rc) return rc;
@@ -323,7 +324,7 @@ int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t s
     if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr) return TRI_ATTN_ENULL;
-    const int mask_dtype = args->mask_dtype & ~TRI_ATTN_MASK_PADDED;
+    const int mask_dtype = args->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);
     if (!(args->mask_dtype & TRI_ATTN_MASK_PADDED) || mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     if (source_dtype < TRI_ATTN_F32 || source_dtype > TRI_ATTN_BOOL) return TRI_ATTN_EDTYPE;
     int rc = check_strides(args->mask_stride);

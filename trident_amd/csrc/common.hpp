@@ -34,6 +34,7 @@ struct KParams {
     int causal;
     int mask_dtype;
     int mask_padded;   // mask rows may be read up to the next multiple of 64 entries (finite values there)
+    int mask_binary;   // every mask value is 0 or -inf
     float scale;       // softmax_scale
     float scale_log2;  // softmax_scale * log2(e)
     float inv_scale;   // 1 / softmax_scale (0 where the scale is 0)

@@ -280,7 +280,10 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
                     for (int g = 0; g < 4; ++g) {
                         const f32x4 l4 = *reinterpret_cast<const f32x4*>(sLse + 32 * qb + 8 * g + 4 * h);
 #pragma unroll
-                        for (int bb = 0; bb < 4; ++bb) pexp[4 * g + bb] = fast_exp2(fmaf(fmaf(mk[4 * g + bb], inv_scale, s[4 * g + bb]), c, -l4[bb]));
+                        for (int bb = 0; bb < 4; ++bb) {  // (a padded mask joins its score behind the scale, as in the forward)
+                            const int i = 4 * g + bb;
+                            pexp[i] = RAGGED ? fast_exp2(fmaf(s[i], c, mk[i] * kLog2e) - l4[bb]) : fast_exp2(fmaf(fmaf(mk[i], inv_scale, s[i]), c, -l4[bb]));
+                        }
                     }
                 } else {
 #pragma unroll
@@ -1225,7 +1228,9 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
             }
         }
         if constexpr (MASK != kNoMask && D == 128) {
-            if (p.ms[2] == 0) {  // (a key-padding mask: as below)
+            // A key-padding mask: as below. Only one of zeros and -inf: this kernel works with S - lse / c, and the lse of a row
+            // whose keys all carry a large finite value would take the score's digits (or, in fp16, not fit at all).
+            if (p.ms[2] == 0 && p.mask_binary) {
                 const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(512);
                 if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, false, true, MASK, true>), grid, block, 0, stream, p);
                 else hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, false, false, MASK, true>), grid, block, 0, stream, p);

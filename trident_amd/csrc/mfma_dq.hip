@@ -305,7 +305,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             float ds[16];
             if (masked) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) ds[i] = fast_exp2(fmaf(fmaf(mk[i], inv_scale, st[i]), c, -lse));  // (s + mask / scale, then the scale)
+                for (int i = 0; i < 16; ++i)  // (s + mask / scale, then the scale; a padded mask behind the scale, as in the forward)
+                    ds[i] = RAGGED ? fast_exp2(fmaf(st[i], c, mk[i] * kLog2e) - lse) : fast_exp2(fmaf(fmaf(mk[i], inv_scale, st[i]), c, -lse));
             } else {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) ds[i] = fast_exp2(fmaf(st[i], c, -lse));

@@ -137,6 +137,9 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     float m_use;  // m, or 0 while no key has been seen (m = -inf): what the exponents are taken against; follows m
     const float c = p.scale_log2;
     const float inv_scale = p.inv_scale;  // (a mask value joins its score before the scale: s + mask / scale)
+    // ... except a padded one (RAGGED), which joins it behind the scale, in the log2 domain: mask / scale would take finite
+    // values below about -3.4e38 * scale to -inf, and a row of nothing else to NaN. One multiplication per score more.
+    constexpr bool kMaskAfter = RAGGED && MASK != kNoMask;
 
     char* mask_lds = smem + kStages * kStageBytes + wave * kMaskBytes;
     auto issue_mask = [&](int t) {  // mask block of tile t -> this wave's region (8 LDS-direct loads), unless it is all zero
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     // to spare, the softmax phase is the one the partner waits for.
     constexpr bool kDefer = !DROPOUT;
     float xd[16];        // deferred exponents and then probabilities
-    float m_def = 0.f;   // the reference exponent they are taken against
+    float m_def = 0.f, c_def = c;   // the reference exponent they are taken against, and their factor
     const uint32_t one2 = Mma<T>::pack2(1.f, 1.f);
     u32x4 ones = {one2, one2, one2, one2};
     asm volatile("" : "+v"(ones));  // (kept in registers: as a constant it would be made anew from scalars in every tile)
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                     for (int e = 0; e < 8; ++e)
                         if (e * ne / 8 == ls) {
                             float& v = xd[8 * (g - 2) + e];
-                            v = fast_exp2(fmaf(v, c, -m_def));
+                            v = fast_exp2(fmaf(v, kMaskAfter ? c_def : c, -m_def));
                             if constexpr (kVectorSum) l += v;
                         }
                     if (ls == pack_step) pb[g] = pack8<T>(&xd[8 * (g - 2)]);
@@ -447,11 +450,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 x[16 + i] = sc[1][i];
             }
             // The scale (to the log2 domain) is folded into the exponent's multiply-add; a mask value is added before it,
-            // divided by the scale: one multiply-add per score, none in a tile whose mask is all zero.
+            // divided by the scale: one multiply-add per score, none in a tile whose mask is all zero. (c_tile: what is left
+            // to multiply by.)
+            const float c_tile = kMaskAfter && !mask_is_zero(j) ? 1.f : c;
             if constexpr (MASK != kNoMask) {
                 if (!mask_is_zero(j)) {
 #pragma unroll
-                    for (int e = 0; e < 32; ++e) x[e] = fmaf(mk[e], inv_scale, x[e]);
+                    for (int e = 0; e < 32; ++e) x[e] = kMaskAfter ? fmaf(mk[e], kLog2e, x[e] * c) : fmaf(mk[e], inv_scale, x[e]);
                 }
             }
             if (CAUSAL && t0 + kBN - 1 > wrow0) {
@@ -476,7 +481,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 mx1 = max3(mx1, x[16 + e], x[17 + e]);
             }
             mx = max_xor32(max3(mx, x[15], max3(mx1, x[31], x[31])));
-            mx *= c;
+            mx *= c_tile;
             // Lazy rescaling: m is the reference exponent of l and of the O accumulators, not
             // necessarily the running maximum. It is only moved (and O rescaled) when some row of
             // the wave outgrew it by more than 2^kTau; until then probabilities may exceed 1 by
@@ -508,7 +513,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             for (int ks = 0; ks < kNow; ++ks) {
 #pragma unroll
                 for (int e = 8 * ks; e < 8 * ks + 8; ++e) {
-                    x[e] = fast_exp2(fmaf(x[e], c, -m_use));
+                    x[e] = fast_exp2(fmaf(x[e], c_tile, -m_use));
                     if constexpr (kVectorSum && !DROPOUT) l += x[e];
                 }
                 if constexpr (!DROPOUT) pb[ks] = pack8<T>(&x[8 * ks]);
@@ -523,6 +528,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
 #pragma unroll
                 for (int e = 0; e < 16; ++e) xd[e] = x[16 + e];
                 m_def = m_use;
+                c_def = c_tile;
             }
             if constexpr (DROPOUT) {
                 // row sum before dropping, in fp32: four interleaved partial sums (a dependent add waits

@@ -167,7 +167,7 @@ class _PreparedMask:
         dtype = query.dtype if boolean else source.dtype
         self.padded = torch.empty(batches * heads * rows * pitch, device=query.device, dtype=dtype)
         self.strides = (heads * rows * pitch if batches > 1 else 0, rows * pitch if heads > 1 else 0, pitch if rows > 1 else 0, 1)
-        self.dtype = util.dtype(dtype) | _lib.MASK_PADDED
+        self.dtype = util.dtype(dtype) | _lib.MASK_PADDED | (_lib.MASK_BINARY if boolean else 0)
         self.classes = None
         args = _lib.TriAttnArgs()
         args.struct_size = _lib.ARGS_PACKER.size
