@@ -646,6 +646,36 @@ def test_backward_through_a_fully_masked_row(device):
     assert torch.isnan(dv.float()).all() == bool(np.isnan(dv_r).all())
 
 
+@pytest.mark.parametrize("kind", ["bool", "f32", "16 bit", "f32+dropout"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 200, 16), (torch.float16, 333, 64), (torch.bfloat16, 300, 128)])
+@pytest.mark.parametrize("where", ["first rows", "last rows", "one row", "all rows"])
+def test_backward_through_fully_masked_rows_of_padded_masks(where, dtype, S, D, kind, device, monkeypatch):
+    """The same at lengths that are no multiple of 128, where row tiles that are masked out over a workgroup's keys are not
+    streamed: rows without a visible key in such tiles, beside rows whose visible keys are another workgroup's."""
+    from trident_amd import operation
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    q, k, v, d_o = _gen((2, 2, S, D), 47 + S, dtype)
+    visible = torch.ones(2, 1, S, S, dtype=torch.bool)
+    lost = {"first rows": slice(0, 64), "last rows": slice(S // 64 * 64, S), "one row": slice(S - 1, S), "all rows": slice(0, S)}[where]
+    visible[1, :, :, S // 2:] = False           # (keys of the second sequence that no row sees: nothing is streamed for them)
+    visible[1, :, S // 64 * 64:, :S // 2] = False
+    visible[1, :, S // 64 * 64:, 0] = True      # (rows that see the first key only)
+    visible[1, :, lost] = False
+    if kind == "bool":
+        given = operation._BooleanMask(visible.to(device))
+    else:
+        given = torch.zeros(visible.shape, dtype=dtype if kind == "16 bit" else torch.float32).masked_fill(~visible, -math.inf).to(device)
+    p, rng = (0.2, (5, 1)) if "dropout" in kind else (0.0, (0, 0))
+    scale = 1.0 / math.sqrt(D)
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    o, lse = operation.Attention._forward(tq, tk, tv, given, p, False, scale, *rng)
+    dq, dk, dv, _ = operation.Attention._backward(tdo, tq, tk, tv, o, lse, given, scale, p, False, *rng, False)
+    hidden = torch.zeros(2, 1, S, 1, dtype=torch.bool)
+    hidden[1, :, lost] = True
+    for name, x, want in (("O", o, hidden), ("dQ", dq, hidden), ("dK", dk, hidden.any(2, keepdim=True)), ("dV", dv, hidden.any(2, keepdim=True))):
+        assert torch.equal(x.isnan().cpu(), want.expand_as(x)), name
+
+
 def test_trace_ranges_switch_on(device):
     """config.use_trace = True: the roctx range calls around the operation and every launch really execute."""
     q, k, v, d_o = _gen((1, 2, 128, 64), 52, torch.bfloat16)

@@ -108,6 +108,10 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
     // With the classes of the mask's blocks at hand: row tiles before the first and behind the last one that is not
     // masked out altogether over the workgroup's keys are not streamed (keys beyond every length: nothing at all, the
     // gradients are zero), and tiles whose mask is all zero over the workgroup's keys are not read.
+    // A row without a single visible key (its lse is -inf) turns all of dK and dV to NaN, as softmax does. Where a padded mask
+    // leaves row tiles out, such rows are looked for among theirs: left_out, a factor of the results, is NaN if there are
+    // any. (Usual padding and length masks leave rows out only of workgroups whose keys nobody sees.)
+    [[maybe_unused]] float left_out = 1.f;
     uint64_t zero_tiles = 0;
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
@@ -119,6 +123,12 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
                 n_tiles = 64 - __builtin_clzll(tc.active);
             } else {
                 n_tiles = 0;
+            }
+            if constexpr (RAGGED) {
+                bool lost = false;
+                for (int r = lane; r < t_begin * kBN; r += 64) lost |= !(lse_base[r] > -INFINITY);
+                for (int r = n_tiles * kBN + lane; r < p.S; r += 64) lost |= !(lse_base[r] > -INFINITY);
+                if (__builtin_amdgcn_ballot_w64(lost) != 0) left_out = __builtin_nanf("");
             }
         }
     }
@@ -353,11 +363,12 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
         char* patch = smem + wave * Store::kPatchBytes;
         char* dk0 = static_cast<char*>(p.dk) + (b * p.dks[0] + hd * p.dks[1] + static_cast<int64_t>(wkey0) * p.dks[2]) * 2;
         char* dv0 = static_cast<char*>(p.dv) + (b * p.dvs[0] + hd * p.dvs[1] + static_cast<int64_t>(wkey0) * p.dvs[2]) * 2;
-        const float sc = kDeltaInAcc ? -p.scale : p.scale;
+        constexpr bool kLeftOut = RAGGED && MASK != kNoMask;
+        const float sc = (kDeltaInAcc ? -p.scale : p.scale) * (kLeftOut ? left_out : 1.f);
         const int keys_here = RAGGED ? p.S - wkey0 : 32;
         Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, lane, keys_here);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
-        Store::run(dv, [](float x) { return x; }, patch, dv0, p.dvs[2] * 2, lane, keys_here);
+        Store::run(dv, [left_out](float x) { return kLeftOut ? x * left_out : x; }, patch, dv0, p.dvs[2] * 2, lane, keys_here);
     }
 }
 
