@@ -127,6 +127,25 @@ def test_value_errors_with_and_without_a_graph():
             f(x, x, x)
 
 
+def test_a_mask_without_memory_for_its_padded_copy_is_handed_over_as_it_is(monkeypatch):
+    """An additive mask at a ragged length that is worth a padded copy (more than 2^29 scores times head size): no copy where
+    there is no memory for it, in the forward (grad mode) and the backward, which take the same decision."""
+    from trident_amd import operation
+    query = torch.empty(1, 1, 1, 1, dtype=torch.bfloat16).expand(8, 16, 1000, 64)
+    asked = []
+
+    def no_memory(*args):
+        asked.append(args)
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(operation, "_PreparedMask", no_memory)
+    for mask in (torch.zeros(1, 1, 1, 1).expand(8, 1, 1000, 1000), torch.zeros(8, 1, 1, 1000, dtype=torch.bfloat16)):
+        assert operation._prepared_mask(mask, query) is None
+    assert len(asked) == 2
+    with pytest.raises(torch.OutOfMemoryError):  # (a boolean mask has no other way)
+        operation._prepared_mask(operation._BooleanMask(torch.ones(8, 1, 1, 1000, dtype=torch.bool)), query)
+
+
 def test_argument_packer_matches_the_structure():
     """_lib.ARGS_PACKER writes TriAttnArgs in one call: every field must land where the ctypes structure (and the
     header) has it."""

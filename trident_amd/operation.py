@@ -206,7 +206,8 @@ def _prepared_mask(mask, query):
     in 16-byte pieces up to the end of a 64-key tile: one more pass over the mask (at the copy rate) in each direction against
     kernels that read masks element by element (bf16, dense fp32 mask, forward + backward: B=16 H=12 S=777 D=64 2.22 -> 0.39 ms,
     S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below _PADS_FROM scores times head size the launches and their arguments cost a call more than
-    the kernels save (S=100 0.15 -> 0.21 ms). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it."""
+    the kernels save (S=100 0.15 -> 0.21 ms). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it.
+    So does one that the GPU has no memory left to copy."""
     if isinstance(mask, _BooleanMask):
         if mask.prepared is None:
             mask.prepared = _PreparedMask(mask.source, query)
@@ -219,7 +220,10 @@ def _prepared_mask(mask, query):
         return None
     if mask.requires_grad and not _sums_mask_gradient(mask, query):
         return None
-    return _PreparedMask(mask.detach(), query)
+    try:
+        return _PreparedMask(mask.detach(), query)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def _expand_mask(mask: torch.Tensor, shape):
