@@ -189,7 +189,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
         const int i = idx % kPerOperand;
         if (RAGGED && (t + 1) * kBN > p.S) {  // the sequence ends inside this tile: clamped rows, offsets from the tile's first row
             int l = lane;
-            if constexpr (D == 128) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
+            if constexpr (D == 128 && MASK != kNoMask) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
             const int last = p.S - 1 - t * kBN;
             if (idx < kPerOperand)
                 lds_direct_load16(kbase + static_cast<int64_t>(t) * kBN * krow_bytes,
@@ -281,15 +281,19 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             // (block 0 precedes tile 0, which has landed)
             if (!mask_is_zero(t)) {
                 if (!first) wait_loads(false, tile_in_flight, v_in_flight);
-                int l32 = threadIdx.x & 31, h = (threadIdx.x >> 5) & 1;
-                if constexpr (RAGGED && D == 128) asm volatile("" : "+v"(l32), "+v"(h));  // (addresses made here, not kept across the loop)
+                int row = l32, half = h;
+                if constexpr (RAGGED && D == 128) {  // (addresses made here, not kept in registers across the loop)
+                    row = threadIdx.x & 31;
+                    half = (threadIdx.x >> 5) & 1;
+                    asm volatile("" : "+v"(row), "+v"(half));
+                }
 #pragma unroll
                 for (int g = 0; g < 8; ++g) {  // keys 32 (g / 4) + 8 (g % 4) + 4 h .. + 3 of this lane's row
                     if constexpr (MASK == kMaskF32) {
-                        const f32x4 v = *reinterpret_cast<const f32x4*>(mask_lds + MaskTile::off(l32, 8 * (g >> 2) + 2 * (g & 3) + h));
+                        const f32x4 v = *reinterpret_cast<const f32x4*>(mask_lds + MaskTile::off(row, 8 * (g >> 2) + 2 * (g & 3) + half));
                         mk[4 * g + 0] = v.x; mk[4 * g + 1] = v.y; mk[4 * g + 2] = v.z; mk[4 * g + 3] = v.w;
                     } else {
-                        const u32x2 v = *reinterpret_cast<const u32x2*>(mask_lds + MaskTile::off(l32, 4 * (g >> 2) + (g & 3)) + 8 * h);
+                        const u32x2 v = *reinterpret_cast<const u32x2*>(mask_lds + MaskTile::off(row, 4 * (g >> 2) + (g & 3)) + 8 * half);
                         mk[4 * g + 0] = Mma<T>::lo(v.x); mk[4 * g + 1] = Mma<T>::hi(v.x);
                         mk[4 * g + 2] = Mma<T>::lo(v.y); mk[4 * g + 3] = Mma<T>::hi(v.y);
                     }
@@ -467,10 +471,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 }
             }
             if (RAGGED && !CAUSAL && t0 + kBN > p.S) {  // keys that do not exist (under the causal mask no existing row sees them)
-                int left = p.S - t0 - 4 * h;
-                asm volatile("" : "+v"(left));  // (made here, not kept in registers across the loop)
+                [[maybe_unused]] int left = p.S - t0 - 4 * h;
+                if constexpr (MASK != kNoMask) asm volatile("" : "+v"(left));  // (made here, not kept in registers across the loop)
 #pragma unroll
-                for (int e = 0; e < 32; ++e) x[e] = 32 * (e >> 4) + c_row(e & 15, 0) < left ? x[e] : -INFINITY;
+                for (int e = 0; e < 32; ++e) {
+                    const int key = t0 + 32 * (e >> 4) + c_row(e & 15, h);
+                    x[e] = (MASK != kNoMask ? 32 * (e >> 4) + c_row(e & 15, 0) < left : key < p.S) ? x[e] : -INFINITY;
+                }
             }
             // two chains (a dependent maximum waits out the ALU latency) of three-operand maxima, written out: through
             // fmaxf the compiler first canonicalises the operands of each chain (a maximum of a value with itself)
