@@ -572,6 +572,15 @@ def test_a_head_does_not_depend_on_its_company(B, H, S, D, causal, device):
     parity.close(dv[B - 1:, hs], dv_r, dtype, "company dV", a_dv)
 
 
+@pytest.mark.parametrize("variant", ["plain", "causal", "dropout", "causal+dropout"])
+@pytest.mark.parametrize("dtype,S,heads", [(torch.float16, 64, 3), (torch.bfloat16, 130, 130), (torch.float16, 300, 90), (torch.bfloat16, 384, 3),
+                                           (torch.bfloat16, 1030, 29)])
+def test_launch_sizes_at_head_size_128(dtype, S, heads, variant, device):
+    """Lengths that are no multiple of 256 on either side of the rules that choose between workgroups of four waves (all on the
+    chip at once, or a single tile) and of eight; causal at S = 1030 with 261 of 128 rows."""
+    _abi_case(device, dtype, S, 128, variant, 4700 + S, batches=1, heads=heads, matrix_cores=True)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_a_head_does_not_depend_on_its_company_at_any_length(causal, device):
     """The same at a length that ends inside a workgroup's rows: 300 items on 256 compute units, so that persistent forward

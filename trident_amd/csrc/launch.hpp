@@ -41,5 +41,9 @@ enum MaskClass { kMaskZero = 0, kMaskNegInf = 1, kMaskMixed = 2 };
 // Number of workgroups for a kernel whose workgroups are persistent (one per CU, each walking several of
 // the `items`): min(items, CUs of the current device).
 int persistent_grid(int items);
+// Whether workgroups of 128 rows are all on the chip at once, one per CU. Causal ones from S = 1024 on also where they are half
+// as many again: the heaviest start first, and the light ones fill up behind them (bf16 with dropout, 288-384 workgroups,
+// S = 1025-2100: forward and dQ 0.85-0.91 of the time of 256-row ones; 384 at S = 300: 1.27).
+bool four_waves_fit_one_round(const KParams& p);
 
 }  // namespace tri

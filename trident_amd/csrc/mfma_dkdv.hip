@@ -1220,21 +1220,25 @@ int launch_dkdv_waves(const KParams& p, hipStream_t stream) {
     return static_cast<int>(hipGetLastError());
 }
 
+// D = 128 without a mask, S no multiple of 128: 32 keys per wave instead of the phased pairs where the rows are one tile, which
+// the pairs pad to four blocks: time over theirs 0.75-0.91, with dropout 0.68-0.81 (S = 65: 1.01-1.19).
+bool dkdv_runs_four_waves(const KParams& p) { return p.S <= 64; }
+
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
     if (p.S % 128 != 0) {
         // any length (no mask): 128-key workgroups with boundary handling
         if constexpr (MASK == kNoMask) {
+            if (D < 128 || dkdv_runs_four_waves(p)) {
+                const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+                return static_cast<int>(hipGetLastError());
+            }
             if constexpr (D == 128) {
                 const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(512);
                 if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, CAUSAL, true, kNoMask, true>), grid, block, 0, stream, p);
                 else hipLaunchKernelGGL((mfma_dkdv_phased_kernel<T, D, CAUSAL, false, kNoMask, true>), grid, block, 0, stream, p);
-                return static_cast<int>(hipGetLastError());
-            }
-            if constexpr (D < 128) {
-                const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-                else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
                 return static_cast<int>(hipGetLastError());
             }
         }

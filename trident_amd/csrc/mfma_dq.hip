@@ -699,15 +699,20 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
                 return static_cast<int>(hipGetLastError());
             }
         }
-        if constexpr (MASK == kNoMask) {
-            if (with_delta) {
-                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
-                else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, false, false, true>), grid, block, 0, stream, p);
-                return static_cast<int>(hipGetLastError());
+        if constexpr (MASK == kNoMask && D == 128) {  // (without dropout: the phased kernel)
+            if (with_delta) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+        } else {
+            if constexpr (MASK == kNoMask) {
+                if (with_delta) {
+                    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
+                    else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, false, false, true>), grid, block, 0, stream, p);
+                    return static_cast<int>(hipGetLastError());
+                }
             }
+            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
         }
-        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
     }
     return static_cast<int>(hipGetLastError());
 }
@@ -724,6 +729,14 @@ bool dq_is_phased(const KParams& p) {
     return D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : D == 64 && p.S % 256 == 0;
 }
 
+// D = 128 without a mask, S no multiple of 256: the unphased kernel in workgroups of four waves. One key tile (S <= 64) is over
+// before phases pay: time over that of the phased kernel 0.81-0.99 (with dropout, against eight unphased waves, 0.92-1.01).
+// With dropout also where all workgroups are on the chip at once: 0.79-0.89 (causal S = 384 1.05; as the forward).
+bool dq_runs_four_waves(const KParams& p) {
+    if (p.S <= 64) return true;
+    return p.thr8 > 0 && p.S > 128 && (!p.causal || p.S % 128 != 0 || p.S >= 640) && four_waves_fit_one_round(p);
+}
+
 // any length (no mask, or a padded one), with boundary handling
 template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
@@ -735,10 +748,10 @@ int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
     }
     if (with_delta) {
         if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
-        else if constexpr (D < 128) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
-        else return TRI_ATTN_ESHAPE;  // (without dropout: the phased kernel)
+        else if constexpr (D < 128 || NW == 4) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
+        else return TRI_ATTN_ESHAPE;  // (eight waves without dropout: the phased kernel)
     } else if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-    else if constexpr (D < 128) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+    else if constexpr (D < 128 || NW == 4) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
     else return TRI_ATTN_ESHAPE;
     return static_cast<int>(hipGetLastError());
 }
@@ -760,6 +773,10 @@ int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
 
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
+    if constexpr (D == 128 && MASK == kNoMask) {
+        if (p.S % 256 != 0 && dq_runs_four_waves(p))
+            return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
+    }
     if constexpr (MASK == kNoMask && D >= 64) {
         if (dq_is_phased<D, MASK>(p)) return p.S % 256 == 0 ? launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta)
                                                            : launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);

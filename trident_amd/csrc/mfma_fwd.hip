@@ -666,12 +666,19 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
         if (p.thr8 > 0) return launch_fwd_ragged<T, D, 4, CAUSAL, MASK>(p, stream);
     }
     const int items = p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW));
+    if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
+        if (p.S % 128 == 0) {  // (causal only with dropout: fwd_runs_four_waves)
+            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), dim3(items), dim3(64 * NW), 0, stream, p);
+            else if constexpr (!CAUSAL) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
+            return static_cast<int>(hipGetLastError());
+        }
+    }
     // (NW == 8: the kernel's kPersistent, one workgroup per CU walks the items)
     const dim3 grid(NW == 8 && MASK == kNoMask ? persistent_grid(items) : items), block(64 * NW);
     if (p.thr8 > 0) {
         if constexpr (!(D == 128 && NW == 8 && MASK != kNoMask))
             hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true, true>), grid, block, 0, stream, p);
-    } else if constexpr (!(D == 128 && NW == 4)) {
+    } else if constexpr (!(D == 128 && NW == 4 && MASK != kNoMask)) {
         hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
     }
     return static_cast<int>(hipGetLastError());
@@ -698,6 +705,18 @@ int launch_fwd_variant(int dtype, const KParams& p, hipStream_t stream) {
     return TRI_ATTN_EDTYPE;
 }
 
+// D = 128 without a mask, S no multiple of 256: 128-row workgroups of four waves where they are all on the chip at once, which
+// then is a matter of one workgroup's time. bf16, time of the four waves over that of the eight: with dropout 0.78-0.98
+// (causal 0.79-0.97, but 1.03 at S = 384, whose last 256 rows are half empty for the eight), without 0.92-0.98 at S = 129 .. 500
+// and from 640 on 1.00-1.12 with boundary handling, 0.88-0.94 at multiples of 128, which need none; causal 0.86-1.00 up to
+// S = 500, 1.02-1.19 beyond and at multiples of 128; S <= 128 without dropout 1.00-1.05.
+bool fwd_runs_four_waves(const KParams& p) {
+    if (!four_waves_fit_one_round(p)) return false;
+    const bool whole = p.S % 128 == 0;
+    if (p.thr8 > 0) return !p.causal || !whole || p.S >= 640;
+    return p.S > 128 && (whole ? !p.causal : p.S <= 512);
+}
+
 template <typename T, int D>
 int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     // 8 waves (256 query rows) when the sequence allows it: two waves per SIMD out of phase. At D = 32 the vector ALU
@@ -708,9 +727,13 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     }
     // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
     // one workgroup per CU, so that four waves are one per SIMD. bf16 causal, heads x S: 768 x 130 0.057 -> 0.034 ms,
-    // 768 x 450 0.168 -> 0.110, 136 x 1531 0.170 -> 0.109, 32 x 3000 0.141 -> 0.084; 768 x 65 0.026 -> 0.022.
+    // 768 x 450 0.168 -> 0.110, 136 x 1531 0.170 -> 0.109, 32 x 3000 0.141 -> 0.084; 768 x 65 0.026 -> 0.022. Launches
+    // that leave CUs idle either way are another matter (above).
     if constexpr (D == 128) {
-        if (p.mask == nullptr) return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
+        if (p.mask == nullptr) {
+            if (fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
+            return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
+        }
     }
     if (p.S % 128 == 0) return launch_fwd_variant<T, D, 4>(dtype, p, stream);
     if (p.mask != nullptr) {

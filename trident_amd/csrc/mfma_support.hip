@@ -227,6 +227,13 @@ int persistent_grid(int items) {
     return items < n ? items : n;
 }
 
+bool four_waves_fit_one_round(const KParams& p) {
+    const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
+    if (items > 1 << 20) return false;
+    const int busy = static_cast<int>(p.causal && p.S >= 1024 ? (2 * items + 2) / 3 : items);
+    return persistent_grid(busy) == busy;
+}
+
 int launch_delta(int dtype, const KParams& p, hipStream_t stream) {
     const bool vec = (dtype == TRI_ATTN_F16 || dtype == TRI_ATTN_BF16) && (p.D == 16 || p.D == 32 || p.D == 64 || p.D == 128) &&
                      aligned16(p.o) && aligned16(p.d_o) && strides8(p.os) && strides8(p.dos);
