@@ -105,6 +105,56 @@ def test_softmax_of_rows_off_the_16_byte_boundaries(x_size, offset, dtype, devic
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [1, 2, 7, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("cols,mask_dtype", [(40, None), (1031, torch.uint8), (2056, torch.int64), (4104, torch.float32)])
+def test_softmax_down_a_few_rows(rows, cols, mask_dtype, dtype, device):
+    """Columns a thread holds whole (up to 16 elements, 8 in the backward) and the first lengths beyond, whole vectors and
+    single elements across the columns, masks, a column that is masked out altogether."""
+    x, g = _pair((rows, cols), 170 + rows, dtype)
+    if mask_dtype is None:
+        _softmax_case(device, x * 3, g, 0, dtype, tag=f"{rows} rows {dtype}")
+        return
+    mask = _build_mask((rows, cols), 171)
+    mask[:, 5] = 1
+    tx = (x * 3).to(device).requires_grad_(True)
+    out = trident.function.masked_softmax(tx, mask.to(mask_dtype).to(device), 0)
+    out.backward(g.to(device))
+    want = rowops.softmax_forward(parity.to64((x * 3).to(dtype)), 0, mask.numpy())
+    live = [c for c in range(cols) if c != 5]
+    assert torch.isnan(out[:, 5]).all() and torch.isnan(tx.grad[:, 5]).all()
+    parity.close(out[:, live], want[:, live], dtype, f"{rows} rows {dtype} {mask_dtype}")
+    gradient = rowops.softmax_backward(parity.to64(out[:, live]), parity.to64(g[:, live]), 0)
+    parity.close(tx.grad[:, live], gradient, dtype, f"{rows} rows grad")
+
+
+def _milliseconds(run):
+    for _ in range(3):
+        run()
+    times = []
+    for _ in range(5):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(10):
+            run()
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end) / 10)
+    return min(times)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_few_long_rows_take_a_streaming_kernels_time(dtype, device):
+    """The forward moves two tensors where the backward moves three: it takes no more than twice the backward's time (in panels,
+    bound by exponentials of elements that do not exist, it took three times)."""
+    from trident_amd.rowops import _softmax_backward, _softmax_forward
+    x = torch.randn(2, 1 << 22, device=device).to(dtype)
+    out = _softmax_forward(x, None, 0, "forward")
+    forward = _milliseconds(lambda: _softmax_forward(x, None, 0, "forward"))
+    backward = _milliseconds(lambda: _softmax_backward(x, out, 0, "backward"))
+    assert forward <= 2 * backward, (forward, backward)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape,mask_dtype", [((2, 40), None), ((129, 2056), torch.uint8), ((4101, 24), torch.int64), ((300, 777), torch.bfloat16),
                                               ((20000, 8), None), ((35001, 3), torch.bool), ((1025, 4096), None)])
 def test_softmax_down_the_columns(shape, mask_dtype, dtype, device):

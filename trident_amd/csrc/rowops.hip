@@ -328,13 +328,12 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
 // stay in registers between statistics and output, so a panel of up to RG x kColHeld elements of length is read once;
 // a longer one is swept twice (the second sweep finds it in L2 or the Infinity Cache as far as it fits). Neighbouring
 // panels go to the same XCD: where a panel row is narrower than a 128-byte line, the other half is then still in its L2.
+// The statistics' LDS is sized by the workgroup, so that single-wave ones fill a CU.
 // fp32 4096 x 4096 along dim 0: forward 0.0257 ms = 5.2 TB/s (what a large copy reaches), backward 0.0447 ms = 4.5 TB/s. One
 // thread per column, which this replaces, took 2.1 and 2.4 ms: 64 waves in flight on the whole chip, each waiting for one
 // load at a time. (Its sums ran in plain order, too: at 65536 elements off by 7.5e-5, these by 1.8e-7.)
 constexpr int kColHeld = 16;        // forward: pieces a thread keeps (64 registers)
 constexpr int kColHeldBwd = 8;      // backward: of each of its two inputs
-constexpr int kColPanel = 128;      // most columns of a panel
-constexpr int kColWaves = 16;       // most waves of a workgroup
 
 struct ColPlace {
     int lane, group, groups;  // lane position in the panel, row group of this thread and their number
@@ -376,7 +375,7 @@ struct ColWalk {
 
 template <typename T, int V, typename M>
 __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams p, int lanes_log2, int64_t panels) {
-    __shared__ Stat part[kColWaves * kColPanel];
+    extern __shared__ Stat part[];  // one per wave and column of the panel
     ColPlace c;
     if (!place_in_panel(p, V, lanes_log2, panels, &c)) return;
     using VT = Vec<T, V>;
@@ -460,7 +459,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
 
 template <typename T, int V>
 __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams p, int lanes_log2, int64_t panels) {
-    __shared__ float part[kColWaves * kColPanel];
+    extern __shared__ float part_sums[];  // one per wave and column of the panel
     ColPlace c;
     if (!place_in_panel(p, V, lanes_log2, panels, &c)) return;
     using VT = Vec<T, V>;
@@ -499,18 +498,18 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
     const int columns = V << lanes_log2, waves = blockDim.x / 64;
     if ((threadIdx.x & 63) < (1 << lanes_log2)) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) part[(threadIdx.x / 64) * columns + c.lane * V + e] = delta[e];
+        for (int e = 0; e < V; ++e) part_sums[(threadIdx.x / 64) * columns + c.lane * V + e] = delta[e];
     }
     __syncthreads();
     for (int i = threadIdx.x; i < columns; i += blockDim.x) {
-        float t = part[i];
-        for (int w = 1; w < waves; ++w) t += part[w * columns + i];
-        part[i] = t;
+        float t = part_sums[i];
+        for (int w = 1; w < waves; ++w) t += part_sums[w * columns + i];
+        part_sums[i] = t;
     }
     __syncthreads();
     if (!c.live) return;
 #pragma unroll
-    for (int e = 0; e < V; ++e) delta[e] = part[c.lane * V + e];
+    for (int e = 0; e < V; ++e) delta[e] = part_sums[c.lane * V + e];
     for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
         if (p.x_size > sweep) load(r0);
         ColWalk w(p, c, r0);
@@ -524,6 +523,105 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
             }
         }
     }
+}
+
+// Columns of a few elements (a few rows of a wide matrix): HBM-bound still, but in panels most of a thread's pieces would not
+// exist, and their exponentials would bound it. Here a thread holds its V columns whole and nothing is exchanged; pieces
+// beyond the last row are skipped by branches the whole launch takes. 2 x 4194304, bf16: forward 0.0835 ms in panels ->
+// 0.0093, backward 0.0231 -> 0.0106; fp32 0.0515 -> 0.0134 and 0.0181 -> 0.0158 (a thread per column, as before the panels,
+// 0.0162 and 0.0192). 16 x 1048576, bf16: forward 0.0296 -> 0.0173; backward at 9 rows the same either way (0.0133).
+constexpr int kFewRows = 16;    // (64 registers)
+constexpr int kFewRowsBwd = 8;  // (of each of its two inputs)
+
+template <typename T, int V, typename M>
+__global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowParams p) {
+    const int64_t col = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V;
+    if (col >= p.y_size) return;
+    const int64_t base = col * p.y_stride;
+    const T* in = static_cast<const T*>(p.input) + base;
+    T* out = static_cast<T*>(p.output) + base;
+    const int rows = static_cast<int>(p.x_size);
+    Piece<T, V> held[kFewRows];
+#pragma unroll
+    for (int k = 0; k < kFewRows; ++k)
+        if (k < rows) held[k].load(in + k * p.x_stride);
+    if constexpr (!std::is_same<M, void>::value) {
+#pragma unroll
+        for (int k = 0; k < kFewRows; ++k)
+            if (k < rows) {
+                const uint32_t hit = mask_bits<M, V>(p.mask, base + k * p.x_stride);
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    if (hit >> e & 1) held[k].set(e, -INFINITY);
+            }
+    }
+    float ms[V], l[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        ms[e] = -INFINITY;
+        l[e] = 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < kFewRows; ++k)
+        if (k < rows) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) ms[e] = fmaxf(ms[e], held[k].get(e));
+            held[k].hide();
+        }
+#pragma unroll
+    for (int e = 0; e < V; ++e) ms[e] = safe(ms[e] * kLog2e);
+#pragma unroll
+    for (int k = 0; k < kFewRows; ++k)
+        if (k < rows) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) l[e] += fast_exp2(fmaf(held[k].get(e), kLog2e, -ms[e]));
+            held[k].hide();
+        }
+#pragma unroll
+    for (int e = 0; e < V; ++e) l[e] = 1.f / l[e];  // a fully masked column: 0 * inf = NaN, as softmax gives
+#pragma unroll
+    for (int k = 0; k < kFewRows; ++k)
+        if (k < rows) {
+            Vec<T, V> o;
+#pragma unroll
+            for (int e = 0; e < V; ++e) o.e[e] = from_f32<T>(fast_exp2(fmaf(held[k].get(e), kLog2e, -ms[e])) * l[e]);
+            *reinterpret_cast<Vec<T, V>*>(out + k * p.x_stride) = o;
+        }
+}
+
+template <typename T, int V>
+__global__ __launch_bounds__(256) void softmax_bwd_few_rows_kernel(const RowParams p) {
+    const int64_t col = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V;
+    if (col >= p.y_size) return;
+    const int64_t base = col * p.y_stride;
+    const T* o = static_cast<const T*>(p.output) + base;
+    const T* g = static_cast<const T*>(p.grad_output) + base;
+    T* gi = static_cast<T*>(p.grad_input) + base;
+    const int rows = static_cast<int>(p.x_size);
+    Piece<T, V> held_o[kFewRowsBwd], held_g[kFewRowsBwd];
+#pragma unroll
+    for (int k = 0; k < kFewRowsBwd; ++k)
+        if (k < rows) {
+            held_o[k].load(o + k * p.x_stride);
+            held_g[k].load(g + k * p.x_stride);
+        }
+    float delta[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) delta[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < kFewRowsBwd; ++k)
+        if (k < rows) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) delta[e] = fmaf(held_o[k].get(e), held_g[k].get(e), delta[e]);
+        }
+#pragma unroll
+    for (int k = 0; k < kFewRowsBwd; ++k)
+        if (k < rows) {
+            Vec<T, V> x;
+#pragma unroll
+            for (int e = 0; e < V; ++e) x.e[e] = from_f32<T>(held_o[k].get(e) * (held_g[k].get(e) - delta[e]));
+            *reinterpret_cast<Vec<T, V>*>(gi + k * p.x_stride) = x;
+        }
 }
 
 // ------------------------------------------------------------------ dropout
@@ -615,10 +713,12 @@ bool aligned16(const void* ptr) { return ptr == nullptr || (reinterpret_cast<uin
 
 // Geometry of a column launch: panels as wide as leaves one for every CU, but no narrower than the 64 bytes HBM moves at
 // a time (16 lanes without vector accesses), and as many threads as give each kColHeld (kColHeldBwd) pieces of its column.
+// A column is never split: a matrix narrower than 256 such panels leaves CUs idle (bf16 65536 x 64: two workgroups, 0.25 ms).
 struct ColLaunch {
     int lanes_log2;
     int64_t panels;
     dim3 grid, block;
+    unsigned stats;  // waves x columns of a panel
 };
 ColLaunch column_launch(const RowParams& p, int v, int held) {
     ColLaunch c;
@@ -634,8 +734,11 @@ ColLaunch column_launch(const RowParams& p, int v, int held) {
     while (threads < 1024 && static_cast<int64_t>(threads >> c.lanes_log2) * held < p.x_size) threads <<= 1;
     c.grid = dim3(static_cast<unsigned>((c.panels + 7) / 8 * 8));
     c.block = dim3(threads);
+    c.stats = static_cast<unsigned>(threads / 64 * (v << c.lanes_log2));
     return c;
 }
+
+dim3 few_rows_grid(const RowParams& p, int v) { return dim3(static_cast<unsigned>((p.y_size + 256 * v - 1) / (256 * v))); }
 
 // Calls launch(V, G, SHIFT) with the variant for rows of this geometry.
 template <typename T, typename Launch>
@@ -668,9 +771,15 @@ int launch_softmax_fwd(const RowParams& p, hipStream_t st) {
     if (p.x_stride != 1 && p.x_size != 1) {
         // 16-byte accesses across the columns when every element row starts on a 16-byte boundary and holds whole vectors
         const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.input) && aligned16(p.output) && aligned16(p.mask);
+        if (p.x_size <= kFewRows) {
+            if (vec) hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, kV, M>), few_rows_grid(p, kV), block, 0, st, p);
+            else hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, 1, M>), few_rows_grid(p, 1), block, 0, st, p);
+            return static_cast<int>(hipGetLastError());
+        }
         const ColLaunch c = column_launch(p, vec ? kV : 1, kColHeld);
-        if (vec) hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, kV, M>), c.grid, c.block, 0, st, p, c.lanes_log2, c.panels);
-        else hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, 1, M>), c.grid, c.block, 0, st, p, c.lanes_log2, c.panels);
+        const unsigned lds = c.stats * sizeof(Stat);
+        if (vec) hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, kV, M>), c.grid, c.block, lds, st, p, c.lanes_log2, c.panels);
+        else hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, 1, M>), c.grid, c.block, lds, st, p, c.lanes_log2, c.panels);
         return static_cast<int>(hipGetLastError());
     }
     const bool base16 = aligned16(p.input) && aligned16(p.output) && aligned16(p.mask);
@@ -686,9 +795,15 @@ int launch_softmax_bwd(const RowParams& p, hipStream_t st) {
     const dim3 block(256);
     if (p.x_stride != 1 && p.x_size != 1) {
         const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input);
+        if (p.x_size <= kFewRowsBwd) {
+            if (vec) hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, kV>), few_rows_grid(p, kV), block, 0, st, p);
+            else hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, 1>), few_rows_grid(p, 1), block, 0, st, p);
+            return static_cast<int>(hipGetLastError());
+        }
         const ColLaunch c = column_launch(p, vec ? kV : 1, kColHeldBwd);
-        if (vec) hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, kV>), c.grid, c.block, 0, st, p, c.lanes_log2, c.panels);
-        else hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, 1>), c.grid, c.block, 0, st, p, c.lanes_log2, c.panels);
+        const unsigned lds = c.stats * sizeof(float);
+        if (vec) hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, kV>), c.grid, c.block, lds, st, p, c.lanes_log2, c.panels);
+        else hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, 1>), c.grid, c.block, lds, st, p, c.lanes_log2, c.panels);
         return static_cast<int>(hipGetLastError());
     }
     const bool base16 = aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input);
