@@ -104,6 +104,28 @@ def test_softmax_of_rows_off_the_16_byte_boundaries(x_size, offset, dtype, devic
     parity.close(grad, rowops.softmax_backward(parity.to64(out), parity.to64(tg), 1), dtype, f"rows {x_size} + {offset} grad")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mask_dtype", [torch.uint8, torch.float16, torch.int64])
+@pytest.mark.parametrize("x_size", [8, 63, 64, 65, 97, 256, 257, 512, 1000, 1001, 1024, 1025])
+def test_softmax_with_a_mask_off_the_16_byte_boundaries(x_size, mask_dtype, dtype, device):
+    """Aligned tensors under a mask that starts one element behind a boundary: rows on 16-byte boundaries and off them, the
+    lengths around which short odd rows and long ones change kernels; and the same data one element behind a boundary."""
+    rows = 7
+    x, g = _pair((rows, x_size), 190 + x_size, dtype)
+    mask = _build_mask((rows, x_size), 191)
+    storage = torch.zeros(rows * x_size + 1, dtype=mask_dtype, device=device)
+    storage[1:] = mask.flatten().to(device)
+    for offset in (0, 1):
+        base = torch.zeros(rows * x_size + offset, dtype=dtype, device=device)
+        base[offset:] = (x * 3).flatten().to(device)
+        tx = base[offset:].view(rows, x_size).requires_grad_(True)
+        out = trident.function.masked_softmax(tx, storage[1:].view(rows, x_size), 1)
+        (grad,) = torch.autograd.grad(out, (tx,), g.to(device))
+        want = rowops.softmax_forward(parity.to64(tx.detach()), 1, mask.numpy())
+        parity.close(out, want, dtype, f"rows {x_size} + {offset} {dtype} {mask_dtype}")
+        parity.close(grad, rowops.softmax_backward(parity.to64(out), parity.to64(g), 1), dtype, f"rows {x_size} + {offset} grad")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows", [1, 2, 7, 8, 9, 15, 16, 17])
 @pytest.mark.parametrize("cols,mask_dtype", [(40, None), (1031, torch.uint8), (2056, torch.int64), (4104, torch.float32)])
@@ -140,6 +162,22 @@ def _milliseconds(run):
         end.synchronize()
         times.append(start.elapsed_time(end) / 10)
     return min(times)
+
+
+@pytest.mark.parametrize("what", ["mask", "data"])
+def test_unaligned_rows_take_a_streaming_kernels_time(what, device):
+    """bf16 rows under a mask, and rows themselves, that start off a 16-byte boundary: no more than 2.5 times the time of the
+    backward, which moves three tensors on boundaries (with a workgroup per row and element-wise loads throughout, more than three
+    times)."""
+    from trident_amd.rowops import _softmax_backward, _softmax_forward
+    rows, cols = 32768, 512
+    x = torch.randn(rows * cols + 1, device=device).bfloat16()
+    mask = (torch.rand(rows * cols + 1, device=device) < 0.25).to(torch.uint8)[1:].view(rows, cols) if what == "mask" else None
+    x = x[1:].view(rows, cols) if what == "data" else x[:-1].view(rows, cols)
+    out = _softmax_forward(x, mask, 1, "forward")
+    forward = _milliseconds(lambda: _softmax_forward(x, mask, 1, "forward"))
+    backward = _milliseconds(lambda: _softmax_backward(out, out, 1, "backward"))
+    assert forward <= 2.5 * backward, (forward, backward)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
