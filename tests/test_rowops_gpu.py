@@ -180,6 +180,19 @@ def test_unaligned_rows_take_a_streaming_kernels_time(what, device):
     assert forward <= 2.5 * backward, (forward, backward)
 
 
+@pytest.mark.parametrize("cols", [17, 33, 49])
+def test_short_odd_rows_take_a_streaming_kernels_time(cols, device):
+    """bf16, 16.7 M elements: backward no longer than three times that of the even length beside it (cut along the tensor's pieces,
+    which are then mostly shared ones, it took four times)."""
+    from trident_amd.rowops import _softmax_backward, _softmax_forward
+    times = []
+    for n in (cols, cols // 8 * 8 + 8):
+        x = torch.randn((1 << 24) // n, n, device=device).bfloat16()
+        out = _softmax_forward(x, None, 1, "forward")
+        times.append(_milliseconds(lambda: _softmax_backward(x, out, 1, "backward")))
+    assert times[0] <= 3 * times[1], times
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_a_few_long_rows_take_a_streaming_kernels_time(dtype, device):
     """The forward moves two tensors where the backward moves three: it takes no more than twice the backward's time (in panels,

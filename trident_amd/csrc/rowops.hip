@@ -119,7 +119,7 @@ struct Piece {
 // SHIFT: rows that do not start on 16-byte boundaries (an odd row length): the pieces are those of the tensor, not of the
 // row, and only a row's first and last piece, which it shares with its neighbours, are read and written element by
 // element. bf16 12288 x 2047 with a uint8 mask: forward 0.0362 ms = 3.5 TB/s, backward 0.0333 ms = 4.5 TB/s; with one element
-// per load, which still serves tensors that are not 16-byte aligned themselves, 0.0545 and 0.0493 ms. Rows on 16-byte
+// per load, which still serves short odd rows and tensors that are not 16-byte aligned themselves, 0.0545 and 0.0493 ms. Rows on 16-byte
 // boundaries: bf16 65536 x 64 forward 0.0092 ms (a wave per row, most of it idle: 0.0265), fp32 8192 x 1536 backward 0.0226
 // (two sweeps: 0.0362), bf16 16384 x 8192 forward 0.1027 (5.2 TB/s), with the mask 0.134 (one mask byte per load: 0.139).
 constexpr int held_pieces(bool shift) { return shift ? 5 : 4; }  // (a shifted row has up to one piece more)
@@ -766,9 +766,15 @@ int launch_rows(const RowParams& p, bool base16, bool backward, Launch launch) {
         else if (worst <= (decltype(v)::value == 1 ? 1024 : 64 * held)) launch(v, integral_constant<int, 64>{}, shift);
         else launch(v, integral_constant<int, 256>{}, shift);
     };
-    // 16-byte accesses when the tensors start on 16-byte boundaries; shifted ones when the rows do not
+    // 16-byte accesses when the tensors start on 16-byte boundaries; shifted ones when the rows do not, but for short rows,
+    // which are little more than their first and last pieces (bf16, 16.7 M elements, shifted -> element by element: 17 per row
+    // forward 0.148 -> 0.061 ms, backward 0.161 -> 0.043; 63: 0.045 -> 0.024 and 0.050 -> 0.020; forward at 65 0.044 -> 0.074).
+    // The backward, with two inputs to read so, turns later: bf16 255 0.030 -> 0.021, 511 0.027 -> 0.022, 1001 0.024 -> 0.029;
+    // fp32 65 0.043 -> 0.049, 255 0.037 -> 0.031, 257 0.033 -> 0.039.
+    const bool by_element = p.x_size <= 64 || (backward && p.x_size > 96 && p.x_size <= (sizeof(T) == 2 ? 512 : 256));
     if (!base16) with_group(One{}, No{});
     else if (p.x_size % kV == 0 && p.y_stride % kV == 0) with_group(Full{}, No{});
+    else if (by_element) with_group(One{}, No{});
     else with_group(Full{}, Yes{});
     return static_cast<int>(hipGetLastError());
 }
