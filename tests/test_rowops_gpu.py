@@ -127,10 +127,10 @@ def test_softmax_with_a_mask_off_the_16_byte_boundaries(x_size, mask_dtype, dtyp
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("rows", [1, 2, 7, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("rows", [1, 2, 4, 5, 8, 9, 15, 16, 17])
 @pytest.mark.parametrize("cols,mask_dtype", [(40, None), (1031, torch.uint8), (2056, torch.int64), (4104, torch.float32)])
 def test_softmax_down_a_few_rows(rows, cols, mask_dtype, dtype, device):
-    """Columns a thread holds whole (up to 16 elements, 8 in the backward) and the first lengths beyond, whole vectors and
+    """Columns a thread holds whole (up to 16 elements, 4 or 8 in the backward) and the first lengths beyond, whole vectors and
     single elements across the columns, masks, a column that is masked out altogether."""
     x, g = _pair((rows, cols), 170 + rows, dtype)
     if mask_dtype is None:

@@ -538,7 +538,8 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
 // 0.0093, backward 0.0231 -> 0.0106; fp32 0.0515 -> 0.0134 and 0.0181 -> 0.0158 (a thread per column, as before the panels,
 // 0.0162 and 0.0192). 16 x 1048576, bf16: forward 0.0296 -> 0.0173; backward at 9 rows the same either way (0.0133).
 constexpr int kFewRows = 16;    // (64 registers)
-constexpr int kFewRowsBwd = 8;  // (of each of its two inputs)
+template <typename T>
+constexpr int kFewRowsBwd = sizeof(T) == 2 ? 8 : 4;  // (of each of its two inputs; fp32 8 x 1048576 0.0178 ms so, in panels 0.0165)
 
 template <typename T, int V, typename M>
 __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowParams p) {
@@ -605,9 +606,10 @@ __global__ __launch_bounds__(256) void softmax_bwd_few_rows_kernel(const RowPara
     const T* g = static_cast<const T*>(p.grad_output) + base;
     T* gi = static_cast<T*>(p.grad_input) + base;
     const int rows = static_cast<int>(p.x_size);
-    Piece<T, V> held_o[kFewRowsBwd], held_g[kFewRowsBwd];
+    constexpr int kRows = kFewRowsBwd<T>;
+    Piece<T, V> held_o[kRows], held_g[kRows];
 #pragma unroll
-    for (int k = 0; k < kFewRowsBwd; ++k)
+    for (int k = 0; k < kRows; ++k)
         if (k < rows) {
             held_o[k].load(o + k * p.x_stride);
             held_g[k].load(g + k * p.x_stride);
@@ -616,13 +618,13 @@ __global__ __launch_bounds__(256) void softmax_bwd_few_rows_kernel(const RowPara
 #pragma unroll
     for (int e = 0; e < V; ++e) delta[e] = 0.f;
 #pragma unroll
-    for (int k = 0; k < kFewRowsBwd; ++k)
+    for (int k = 0; k < kRows; ++k)
         if (k < rows) {
 #pragma unroll
             for (int e = 0; e < V; ++e) delta[e] = fmaf(held_o[k].get(e), held_g[k].get(e), delta[e]);
         }
 #pragma unroll
-    for (int k = 0; k < kFewRowsBwd; ++k)
+    for (int k = 0; k < kRows; ++k)
         if (k < rows) {
             Vec<T, V> x;
 #pragma unroll
@@ -819,7 +821,7 @@ int launch_softmax_bwd(const RowParams& p, hipStream_t st) {
     const dim3 block(256);
     if (p.x_stride != 1 && p.x_size != 1) {
         const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input);
-        if (p.x_size <= kFewRowsBwd) {
+        if (p.x_size <= kFewRowsBwd<T>) {
             if (vec) hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, kV>), few_rows_grid(p, kV), block, 0, st, p);
             else hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, 1>), few_rows_grid(p, 1), block, 0, st, p);
             return static_cast<int>(hipGetLastError());
