@@ -245,6 +245,27 @@ def test_softmax_of_a_transposed_view_and_large_values(device):
     parity.close(out, rowops.softmax_forward(parity.to64(big), 1), torch.float32, "large values")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("shape,dim", [((5, 100), 1), ((5, 128), 1), ((3, 4096), 1), ((3, 2047), 1), ((2, 20000), 1), ((9, 33), 0), ((40, 64), 0),
+                                       ((300, 33), 0), ((3000, 64), 0)])
+def test_softmax_of_elements_far_from_zero(shape, dim, masked, dtype, device):
+    """Rows and columns around a large number, as masks that fill with one leave them: all alike, differences of a few units,
+    sizes around that from which the maximum is subtracted before the product with log2 e, and such elements among ordinary ones."""
+    x, g = _pair(shape, 193)
+    g = g.to(dtype)
+    mask = _build_mask(shape, 194) if masked else None
+    for centre in (-1e9, 1e9, -1e10, 1e10, -1e30, -2e38, 2e38):
+        _softmax_case(device, torch.full(shape, centre, dtype=dtype), g, dim, dtype, mask, f"{centre}")
+    for centre in (3e6, -1.04e9, 1.04e9, -1e10, 1e38):
+        _softmax_case(device, (x.double() + centre).to(dtype), g, dim, dtype, mask, f"around {centre}")
+    place = torch.arange(shape[dim]).view((-1, 1) if dim == 0 else (1, -1))
+    for fill in (-1e9, -1e10, -1e30):
+        _softmax_case(device, torch.where(place >= 7, fill, x).to(dtype), g, dim, dtype, mask, f"{fill} from the eighth on")
+    lines = torch.arange(shape[1 - dim]).view((1, -1) if dim == 0 else (-1, 1))
+    _softmax_case(device, torch.where(lines % 2 == 0, -1e20, x).to(dtype), g, dim, dtype, mask, "every other one far")
+
+
 # ------------------------------------------------------------------ dropout
 @pytest.mark.parametrize("x_size, p", [(256, 0.0), (512, 1.0)])
 def test_dropout_reference_cases(x_size, p, device):

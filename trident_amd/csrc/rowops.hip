@@ -41,9 +41,15 @@ __device__ __forceinline__ bool mask_hit(const void* base, int64_t off) {
 struct Stat {
     float m, l;
 };
-__device__ __forceinline__ float safe(float m) { return m == -INFINITY ? 0.f : m; }
+// Exponents are fma(x, log2 e, -reference(m)) with m, the maximum times log2 e, rounded: a factor common to all exponentials,
+// which the division by their sum takes out again. Half a unit in the last place of m is 64 at 1.6e9 and overflows beyond, so
+// that the reference goes no lower (elements below it are 0 beside any that are not, also where a thread or a wave sees no
+// other), and rows whose maximum is that far from 0 are computed once more with the maximum subtracted from their elements
+// before the product (far_from_zero; a row of nothing but -1e10 would have the sum 0 or infinity).
+__device__ __forceinline__ float reference(float m) { return fmaxf(m, -1.6e9f); }
+__device__ __forceinline__ bool far_from_zero(float m) { return fabsf(m) > 1.5e9f && m > -INFINITY; }
 __device__ __forceinline__ Stat merge(Stat a, Stat b) {
-    const float m = fmaxf(a.m, b.m), ms = safe(m);
+    const float m = fmaxf(a.m, b.m), ms = reference(m);
     return Stat{m, a.l * fast_exp2(a.m - ms) + b.l * fast_exp2(b.m - ms)};
 }
 
@@ -197,6 +203,48 @@ struct RowPlace {
     }
 };
 
+// Softmax of a row or column whose maximum is far from zero, element by element: one of the threads t, t + threads, ... that
+// share it. maximum and sum reduce over them.
+template <typename T, typename M, typename Maximum, typename Sum>
+__device__ __forceinline__ void softmax_far(const RowParams& p, int64_t base, int64_t stride, int64_t size, int t, int threads, Maximum maximum, Sum sum) {
+    const auto element = [&](int64_t i) {
+        const int64_t at = base + i * stride;
+        return mask_hit<M>(p.mask, at) ? -INFINITY : to_f32(static_cast<const T*>(p.input)[at]);
+    };
+    float m = -INFINITY, l = 0.f;
+#pragma unroll 1
+    for (int64_t i = t; i < size; i += threads) m = fmaxf(m, element(i));
+    m = maximum(m);
+    const float ms = m == -INFINITY ? 0.f : m;
+#pragma unroll 1
+    for (int64_t i = t; i < size; i += threads) l += fast_exp2((element(i) - ms) * kLog2e);
+    const float inv = 1.f / sum(l);
+#pragma unroll 1
+    for (int64_t i = t; i < size; i += threads)
+        static_cast<T*>(p.output)[base + i * stride] = from_f32<T>(fast_exp2((element(i) - ms) * kLog2e) * inv);
+}
+
+// Reduction over the lanes of a wave from distance `from` up to `to`, and over the waves of the workgroup through LDS if there are
+// several.
+template <typename Op>
+__device__ __forceinline__ float reduce(float x, int from, int to, int waves, float* shared, Op op) {
+    for (int d = from; d < to; d <<= 1) x = op(x, __shfl_xor(x, d));
+    if (waves > 1) {
+        __syncthreads();  // (what was there has been read)
+        if ((threadIdx.x & 63) == 0) shared[threadIdx.x >> 6] = x;
+        __syncthreads();
+        x = shared[0];
+        for (int w = 1; w < waves; ++w) x = op(x, shared[w]);
+    }
+    return x;
+}
+struct MaxOp {
+    __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+struct SumOp {
+    __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+
 // PIECES: the mask, too, starts on a 16-byte boundary; otherwise it alone is read element by element (bf16 4096 x 8192, uint8
 // mask one byte off: 0.0305 ms, with everything read so 0.0750; 16384 x 1024 0.0180 and 0.0347).
 template <typename T, int V, int G, bool SHIFT, typename M, bool PIECES = true>
@@ -239,7 +287,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_rows_kernel(const RowParams p
                 for (int e = 0; e < V; ++e) mx = fmaxf(mx, held[k].get(e));
                 held[k].hide();
             }
-        const float m = fmaxf(s.m, mx * kLog2e), ms = safe(m);
+        const float m = fmaxf(s.m, mx * kLog2e), ms = reference(m);
         float l = s.l * fast_exp2(s.m - ms);
 #pragma unroll
         for (int k = 0; k < kHeld; ++k)
@@ -257,7 +305,15 @@ __global__ __launch_bounds__(256) void softmax_fwd_rows_kernel(const RowParams p
         __syncthreads();
         s = merge(merge(part[0], part[1]), merge(part[2], part[3]));
     }
-    const float ms = safe(s.m), inv = 1.f / s.l;  // a fully masked row: 0 * inf = NaN, as softmax gives
+    if (__builtin_amdgcn_ballot_w64(far_from_zero(s.m)) != 0) {  // (G == 256: the same in all waves)
+        constexpr int kLanes = G < 64 ? G : 64;
+        float* const shared = &part[0].m;
+        softmax_far<T, M>(p, row.at0 + row.shift, 1, row.live ? p.x_size : 0, row.t, G,
+                          [&](float x) { return reduce(x, 1, kLanes, G / kLanes, shared, MaxOp{}); },
+                          [&](float x) { return reduce(x, 1, kLanes, G / kLanes, shared, SumOp{}); });
+        return;
+    }
+    const float ms = reference(s.m), inv = 1.f / s.l;  // a fully masked row: 0 * inf = NaN, as softmax gives
     for (int64_t c0 = 0; c0 < row.pieces; c0 += G * kHeld) {
         if (row.pieces > G * kHeld) load(c0);
 #pragma unroll
@@ -344,6 +400,7 @@ constexpr int kColHeldBwd = 8;      // backward: of each of its two inputs
 
 struct ColPlace {
     int lane, group, groups;  // lane position in the panel, row group of this thread and their number
+    int64_t first;            // the panel's first column
     int64_t base;             // element offset of this thread's first column
     bool live;
 };
@@ -354,7 +411,8 @@ __device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int la
     c->lane = threadIdx.x & ((1 << lanes_log2) - 1);
     c->group = threadIdx.x >> lanes_log2;
     c->groups = blockDim.x >> lanes_log2;
-    const int64_t col = ((panel << lanes_log2) + c->lane) * v;
+    c->first = (panel << lanes_log2) * v;
+    const int64_t col = c->first + c->lane * v;
     c->live = col < p.y_size;
     c->base = c->live ? col * p.y_stride : 0;
     return true;
@@ -421,7 +479,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
             float mx = held[0].get(e);
 #pragma unroll
             for (int k = 1; k < kColHeld; ++k) mx = fmaxf(mx, held[k].get(e));
-            const float m = fmaxf(s[e].m, mx * kLog2e), ms = safe(m);
+            const float m = fmaxf(s[e].m, mx * kLog2e), ms = reference(m);
             float l = s[e].l * fast_exp2(s[e].m - ms);
 #pragma unroll
             for (int k = 0; k < kColHeld; ++k) l += fast_exp2(fmaf(held[k].get(e), kLog2e, -ms));
@@ -443,12 +501,25 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
     for (int i = threadIdx.x; i < columns; i += blockDim.x) {
         Stat t = part[i];
         for (int w = 1; w < waves; ++w) t = merge(t, part[w * columns + i]);
-        part[i] = Stat{safe(t.m), 1.f / t.l};  // a fully masked column: 0 * inf = NaN, as softmax gives
+        part[i] = Stat{t.m, 1.f / t.l};  // a fully masked column: 0 * inf = NaN, as softmax gives
     }
     __syncthreads();
-    if (!c.live) return;
+    bool far = false;
 #pragma unroll
-    for (int e = 0; e < V; ++e) s[e] = part[c.lane * V + e];
+    for (int e = 0; e < V; ++e) {
+        s[e] = part[c.lane * V + e];
+        far |= far_from_zero(s[e].m);
+        s[e].m = reference(s[e].m);
+    }
+    if (__builtin_amdgcn_ballot_w64(far) != 0) {  // (a wave has all columns of the panel: the same in all waves)
+        float* const shared = &part[0].m;
+        for (int i = 0; i < columns && c.first + i < p.y_size; ++i)
+            softmax_far<T, M>(p, (c.first + i) * p.y_stride, p.x_stride, p.x_size, threadIdx.x, blockDim.x,
+                              [&](float x) { return reduce(x, 1, 64, waves, shared, MaxOp{}); },
+                              [&](float x) { return reduce(x, 1, 64, waves, shared, SumOp{}); });
+        return;
+    }
+    if (!c.live) return;
     for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
         if (p.x_size > sweep) load(r0);
         ColWalk w(p, c, r0);
@@ -564,6 +635,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
             }
     }
     float ms[V], l[V];
+    bool far = false;
 #pragma unroll
     for (int e = 0; e < V; ++e) {
         ms[e] = -INFINITY;
@@ -577,7 +649,15 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
             held[k].hide();
         }
 #pragma unroll
-    for (int e = 0; e < V; ++e) ms[e] = safe(ms[e] * kLog2e);
+    for (int e = 0; e < V; ++e) {
+        far |= far_from_zero(ms[e] * kLog2e);
+        ms[e] = reference(ms[e] * kLog2e);
+    }
+    if (__builtin_amdgcn_ballot_w64(far) != 0) {
+        const auto own = [](float x) { return x; };
+        for (int e = 0; e < V; ++e) softmax_far<T, M>(p, base + e * p.y_stride, p.x_stride, p.x_size, 0, 1, own, own);
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < kFewRows; ++k)
         if (k < rows) {
