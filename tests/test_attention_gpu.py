@@ -1028,15 +1028,28 @@ def test_config3_full_size_properties(device):
 
 
 # ------------------------------------------------------------------ padded masks
-@pytest.mark.parametrize("kind", ["bool keys", "bool", "f32", "16 bit", "16 bit+dropout", "bool keys+dropout"])
+def _assert_padded_mask_family(prepared, query, dropout_p):
+    """Forward, dK/dV and dQ of a call with this prepared mask run on the 16-bit matrix-core kernels."""
+    import ctypes
+    from trident_amd import _lib, operation
+    lse = torch.empty(query.shape[:3], dtype=torch.float32, device=query.device)
+    args = operation._make_args(query, query, query, query, lse, None, dropout_p, False, 0.1, 0, 0, query, query, query, query, None, lse)
+    prepared.describe(args)
+    assert [_lib.lib().tri_attn_uses_matrix_cores(ctypes.byref(args), which) for which in (0, 1, 2)] == [1, 1, 1]
+
+
+@pytest.mark.parametrize("kind", ["bool keys", "bool", "f32", "f32 length", "16 bit", "f32+dropout", "16 bit+dropout", "bool keys+dropout"])
 @pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 1, 64), (torch.float16, 65, 64), (torch.bfloat16, 129, 128),
                                        (torch.float16, 255, 128), (torch.bfloat16, 321, 64), (torch.float16, 200, 32),
                                        (torch.bfloat16, 333, 16), (torch.bfloat16, 384, 64), (torch.float16, 577, 128)])
-def test_masks_at_any_length(dtype, S, D, kind, device):
+def test_masks_at_any_length(dtype, S, D, kind, device, monkeypatch):
     """Boolean masks and additive ones at lengths that are no multiple of 128 go through tri_attn_prepare_mask to the 16-bit
     kernels with boundary handling: a single key, one key beyond a tile, beyond a workgroup's rows, whole waves without
-    rows, blocks of keys that are masked out behind the last active one (classes), dropout."""
+    rows, blocks of keys that are masked out behind the last active one (classes), dropout. (Small calls hand additive masks over
+    unpadded: the threshold is taken away.)"""
+    from trident_amd import operation
     from trident_amd.operation import Attention, _BooleanMask
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
     q, k, v, d_o = _gen((2, 3, S, D), 5200 + S + D, dtype)
     g = torch.Generator().manual_seed(S)
     p = 0.2 if "dropout" in kind else 0.0
@@ -1046,11 +1059,20 @@ def test_masks_at_any_length(dtype, S, D, kind, device):
         keep[..., 0] = True
         mask = torch.zeros(keep.shape).masked_fill(~keep, float("-inf"))
         given = _BooleanMask(keep.to(device))
+    elif "length" in kind:  # (blocks of all three classes)
+        mask = torch.zeros(2, 1, S, S)
+        mask[0, :, :, (3 * S + 3) // 4:] = float("-inf")
+        mask[1, :, :, (S + 1) // 2:] = float("-inf")
+        given = mask.to(device)
     else:
-        mask = torch.randn(1, 3, S, S, generator=g).to(torch.float32 if kind == "f32" else dtype)
+        mask = torch.randn(1, 3, S, S, generator=g).to(torch.float32 if "f32" in kind else dtype)
         given = mask.to(device)
     scale, rng = 1.0 / math.sqrt(D), (31, 2) if p > 0 else (0, 0)
     tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    prepared = operation._prepared_mask(given, tq)
+    assert (prepared is None) == ("bool" not in kind and S % 128 == 0)
+    if prepared is not None:
+        _assert_padded_mask_family(prepared, tq, p)
     o, lse = Attention._forward(tq, tk, tv, given, p, False, scale, *rng)
     dq, dk, dv, _ = Attention._backward(tdo, tq, tk, tv, o, lse, given, scale, p, False, *rng, False)
     kw = dict(mask=mask, dropout_p=p, is_causal=False, scale=scale, seed=rng[0], offset=rng[1])
@@ -1061,6 +1083,63 @@ def test_masks_at_any_length(dtype, S, D, kind, device):
     parity.close(dq, dq_r, dtype, f"{kind} dQ", a_dq)
     parity.close(dk, dk_r, dtype, f"{kind} dK", a_dk)
     parity.close(dv, dv_r, dtype, f"{kind} dV", a_dv)
+
+
+@pytest.mark.parametrize("kind", ["bool keys", "f32", "16 bit"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 4161, 64), (torch.float16, 4161, 128)])
+def test_padded_masks_of_more_tiles_than_a_class_word_holds(dtype, S, D, kind, device, monkeypatch):
+    """66 key tiles: the kernels then read every block of the mask."""
+    from trident_amd import operation
+    from trident_amd.operation import Attention, _BooleanMask
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    q, k, v, d_o = _gen((1, 1, S, D), 5300 + D, dtype)
+    keep = torch.ones(1, 1, 1 if "keys" in kind else S, S, dtype=torch.bool)
+    keep[..., 3000:] = False
+    mask = torch.zeros(keep.shape, dtype=dtype if kind == "16 bit" else torch.float32).masked_fill(~keep, float("-inf"))
+    given = _BooleanMask(keep.to(device)) if kind == "bool keys" else mask.to(device)
+    scale = 1.0 / math.sqrt(D)
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    _assert_padded_mask_family(operation._prepared_mask(_BooleanMask(keep.to(device)) if kind == "bool keys" else given, tq), tq, 0.0)
+    o, lse = Attention._forward(tq, tk, tv, given, 0.0, False, scale, 0, 0)
+    dq, dk, dv, _ = Attention._backward(tdo, tq, tk, tv, o, lse, given, scale, 0.0, False, 0, 0, False)
+    kw = dict(mask=mask.float(), dropout_p=0.0, is_causal=False, scale=scale)
+    parity.close(o, parity.oracle_forward(q, k, v, **kw)[0], dtype, f"{kind} O")
+    dq_r, dk_r, dv_r, _, _ = parity.oracle_backward(q, k, v, d_o, o=o, **kw)
+    _, a_dq, a_dk, a_dv = parity.oracle_abs_sums(q, k, v, d_o, o=o, **kw)
+    parity.close(dq, dq_r, dtype, f"{kind} dQ", a_dq)
+    parity.close(dk, dk_r, dtype, f"{kind} dK", a_dk)
+    parity.close(dv, dv_r, dtype, f"{kind} dV", a_dv)
+
+
+@pytest.mark.parametrize("kind", ["bool keys", "f32", "16 bit+dropout", "f32 shared, learned"])
+@pytest.mark.parametrize("dtype,S,D", [(torch.float16, 333, 64), (torch.bfloat16, 200, 128)])
+def test_padded_masks_on_strided_views_and_twice_backward(dtype, S, D, kind, device, monkeypatch):
+    """[B,S,H,D] tensors seen as [B,H,S,D] give the bits of dense ones, and so does a second backward through the kept graph."""
+    from trident_amd import operation
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    monkeypatch.setattr(trident.config, "dropout_seed", None)
+    shape = (2, 3, S, D)
+    q, k, v, d_o = [x.to(device) for x in _gen(shape, 5400 + S, dtype)]
+    if kind == "bool keys":
+        mask = (torch.arange(S) < S - 70).view(1, 1, 1, S).to(device)
+    else:
+        mask = torch.randn((1, 3, S, S) if "shared" in kind else (2, 1, S, S), generator=torch.Generator().manual_seed(S))
+        mask = mask.to(dtype if "16 bit" in kind else torch.float32).to(device)
+    learned = "learned" in kind
+    results = []
+    for strided in (False, True):
+        tensors = [x.transpose(1, 2).contiguous().transpose(1, 2) if strided else x.clone() for x in (q, k, v)]
+        trident.config.dropout_seed = (11, 0)
+        inputs = [x.requires_grad_(True) for x in tensors] + ([mask.clone().requires_grad_(True)] if learned else [])
+        out = trident.function.scaled_dot_product_attention(*inputs[:3], inputs[3] if learned else mask, 0.2 if "dropout" in kind else 0.0)
+        first = torch.autograd.grad(out, inputs, d_o, retain_graph=True)
+        second = torch.autograd.grad(out, inputs, d_o)
+        for a, b in zip(first, second):
+            assert torch.equal(a, b)
+        results.append((out.detach(), *first))
+    for name, a, b in zip(("O", "dQ", "dK", "dV", "dMask"), *results):
+        assert torch.equal(a, b), name
 
 
 @pytest.mark.parametrize("source", [torch.bool, torch.float32, torch.bfloat16])
@@ -1175,14 +1254,18 @@ def test_padded_masks_of_large_finite_values(dtype, mask_dtype, S, D, value, sha
 
 
 # ------------------------------------------------------------------ mask gradients summed over batches and heads
+@pytest.mark.parametrize("padded", [False, True])
 @pytest.mark.parametrize("shape", ["1HSS", "B1SS", "11SS"])
 @pytest.mark.parametrize("dtype,mask_dtype,B,H,S,D", [(torch.bfloat16, torch.bfloat16, 3, 2, 1, 64), (torch.float16, torch.float32, 2, 3, 31, 16),
                                                       (torch.bfloat16, torch.float32, 5, 2, 65, 32), (torch.bfloat16, torch.bfloat16, 2, 2, 130, 128),
                                                       (torch.float16, torch.float16, 2, 2, 256, 64), (torch.bfloat16, torch.float16, 2, 20, 260, 64)])
-def test_mask_gradient_of_a_shared_mask(dtype, mask_dtype, B, H, S, D, shape, device):
-    """tri_attn_bwd_dmask: one row, lengths that end inside a key block, a key tile and a row block, store pieces that are not
+def test_mask_gradient_of_a_shared_mask(dtype, mask_dtype, B, H, S, D, shape, padded, device, monkeypatch):
+    """tri_attn_bwd_dmask beside passes that read the mask as it is, and beside ones that read a padded copy: one row, lengths that end inside a key block, a key tile and a row block, store pieces that are not
     aligned, more and fewer pairs than waves, enough tiles for one row block per wave (the last case with 1HSS: 20 x 5 x 3
     workgroups) and too few; the same bits twice."""
+    if padded:
+        from trident_amd import operation
+        monkeypatch.setattr(operation, "_PADS_FROM", 0)
     q, k, v, d_o = _gen((B, H, S, D), 6100 + S + D, dtype)
     mshape = {"1HSS": (1, H, S, S), "B1SS": (B, 1, S, S), "11SS": (1, 1, S, S)}[shape]
     mask = (0.5 * torch.randn(mshape, generator=torch.Generator().manual_seed(S))).to(mask_dtype)
