@@ -378,6 +378,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
 // not stored), a wave without a single row of its own only fetches and meets the barriers.
 template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false>
 __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p) {
+    static_assert(!RAGGED || D == 128, "boundary handling: D = 128 only");
     using Tile = SwzTile<D>;
     constexpr int NW = 8;
     constexpr int kRows = 32 * NW;
@@ -519,7 +520,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     // Without dropout the subtraction in dS = P (dP - delta) is left to the matrix pipe: the dP^T accumulators start from
     // delta and take the product with the dO rows negated (delta - dP^T); dS^T comes out negated and the sign goes into
     // the scale of the final store.
-    constexpr bool kDeltaInAcc = !DROPOUT && !(RAGGED && D == 128);  // (boundary handling leaves no registers for it at D = 128)
+    constexpr bool kDeltaInAcc = !DROPOUT && !RAGGED;  // (boundary handling leaves no registers for it)
     f32x16 dlt16;
     if constexpr (kDeltaInAcc) {
 #pragma unroll
@@ -746,13 +747,14 @@ int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
         else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
         return static_cast<int>(hipGetLastError());
     }
-    if (with_delta) {
-        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
-        else if constexpr (D < 128 || NW == 4) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
-        else return TRI_ATTN_ESHAPE;  // (eight waves without dropout: the phased kernel)
-    } else if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-    else if constexpr (D < 128 || NW == 4) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
-    else return TRI_ATTN_ESHAPE;
+    constexpr bool kDropoutOnly = D == 128 && NW == 8;  // (eight waves without dropout: the phased kernel)
+    if (kDropoutOnly || p.thr8 > 0) {
+        if (with_delta) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true, false, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+    } else if constexpr (!kDropoutOnly) {
+        if (with_delta) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true, false, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+    }
     return static_cast<int>(hipGetLastError());
 }
 
@@ -778,8 +780,12 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
     }
     if constexpr (MASK == kNoMask && D >= 64) {
-        if (dq_is_phased<D, MASK>(p)) return p.S % 256 == 0 ? launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta)
-                                                           : launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);
+        if (dq_is_phased<D, MASK>(p)) {
+            if constexpr (D == 128) {
+                if (p.S % 256 != 0) return launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);
+            }
+            return launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta);
+        }
     }
     if (with_delta && MASK != kNoMask) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
     // 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows)
