@@ -170,8 +170,8 @@ int tri_attn_bwd_dmask(const TriAttnArgs* args);
 
 /* The whole backward (trident/operation/attention.py:137-202): the results of bwd_delta, bwd_dkdv and
  * bwd_dq called in that order, written to delta, dk, dv, dq[, dmask]. The library may launch fewer
- * kernels and in another order: without a mask, for sequence lengths that are multiples of 256 (and
- * without dropout at D = 128) the dQ kernel computes delta on its way and runs before dK/dV. */
+ * kernels and in another order: where tri_attn_bwd_dq_delta applies (16-bit matrix-core kernels
+ * without a mask, any S) the dQ kernel computes delta on its way and runs before dK/dV. */
 int tri_attn_bwd(const TriAttnArgs* args);
 
 /* tri_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving

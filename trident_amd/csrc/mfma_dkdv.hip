@@ -886,13 +886,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
                 lds_direct_load16(g_from, Tile::src_off_clamped(kb + 4, lane, grow_bytes, last), slot + kHalfBytes + (kb + 4) * 1024);
                 lds_direct_load4(((kb & 1) ? delta_base : lse_base) + from, min(lane & 31, last) * 4, slot + aux_lds);
             } else {
-            lds_direct_load16(next_q, qoff, slot + kb * 1024);
-            lds_direct_load16(next_g, goff, slot + kHalfBytes + kb * 1024);
-            lds_direct_load16(next_q + 16 * qrow_bytes, qoff, slot + (kb + 4) * 1024);
-            lds_direct_load16(next_g + 16 * grow_bytes, goff, slot + kHalfBytes + (kb + 4) * 1024);
-            int aux = threadIdx.x & 31;
-            if constexpr (RAGGED) asm volatile("" : "+v"(aux));
-            lds_direct_load4(next_aux, aux * 4, slot + aux_lds);
+                lds_direct_load16(next_q, qoff, slot + kb * 1024);
+                lds_direct_load16(next_g, goff, slot + kHalfBytes + kb * 1024);
+                lds_direct_load16(next_q + 16 * qrow_bytes, qoff, slot + (kb + 4) * 1024);
+                lds_direct_load16(next_g + 16 * grow_bytes, goff, slot + kHalfBytes + (kb + 4) * 1024);
+                int aux = threadIdx.x & 31;
+                if constexpr (RAGGED) asm volatile("" : "+v"(aux));
+                lds_direct_load4(next_aux, aux * 4, slot + aux_lds);
             }
         }
         next_block += 2;
