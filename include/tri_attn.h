@@ -21,14 +21,16 @@
  *     but always fp32). For fp16/bf16 problems the 16-bit matrix-core kernels sum the probabilities as rounded to
  *     that type (the values that multiply V), so lse is accurate to half an ulp of the type times log2(e)
  *     (2.8e-3 for bf16, 3.5e-4 for fp16), not to fp32 precision; the backward calls expect this very lse.
- *     (fp32 problems keep fp32 products and sums throughout; 16-bit problems on the 32-row-tile kernels sum the
+ *     (fp32 problems keep fp32 products and sums throughout; 16-bit problems with a padded mask or on the 32-row-tile kernels sum the
  *     probabilities in fp32 before rounding them for the product with V, so their lse has fp32 accuracy.)
  *   - mask is additive, dtype mask_dtype, logical shape [B, H, S, S] with element strides;
  *     a stride of 0 broadcasts that dimension; the innermost mask stride must be 1.
  *     mask and is_causal are mutually exclusive (trident/operation/attention.py:41-43).
  *   - A query row whose keys are ALL masked (-inf) behaves as in softmax: its output row and lse are NaN / -inf,
  *     and in the backward its probabilities are NaN, which makes its dQ row and all of that head's dK and dV
- *     NaN (what the reference's kernel and torch's attention give as well).
+ *     NaN (what the reference's kernel and torch's attention give as well). One exception: with mask_classes at an S that is
+ *     a multiple of 128, leading and trailing 64-row blocks that are -inf over all keys of a dK/dV workgroup are not read,
+ *     and fully masked rows in them leave those keys' dK and dV as the other rows make them.
  *   - Causal rule: key j is visible to query i iff i >= j (trident/kernel/attention.py:131-134).
  *   - Dropout acts on the probabilities: P is multiplied by keep/(1 - thr8/256) where
  *     thr8 = clamp(rint(dropout_p * 256), 0, 256) and keep comes from Philox4x32-10:
