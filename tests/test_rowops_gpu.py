@@ -127,6 +127,24 @@ def test_softmax_with_a_mask_off_the_16_byte_boundaries(x_size, mask_dtype, dtyp
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mask_dtype", [torch.uint8, torch.bool, torch.bfloat16, torch.int32, torch.int64])
+@pytest.mark.parametrize("x_size", [1280, 4096, 4100, 8192, 8193, 8200, 16384, 24584])
+def test_masked_softmax_of_long_rows(x_size, mask_dtype, dtype, device):
+    """Rows that a workgroup just holds, and rows of two to six sweeps, whole vectors and shifted ones, masks that a thread keeps
+    as they lie in memory and as bits; every byte but 0 of a uint8 mask counts."""
+    x, g = _pair((3, x_size), 198, dtype)
+    mask = _build_mask((3, x_size), 199)
+    given = mask.to(mask_dtype)
+    if mask_dtype == torch.uint8:
+        given = given * torch.randint(1, 256, given.shape, generator=torch.Generator().manual_seed(1)).to(torch.uint8)
+    tx = (x * 3).to(device).requires_grad_(True)
+    out = trident.function.masked_softmax(tx, given.to(device), 1)
+    out.backward(g.to(device))
+    parity.close(out, rowops.softmax_forward(parity.to64((x * 3).to(dtype)), 1, mask.numpy()), dtype, f"{x_size} {mask_dtype} out")
+    parity.close(tx.grad, rowops.softmax_backward(parity.to64(out), parity.to64(g), 1), dtype, f"{x_size} {mask_dtype} grad")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows", [1, 2, 4, 5, 8, 9, 15, 16, 17])
 @pytest.mark.parametrize("cols,mask_dtype", [(40, None), (1031, torch.uint8), (2056, torch.int64), (4104, torch.float32)])
 def test_softmax_down_a_few_rows(rows, cols, mask_dtype, dtype, device):
