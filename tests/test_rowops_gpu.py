@@ -167,6 +167,20 @@ def test_softmax_down_a_few_rows(rows, cols, mask_dtype, dtype, device):
     parity.close(tx.grad[:, live], gradient, dtype, f"{rows} rows grad")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("mask_dtype", [None, torch.uint8, torch.int64])
+@pytest.mark.parametrize("rows,cols", [(18, 40), (31, 1031), (32, 2048), (33, 2048), (3, 524288), (16, 524296), (2, 524287), (17, 262144), (17, 262152)])
+def test_softmax_down_a_few_rows_of_many_columns(rows, cols, mask_dtype, dtype, device):
+    """The lengths and widths at which columns change between one per thread, whole vectors of them and panels."""
+    x, g = _pair((rows, cols), 175 + rows, dtype)
+    mask = None if mask_dtype is None else _build_mask((rows, cols), 176)
+    tx = (x * 3).to(device).requires_grad_(True)
+    out = trident.function.softmax(tx, 0) if mask is None else trident.function.masked_softmax(tx, mask.to(mask_dtype).to(device), 0)
+    out.backward(g.to(device))
+    parity.close(out, rowops.softmax_forward(parity.to64((x * 3).to(dtype)), 0, None if mask is None else mask.numpy()), dtype, f"{rows} x {cols} out")
+    parity.close(tx.grad, rowops.softmax_backward(parity.to64(out), parity.to64(g), 0), dtype, f"{rows} x {cols} grad")
+
+
 def _milliseconds(run):
     for _ in range(3):
         run()

@@ -144,6 +144,7 @@ struct MaskPiece {
             else if (live && mask_hit<M>(base, off + e)) bits |= 1u << e;
         }
     }
+    __device__ __forceinline__ void clear() { load(nullptr, 0, 0, 0); }  // nothing masked
     // masked elements: -inf
     template <typename T>
     __device__ __forceinline__ void apply(Piece<T, V>& piece) const {
@@ -518,12 +519,27 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
         }
         if constexpr (!std::is_same<M, void>::value) {
             ColWalk m(p, c, r0);
+            if constexpr (V == 8) {  // (bits, one piece at a time: there are no registers left for more)
 #pragma unroll
-            for (int k = 0; k < kColHeld; ++k, m.next()) {
-                const uint32_t hit = m.exists() ? mask_bits<M, V>(p.mask, c.base + m.at) : 0u;
+                for (int k = 0; k < kColHeld; ++k, m.next()) {
+                    const uint32_t hit = m.exists() ? mask_bits<M, V>(p.mask, c.base + m.at) : 0u;
 #pragma unroll
-                for (int e = 0; e < V; ++e)
-                    if (hit >> e & 1) held[k].set(e, -INFINITY);
+                    for (int e = 0; e < V; ++e)
+                        if (hit >> e & 1) held[k].set(e, -INFINITY);
+                }
+            } else {
+                constexpr int kGroup = 4;
+                MaskPiece<M, V> masks[kGroup];
+#pragma unroll
+                for (int k = 0; k < kColHeld; k += kGroup) {
+#pragma unroll
+                    for (int i = 0; i < kGroup; ++i, m.next()) {
+                        if (m.exists()) masks[i].load(p.mask, c.base + m.at);
+                        else masks[i].clear();
+                    }
+#pragma unroll
+                    for (int i = 0; i < kGroup; ++i) masks[i].apply(held[k + i]);
+                }
             }
         }
     };
@@ -666,11 +682,11 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
 // beyond the last row are skipped by branches the whole launch takes. 2 x 4194304, bf16: forward 0.0835 ms in panels ->
 // 0.0093, backward 0.0231 -> 0.0106; fp32 0.0515 -> 0.0134 and 0.0181 -> 0.0158 (a thread per column, as before the panels,
 // 0.0162 and 0.0192). 16 x 1048576, bf16: forward 0.0296 -> 0.0173; backward at 9 rows the same either way (0.0133).
-constexpr int kFewRows = 16;    // (64 registers)
+constexpr int kFewRows = 16;    // (64 registers; 16-bit columns one per thread: 32 rows)
 template <typename T>
 constexpr int kFewRowsBwd = sizeof(T) == 2 ? 8 : 4;  // (of each of its two inputs; fp32 8 x 1048576 0.0178 ms so, in panels 0.0165)
 
-template <typename T, int V, typename M>
+template <typename T, int V, typename M, int ROWS = kFewRows>
 __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowParams p) {
     const int64_t col = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V;
     if (col >= p.y_size) return;
@@ -678,19 +694,21 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
     const T* in = static_cast<const T*>(p.input) + base;
     T* out = static_cast<T*>(p.output) + base;
     const int rows = static_cast<int>(p.x_size);
-    Piece<T, V> held[kFewRows];
+    Piece<T, V> held[ROWS];
 #pragma unroll
-    for (int k = 0; k < kFewRows; ++k)
+    for (int k = 0; k < ROWS; ++k)
         if (k < rows) held[k].load(in + k * p.x_stride);
     if constexpr (!std::is_same<M, void>::value) {
+        MaskPiece<M, V> masks[8];
 #pragma unroll
-        for (int k = 0; k < kFewRows; ++k)
-            if (k < rows) {
-                const uint32_t hit = mask_bits<M, V>(p.mask, base + k * p.x_stride);
+        for (int k = 0; k < ROWS; k += 8) {
 #pragma unroll
-                for (int e = 0; e < V; ++e)
-                    if (hit >> e & 1) held[k].set(e, -INFINITY);
-            }
+            for (int i = 0; i < 8; ++i)
+                if (k + i < rows) masks[i].load(p.mask, base + (k + i) * p.x_stride);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (k + i < rows) masks[i].apply(held[k + i]);
+        }
     }
     float ms[V], l[V];
     bool far = false;
@@ -700,7 +718,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
         l[e] = 0.f;
     }
 #pragma unroll
-    for (int k = 0; k < kFewRows; ++k)
+    for (int k = 0; k < ROWS; ++k)
         if (k < rows) {
 #pragma unroll
             for (int e = 0; e < V; ++e) ms[e] = fmaxf(ms[e], held[k].get(e));
@@ -717,7 +735,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
         return;
     }
 #pragma unroll
-    for (int k = 0; k < kFewRows; ++k)
+    for (int k = 0; k < ROWS; ++k)
         if (k < rows) {
 #pragma unroll
             for (int e = 0; e < V; ++e) l[e] += fast_exp2(fmaf(held[k].get(e), kLog2e, -ms[e]));
@@ -726,7 +744,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_few_rows_kernel(const RowPara
 #pragma unroll
     for (int e = 0; e < V; ++e) l[e] = 1.f / l[e];  // a fully masked column: 0 * inf = NaN, as softmax gives
 #pragma unroll
-    for (int k = 0; k < kFewRows; ++k)
+    for (int k = 0; k < ROWS; ++k)
         if (k < rows) {
             Vec<T, V> o;
 #pragma unroll
@@ -926,10 +944,20 @@ int launch_softmax_fwd(const RowParams& p, hipStream_t st) {
     if (p.x_stride != 1 && p.x_size != 1) {
         // 16-byte accesses across the columns when every element row starts on a 16-byte boundary and holds whole vectors
         const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.input) && aligned16(p.output) && aligned16(p.mask);
+        // Whole vectors where they leave two workgroups and more per CU: below, one column per thread is faster (forward, bf16 16 x
+        // 16384 0.0094 -> 0.0057 ms, 262144 columns 0.0110 -> 0.0079; from 524288 columns on the vectors, 16 x 1048576 0.0180 to 0.0207).
+        // 16-bit columns of up to 32 elements go one per thread, too, with a mask, which the panels work through piece by piece
+        // (bf16 17 x 16384 0.0093 -> 0.0064 ms, 17 x 1048576 0.0363 -> 0.0259), or up to 262144 of them (24 x 1048576 0.0265 in panels).
         if (p.x_size <= kFewRows) {
-            if (vec) hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, kV, M>), few_rows_grid(p, kV), block, 0, st, p);
+            if (vec && p.y_size >= 1 << 19) hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, kV, M>), few_rows_grid(p, kV), block, 0, st, p);
             else hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, 1, M>), few_rows_grid(p, 1), block, 0, st, p);
             return static_cast<int>(hipGetLastError());
+        }
+        if constexpr (sizeof(T) == 2) {
+            if (p.x_size <= 32 && (!std::is_same<M, void>::value || p.y_size <= 1 << 18)) {
+                hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, 1, M, 32>), few_rows_grid(p, 1), block, 0, st, p);
+                return static_cast<int>(hipGetLastError());
+            }
         }
         const ColLaunch c = column_launch(p, vec ? kV : 1, kColHeld);
         const unsigned lds = c.stats * sizeof(Stat);
