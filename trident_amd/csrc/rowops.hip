@@ -180,7 +180,7 @@ private:
 // output; a longer one takes two sweeps, the second of which finds the row in the L2 it was just read through.
 // SHIFT: rows that do not start on 16-byte boundaries (an odd row length): the pieces are those of the tensor, not of the
 // row, and only a row's first and last piece, which it shares with its neighbours, are read and written element by
-// element. Launches in a row, bf16 12288 x 2047 with a uint8 mask: forward 0.0362 ms = 3.5 TB/s, backward 0.0333 ms = 4.5 TB/s; with one element
+// element. Launches in a row, bf16 12288 x 2047 with a uint8 mask: forward 0.0336 ms = 3.7 TB/s, backward 0.0333 ms = 4.5 TB/s; with one element
 // per load, which still serves short odd rows and tensors that are not 16-byte aligned themselves, 0.0545 and 0.0493 ms. Rows on 16-byte
 // boundaries: bf16 65536 x 64 forward 0.0092 ms (a wave per row, most of it idle: 0.0265), fp32 8192 x 1536 backward 0.0226
 // (two sweeps: 0.0362), bf16 16384 x 8192 forward 0.1027 (5.2 TB/s), with the mask 0.134 (one mask byte per load: 0.139).
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
 // panels go to the same XCD: where a panel row is narrower than a 128-byte line, the other half is then still in its L2.
 // The statistics' LDS is sized by the workgroup, so that single-wave ones fill a CU.
 // fp32 4096 x 4096 along dim 0, launches in a row: forward 0.0254 ms = 5.3 TB/s (what a large copy reaches), backward 0.0435 ms =
-// 4.6 TB/s (in a training step, whose four tensors fill the Infinity Cache, 0.032 and 0.069 ms). One
+// 4.6 TB/s (in a training step, whose four tensors fill the Infinity Cache, 0.031 and 0.068 ms). One
 // thread per column, which this replaces, took 2.1 and 2.4 ms: 64 waves in flight on the whole chip, each waiting for one
 // load at a time. (Its sums ran in plain order, too: at 65536 elements off by 7.5e-5, these by 1.8e-7.)
 constexpr int kColHeld = 16;        // forward: pieces a thread keeps (64 registers)
