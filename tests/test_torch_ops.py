@@ -1,0 +1,132 @@
+"""The C++ host path (csrc_torch/torch_ops.cpp) against the Python autograd Functions it stands in for: the same launches, so the
+same bits; and the calls it hands back to them."""
+import pytest
+import torch
+
+import trident_amd as trident
+from trident_amd import _lib, operation
+
+
+def test_calls_that_are_not_plain_are_handed_back():
+    """CPU tensors, subclasses, other argument types: None and no exception (the Python Functions raise what there is to raise)."""
+    ops = _lib.torch_ops()
+    x = torch.zeros(1, 1, 8, 16)
+    for args in ((x, x, x, None, 0.0, False, 0.25), (x, x, None, None, 0.0, False, 0.25), (x, x, x, "mask", 0.0, False, 0.25)):
+        assert ops.attention(*args) is None
+    assert ops.softmax(x[0, 0], None, 1) is None
+    assert ops.dropout(x[0, 0], 0.5) is None
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@pytest.mark.gpu
+def test_watched_calls_are_handed_back(device):
+    ops = _lib.torch_ops()
+    x = torch.zeros(1, 1, 64, 16, dtype=torch.float16, device=device)
+
+    def native(t=x):
+        return ops.attention(t, t, t, None, 0.0, False, 0.25) is not None
+
+    assert native()
+    assert not native(x.as_subclass(_Subclass))
+    with torch.device("cpu"):  # (a torch function mode)
+        assert not native()
+    with torch.autograd.forward_ad.dual_level():
+        assert not native()
+    seen = []
+    torch.func.vmap(lambda t: seen.append(native()) or t)(torch.zeros(2))
+    assert seen == [False]
+    trident.config.use_trace = True
+    try:
+        assert not native()
+    finally:
+        trident.config.use_trace = False
+
+
+def _mask(kind, B, H, S, dtype, device):
+    g = torch.Generator(device=device).manual_seed(S)
+    if kind == "none":
+        return None
+    if kind == "bool":
+        keep = torch.rand(B, 1, 1, S, generator=g, device=device) > 0.3
+        keep[..., 0] = True
+        return keep
+    shape = {"full grad": (B, H, S, S), "shared grad": (1, H, S, S), "keys grad": (B, 1, 1, S), "matrix": (S, S), "length": (B, 1, S, S)}[kind]
+    mask = torch.randn(shape, generator=g, device=device)
+    if kind == "length":
+        mask = torch.zeros(shape, device=device)
+        mask[..., S // 2:] = float("-inf")
+    return (mask.to(dtype) if "grad" in kind else mask).requires_grad_("grad" in kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["none", "bool", "full grad", "shared grad", "keys grad", "matrix", "length"])
+@pytest.mark.parametrize("dtype,S,D,p,layout", [(torch.bfloat16, 128, 64, 0.0, "bhsd"), (torch.float16, 100, 32, 0.2, "bshd"),
+                                                (torch.float32, 65, 16, 0.2, "bhsd"), (torch.bfloat16, 777, 128, 0.0, "bshd")])
+def test_attention_is_the_function_it_stands_in_for(kind, dtype, S, D, p, layout, device, monkeypatch):
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    B, H = 2, 3
+    g = torch.Generator(device=device).manual_seed(S + D)
+    make = (lambda: torch.randn(B, S, H, D, generator=g, device=device).to(dtype).transpose(1, 2)) if layout == "bshd" else \
+        (lambda: torch.randn(B, H, S, D, generator=g, device=device).to(dtype))
+    q, k, v, grad = make().requires_grad_(), make(), make().requires_grad_(), make()
+    mask = _mask(kind, B, H, S, dtype, device)
+    inputs = [q, v] + ([mask] if "grad" in kind else [])
+    results = []
+    for f in (operation.Attention.call, operation.Attention.apply):
+        monkeypatch.setattr(trident.config, "dropout_seed", (5, 1))
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(tuple(t.shape)) or t, lambda t: t):
+            out = f(q, k, v, mask, p, False, 0.125, False)
+        first = torch.autograd.grad(out, inputs, grad, retain_graph=True)
+        results.append(([out.detach(), *first], packed))
+        for a, b in zip(first, torch.autograd.grad(out, inputs, grad)):
+            if a is not first[-1] or kind != "keys grad":  # (that gradient is added up atomically)
+                assert torch.equal(a, b)
+        with torch.no_grad():
+            monkeypatch.setattr(trident.config, "dropout_seed", (5, 1))
+            assert torch.equal(f(q, k, v, mask, p, False, 0.125, False), out)
+    assert results[0][1] == results[1][1]
+    for n, (a, b) in enumerate(zip(results[0][0], results[1][0])):
+        assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride()
+        if kind == "keys grad" and n == 3:
+            assert (a - b).abs().max() <= 1e-2 * b.abs().max()  # (fp32 atomic adds in another order, rounded to the mask's type)
+        else:
+            assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,dim", [((40, 33), 0), ((40, 33), 1), ((40, 33), None), ((3, 5, 16), -1)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_row_operations_are_the_functions_they_stand_in_for(shape, dim, masked, device, monkeypatch):
+    g = torch.Generator(device=device).manual_seed(7)
+    x = torch.randn(shape, generator=g, device=device).requires_grad_()
+    grad = torch.randn(shape[::-1], generator=g, device=device).permute(*reversed(range(len(shape))))
+    mask = torch.rand(shape[-1:], generator=g, device=device) > 0.7  # (broadcast over the rows)
+    mask[0] = False
+
+    def run(softmax, dropout):
+        monkeypatch.setattr(trident.config, "dropout_seed", (9, 4))
+        y = softmax()
+        z = dropout(y) if len(shape) == 2 else y
+        return [y.detach(), z.detach(), *torch.autograd.grad(z, x, grad)]
+
+    got = run(lambda: trident.function.masked_softmax(x, mask, dim) if masked else trident.function.softmax(x, dim),
+              lambda y: trident.function.dropout(y, 0.25))
+    want = run(lambda: operation.MaskedSoftmax.apply(x, mask, dim) if masked else operation.Softmax.apply(x, dim),
+               lambda y: operation.Dropout.apply(y, 0.25))
+    for a, b in zip(got, want):
+        assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)) and a.stride() == b.stride()  # (masked out columns: NaN)
+
+
+@pytest.mark.gpu
+def test_a_call_that_fails_raises_as_before(device):
+    x = torch.zeros(1, 1, 64, 16, dtype=torch.float16, device=device)
+    with pytest.raises(RuntimeError, match="dropout_p must lie in"):
+        trident.function.scaled_dot_product_attention(x, x, x, None, 1.5)
+    with pytest.raises(RuntimeError, match="expanded size"):
+        trident.function.scaled_dot_product_attention(x, x, x, torch.zeros(3, 64, device=device))
+    with pytest.raises(RuntimeError, match="dropout_p must lie in"):
+        trident.function.dropout(x[0, 0], 1.5)

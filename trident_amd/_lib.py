@@ -173,6 +173,27 @@ def probe_lib():
     return _probe
 
 
+_torch_ops = None
+
+
+def torch_ops():
+    """The C++ host path (csrc_torch/torch_ops.cpp), bound to the loaded library. Raises if it has not been built."""
+    global _torch_ops
+    if _torch_ops is None:
+        try:
+            from . import _torch_ops as module
+        except ImportError as error:
+            raise RuntimeError("trident_amd/_torch_ops.so is missing or does not fit this torch: build it with "
+                               "`python -m trident_amd.build`") from error
+        from . import config, operation
+
+        library = lib()
+        module.bind(vars(config), vars(operation), {name: ctypes.cast(getattr(library, name), ctypes.c_void_p).value
+                                                    for name in EXPORTS + ROW_EXPORTS})
+        _torch_ops = module
+    return _torch_ops
+
+
 def check(status):
     if status != 0:
         raise RuntimeError("tri_attn: " + lib().tri_attn_strerror(status).decode())

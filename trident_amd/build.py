@@ -1,4 +1,5 @@
-"""Builds libtrident_attn.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc.
+"""Builds libtrident_attn.so (the C-ABI library with the gfx950 kernels) in-tree with hipcc, and _torch_ops.so (the operator's
+host path, csrc_torch/torch_ops.cpp) with the host compiler.
 
     python -m trident_amd.build               # compile every csrc/*.hip and link
     python -m trident_amd.build --resources   # also print the per-kernel register / LDS / scratch table
@@ -21,6 +22,8 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT = os.path.join(HERE, "libtrident_attn.so")
 PROBE_SRC = os.path.join(HERE, "probe", "probe.hip")   # calibration kernels: a library of their own (include/tri_probe.h)
 PROBE_OUT = os.path.join(HERE, "libtri_probe.so")
+TORCH_SRC = os.path.join(HERE, "csrc_torch", "torch_ops.cpp")  # the operator's host path, against torch's C++ interface
+TORCH_OUT = os.path.join(HERE, "_torch_ops.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -126,6 +129,24 @@ def _compile(src):
     return obj, _parse_resources(res.stderr)
 
 
+def _compile_torch_ops():
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-I", INCLUDE,
+           "-isystem", sysconfig.get_paths()["include"]]
+    for path in include_paths("cuda"):
+        cmd += ["-isystem", path]
+    cmd += [TORCH_SRC, "-o", TORCH_OUT, "-L", libs]
+    cmd += ["-l" + name for name in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python")]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"the host compiler failed on {TORCH_SRC}:\n{res.stderr}")
+
+
 def resource_table(resources):
     names = _demangle(sorted(resources))
     rows = sorted(((names[m], r) for m, r in resources.items()), key=lambda x: x[0])
@@ -154,8 +175,10 @@ def check_baseline_kernels(resources):
 def build(verbose=True, resources=False):
     os.makedirs(OBJ_DIR, exist_ok=True)
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 2)) as pool:
+        host = pool.submit(_compile_torch_ops)
         results = list(pool.map(_compile, sources + [PROBE_SRC]))
+        host.result()
     probe_obj = results.pop()[0]
     objs = [o for o, _ in results]
     usage = {}

@@ -1,9 +1,10 @@
-"""Functional entry points (reference: trident/function/function.py:58-67, 166-172, 238-262)."""
+"""Functional entry points (reference: trident/function/function.py:58-67, 166-172, 238-262). Plain calls of the operations run in
+C++ (csrc_torch/torch_ops.cpp); what that returns None for goes through the autograd Functions of operation.py and rowops.py."""
 import math
 
 import torch
 
-from . import operation
+from . import _lib, operation
 
 
 def dropout(input, p=0.5, training=True):
@@ -14,7 +15,8 @@ def dropout(input, p=0.5, training=True):
     """
     if training:
         if input.dim() == 2 and input.numel() > 0:  # (a view of the same shape is two more nodes of the graph)
-            return operation.Dropout.apply(input, p)
+            output = _lib.torch_ops().dropout(input, p)
+            return operation.Dropout.apply(input, p) if output is None else output
         return operation.Dropout.apply(input.view(-1, input.shape[-1]), p).view(input.shape)
     else:
         return input.clone()
@@ -26,7 +28,8 @@ def masked_softmax(input: torch.Tensor, mask: torch.Tensor, dim: int):
 
     See MaskedSoftmax for more details.
     """
-    return operation.MaskedSoftmax.apply(input, mask, dim)
+    output = _lib.torch_ops().softmax(input, mask, dim) if mask is not None else None
+    return operation.MaskedSoftmax.apply(input, mask, dim) if output is None else output
 
 
 def softmax(input: torch.Tensor, dim: int = None):
@@ -35,7 +38,8 @@ def softmax(input: torch.Tensor, dim: int = None):
 
     See Softmax for more details.
     """
-    return operation.Softmax.apply(input, dim)
+    output = _lib.torch_ops().softmax(input, None, dim)
+    return operation.Softmax.apply(input, dim) if output is None else output
 
 
 def scaled_dot_product_attention(

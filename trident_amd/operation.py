@@ -6,7 +6,6 @@ Triton launches of the reference (attention.py:109, 161, 170) become calls into
 libtrident_attn.so (include/tri_attn.h).
 """
 import ctypes
-import weakref
 from typing import Any
 
 import torch
@@ -84,51 +83,24 @@ def _make_args(query, key, value, output, log2sum, mask, dropout_p, is_causal, s
     return args
 
 
-# Classes of a mask's 64 x 64 blocks (tri_attn_classify_mask), kept per mask tensor: the forward call computes them, the
-# backward call and later calls with the same, unmodified tensor (other layers, other steps) find them here. An entry
-# dies with its tensor (weak reference) and is recomputed when the tensor was written to through torch (its version
-# counter moved), when another stream asks for it (no event orders the two), and it is neither made nor used while a
-# stream is being captured (the classification would be recorded, not run). A write that torch does not see (through
+# Classes of a mask's 64 x 64 blocks (tri_attn_classify_mask), kept per mask tensor (csrc_torch/torch_ops.cpp): the forward
+# call computes them, the backward call and later calls with the same, unmodified tensor (other layers, other steps) find
+# them there. An entry ends with its tensor (weak reference) and is recomputed when the tensor was written to through torch
+# (its version counter moved), when another stream asks for it (no event orders the two), and it is neither made nor used
+# while a stream is being captured (the classification would be recorded, not run). A write that torch does not see (through
 # ``.data``, a raw pointer, a graph replay into the mask's memory) leaves stale classes behind, and the kernels skip
 # tiles on their word: such callers set ``config.cache_mask_classes = False`` (every call classifies the mask again)
 # or call ``forget_mask_classes()`` after the write.
-_MASK_CLASSES = {}
-
-
 def forget_mask_classes():
     """Drops every cached block classification (after a write to a mask's memory that torch's version counter did not see)."""
-    _MASK_CLASSES.clear()
+    _lib.torch_ops().forget_mask_classes()
 
 
 def _mask_classes(mask: torch.Tensor, args):
     """Sets args.mask_classes for the mask already described in ``args``; returns the tensor to keep alive, or None
-    where the library has no use for classes (nothing is launched then)."""
-    if args.S % 128 != 0:  # (padded masks bring theirs along; the kernels use no other classes at such lengths)
-        return None
-    lib = _lib.lib()
-    size = lib.tri_attn_mask_classes_size(ctypes.byref(args))
-    if size <= 0:
-        return None
-    use_cache = config.cache_mask_classes and not torch.cuda.is_current_stream_capturing()
-    key = id(mask)
-    entry = _MASK_CLASSES.get(key) if use_cache else None
-    signature = (mask._version, tuple(mask.shape), mask.stride(), mask.dtype, args.B, args.H, args.S, args.mask, args.stream)
-    if entry is not None and entry[0]() is mask and entry[1] == signature:
-        classes = entry[2]
-    else:
-        classes = torch.empty(size, dtype=torch.uint8, device=mask.device)
-        args.mask_classes = classes.data_ptr()
-        status = lib.tri_attn_classify_mask(ctypes.byref(args))
-        if status in (_lib.ENOFUSE, _lib.EALIGN):
-            args.mask_classes = None
-            return None
-        _lib.check(status)
-        if use_cache:
-            if len(_MASK_CLASSES) >= 64:
-                _MASK_CLASSES.clear()
-            _MASK_CLASSES[key] = (weakref.ref(mask, lambda _r, k=key: _MASK_CLASSES.pop(k, None)), signature, classes)
-    args.mask_classes = classes.data_ptr()
-    return classes
+    where the library has no use for classes (nothing is launched then; padded masks bring theirs along, and the kernels use
+    no others at lengths that are no multiple of 128)."""
+    return _lib.torch_ops().mask_classes(mask, ctypes.addressof(args), bool(config.cache_mask_classes))
 
 
 class _BooleanMask:
@@ -247,8 +219,12 @@ class _NoGraph:
 class Attention(torch.autograd.Function):
     @staticmethod
     def call(query, key, value, mask, dropout_p, is_causal, softmax_scale, use_accelerator):
-        """``apply`` with the same arguments, checks and result; when no input asks for a gradient (or gradients are
-        switched off) the forward runs without autograd's bookkeeping, which a small problem would feel."""
+        """``apply`` with the same arguments, checks and result. Plain calls run in C++ (csrc_torch/torch_ops.cpp), which
+        returns None for all others; when no input asks for a gradient (or gradients are switched off) the forward runs
+        without autograd's bookkeeping, which a small problem would feel."""
+        output = _lib.torch_ops().attention(query, key, value, mask, dropout_p, is_causal, softmax_scale)
+        if output is not None:
+            return output
         if torch.is_grad_enabled() and (
             query.requires_grad or key.requires_grad or value.requires_grad or (mask is not None and mask.requires_grad)
         ):
