@@ -127,6 +127,10 @@ typedef struct TriAttnArgs {
                                   mask_stride[0] == 0), MH = H (1 if mask_stride[1] == 0), RB = S/64 (1 if mask_stride[2] == 0);
                                   0 = every entry of the block is 0, 1 = every entry is -inf, 2 = anything else.
                                   Only used where S is a multiple of 128, or with TRI_ATTN_MASK_PADDED (S/64 rounded up). */
+
+    void* workspace;           /* NULL, or scratch memory for this call (16-byte aligned, used until the stream has passed it): with at
+                                  least tri_attn_workspace_size bytes of it, calls of few heads run split along the sequence */
+    int64_t workspace_size;    /* its bytes. A struct_size without these two fields (offsetof(TriAttnArgs, workspace)) is taken too */
 } TriAttnArgs;
 
 /* ABI version of the loaded library (TRI_ATTN_ABI_VERSION it was built with). */
@@ -186,6 +190,14 @@ int tri_attn_bwd(const TriAttnArgs* args);
  * or threads) race on it and must be serialised by the caller; calls on one stream are ordered. */
 #define TRI_ATTN_NOALLOC_MAX_ROWS (1 << 20)
 int tri_attn_bwd_noalloc(const TriAttnArgs* args);
+
+/* Bytes of args->workspace with which a call on these arguments runs split along the streamed dimension, 0 where it never does
+ * (enough heads to fill the GPU, fewer than 20 tiles of 64, kernels other than the 16-bit matrix-core ones), or a negative
+ * TRI_ATTN_E* code. pass 0 = tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq, 3 = tri_attn_bwd (its passes share the
+ * workspace, one after the other). A split call adds the parts' fp32 sums up in a fixed order: its results differ from an
+ * unsplit call's by fp32 rounding, and do not depend on how the GPU schedules it. The reference launches one program per
+ * row or key tile whatever the number of heads (trident/operation/attention.py:106-108). */
+int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass);
 
 /* Classifies the 64 x 64 blocks of args->mask into args->mask_classes (see there; caller-allocated, size
  * tri_attn_mask_classes_size(args) bytes). It has no counterpart in the reference, whose kernel adds every mask

@@ -1,0 +1,156 @@
+"""Launches split along the sequence (few heads, at least 20 tiles of 64) against whole ones and 64-bit results: the operator gives
+its calls a workspace and so splits them, the same call without one does not."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from trident_amd import _lib, operation
+
+pytestmark = pytest.mark.gpu
+
+
+def _exact(q, k, v, d_o, mask, keep, zscale, causal, scale):
+    """O, dQ, dK, dV in 64 bits, head by head."""
+    B, H, S, D = q.shape
+    out = [torch.empty(B, H, S, D, dtype=torch.float64, device=q.device) for _ in range(4)]
+    hidden = torch.ones(S, S, dtype=torch.bool, device=q.device).triu_(1) if causal else None
+    for b in range(B):
+        for h in range(H):
+            qq, kk, vv, g = [x[b, h].double() for x in (q, k, v, d_o)]
+            s = qq @ kk.t() * scale
+            if mask is not None:
+                s += mask.expand(B, H, S, S)[b, h].double()
+            if causal:
+                s.masked_fill_(hidden, -math.inf)
+            p = s.softmax(1)
+            z = keep[b * H + h] * zscale if keep is not None else None
+            pz = p if z is None else p * z
+            dp = g @ vv.t()
+            dp = dp if z is None else dp * z
+            out[0][b, h] = pz @ vv
+            ds = p * (dp - (dp * p).sum(1, keepdim=True))
+            out[1][b, h] = ds @ kk * scale
+            out[2][b, h] = ds.t() @ qq * scale
+            out[3][b, h] = pz.t() @ g
+    return out
+
+
+def _mask(kind, B, H, S, dtype, device):
+    g = torch.Generator(device=device).manual_seed(S)
+    lengths = torch.tensor([S - 70 * i - S // 3 * (i % 2) for i in range(B)], device=device)
+    exists = torch.arange(S, device=device)[None, :] < lengths[:, None]
+    if kind == "bool keys":
+        return exists[:, None, None, :].contiguous()
+    if kind == "length":
+        return torch.zeros(B, 1, S, S, device=device).masked_fill_(~exists[:, None, None, :], -math.inf)
+    if kind == "dense":
+        return torch.randn(B, 1, S, S, generator=g, device=device)
+    if kind == "16 bit":
+        return torch.randn(1, H, S, S, generator=g, device=device).to(dtype)
+    return None
+
+
+def _run(q, k, v, d_o, mask, p, causal, scale, rng, split, monkeypatch):
+    """O, lse, dQ, dK, dV and whether any launch was split."""
+    used = []
+    take = operation._take_workspace
+
+    def spy(args, which, device):
+        workspace = take(args, which, device) if split else None
+        used.append(workspace is not None)
+        return workspace
+
+    with monkeypatch.context() as m:
+        m.setattr(operation, "_take_workspace", spy)
+        m.setattr(operation, "_PADS_FROM", 0)
+        given = operation._BooleanMask(mask) if mask is not None and mask.dtype == torch.bool else mask
+        o, lse = operation.Attention._forward(q, k, v, given, p, causal, scale, *rng)
+        dq, dk, dv, _ = operation.Attention._backward(d_o, q, k, v, o, lse, given, scale, p, causal, *rng, False)
+    return (o, lse, dq, dk, dv), used
+
+
+VARIANTS = ["plain", "causal", "dropout", "causal+dropout", "bool keys", "length", "dense", "16 bit", "bool keys+dropout", "dense+dropout"]
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("dtype,B,H,S,D", [
+    (torch.bfloat16, 1, 2, 2048, 128), (torch.float16, 1, 3, 1281, 128), (torch.bfloat16, 2, 1, 2047, 128), (torch.float16, 1, 1, 4160, 128),
+    (torch.bfloat16, 1, 3, 1345, 64), (torch.float16, 2, 1, 2176, 64), (torch.bfloat16, 1, 1, 5000, 64),
+    (torch.float16, 1, 4, 1343, 32), (torch.bfloat16, 2, 1, 2304, 32), (torch.bfloat16, 1, 2, 1409, 16), (torch.float16, 1, 5, 1920, 16)])
+def test_split_launches(dtype, B, H, S, D, variant, device, monkeypatch):
+    """As close to the 64-bit result as the whole launch: the parts' sums are fp32, what differs is which rounding of P to 16 bits
+    goes with which row maximum (a few per cent of the error; 10 % allowed, and fp32 rounding on top of it)."""
+    p, causal = (0.2 if "dropout" in variant else 0.0), "causal" in variant
+    rng = (77, 3) if p else (0, 0)
+    scale = 1.0 / math.sqrt(D)
+    g = torch.Generator(device=device).manual_seed(S + D)
+    q, k, v, d_o = [torch.randn(B, S, H, D, generator=g, device=device).to(dtype).transpose(1, 2) for _ in range(4)]
+    mask = _mask(variant.split("+")[0], B, H, S, dtype, device)
+    keep = None
+    if p:
+        keep = torch.empty(B * H, S, S, dtype=torch.uint8, device=device)
+        for bh in range(B * H):
+            _lib.check(_lib.lib().tri_attn_dropout_mask(*rng, p, bh, 0, S, 0, S, keep[bh].data_ptr(), torch.cuda.current_stream().cuda_stream))
+    thr = round(p * 256)
+    additive = mask if mask is None or mask.dtype != torch.bool else torch.zeros(mask.shape, device=device).masked_fill(~mask, -math.inf)
+    exact = _exact(q, k, v, d_o, additive, keep, 256 / (256 - thr), causal, scale)
+    whole, used = _run(q, k, v, d_o, mask, p, causal, scale, rng, False, monkeypatch)
+    assert not any(used)
+    split, used = _run(q, k, v, d_o, mask, p, causal, scale, rng, True, monkeypatch)
+    assert all(used), "the call was not split"
+    again, _ = _run(q, k, v, d_o, mask, p, causal, scale, rng, True, monkeypatch)
+    for name, a, b, c in zip(("O", "lse", "dQ", "dK", "dV"), split, whole, again):
+        assert torch.equal(a, c), f"{name} differs between two runs"
+        if name == "lse":
+            assert (a - b).abs().max() <= 2.0 ** -8 * 1.5, name  # (whole launches sum P as rounded, padded masks as it is)
+    for name, a, b, e in zip(("O", "dQ", "dK", "dV"), (split[0], *split[2:]), (whole[0], *whole[2:]), exact):
+        off, off_whole = [((x.double() - e).norm() / e.norm()).item() for x in (a, b)]
+        assert off <= 1.1 * off_whole + 1e-6, (name, off, off_whole)
+        half_ulp = e.abs().max() * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)  # (the result's own rounding)
+        assert (a.double() - e).abs().max() <= 2 * (b.double() - e).abs().max() + half_ulp + 1e-6, name
+
+
+@pytest.mark.parametrize("S,D", [(2048, 64), (1300, 128), (1300, 32), (2176, 128)])
+@pytest.mark.parametrize("where", ["first rows", "last rows", "middle", "one row"])
+def test_rows_without_a_visible_key(S, D, where, device, monkeypatch):
+    """NaN where the whole launch gives NaN, and only there."""
+    dtype = torch.bfloat16
+    g = torch.Generator(device=device).manual_seed(S)
+    q, k, v, d_o = [torch.randn(2, 1, S, D, generator=g, device=device).to(dtype) for _ in range(4)]
+    lost = {"first rows": slice(0, 448), "last rows": slice(S - 400, S), "middle": slice(512, 960), "one row": slice(700, 701)}[where]
+    mask = torch.zeros(2, 1, S, S, device=device)
+    mask[1, :, lost] = -math.inf
+    mask[1, ..., S // 2:] = -math.inf
+    whole, _ = _run(q, k, v, d_o, mask, 0.0, False, 0.125, (0, 0), False, monkeypatch)
+    split, used = _run(q, k, v, d_o, mask, 0.0, False, 0.125, (0, 0), True, monkeypatch)
+    assert all(used)
+    for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), split, whole):
+        assert torch.equal(a.isnan(), b.isnan()), name
+        a, b = a.float().nan_to_num(0.0, neginf=-1e4), b.float().nan_to_num(0.0, neginf=-1e4)
+        assert (a - b).norm() <= 2.0 ** -6 * b.norm(), name
+
+
+def test_workspaces_that_do_not_do(device):
+    """Too small, misaligned or absent (also by the size of the structure): the whole launch, bit for bit."""
+    B, H, S, D = 1, 2, 1400, 64
+    q, k, v = [torch.randn(B, H, S, D, device=device).half() for _ in range(3)]
+    results = []
+    for case in ("none", "small", "misaligned", "old structure"):
+        o, lse = torch.empty_like(q), torch.empty(B, H, S, device=device)
+        args = operation._make_args(q, k, v, o, lse, None, 0.0, True, 0.125, 0, 0)
+        size = _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 0)
+        assert size > 0
+        workspace = torch.empty(size + 16, dtype=torch.uint8, device=device)
+        if case != "none":
+            args.workspace, args.workspace_size = workspace.data_ptr() + (8 if case == "misaligned" else 0), size - (case == "small")
+        if case == "old structure":
+            args.struct_size = _lib.TriAttnArgs.workspace.offset
+        _lib.check(_lib.lib().tri_attn_fwd(ctypes.byref(args)))
+        results.append((o, lse))
+    for o, lse in results[1:]:
+        assert torch.equal(o, results[0][0]) and torch.equal(lse, results[0][1])
+    many = torch.empty(64, 16, 1024, 64, dtype=torch.float16, device=device)
+    args = operation._make_args(many, many, many, many, torch.empty(64, 16, 1024, device=device), None, 0.0, True, 0.125, 0, 0)
+    assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 0) == 0

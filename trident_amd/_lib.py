@@ -55,12 +55,14 @@ class TriAttnArgs(ctypes.Structure):
         ("dmask_stride", _i64x4),
         ("stream", ctypes.c_void_p),
         ("mask_classes", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p),
+        ("workspace_size", ctypes.c_int64),
     ]
 
 
 # TriAttnArgs as one struct.pack_into call (an argument structure filled field by field costs a small call several
-# microseconds): scalars, the twelve pointers, the ten stride arrays, stream and mask_classes, in declaration order.
-ARGS_PACKER = struct.Struct("@Iiiiiiiiff" "QQ" "12P" "40q" "PP")
+# microseconds): scalars, the twelve pointers, the ten stride arrays, stream, mask_classes and the workspace, in declaration order.
+ARGS_PACKER = struct.Struct("@Iiiiiiiiff" "QQ" "12P" "40q" "PP" "Pq")
 assert ARGS_PACKER.size == ctypes.sizeof(TriAttnArgs)
 
 
@@ -101,6 +103,7 @@ EXPORTS = (
     "tri_attn_bwd_noalloc",
     "tri_attn_dropout_mask",
     "tri_attn_uses_matrix_cores",
+    "tri_attn_workspace_size",
     "tri_attn_classify_mask",
     "tri_attn_mask_classes_size",
     "tri_attn_prepare_mask",
@@ -129,6 +132,8 @@ def lib():
             fn = getattr(cdll, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(TriAttnArgs)]
+        cdll.tri_attn_workspace_size.restype = ctypes.c_int64
+        cdll.tri_attn_workspace_size.argtypes = [ctypes.POINTER(TriAttnArgs), ctypes.c_int]
         cdll.tri_attn_mask_classes_size.restype = ctypes.c_int64
         cdll.tri_attn_mask_classes_size.argtypes = [ctypes.POINTER(TriAttnArgs)]
         cdll.tri_attn_prepare_mask.restype = ctypes.c_int

@@ -1,7 +1,9 @@
 // C ABI of libtrident_attn.so: argument checks, kernel selection, launches.
 #include <math.h>
+#include <stddef.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "common.hpp"
@@ -29,6 +31,9 @@ void copy3(int64_t* dst, const int64_t* src) {
     dst[2] = src[2];
 }
 
+// Structures of callers built before the workspace fields were added end there.
+bool size_ok(const TriAttnArgs* a) { return a->struct_size == sizeof(TriAttnArgs) || a->struct_size == offsetof(TriAttnArgs, workspace); }
+
 // Layout of the classes of the mask's 64 x 64 blocks, broadcast like the mask itself.
 void set_class_strides(int64_t* mcs, const TriAttnArgs* a) {
     const int64_t cb = (a->S + 63) / 64, rb = a->mask_stride[2] == 0 ? 1 : cb, mh = a->mask_stride[1] == 0 ? 1 : a->H;
@@ -40,7 +45,7 @@ void set_class_strides(int64_t* mcs, const TriAttnArgs* a) {
 // Common validation + translation. `need` bits: 1 = forward, 2 = delta, 4 = dK/dV, 8 = dQ (and dMask), 16 = summed dMask.
 int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (a == nullptr) return TRI_ATTN_ENULL;
-    if (a->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (!size_ok(a)) return TRI_ATTN_ESIZE;
     if (a->dtype < TRI_ATTN_F32 || a->dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     if (a->B <= 0 || a->H <= 0 || a->S <= 0 || !valid_d(a->D)) return TRI_ATTN_ESHAPE;
     if (static_cast<int64_t>(a->B) * a->H > 2147483647LL / 64) return TRI_ATTN_ESHAPE;
@@ -120,6 +125,10 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (a->mask != nullptr && (a->S % 128 == 0 || padded)) {
         set_class_strides(p->mcs, a);
         p->mcls = a->mask_classes;
+    }
+    if (a->struct_size == sizeof(TriAttnArgs)) {
+        p->workspace = a->workspace;
+        p->workspace_bytes = a->workspace_size;
     }
     p->B = a->B;
     p->H = a->H;
@@ -277,10 +286,13 @@ int tri_attn_bwd_dmask(const TriAttnArgs* args) {
 
 int tri_attn_bwd_noalloc(const TriAttnArgs* args) {
     if (args == nullptr) return TRI_ATTN_ENULL;
-    if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (!size_ok(args)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (static_cast<int64_t>(args->B) * args->H * args->S > kScratchRows) return TRI_ATTN_ESCRATCH;
-    TriAttnArgs a = *args;  // (host copy of a plain struct)
+    TriAttnArgs a;  // (host copy of a plain struct; no workspace: whoever cannot allocate delta has none)
+    memset(&a, 0, sizeof(a));
+    memcpy(&a, args, offsetof(TriAttnArgs, workspace));
+    a.struct_size = sizeof(a);
     const int rc = scratch_for_current_device(&a.delta);
     if (rc) return rc;
     // every row of delta that dK/dV reads is written first by this call's dQ kernel or delta pre-pass:
@@ -288,9 +300,22 @@ int tri_attn_bwd_noalloc(const TriAttnArgs* args) {
     return tri_attn_bwd(&a);
 }
 
+int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass) {
+    if (pass < 0 || pass > 3) return TRI_ATTN_ESHAPE;
+    KParams p;
+    const int rc = make_params(args, pass == 0 ? 1 : pass == 1 ? 4 : pass == 2 ? 8 : 4 | 8, &p);
+    if (rc) return rc;
+    const int dtype = args->dtype;
+    if (pass == 0) return mfma_supported(kMfmaFwd, dtype, p) ? mfma_fwd_workspace(p) : 0;
+    int64_t bytes = 0;
+    if ((pass & 1) && mfma_supported(kMfmaDkdv, dtype, p)) bytes = mfma_dkdv_workspace(p);
+    if ((pass & 2) && mfma_supported(kMfmaDq, dtype, p)) bytes = std::max(bytes, mfma_dq_workspace(p, pass == 3 && mfma_dq_fuses_delta(p)));
+    return bytes;
+}
+
 int64_t tri_attn_mask_classes_size(const TriAttnArgs* args) {
     if (args == nullptr) return TRI_ATTN_ENULL;
-    if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (!size_ok(args)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr || (args->S % 128 != 0 && !(args->mask_dtype & TRI_ATTN_MASK_PADDED))) return 0;
     const int64_t cb = (args->S + 63) / 64, rb = args->mask_stride[2] == 0 ? 1 : cb;
@@ -299,7 +324,7 @@ int64_t tri_attn_mask_classes_size(const TriAttnArgs* args) {
 
 int tri_attn_classify_mask(const TriAttnArgs* args) {
     if (args == nullptr) return TRI_ATTN_ENULL;
-    if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (!size_ok(args)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr || args->mask_classes == nullptr) return TRI_ATTN_ENULL;
     const int mask_dtype = args->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);
@@ -321,7 +346,7 @@ int tri_attn_classify_mask(const TriAttnArgs* args) {
 
 int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t source_dtype, const int64_t* source_stride) {
     if (args == nullptr || source == nullptr || source_stride == nullptr) return TRI_ATTN_ENULL;
-    if (args->struct_size != sizeof(TriAttnArgs)) return TRI_ATTN_ESIZE;
+    if (!size_ok(args)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
     if (args->mask == nullptr) return TRI_ATTN_ENULL;
     const int mask_dtype = args->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);

@@ -42,6 +42,13 @@ struct KParams {
     int dmask_acc;     // dmask is summed over a broadcast dimension (stride 0): fp32 buffer, atomic adds
     int thr8;          // 0 = no dropout; keep iff u8 >= thr8
     float zscale;      // 256 / (256 - thr8), 0 when thr8 == 256
+    // A launch whose items are split along the streamed dimension (split.hpp): 0 units = it is not.
+    int part_units;    // workgroups per head
+    int part_tiles;    // 64-row tiles of a part
+    int part_group;    // causal: how many items in a row have the same number of parts; 0: all have the same
+    float* partial;    // fp32 accumulators of the parts, then (forward) their row statistics
+    void* workspace;   // what the caller has for them
+    int64_t workspace_bytes;
 };
 
 template <typename T>

@@ -21,6 +21,10 @@ int launch_mfma_fwd(int dtype, const KParams& p, hipStream_t stream);
 int launch_mfma_dq(int dtype, const KParams& p, hipStream_t stream, bool with_delta = false);
 bool mfma_dq_fuses_delta(const KParams& p);
 int launch_mfma_dkdv(int dtype, const KParams& p, hipStream_t stream);
+// Bytes of workspace (KParams::workspace) with which these launches run split along the streamed dimension; 0: they never do.
+int64_t mfma_fwd_workspace(const KParams& p);
+int64_t mfma_dq_workspace(const KParams& p, bool with_delta);
+int64_t mfma_dkdv_workspace(const KParams& p);
 int launch_delta(int dtype, const KParams& p, hipStream_t stream);
 
 // mfma_dmask.hip: gradient of a mask shared by batches or heads, summed over them.

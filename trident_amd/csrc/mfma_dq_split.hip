@@ -1,0 +1,68 @@
+// Launches of the dQ kernels whose items are split along the keys (split.hpp).
+#include "mfma_dq.hpp"
+
+namespace tri {
+namespace {
+
+// Few heads: items split along the keys, in workgroups with boundary handling: at D = 128 without mask and dropout the phased
+// kernel, else the one above with as many waves as a ragged length has.
+SplitShape dq_split_shape(const KParams& p) {
+    const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
+    const int waves = (p.D == 128 && p.mask == nullptr && p.thr8 <= 0) || (p.D == 64 && f32_mask) ? 8 : 4;
+    return SplitShape{32 * waves, p.D == 128 || waves == 8 ? 1 : p.D == 64 || f32_mask ? 2 : 4, 1, false, p.D == 128 ? 1.6 : 1.0, split_gain(p)};
+}
+
+template <typename T, int D, bool CAUSAL, int MASK>
+int launch_dq_split(const KParams& p, hipStream_t stream, bool with_delta) {
+    constexpr int NW = D == 64 && MASK == kMaskF32 ? 8 : 4;
+    constexpr bool kDelta = MASK == kNoMask;
+    const dim3 grid = split_grid(p);
+    if (kDelta && !with_delta) return TRI_ATTN_ESHAPE;  // (dq_splits)
+    if constexpr (D == 128 && MASK == kNoMask) {
+        if (p.thr8 <= 0) {
+            hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, true, true>), grid, dim3(512), 0, stream, p);
+            return static_cast<int>(hipGetLastError());
+        }
+    }
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
+    else if constexpr (!(D == 128 && MASK == kNoMask))
+        hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
+template <typename T, int D>
+int launch_dq_split_variant(int dtype, const KParams& p, hipStream_t stream, bool with_delta) {
+    if (p.causal) return launch_dq_split<T, D, true, kNoMask>(p, stream, with_delta);
+    if (p.mask == nullptr) return launch_dq_split<T, D, false, kNoMask>(p, stream, with_delta);
+    if (p.mask_dtype == TRI_ATTN_F32) return launch_dq_split<T, D, false, kMaskF32>(p, stream, with_delta);
+    if (p.mask_dtype == dtype) return launch_dq_split<T, D, false, kMaskT>(p, stream, with_delta);
+    return TRI_ATTN_EDTYPE;
+}
+
+// (a mask gradient is written by whole items only; without a mask the parts bring delta along)
+bool dq_splits(const KParams& p, bool with_delta) { return p.dmask == nullptr && with_delta == (p.mask == nullptr); }
+
+template <typename T>
+int launch_dq_split_head(int dtype, const KParams& p, hipStream_t stream, bool with_delta) {
+    if (p.D == 128) return launch_dq_split_variant<T, 128>(dtype, p, stream, with_delta);
+    if (p.D == 64) return launch_dq_split_variant<T, 64>(dtype, p, stream, with_delta);
+    if (p.D == 32) return launch_dq_split_variant<T, 32>(dtype, p, stream, with_delta);
+    return launch_dq_split_variant<T, 16>(dtype, p, stream, with_delta);
+}
+
+}  // namespace
+
+int64_t mfma_dq_workspace(const KParams& p, bool with_delta) {
+    KParams plan = p;
+    return dq_splits(p, with_delta) ? plan_split(dq_split_shape(p), p.causal != 0, &plan) : 0;
+}
+
+int launch_mfma_dq_split(int dtype, KParams p, hipStream_t stream, bool with_delta) {
+    const SplitShape shape = dq_split_shape(p);
+    if (!dq_splits(p, with_delta) || !take_workspace(plan_split(shape, p.causal != 0, &p), &p)) return TRI_ATTN_ENOFUSE;
+    const int rc = dtype == TRI_ATTN_BF16 ? launch_dq_split_head<bf16_t>(dtype, p, stream, with_delta)
+                                          : launch_dq_split_head<f16_t>(dtype, p, stream, with_delta);
+    return rc ? rc : launch_combine_backward(dtype, p, shape.rows, false, stream);
+}
+
+}  // namespace tri

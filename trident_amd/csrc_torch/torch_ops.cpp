@@ -35,6 +35,7 @@ struct Library {
     decltype(&tri_attn_bwd) bwd = nullptr;
     decltype(&tri_attn_bwd_dmask) bwd_dmask = nullptr;
     decltype(&tri_attn_uses_matrix_cores) uses_matrix_cores = nullptr;
+    decltype(&tri_attn_workspace_size) workspace_size = nullptr;
     decltype(&tri_attn_mask_classes_size) mask_classes_size = nullptr;
     decltype(&tri_attn_classify_mask) classify_mask = nullptr;
     decltype(&tri_attn_prepare_mask) prepare_mask = nullptr;
@@ -308,6 +309,20 @@ TriAttnArgs make_args(const Call& call, const Tensor& q, const Tensor& k, const 
     return a;
 }
 
+// operation._take_workspace
+Tensor take_workspace(TriAttnArgs& a, int pass, const Tensor& q) {
+    const int64_t size = lib.workspace_size(&a, pass);
+    if (size <= 0) return Tensor();
+    try {
+        Tensor workspace = at::empty({size}, q.options().dtype(at::kByte).requires_grad(false));
+        a.workspace = workspace.data_ptr();
+        a.workspace_size = size;
+        return workspace;
+    } catch (const c10::OutOfMemoryError&) {
+        return Tensor();
+    }
+}
+
 // operation.Attention._forward
 std::pair<Tensor, Tensor> attention_forward(Call& call, const Tensor& query, const Tensor& key, const Tensor& value) {
     const c10::DeviceGuard device(query.device());
@@ -331,6 +346,7 @@ std::pair<Tensor, Tensor> attention_forward(Call& call, const Tensor& query, con
     if (prepared) prepared->describe(a);
     Tensor classes;  // (kept alive until the call is enqueued)
     if (mask_view.defined()) classes = mask_classes(call.mask, a, switches.cache);
+    const Tensor workspace = take_workspace(a, 0, q);
     check(lib.fwd(&a));
     return {output, lse};
 }
@@ -404,6 +420,7 @@ std::array<Tensor, 4> attention_backward(const Call& call, const Tensor& grad_ou
         }
         if (mask_view.scalar_type() == mask.scalar_type()) classes = mask_classes(mask, a, switches.cache);
     }
+    const Tensor workspace = take_workspace(a, 3, q);
     check(lib.bwd(&a));
     if (summed) {
         set_mask(mask_view);
@@ -714,6 +731,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     entry("tri_attn_bwd", lib.bwd);
     entry("tri_attn_bwd_dmask", lib.bwd_dmask);
     entry("tri_attn_uses_matrix_cores", lib.uses_matrix_cores);
+    entry("tri_attn_workspace_size", lib.workspace_size);
     entry("tri_attn_mask_classes_size", lib.mask_classes_size);
     entry("tri_attn_classify_mask", lib.classify_mask);
     entry("tri_attn_prepare_mask", lib.prepare_mask);

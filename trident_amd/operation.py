@@ -78,9 +78,23 @@ def _make_args(query, key, value, output, log2sum, mask, dropout_p, is_causal, s
         *query.stride(), *key.stride(), *value.stride(), *output.stride(),
         *_strides_or_zero(grad_output), *_strides_or_zero(grad_query), *_strides_or_zero(grad_key),
         *_strides_or_zero(grad_value), *_strides_or_zero(mask), *_strides_or_zero(grad_mask),
-        torch._C._cuda_getCurrentRawStream(query.device.index), 0,
+        torch._C._cuda_getCurrentRawStream(query.device.index), 0, 0, 0,
     )
     return args
+
+
+def _take_workspace(args, which, device):
+    """Gives the call (0: forward, 3: backward) the scratch memory with which it runs split along the sequence, where it does and
+    the GPU has that much left; returns the tensor to keep alive until the call is enqueued."""
+    size = _lib.lib().tri_attn_workspace_size(ctypes.byref(args), which)
+    if size <= 0:
+        return None
+    try:
+        workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+    args.workspace, args.workspace_size = workspace.data_ptr(), size
+    return workspace
 
 
 # Classes of a mask's 64 x 64 blocks (tri_attn_classify_mask), kept per mask tensor (csrc_torch/torch_ops.cpp): the forward
@@ -333,6 +347,8 @@ class Attention(torch.autograd.Function):
             prepared.describe(args)
         classes = _mask_classes(mask, args) if mask_view is not None else None  # (kept alive until the call is enqueued)
 
+        workspace = _take_workspace(args, 0, query.device)  # noqa: F841  (kept alive until the call is enqueued)
+
         util.push_trace("kernel.Attention.forward")
         _lib.check(lib.tri_attn_fwd(ctypes.byref(args)))
         util.pop_trace()
@@ -404,6 +420,7 @@ class Attention(torch.autograd.Function):
         # one call for the three backward launches (trident/operation/attention.py:161-199 launches the
         # delta pre-pass and the backward kernel): the library orders them, and where the dQ kernel can
         # compute delta on its way the pre-pass disappears into it
+        workspace = _take_workspace(args, 3, query.device)  # noqa: F841  (kept alive until the call is enqueued)
         util.push_trace("kernel.Attention.backward")
         _lib.check(lib.tri_attn_bwd(ctypes.byref(args)))
         if summed:
