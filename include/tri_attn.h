@@ -62,7 +62,7 @@ enum {
 
 /* Or-ed to mask_dtype: every row of the mask may be read up to the next multiple of 64 entries beyond S and holds finite
  * values there (they are not used), and mask_classes, where given, also covers the blocks that S cuts. The 16-bit
- * matrix-core kernels take masked lengths that are no multiple of 128 only so; tri_attn_prepare_mask makes such a mask. */
+ * matrix-core kernels take masked lengths that are no multiple of 64 only so; tri_attn_prepare_mask makes such a mask. */
 #define TRI_ATTN_MASK_PADDED 0x100
 
 /* Or-ed to mask_dtype: every value of the mask is 0 or -inf (what tri_attn_prepare_mask makes of a boolean mask). Only a hint:
@@ -126,7 +126,7 @@ typedef struct TriAttnArgs {
                                   read by tri_attn_fwd / tri_attn_bwd*: dense [MB][MH][RB][S/64] bytes with MB = B (1 if
                                   mask_stride[0] == 0), MH = H (1 if mask_stride[1] == 0), RB = S/64 (1 if mask_stride[2] == 0);
                                   0 = every entry of the block is 0, 1 = every entry is -inf, 2 = anything else.
-                                  Only used where S is a multiple of 128, or with TRI_ATTN_MASK_PADDED (S/64 rounded up). */
+                                  Only used where S is a multiple of 64, or with TRI_ATTN_MASK_PADDED (S/64 rounded up). */
 
     void* workspace;           /* NULL, or scratch memory for this call (16-byte aligned, used until the stream has passed it): with at
                                   least tri_attn_workspace_size bytes of it, calls of few heads run split along the sequence */
@@ -167,7 +167,7 @@ int tri_attn_bwd_dq(const TriAttnArgs* args);
 int tri_attn_bwd_dq_delta(const TriAttnArgs* args);
 
 /* The gradient of a mask that batches or heads share (dmask_stride 0 over one or both; the mask broadcast the same way),
- * summed over them: written, not added, to args->dmask in mask_dtype, with a fixed order of summation. For the 16-bit types,
+ * summed over them, or of any mask with rows and keys of its own where S is no multiple of 128: written, not added, to args->dmask in mask_dtype, with a fixed order of summation. For the 16-bit types,
  * any S, 16-byte aligned rows of q, k, v, d_o, and a row stride of dmask that is not 0. Reads q,k,v,d_o,lse,delta,mask: it
  * follows a tri_attn_bwd (with dmask NULL) or whatever computed delta. Returns TRI_ATTN_ENOFUSE without launching anything
  * where it does not apply: tri_attn_bwd / tri_attn_bwd_dq with dmask set then adds the gradient up atomically. The reference
@@ -207,7 +207,7 @@ int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass);
  * without a mask (the scale folded into one fused multiply-add per score instead of a product, a sum and a
  * difference): results agree with those computed without classes to the last fp32 rounding of a score's exponent, i.e.
  * to within an ulp of the 16-bit outputs, not bit for bit. Reads mask; writes mask_classes.
- * Returns TRI_ATTN_ENOFUSE (nothing launched) where the classes would not be used: S not a multiple of 128. */
+ * Returns TRI_ATTN_ENOFUSE (nothing launched) where the classes would not be used: S not a multiple of 64. */
 int tri_attn_classify_mask(const TriAttnArgs* args);
 /* Bytes of mask_classes for these arguments (MB * MH * RB * S/64), 0 where tri_attn_classify_mask does not apply, or a
  * negative TRI_ATTN_E* code. */
@@ -225,9 +225,9 @@ int tri_attn_prepare_mask(const TriAttnArgs* args, const void* source, int32_t s
 /* Which kernel family a call would run, without launching anything (no counterpart in the reference): pass 0 =
  * tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq, 3 = tri_attn_bwd_dmask (1 or 0: applies or not) on these arguments. Returns 1 for the 16-bit matrix-core
  * (MFMA) kernels (fp16/bf16, D in {16,32,64,128}, 16-byte aligned rows; any S without a mask or with
- * a padded one, S a multiple of 128 with any other); 2 for the 32-row-tile matrix-core kernels (everything else whose pointers and strides are multiples of
+ * a padded one, S a multiple of 64 with any other, of 128 where tri_attn_bwd_dq writes dmask); 2 for the 32-row-tile matrix-core kernels (everything else whose pointers and strides are multiples of
  * four elements: fp32 problems on the fp32 matrix instruction with fp32 products and sums; fp16/bf16 problems with
- * unpadded masks at lengths that are no multiple of 128 on the 16-bit 32x32x8 instruction);
+ * unpadded masks at other lengths on the 16-bit 32x32x8 instruction);
  * 0 for the general vector-ALU kernels (views that are not aligned so); or a negative TRI_ATTN_E* code. */
 int tri_attn_uses_matrix_cores(const TriAttnArgs* args, int pass);
 

@@ -1,0 +1,66 @@
+"""Masks at lengths that are multiples of 64 but not of 128 run the 16-bit kernels as they are, with classes, and learned masks of any
+kind at lengths that are no multiple of 128 get their gradient from tri_attn_bwd_dmask."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+import trident_amd as trident
+from tests import parity
+from trident_amd import _lib, operation
+from trident_amd.operation import Attention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", ["dense", "length", "16 bit", "keys", "dense+dropout"])
+@pytest.mark.parametrize("dtype,B,H,S,D", [(torch.bfloat16, 2, 3, 64, 64), (torch.float16, 1, 3, 192, 128), (torch.bfloat16, 2, 2, 320, 32),
+                                           (torch.float16, 2, 2, 192, 16), (torch.bfloat16, 1, 2, 576, 64), (torch.bfloat16, 2, 1, 448, 128)])
+def test_multiples_of_64(dtype, B, H, S, D, kind, device):
+    g = torch.Generator().manual_seed(S + D)
+    q, k, v, d_o = [torch.randn(B, H, S, D, generator=g).to(dtype) for _ in range(4)]
+    p, rng = (0.2, (31, 2)) if "dropout" in kind else (0.0, (0, 0))
+    mask = 0.5 * torch.randn(1, H, S, S, generator=g) if kind == "16 bit" else torch.randn(B, 1, 1 if kind == "keys" else S, S, generator=g)
+    if kind == "length":
+        mask = torch.zeros(B, 1, S, S)
+        mask[0, ..., S - 70 if S > 70 else 40:] = -math.inf
+    mask = mask.to(dtype) if kind == "16 bit" else mask
+    tq, tk, tv, tdo, tm = [x.to(device) for x in (q, k, v, d_o, mask)]
+    assert operation._prepared_mask(tm, tq) is None
+    o, lse = torch.empty_like(tq), torch.empty(B, H, S, device=device)
+    args = operation._make_args(tq, tk, tv, o, lse, operation._expand_mask(tm, (B, H, S, S)), p, False, 0.125, 0, 0, tdo, o, o, o, None, lse)
+    assert [_lib.lib().tri_attn_uses_matrix_cores(ctypes.byref(args), which) for which in (0, 1, 2)] == [1, 1, 1]
+    assert operation._mask_classes(tm, args) is not None
+    scale = 1.0 / math.sqrt(D)
+    o, lse = Attention._forward(tq, tk, tv, tm, p, False, scale, *rng)
+    dq, dk, dv, _ = Attention._backward(tdo, tq, tk, tv, o, lse, tm, scale, p, False, *rng, False)
+    kw = dict(mask=mask.float(), dropout_p=p, is_causal=False, scale=scale, seed=rng[0], offset=rng[1])
+    parity.close(o, parity.oracle_forward(q, k, v, **kw)[0], dtype, f"{kind} O")
+    dq_r, dk_r, dv_r, _, _ = parity.oracle_backward(q, k, v, d_o, o=o, **kw)
+    _, a_dq, a_dk, a_dv = parity.oracle_abs_sums(q, k, v, d_o, o=o, **kw)
+    parity.close(dq, dq_r, dtype, f"{kind} dQ", a_dq)
+    parity.close(dk, dk_r, dtype, f"{kind} dK", a_dk)
+    parity.close(dv, dv_r, dtype, f"{kind} dV", a_dv)
+
+
+@pytest.mark.parametrize("S,D", [(1, 64), (63, 32), (64, 64), (130, 128), (192, 16), (260, 64)])
+@pytest.mark.parametrize("shape", ["BHSS", "1HSS", "SS"])
+@pytest.mark.parametrize("small", [False, True])
+def test_learned_masks_at_lengths_that_are_no_multiple_of_128(S, D, shape, small, device, monkeypatch):
+    """B = 1, so that [1,H,S,S] is a mask of its own for every head; as a large call has it (padded) and as a small one."""
+    monkeypatch.setattr(operation, "_PADS_FROM", 1 << 62 if small else 0)
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    B, H = (2, 2) if shape == "BHSS" else (1, 3)
+    g = torch.Generator().manual_seed(S)
+    q, k, v, d_o = [torch.randn(B, H, S, D, generator=g).to(torch.bfloat16) for _ in range(4)]
+    mask = (0.5 * torch.randn({"BHSS": (B, H, S, S), "1HSS": (1, H, S, S), "SS": (S, S)}[shape], generator=g)).to(torch.bfloat16)
+    tq, tk, tv, tm = [x.to(device).requires_grad_() for x in (q, k, v, mask)]
+    out = trident.function.scaled_dot_product_attention(tq, tk, tv, tm)
+    grads = torch.autograd.grad(out, (tq, tk, tv, tm), d_o.to(device))
+    full = mask.float() if mask.dim() == 4 else mask.float()[None, None]
+    dq, dk, dv, dm, _ = parity.oracle_backward(q, k, v, d_o, mask=full, want_dmask=True, o=out.detach())
+    _, a_dq, a_dk, a_dv = parity.oracle_abs_sums(q, k, v, d_o, mask=full, o=out.detach())
+    for name, got, want, terms in (("dQ", grads[0], dq, a_dq), ("dK", grads[1], dk, a_dk), ("dV", grads[2], dv, a_dv)):
+        parity.close(got, want, torch.bfloat16, name, terms)
+    parity.close(grads[3].reshape(full.shape), dm, torch.bfloat16, "dMask")

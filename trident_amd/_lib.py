@@ -61,8 +61,8 @@ class TriAttnArgs(ctypes.Structure):
 
 
 # TriAttnArgs as one struct.pack_into call (an argument structure filled field by field costs a small call several
-# microseconds): scalars, the twelve pointers, the ten stride arrays, stream, mask_classes and the workspace, in declaration order.
-ARGS_PACKER = struct.Struct("@Iiiiiiiiff" "QQ" "12P" "40q" "PP" "Pq")
+# microseconds): scalars, the twelve pointers, the ten stride arrays, stream and mask_classes, in declaration order; no workspace.
+ARGS_PACKER = struct.Struct("@Iiiiiiiiff" "QQ" "12P" "40q" "PP" "16x")
 assert ARGS_PACKER.size == ctypes.sizeof(TriAttnArgs)
 
 

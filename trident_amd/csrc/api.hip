@@ -52,7 +52,8 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
     if (!(a->dropout_p >= 0.f && a->dropout_p <= 1.f)) return TRI_ATTN_EDROPOUT;
     if (a->mask != nullptr && a->is_causal) return TRI_ATTN_EMASKCAUSAL;
     const int mask_dtype = a->mask_dtype & ~(TRI_ATTN_MASK_PADDED | TRI_ATTN_MASK_BINARY);
-    const bool padded = a->mask != nullptr && (a->mask_dtype & TRI_ATTN_MASK_PADDED) != 0;
+    // (rows of a multiple of 64 keys are whole pieces as they are)
+    const bool padded = a->mask != nullptr && ((a->mask_dtype & TRI_ATTN_MASK_PADDED) != 0 || a->S % 64 == 0);
     if (a->mask != nullptr || a->dmask != nullptr) {
         if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     }
@@ -122,7 +123,7 @@ int make_params(const TriAttnArgs* a, int need, KParams* p) {
                        (a->S > 1 && a->dmask_stride[2] == 0);
         if (p->dmask_acc && mask_dtype != TRI_ATTN_F32 && (need & 8)) return TRI_ATTN_EDTYPE;
     }
-    if (a->mask != nullptr && (a->S % 128 == 0 || padded)) {
+    if (padded) {
         set_class_strides(p->mcs, a);
         p->mcls = a->mask_classes;
     }
@@ -317,7 +318,7 @@ int64_t tri_attn_mask_classes_size(const TriAttnArgs* args) {
     if (args == nullptr) return TRI_ATTN_ENULL;
     if (!size_ok(args)) return TRI_ATTN_ESIZE;
     if (args->B <= 0 || args->H <= 0 || args->S <= 0) return TRI_ATTN_ESHAPE;
-    if (args->mask == nullptr || (args->S % 128 != 0 && !(args->mask_dtype & TRI_ATTN_MASK_PADDED))) return 0;
+    if (args->mask == nullptr || (args->S % 64 != 0 && !(args->mask_dtype & TRI_ATTN_MASK_PADDED))) return 0;
     const int64_t cb = (args->S + 63) / 64, rb = args->mask_stride[2] == 0 ? 1 : cb;
     return (args->mask_stride[0] == 0 ? 1 : args->B) * (args->mask_stride[1] == 0 ? 1 : args->H) * rb * cb;
 }
@@ -331,7 +332,7 @@ int tri_attn_classify_mask(const TriAttnArgs* args) {
     if (mask_dtype < TRI_ATTN_F32 || mask_dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     int rc = check_strides(args->mask_stride);
     if (rc) return rc;
-    if (args->S % 128 != 0) return TRI_ATTN_ENOFUSE;
+    if (args->S % 64 != 0) return TRI_ATTN_ENOFUSE;
     KParams p;
     memset(&p, 0, sizeof(p));
     p.mask = args->mask;

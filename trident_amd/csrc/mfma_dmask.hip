@@ -250,7 +250,7 @@ bool mfma_dmask_supported(int dtype, const KParams& p) {
     if (dtype != TRI_ATTN_F16 && dtype != TRI_ATTN_BF16) return false;
     if (p.mask == nullptr || p.dmask == nullptr || p.causal) return false;
     const bool over_b = p.dms[0] == 0 && p.B > 1, over_h = p.dms[1] == 0 && p.H > 1;
-    if (!over_b && !over_h) return false;                                        // (written in place by the dQ pass)
+    if (!over_b && !over_h && p.S % 128 == 0) return false;                      // (written in place by the dQ pass)
     if (p.dms[2] == 0 && p.S > 1) return false;                                  // (summed over the rows: atomics)
     if ((over_b && p.ms[0] != 0) || (over_h && p.ms[1] != 0)) return false;      // (one mask tile for all pairs)
     // A wave's pairs follow one another (about 0.75 us each per 16 columns of the head size: latency), while the atomic adds of

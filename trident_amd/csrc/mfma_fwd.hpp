@@ -1,5 +1,5 @@
 // Forward attention on the matrix cores: online-softmax flash kernel for fp16/bf16,
-// D in {16,32,64,128}; any S without a mask or with a padded one, multiples of 128 with any other (replaces trident/kernel/attention.py:33-165).
+// D in {16,32,64,128}; any S without a mask or with a padded one, multiples of 64 with any other (replaces trident/kernel/attention.py:33-165).
 //
 // A workgroup of NW waves owns 32*NW query rows, one wave 32 of them. Q stays in registers as
 // the B operand of S^T = K Q^T; K and V tiles of 64 keys live row-major (swizzled) in a four-stage

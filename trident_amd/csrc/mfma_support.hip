@@ -171,8 +171,8 @@ static bool tile_offsets_fit(const int64_t* strides) { return strides[2] >= 0 &&
 bool mfma_supported(int which, int dtype, const KParams& p) {
     if (dtype != TRI_ATTN_F16 && dtype != TRI_ATTN_BF16) return false;
     if (p.D != 16 && p.D != 32 && p.D != 64 && p.D != 128) return false;
-    // lengths that are not multiples of 128 run with boundary handling, which reads whole pieces of padded masks only and
-    // does not write a mask gradient
+    // lengths that are not multiples of 128 run with boundary handling, which reads whole pieces of 64 keys of a mask (so that its
+    // rows are padded where S is no multiple of 64) and does not write a mask gradient
     if (p.S % 128 != 0 && p.mask != nullptr && (!p.mask_padded || p.dmask != nullptr)) return false;
     if (!(p.scale > 0.f)) return false;  // the kernels take row maxima before scaling
     if (!aligned16(p.q) || !aligned16(p.k) || !aligned16(p.v)) return false;

@@ -172,18 +172,27 @@ std::shared_ptr<Prepared> prepare(const Tensor& source, const Tensor& query) {
     return m;
 }
 
+constexpr int64_t kPadsLong = int64_t{1} << 28;  // operation._PADS_LONG
+constexpr int64_t kKeptBytes = int64_t{1} << 22;
+
+// operation._worth_padding
+bool worth_padding(const Tensor& query, int64_t pads_from) {
+    const int64_t S = query.size(2), work = query.size(0) * query.size(1) * S * S * std::max<int64_t>(query.size(3), 32);
+    return std::max(work, S > 128 ? kPadsLong : int64_t{0}) >= pads_from;
+}
+
 // operation._sums_mask_gradient
-bool sums_mask_gradient(const Tensor& mask, const Tensor& query) {
+bool sums_mask_gradient(const Tensor& mask, const Tensor& query, int64_t pads_from) {
     const int64_t S = query.size(2);
     if (query.scalar_type() == at::kFloat || mask.dim() < 2 || mask.size(-1) != S || mask.size(-2) != S) return false;
     const int64_t b = mask.dim() >= 4 ? mask.size(-4) : 1, h = mask.dim() >= 3 ? mask.size(-3) : 1;
-    return b != query.size(0) || h != query.size(1);
+    return b != query.size(0) || h != query.size(1) || (S % 128 != 0 && (S % 64 == 0 || worth_padding(query, pads_from)));
 }
 
 // What a call was asked for, kept for its backward.
 struct Call : torch::CustomClassHolder {
     Tensor mask;                         // as given; of a boolean one the prepared mask is kept in its place
-    std::shared_ptr<Prepared> prepared;  // a boolean mask on its way through forward and backward
+    std::shared_ptr<Prepared> prepared;  // a boolean mask, or a small padded one, on its way through forward and backward
     bool boolean = false;
     double dropout_p = 0.0, scale = 1.0;
     bool causal = false;
@@ -192,12 +201,11 @@ struct Call : torch::CustomClassHolder {
 
 // operation._prepared_mask
 std::shared_ptr<Prepared> prepared_mask(const Call& call, const Tensor& query, int64_t pads_from) {
-    if (call.boolean) return call.prepared;
+    if (call.prepared) return call.prepared;
     const Tensor& mask = call.mask;
-    const int64_t S = query.size(2);
-    if (S % 128 == 0 || query.size(0) * query.size(1) * S * S * std::max<int64_t>(query.size(3), 32) < pads_from) return nullptr;
+    if (query.size(2) % 64 == 0 || !worth_padding(query, pads_from)) return nullptr;
     if (query.scalar_type() == at::kFloat || (mask.scalar_type() != at::kFloat && mask.scalar_type() != query.scalar_type())) return nullptr;
-    if (mask.requires_grad() && !sums_mask_gradient(mask, query)) return nullptr;
+    if (mask.requires_grad() && !sums_mask_gradient(mask, query, pads_from)) return nullptr;
     try {
         return prepare(mask.detach(), query);
     } catch (const c10::OutOfMemoryError&) {
@@ -229,7 +237,6 @@ std::vector<int64_t> classes_signature(const Tensor& mask, const TriAttnArgs& a)
 }
 
 Tensor mask_classes(const Tensor& mask, TriAttnArgs& a, bool may_cache) {
-    if (a.S % 128 != 0) return Tensor();
     const int64_t size = lib.mask_classes_size(&a);
     if (size <= 0) return Tensor();
     const bool use_cache = may_cache && !stream_is_capturing() && !mask.is_inference();
@@ -341,6 +348,8 @@ std::pair<Tensor, Tensor> attention_forward(Call& call, const Tensor& query, con
         }
         prepared = prepared_mask(call, q, switches.pads_from);
         if (prepared == nullptr) mask_view = expand_mask(call.mask, {B, H, S, S});
+        // (for the backward, which pads a larger mask again instead of holding the memory until then)
+        else if (prepared->padded.nbytes() <= kKeptBytes) call.prepared = prepared;
     }
     TriAttnArgs a = make_args(call, q, k, v, output, lse, mask_view);
     if (prepared) prepared->describe(a);
@@ -365,7 +374,7 @@ std::array<Tensor, 4> attention_backward(const Call& call, const Tensor& grad_ou
     MaskSwitches switches;
     if (masked) switches = mask_switches();
     const Tensor& mask = call.mask;
-    bool summed = want_grad_mask && sums_mask_gradient(mask, q);
+    bool summed = want_grad_mask && sums_mask_gradient(mask, q, switches.pads_from);  // (a mask whose gradient the dQ pass writes was not padded)
     std::shared_ptr<Prepared> prepared;
     if (masked && !want_grad_mask) prepared = prepared_mask(call, q, switches.pads_from);
     Tensor mask_view, grad_mask_buf, grad_mask_view;

@@ -78,7 +78,7 @@ def _make_args(query, key, value, output, log2sum, mask, dropout_p, is_causal, s
         *query.stride(), *key.stride(), *value.stride(), *output.stride(),
         *_strides_or_zero(grad_output), *_strides_or_zero(grad_query), *_strides_or_zero(grad_key),
         *_strides_or_zero(grad_value), *_strides_or_zero(mask), *_strides_or_zero(grad_mask),
-        torch._C._cuda_getCurrentRawStream(query.device.index), 0, 0, 0,
+        torch._C._cuda_getCurrentRawStream(query.device.index), 0,
     )
     return args
 
@@ -113,7 +113,7 @@ def forget_mask_classes():
 def _mask_classes(mask: torch.Tensor, args):
     """Sets args.mask_classes for the mask already described in ``args``; returns the tensor to keep alive, or None
     where the library has no use for classes (nothing is launched then; padded masks bring theirs along, and the kernels use
-    no others at lengths that are no multiple of 128)."""
+    no others at lengths that are no multiple of 64)."""
     return _lib.torch_ops().mask_classes(mask, ctypes.addressof(args), bool(config.cache_mask_classes))
 
 
@@ -175,32 +175,44 @@ class _PreparedMask:
             args.mask_classes = self.classes.data_ptr()
 
 
-# Scores times head size from which an additive mask at a ragged length is copied into padded rows (_prepared_mask).
-_PADS_FROM = 1 << 29
+# Scores times head size from which an additive mask at a ragged length is copied into padded rows (_prepared_mask), and what
+# lengths beyond 128 count as at least.
+_PADS_FROM = 1 << 28
+_PADS_LONG = 1 << 28
+
+
+def _worth_padding(query):
+    num_batches, num_heads, y_size, x_size = query.shape
+    work = num_batches * num_heads * y_size * y_size * max(x_size, 32)
+    return max(work, _PADS_LONG if y_size > 128 else 0) >= _PADS_FROM
 
 
 def _sums_mask_gradient(mask, query):
-    """Whether the gradient of ``mask`` is summed over batches or heads, with rows and keys of its own (16-bit problems)."""
+    """Whether the gradient of ``mask`` is made by a kernel of its own (tri_attn_bwd_dmask) behind the backward: 16-bit problems, a
+    mask with rows and keys of its own that batches or heads share, or any such mask at a length that is no multiple of 128,
+    where the dQ pass of the 16-bit kernels does not write it (and the call is large enough for them)."""
     shape4 = (1,) * (4 - mask.dim()) + tuple(mask.shape)
     num_batches, num_heads, y_size, _ = query.shape
-    return query.dtype != torch.float32 and shape4[2:] == (y_size, y_size) and shape4[:2] != (num_batches, num_heads)
+    return query.dtype != torch.float32 and shape4[2:] == (y_size, y_size) and (
+        shape4[:2] != (num_batches, num_heads) or (y_size % 128 != 0 and (y_size % 64 == 0 or _worth_padding(query))))
 
 
 def _prepared_mask(mask, query):
     """The _PreparedMask of a call, or None where the mask is handed over as it is. Boolean masks always have one. Additive
-    ones are copied into padded rows for 16-bit problems at lengths that are no multiple of 128, whose kernels fetch mask rows
+    ones are copied into padded rows for 16-bit problems at lengths that are no multiple of 64, whose kernels fetch mask rows
     in 16-byte pieces up to the end of a 64-key tile: one more pass over the mask (at the copy rate) in each direction against
     kernels that read masks element by element (bf16, dense fp32 mask, forward + backward: B=16 H=12 S=777 D=64 2.22 -> 0.39 ms,
-    S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Below _PADS_FROM scores times head size the launches and their arguments cost a call more than
-    the kernels save (S=100 0.15 -> 0.21 ms). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it.
+    S=500 D=16 0.38 -> 0.21, S=333 D=128 0.93 -> 0.22). Those kernels take their time per row whatever the number of heads (B=1
+    H=4 D=64: S=400 57 -> 20 us forward, 190 -> 80 with the backward; S=200 32 -> 15 forward), so that only at lengths up to 128, below
+    _PADS_FROM scores times head size, the launches and their arguments cost a call more than the kernels save (S=100, 64 heads,
+    with the backward: 70 -> 81 us). A mask whose gradient the dQ pass writes stays as it is: the gradient is laid out like it.
     So does one that the GPU has no memory left to copy."""
     if isinstance(mask, _BooleanMask):
         if mask.prepared is None:
             mask.prepared = _PreparedMask(mask.source, query)
             mask.source = None
         return mask.prepared
-    num_batches, num_heads, y_size, x_size = query.shape
-    if y_size % 128 == 0 or num_batches * num_heads * y_size * y_size * max(x_size, 32) < _PADS_FROM:
+    if query.shape[2] % 64 == 0 or not _worth_padding(query):
         return None
     if query.dtype == torch.float32 or mask.dtype not in (torch.float32, query.dtype):
         return None
