@@ -64,3 +64,43 @@ def test_learned_masks_at_lengths_that_are_no_multiple_of_128(S, D, shape, small
     for name, got, want, terms in (("dQ", grads[0], dq, a_dq), ("dK", grads[1], dk, a_dk), ("dV", grads[2], dv, a_dv)):
         parity.close(got, want, torch.bfloat16, name, terms)
     parity.close(grads[3].reshape(full.shape), dm, torch.bfloat16, "dMask")
+
+
+@pytest.mark.parametrize("p", [0.0, 0.2])
+@pytest.mark.parametrize("shape", ["1HSS", "11SS"])
+@pytest.mark.parametrize("B,H,S,D,mask_dtype", [(40, 3, 70, 64, torch.bfloat16), (50, 2, 130, 128, torch.float32), (33, 4, 64, 32, torch.bfloat16),
+                                                (64, 1, 33, 16, torch.float16), (9, 2, 257, 128, torch.bfloat16), (5, 1, 128, 64, torch.float32)])
+def test_pairs_of_a_tile_dealt_to_several_workgroups(B, H, S, D, mask_dtype, shape, p, device):
+    """Few tiles under many pairs: parts of unequal length and empty ones, with and without the workspace, against fp64. The sums
+    are fp32 in both: apart by the rounding of `pairs` additions at most."""
+    g = torch.Generator(device=device).manual_seed(S + D)
+    q, k, v, d_o = [torch.randn(B, H, S, D, generator=g, device=device).to(torch.bfloat16) for _ in range(4)]
+    mask = (0.5 * torch.randn(1, H if shape == "1HSS" else 1, S, S, generator=g, device=device)).to(mask_dtype)
+    scale, rng, full = 1.0 / math.sqrt(D), ((5, 2) if p else (0, 0)), (B, H, S, S)
+    o, lse = Attention._forward(q, k, v, mask, p, False, scale, *rng)
+    delta = (o.float() * d_o.float()).sum(-1)
+    results = []
+    for split in (True, False):
+        dmask = torch.full(mask.shape, float("nan"), dtype=mask_dtype, device=device)
+        args = operation._make_args(q, k, v, o, lse, mask.expand(full), p, False, scale, *rng, d_o, None, None, None, dmask.expand(full), delta)
+        size = _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 4)
+        assert size > 0
+        if split:
+            workspace = torch.full((size,), 255, dtype=torch.uint8, device=device)
+            args.workspace, args.workspace_size = workspace.data_ptr(), size
+        _lib.check(_lib.lib().tri_attn_bwd_dmask(ctypes.byref(args)))
+        results.append(dmask)
+    s = q.double() @ k.double().transpose(-1, -2).contiguous() * scale + mask.double()
+    dp = d_o.double() @ v.double().transpose(-1, -2).contiguous()
+    if p:
+        keep = torch.empty(B * H, S, S, dtype=torch.uint8, device=device)
+        for bh in range(B * H):
+            _lib.check(_lib.lib().tri_attn_dropout_mask(*rng, p, bh, 0, S, 0, S, keep[bh].data_ptr(), torch.cuda.current_stream().cuda_stream))
+        dp *= keep.view(full) * (256 / (256 - round(p * 256)))
+    ds = torch.exp2(s * math.log2(math.e) - lse.double()[..., None]) * (dp - delta.double()[..., None])
+    want = ds.sum((0,) if shape == "1HSS" else (0, 1), keepdim=True).reshape(mask.shape)
+    terms = ds.abs().sum((0,) if shape == "1HSS" else (0, 1), keepdim=True).reshape(mask.shape)
+    half_ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[mask_dtype]
+    for dmask in results:
+        # (scores of D products and their exponentials in fp32: a few 2^-20 of every term)
+        assert ((dmask.double() - want).abs() <= half_ulp * want.abs() * 1.01 + 2.0 ** -17 * terms + 1e-7).all()

@@ -302,11 +302,12 @@ int tri_attn_bwd_noalloc(const TriAttnArgs* args) {
 }
 
 int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass) {
-    if (pass < 0 || pass > 3) return TRI_ATTN_ESHAPE;
+    if (pass < 0 || pass > 4) return TRI_ATTN_ESHAPE;
     KParams p;
-    const int rc = make_params(args, pass == 0 ? 1 : pass == 1 ? 4 : pass == 2 ? 8 : 4 | 8, &p);
+    const int rc = make_params(args, pass == 0 ? 1 : pass == 1 ? 4 : pass == 2 ? 8 : pass == 3 ? 4 | 8 : 16, &p);
     if (rc) return rc;
     const int dtype = args->dtype;
+    if (pass == 4) return mfma_dmask_supported(dtype, p) ? mfma_dmask_workspace(p) : 0;
     if (pass == 0) return mfma_supported(kMfmaFwd, dtype, p) ? mfma_fwd_workspace(p) : 0;
     int64_t bytes = 0;
     if ((pass & 1) && mfma_supported(kMfmaDkdv, dtype, p)) bytes = mfma_dkdv_workspace(p);

@@ -27,9 +27,10 @@ int64_t mfma_dq_workspace(const KParams& p, bool with_delta);
 int64_t mfma_dkdv_workspace(const KParams& p);
 int launch_delta(int dtype, const KParams& p, hipStream_t stream);
 
-// mfma_dmask.hip: gradient of a mask shared by batches or heads, summed over them.
+// mfma_dmask.hip: gradient of a mask, summed over the batches or heads that share it.
 bool mfma_dmask_supported(int dtype, const KParams& p);
-int launch_mfma_dmask(int dtype, const KParams& p, hipStream_t stream);
+int launch_mfma_dmask(int dtype, KParams p, hipStream_t stream);
+int64_t mfma_dmask_workspace(const KParams& p);  // bytes with which it deals the pairs of a tile to several workgroups; 0: it never does
 
 // mfma32.hip: the fp32 matrix instruction. fp32 / fp16 / bf16 storage, D in {16,32,64,128}, any S, any mask, rows
 // aligned to four elements. `which` is a MfmaKernel.

@@ -434,6 +434,9 @@ std::array<Tensor, 4> attention_backward(const Call& call, const Tensor& grad_ou
     if (summed) {
         set_mask(mask_view);
         a.dmask = grad_mask_buf.data_ptr();
+        a.workspace = nullptr;
+        a.workspace_size = 0;
+        const Tensor sums = take_workspace(a, 4, q);
         check(lib.bwd_dmask(&a));
     }
     Tensor grad_mask;

@@ -84,7 +84,7 @@ def _make_args(query, key, value, output, log2sum, mask, dropout_p, is_causal, s
 
 
 def _take_workspace(args, which, device):
-    """Gives the call (0: forward, 3: backward) the scratch memory with which it runs split along the sequence, where it does and
+    """Gives the call (0: forward, 3: backward, 4: mask gradient) the scratch memory with which it runs split along the sequence, where it does and
     the GPU has that much left; returns the tensor to keep alive until the call is enqueued."""
     size = _lib.lib().tri_attn_workspace_size(ctypes.byref(args), which)
     if size <= 0:
@@ -440,6 +440,8 @@ class Attention(torch.autograd.Function):
             args.mask_dtype = util.dtype(mask_view.dtype)
             args.mask_stride[:] = _strides_or_zero(mask_view)
             args.dmask = grad_mask_buf.data_ptr()
+            args.workspace, args.workspace_size = None, 0
+            sums = _take_workspace(args, 4, query.device)  # noqa: F841  (kept alive until the call is enqueued)
             _lib.check(lib.tri_attn_bwd_dmask(ctypes.byref(args)))
         util.pop_trace()
 
