@@ -1,4 +1,4 @@
-"""Launches split along the sequence (few heads, at least 20 tiles of 64) against whole ones and 64-bit results: the operator gives
+"""Launches split along the sequence (few heads, at least 20 tiles of 64, 4 in fp32) against whole ones and 64-bit results: the operator gives
 its calls a workspace and so splits them, the same call without one does not."""
 import ctypes
 import math
@@ -78,7 +78,9 @@ VARIANTS = ["plain", "causal", "dropout", "causal+dropout", "bool keys", "length
 @pytest.mark.parametrize("dtype,B,H,S,D", [
     (torch.bfloat16, 1, 2, 2048, 128), (torch.float16, 1, 3, 1281, 128), (torch.bfloat16, 2, 1, 2047, 128), (torch.float16, 1, 1, 4160, 128),
     (torch.bfloat16, 1, 3, 1345, 64), (torch.float16, 2, 1, 2176, 64), (torch.bfloat16, 1, 1, 5000, 64),
-    (torch.float16, 1, 4, 1343, 32), (torch.bfloat16, 2, 1, 2304, 32), (torch.bfloat16, 1, 2, 1409, 16), (torch.float16, 1, 5, 1920, 16)])
+    (torch.float16, 1, 4, 1343, 32), (torch.bfloat16, 2, 1, 2304, 32), (torch.bfloat16, 1, 2, 1409, 16), (torch.float16, 1, 5, 1920, 16),
+    (torch.float32, 1, 3, 1281, 128), (torch.float32, 2, 1, 513, 128), (torch.float32, 1, 4, 640, 64), (torch.float32, 1, 2, 420, 32),
+    (torch.float32, 1, 4, 1000, 16)])
 def test_split_launches(dtype, B, H, S, D, variant, device, monkeypatch):
     """As close to the 64-bit result as the whole launch: the parts' sums are fp32, what differs is which rounding of P to 16 bits
     goes with which row maximum (a few per cent of the error; 10 % allowed, and fp32 rounding on top of it)."""
@@ -104,11 +106,11 @@ def test_split_launches(dtype, B, H, S, D, variant, device, monkeypatch):
     for name, a, b, c in zip(("O", "lse", "dQ", "dK", "dV"), split, whole, again):
         assert torch.equal(a, c), f"{name} differs between two runs"
         if name == "lse":
-            assert (a - b).abs().max() <= 2.0 ** -8 * 1.5, name  # (whole launches sum P as rounded, padded masks as it is)
+            assert (a - b).abs().max() <= (1e-5 if dtype == torch.float32 else 2.0 ** -8 * 1.5), name  # (whole launches sum P as rounded, padded masks as it is)
     for name, a, b, e in zip(("O", "dQ", "dK", "dV"), (split[0], *split[2:]), (whole[0], *whole[2:]), exact):
         off, off_whole = [((x.double() - e).norm() / e.norm()).item() for x in (a, b)]
-        assert off <= 1.1 * off_whole + 1e-6, (name, off, off_whole)
-        half_ulp = e.abs().max() * (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)  # (the result's own rounding)
+        assert off <= 1.1 * off_whole + (1e-8 if dtype == torch.float32 else 1e-6), (name, off, off_whole)
+        half_ulp = e.abs().max() * {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12, torch.float32: 2.0 ** -25}[dtype]  # (the result's own rounding)
         assert (a.double() - e).abs().max() <= 2 * (b.double() - e).abs().max() + half_ulp + 1e-6, name
 
 

@@ -308,11 +308,13 @@ int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass) {
     if (rc) return rc;
     const int dtype = args->dtype;
     if (pass == 4) return mfma_dmask_supported(dtype, p) ? mfma_dmask_workspace(p) : 0;
-    if (pass == 0) return mfma_supported(kMfmaFwd, dtype, p) ? mfma_fwd_workspace(p) : 0;
-    int64_t bytes = 0;
-    if ((pass & 1) && mfma_supported(kMfmaDkdv, dtype, p)) bytes = mfma_dkdv_workspace(p);
-    if ((pass & 2) && mfma_supported(kMfmaDq, dtype, p)) bytes = std::max(bytes, mfma_dq_workspace(p, pass == 3 && mfma_dq_fuses_delta(p)));
-    return bytes;
+    const auto bytes_of = [&](int which) -> int64_t {
+        if (mfma_supported(which, dtype, p))
+            return which == kMfmaFwd ? mfma_fwd_workspace(p) : which == kMfmaDkdv ? mfma_dkdv_workspace(p) : mfma_dq_workspace(p, pass == 3 && mfma_dq_fuses_delta(p));
+        return mfma32_supported(which, dtype, p) ? mfma32_workspace(which, dtype, p) : 0;
+    };
+    if (pass == 0) return bytes_of(kMfmaFwd);
+    return std::max(pass & 1 ? bytes_of(kMfmaDkdv) : 0, pass & 2 ? bytes_of(kMfmaDq) : 0);
 }
 
 int64_t tri_attn_mask_classes_size(const TriAttnArgs* args) {

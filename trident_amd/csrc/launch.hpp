@@ -35,6 +35,7 @@ int64_t mfma_dmask_workspace(const KParams& p);  // bytes with which it deals th
 // mfma32.hip: the fp32 matrix instruction. fp32 / fp16 / bf16 storage, D in {16,32,64,128}, any S, any mask, rows
 // aligned to four elements. `which` is a MfmaKernel.
 bool mfma32_supported(int which, int dtype, const KParams& p);
+int64_t mfma32_workspace(int which, int dtype, const KParams& p);  // as mfma_fwd_workspace below
 int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream);
 // Classes of the mask's 64 x 64 blocks (0 all zero, 1 all -inf, 2 mixed) into `out`, laid out as p.mcs says.
 int launch_classify_mask(const KParams& p, uint8_t* out, hipStream_t stream);

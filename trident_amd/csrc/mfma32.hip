@@ -23,7 +23,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
-#include "mfma_common.hpp"
+#include "split.hpp"
 
 namespace tri {
 namespace {
@@ -137,7 +137,8 @@ __device__ __forceinline__ uint32_t pick_word(const Philox4& r, int s) {
 }
 
 // ------------------------------------------------------------------------------------------------ forward
-template <typename T, int D>
+// SPLIT (here and below): a workgroup streams one part of its item's rows (split.hpp).
+template <typename T, int D, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
     constexpr int LD = D + 4;
     constexpr int DB = D >= 32 ? D / 32 : 1;  // 32-wide blocks of the head dimension (D = 16: one, half empty)
@@ -148,7 +149,14 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     int bh, qt;
-    map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyLast : kUniformTiles, &bh, &qt);
+    [[maybe_unused]] Part part{};
+    if constexpr (SPLIT) {
+        if (!map_part(p, blockIdx.x, gridDim.x, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, (p.S + 63) / 64, false, &part)) return;
+        bh = part.bh;
+        qt = part.tile;
+    } else {
+        map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyLast : kUniformTiles, &bh, &qt);
+    }
     const int b = bh / p.H, hd = bh % p.H;
     const int q0 = qt * kRowsPerGroup, wrow0 = q0 + 32 * wave, qrow = wrow0 + l32;
     const bool row_ok = qrow < p.S;
@@ -171,14 +179,16 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
     float m = -INFINITY, l = 0.f;
 
     const int n_keys = p.causal ? min(p.S, q0 + kRowsPerGroup) : p.S;  // keys some row of the workgroup sees
-    const int n_tiles = (n_keys + kTile32 - 1) / kTile32;
+    const int first_key = SPLIT ? part.index * p.part_tiles * 64 : 0;
+    const int keys_here = SPLIT ? min(n_keys - first_key, p.part_tiles * 64) : n_keys;
+    const int n_tiles = (max(keys_here, 0) + kTile32 - 1) / kTile32;
     Stage32<T, D> kst, vst;
-    kst.fetch(kbase, p.ks[2], 0, p.S);
-    vst.fetch(vbase, p.vs[2], 0, p.S);
+    kst.fetch(kbase, p.ks[2], first_key, p.S);
+    vst.fetch(vbase, p.vs[2], first_key, p.S);
     kst.commit(sK);
     vst.commit(sV);
     for (int t = 0; t < n_tiles; ++t) {
-        const int k0 = t * kTile32;
+        const int k0 = first_key + t * kTile32;
         if (t + 1 < n_tiles) {
             kst.fetch(kbase, p.ks[2], k0 + kTile32, p.S);
             vst.fetch(vbase, p.vs[2], k0 + kTile32, p.S);
@@ -271,6 +281,15 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
         }
     }
     l = sum_xor32(l);
+    if constexpr (SPLIT) {
+        if (part.count > 1) {
+            const int64_t row = static_cast<int64_t>(part.unit) * kRowsPerGroup + 32 * wave;
+            store_partial<DB, D>(oacc, p.partial + row * D, 0, lane, 1.f);
+            float2* const stats = reinterpret_cast<float2*>(p.partial + static_cast<int64_t>(p.B) * p.H * p.part_units * kRowsPerGroup * D);
+            if (h == 0) stats[row + l32] = make_float2(m, l);
+            return;
+        }
+    }
     const float inv = 1.f / l;
     if (row_ok) {
         // O^T accumulators: register 4 g + e of block db is dim 32 db + 8 g + 4 h + e of this lane's query
@@ -291,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
 // ------------------------------------------------------------------------------------------------ dQ (and dMask)
 // Same data flow as the forward kernel: S^T = K Q^T and dP^T = V dO^T against the wave's Q and dO rows in registers,
 // P and dS on the vector ALU (this lane: its query, 16 keys), dQ^T += K^T dS^T walking the keys in accumulator order.
-template <typename T, int D>
+template <typename T, int D, bool SPLIT>
 __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const KParams p) {
     constexpr int LD = D + 4;
     constexpr int DB = D >= 32 ? D / 32 : 1;
@@ -302,7 +321,14 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     int bh, qt;
-    map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyLast : kUniformTiles, &bh, &qt);
+    [[maybe_unused]] Part part{};
+    if constexpr (SPLIT) {
+        if (!map_part(p, blockIdx.x, gridDim.x, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, (p.S + 63) / 64, false, &part)) return;
+        bh = part.bh;
+        qt = part.tile;
+    } else {
+        map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyLast : kUniformTiles, &bh, &qt);
+    }
     const int b = bh / p.H, hd = bh % p.H;
     const int q0 = qt * kRowsPerGroup, wrow0 = q0 + 32 * wave, qrow = wrow0 + l32;
     const bool row_ok = qrow < p.S;
@@ -330,14 +356,16 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
     for (int db = 0; db < DB; ++db) acc[db] = zero16();
 
     const int n_keys = p.causal ? min(p.S, q0 + kRowsPerGroup) : p.S;
-    const int n_tiles = (n_keys + kTile32 - 1) / kTile32;
+    const int first_key = SPLIT ? part.index * p.part_tiles * 64 : 0;
+    const int keys_here = SPLIT ? min(n_keys - first_key, p.part_tiles * 64) : n_keys;
+    const int n_tiles = (max(keys_here, 0) + kTile32 - 1) / kTile32;
     Stage32<T, D> kst, vst;
-    kst.fetch(kbase, p.ks[2], 0, p.S);
-    vst.fetch(vbase, p.vs[2], 0, p.S);
+    kst.fetch(kbase, p.ks[2], first_key, p.S);
+    vst.fetch(vbase, p.vs[2], first_key, p.S);
     kst.commit(sK);
     vst.commit(sV);
     for (int t = 0; t < n_tiles; ++t) {
-        const int k0 = t * kTile32;
+        const int k0 = first_key + t * kTile32;
         if (t + 1 < n_tiles) {
             kst.fetch(kbase, p.ks[2], k0 + kTile32, p.S);
             vst.fetch(vbase, p.vs[2], k0 + kTile32, p.S);
@@ -417,6 +445,12 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
             vst.commit(sV);
         }
     }
+    if constexpr (SPLIT) {
+        if (part.count > 1) {
+            store_partial<DB, D>(acc, p.partial + (static_cast<int64_t>(part.unit) * kRowsPerGroup + 32 * wave) * D, 0, lane, 1.f);
+            return;
+        }
+    }
     if (row_ok) {
         T* dqrow = static_cast<T*>(p.dq) + b * p.dqs[0] + hd * p.dqs[1] + static_cast<int64_t>(qrow) * p.dqs[2];
         const float sc = p.scale;
@@ -436,8 +470,8 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
 // Roles exchanged: a wave owns 32 keys (K and V rows in registers, as B operands), Q and dO stream through LDS in
 // 32-row tiles with their lse and delta. S = Q K^T and dP = dO V^T leave lane (h, l32) with key l32 and rows
 // c_row(r, h); dV^T += dO^T P and dK^T += Q^T dS walk the rows in that order.
-template <typename T, int D>
-__global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void mfma32_dkdv_kernel(const KParams p) {
+template <typename T, int D, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void mfma32_dkdv_kernel(const KParams p) {
     constexpr int LD = D + 4;
     constexpr int DB = D >= 32 ? D / 32 : 1;
     constexpr int KJ = D / 8;
@@ -449,7 +483,14 @@ __global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void mfma32_dkdv_kernel(const
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     int bh, kt;
-    map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyFirst : kUniformTiles, &bh, &kt);
+    [[maybe_unused]] Part part{};
+    if constexpr (SPLIT) {
+        if (!map_part(p, blockIdx.x, gridDim.x, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, (p.S + 63) / 64, p.causal, &part)) return;
+        bh = part.bh;
+        kt = part.tile;
+    } else {
+        map_block(blockIdx.x, p.B * p.H, (p.S + kRowsPerGroup - 1) / kRowsPerGroup, p.causal ? kHeavyFirst : kUniformTiles, &bh, &kt);
+    }
     const int b = bh / p.H, hd = bh % p.H;
     const int g0 = kt * kRowsPerGroup, wkey0 = g0 + 32 * wave, key = wkey0 + l32;
     const bool key_ok = key < p.S;
@@ -478,8 +519,10 @@ __global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void mfma32_dkdv_kernel(const
         dv[db] = zero16();
     }
 
-    const int r_begin = p.causal ? g0 : 0;  // rows above the workgroup's first key see none of its keys
-    const int n_tiles = (p.S - r_begin + kTile32 - 1) / kTile32;
+    // rows above the workgroup's first key see none of its keys
+    const int r_begin = (p.causal ? g0 : 0) + (SPLIT ? part.index * p.part_tiles * 64 : 0);
+    const int rows_here = SPLIT ? min(p.S - r_begin, p.part_tiles * 64) : p.S - r_begin;
+    const int n_tiles = (max(rows_here, 0) + kTile32 - 1) / kTile32;
     Stage32<T, D> qst, gst;
     float aux = 0.f;  // threads 0-31: lse of a row of the tile, threads 32-63: its delta
     auto fetch_tile = [&](int r0) {
@@ -569,6 +612,14 @@ __global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void mfma32_dkdv_kernel(const
         __syncthreads();
         if (t + 1 < n_tiles) commit_tile();
     }
+    if constexpr (SPLIT) {
+        if (part.count > 1) {
+            float* const sums = p.partial + (static_cast<int64_t>(part.unit) * 2 * kRowsPerGroup + 32 * wave) * D;
+            store_partial<DB, D>(dk, sums, 0, lane, 1.f);
+            store_partial<DB, D>(dv, sums + static_cast<int64_t>(kRowsPerGroup) * D, 0, lane, 1.f);
+            return;
+        }
+    }
     if (key_ok) {
         T* dkrow = static_cast<T*>(p.dk) + b * p.dks[0] + hd * p.dks[1] + static_cast<int64_t>(key) * p.dks[2];
         T* dvrow = static_cast<T*>(p.dv) + b * p.dvs[0] + hd * p.dvs[1] + static_cast<int64_t>(key) * p.dvs[2];
@@ -592,7 +643,7 @@ __global__ __launch_bounds__(256, D >= 64 ? 1 : 2) void mfma32_dkdv_kernel(const
 // 16 bytes per four steps, like the A operands), and the two waves of a key block share its query rows: wave (kb, rh)
 // takes the 32-row tiles 2 u + rh, both accumulate the full head dimension, and at the end the rh = 1 wave hands its
 // accumulators to its partner through LDS.
-template <typename T, int D>
+template <typename T, int D, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams p) {
     constexpr int LD = D + 4;
     constexpr int DB = D / 32;
@@ -610,7 +661,14 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
     const int kb = wave & 1, rh = wave >> 1;
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     int bh, kt;
-    map_block(blockIdx.x, p.B * p.H, (p.S + kKeys - 1) / kKeys, p.causal ? kHeavyFirst : kUniformTiles, &bh, &kt);
+    [[maybe_unused]] Part part{};
+    if constexpr (SPLIT) {
+        if (!map_part(p, blockIdx.x, gridDim.x, (p.S + kKeys - 1) / kKeys, (p.S + 63) / 64, p.causal, &part)) return;
+        bh = part.bh;
+        kt = part.tile;
+    } else {
+        map_block(blockIdx.x, p.B * p.H, (p.S + kKeys - 1) / kKeys, p.causal ? kHeavyFirst : kUniformTiles, &bh, &kt);
+    }
     const int b = bh / p.H, hd = bh % p.H;
     const int g0 = kt * kKeys, wkey0 = g0 + 32 * kb, key = wkey0 + l32;
     const bool key_ok = key < p.S;
@@ -665,8 +723,9 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
         dk[db] = zero16();
         dv[db] = zero16();
     }
-    const int r_begin = p.causal ? g0 : 0;
-    const int n_steps = (p.S - r_begin + 2 * kTile32 - 1) / (2 * kTile32);
+    const int r_begin = (p.causal ? g0 : 0) + (SPLIT ? part.index * p.part_tiles * 64 : 0);
+    const int rows_here = SPLIT ? min(p.S - r_begin, p.part_tiles * 64) : p.S - r_begin;
+    const int n_steps = (max(rows_here, 0) + 2 * kTile32 - 1) / (2 * kTile32);
     fetch_rows(r_begin);
     commit_rows();
     const float* myK = sK + (32 * kb + l32) * LD + 4 * h;
@@ -760,6 +819,23 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
                 }
         }
         __syncthreads();
+        if constexpr (SPLIT) {
+            if (part.count > 1) {
+                if (rh == 0) {
+#pragma unroll
+                    for (int db = 0; db < DB; ++db)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            dk[db][i] += xch[((2 * db + 0) * 4 + (i >> 2)) * 256 + lane * 4 + (i & 3)];
+                            dv[db][i] += xch[((2 * db + 1) * 4 + (i >> 2)) * 256 + lane * 4 + (i & 3)];
+                        }
+                    float* const sums = p.partial + (static_cast<int64_t>(part.unit) * 2 * kKeys + 32 * kb) * D;
+                    store_partial<DB, D>(dk, sums, 0, lane, 1.f);
+                    store_partial<DB, D>(dv, sums + static_cast<int64_t>(kKeys) * D, 0, lane, 1.f);
+                }
+                return;
+            }
+        }
         if (rh == 0 && key_ok) {
             T* dkrow = static_cast<T*>(p.dk) + b * p.dks[0] + hd * p.dks[1] + static_cast<int64_t>(key) * p.dks[2];
             T* dvrow = static_cast<T*>(p.dv) + b * p.dvs[0] + hd * p.dvs[1] + static_cast<int64_t>(key) * p.dvs[2];
@@ -780,6 +856,30 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
     }
 }
 
+// fp32 launches of few heads, split along the streamed rows (split.hpp). A tile of 64 rows takes a workgroup its products at about
+// 70 % of the fp32 matrix rate of a CU, so that parts pay from a few tiles on; a second workgroup on a CU adds little.
+SplitShape split_shape32(int which, const KParams& p) {
+    const double fwd_us = p.D == 128 ? 9.5 : p.D == 64 ? 4.9 : p.D == 32 ? 2.6 : 2.0;
+    if (which == kMfmaFwd) return SplitShape{kRowsPerGroup, 1, 1, true, 4, fwd_us, 0.85};
+    if (which == kMfmaDq) return SplitShape{kRowsPerGroup, 1, 1, false, 4, 1.5 * fwd_us, 0.85};
+    return SplitShape{p.D == 128 ? 64 : kRowsPerGroup, 1, 2, false, 4, p.D == 128 ? 10.0 : 2 * fwd_us, 0.85};
+}
+// (a mask gradient is written by whole items only)
+bool splits32(int which, int dtype, const KParams& p) { return dtype == TRI_ATTN_F32 && !(which == kMfmaDq && p.dmask != nullptr); }
+
+template <int D>
+int launch32_split(int which, const KParams& p, int rows, hipStream_t stream) {
+    const dim3 grid = split_grid(p), block(256);
+    if (which == kMfmaFwd) hipLaunchKernelGGL((mfma32_fwd_kernel<float, D, true>), grid, block, 0, stream, p);
+    else if (which == kMfmaDq) hipLaunchKernelGGL((mfma32_dq_kernel<float, D, true>), grid, block, 0, stream, p);
+    else if constexpr (D == 128) hipLaunchKernelGGL((mfma32_dkdv_split_kernel<float, D, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma32_dkdv_kernel<float, D, true>), grid, block, 0, stream, p);
+    const int rc = static_cast<int>(hipGetLastError());
+    if (rc) return rc;
+    return which == kMfmaFwd ? launch_combine_forward(TRI_ATTN_F32, p, rows, stream)
+                             : launch_combine_backward(TRI_ATTN_F32, p, rows, which == kMfmaDkdv, stream);
+}
+
 template <typename T, int D>
 int launch32(int which, const KParams& p, hipStream_t stream) {
     const int64_t groups = static_cast<int64_t>((p.S + kRowsPerGroup - 1) / kRowsPerGroup) * p.B * p.H;
@@ -787,18 +887,18 @@ int launch32(int which, const KParams& p, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(groups)), block(256);
     switch (which) {
         case kMfmaFwd:
-            hipLaunchKernelGGL((mfma32_fwd_kernel<T, D>), grid, block, 0, stream, p);
+            hipLaunchKernelGGL((mfma32_fwd_kernel<T, D, false>), grid, block, 0, stream, p);
             break;
         case kMfmaDq:
-            hipLaunchKernelGGL((mfma32_dq_kernel<T, D>), grid, block, 0, stream, p);
+            hipLaunchKernelGGL((mfma32_dq_kernel<T, D, false>), grid, block, 0, stream, p);
             break;
         case kMfmaDkdv:
             if constexpr (D == 128) {
                 const int64_t groups64 = static_cast<int64_t>((p.S + 63) / 64) * p.B * p.H;
                 if (groups64 > 2147483647LL) return TRI_ATTN_ESHAPE;
-                hipLaunchKernelGGL((mfma32_dkdv_split_kernel<T, D>), dim3(static_cast<unsigned>(groups64)), block, 0, stream, p);
+                hipLaunchKernelGGL((mfma32_dkdv_split_kernel<T, D, false>), dim3(static_cast<unsigned>(groups64)), block, 0, stream, p);
             } else {
-                hipLaunchKernelGGL((mfma32_dkdv_kernel<T, D>), grid, block, 0, stream, p);
+                hipLaunchKernelGGL((mfma32_dkdv_kernel<T, D, false>), grid, block, 0, stream, p);
             }
             break;
         default:
@@ -839,7 +939,21 @@ bool mfma32_supported(int which, int dtype, const KParams& p) {
     }
 }
 
+int64_t mfma32_workspace(int which, int dtype, const KParams& p) {
+    KParams plan = p;
+    return splits32(which, dtype, p) ? plan_split(split_shape32(which, p), p.causal != 0, &plan) : 0;
+}
+
 int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream) {
+    if (p.workspace != nullptr && splits32(which, dtype, p)) {
+        KParams plan = p;
+        const SplitShape shape = split_shape32(which, p);
+        if (take_workspace(plan_split(shape, p.causal != 0, &plan), &plan))
+            return p.D == 128  ? launch32_split<128>(which, plan, shape.rows, stream)
+                   : p.D == 64 ? launch32_split<64>(which, plan, shape.rows, stream)
+                   : p.D == 32 ? launch32_split<32>(which, plan, shape.rows, stream)
+                               : launch32_split<16>(which, plan, shape.rows, stream);
+    }
     switch (dtype) {
         case TRI_ATTN_F32: return launch32_d<float>(which, p, stream);
         case TRI_ATTN_F16: return launch32_d<f16_t>(which, p, stream);

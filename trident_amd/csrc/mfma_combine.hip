@@ -32,10 +32,27 @@ __device__ __forceinline__ Place place_of(const KParams& p, int rows) {
     return r;
 }
 
+// Where a wave's block goes: 16-bit results through the epilogue's transposition patch, fp32 ones 16 bytes per lane and row.
+template <typename T, int COLS>
+struct BlockStore : RowBlockStore<T, 1, COLS> {};
+template <int COLS>
+struct BlockStore<float, COLS> {
+    static constexpr int kPatchBytes = 16;
+    template <typename Scale>
+    static __device__ __forceinline__ void run(const f32x16 (&acc)[1], Scale scale, char*, char* row0, int64_t row_stride_bytes, int lane, int rows) {
+        const int l32 = lane & 31, h = lane >> 5;
+        if (l32 >= rows) return;
+#pragma unroll
+        for (int g = 0; g < COLS / 8; ++g)
+            *reinterpret_cast<f32x4*>(row0 + l32 * row_stride_bytes + (8 * g + 4 * h) * 4) =
+                f32x4{scale(acc[0][4 * g]), scale(acc[0][4 * g + 1]), scale(acc[0][4 * g + 2]), scale(acc[0][4 * g + 3])};
+    }
+};
+
 template <typename T, int D>
 __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, int rows) {
     constexpr int G = D < 32 ? 2 : 4;
-    using Store = RowBlockStore<T, 1, D < 32 ? D : 32>;
+    using Store = BlockStore<T, D < 32 ? D : 32>;
     __shared__ __attribute__((aligned(1024))) char smem[4 * Store::kPatchBytes];
     const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
     const Place at = place_of<D>(p, rows);
@@ -72,10 +89,10 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
             for (int e = 0; e < 4; ++e) acc[0][4 * g + e] = fmaf(w, none ? 0.f : v[e], acc[0][4 * g + e]);
         }
     }
-    const float inv = (p.thr8 > 0 ? p.zscale : 1.f) / l;
+    const float inv = (sizeof(T) == 2 && p.thr8 > 0 ? p.zscale : 1.f) / l;  // (the fp32 kernels scale what they keep at once)
     const int b = at.bh / p.H, hd = at.bh % p.H, rows_here = p.S - at.row0;
-    char* o0 = static_cast<char*>(p.o) + (b * p.os[0] + hd * p.os[1] + at.row0 * p.os[2] + 32 * at.column) * 2;
-    Store::run(acc, [inv](float x) { return x * inv; }, smem + (threadIdx.x >> 6) * Store::kPatchBytes, o0, p.os[2] * 2, lane, rows_here);
+    char* o0 = static_cast<char*>(p.o) + (b * p.os[0] + hd * p.os[1] + at.row0 * p.os[2] + 32 * at.column) * sizeof(T);
+    Store::run(acc, [inv](float x) { return x * inv; }, smem + (threadIdx.x >> 6) * Store::kPatchBytes, o0, p.os[2] * sizeof(T), lane, rows_here);
     if (at.column == 0 && h == 0 && l32 < rows_here) p.lse[static_cast<int64_t>(at.bh) * p.S + at.row0 + l32] = m == -INFINITY ? m : m + fast_log2(l);
 }
 
@@ -83,7 +100,7 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
 template <typename T, int D, int OUTPUTS>
 __global__ __launch_bounds__(256) void combine_backward_kernel(const KParams p, int rows) {
     constexpr int G = D < 32 ? 2 : 4;
-    using Store = RowBlockStore<T, 1, D < 32 ? D : 32>;
+    using Store = BlockStore<T, D < 32 ? D : 32>;
     __shared__ __attribute__((aligned(1024))) char smem[4 * Store::kPatchBytes];
     const int lane = threadIdx.x & 63;
     const Place at = place_of<D>(p, rows);
@@ -110,7 +127,7 @@ __global__ __launch_bounds__(256) void combine_backward_kernel(const KParams p, 
     const int64_t* s = OUTPUTS == 1 ? p.dqs : n == 0 ? p.dks : p.dvs;
     const float scale = n == 1 ? 1.f : p.scale;
     Store::run(acc, [scale](float x) { return x * scale; }, smem + (threadIdx.x >> 6) * Store::kPatchBytes,
-               to + (b * s[0] + hd * s[1] + at.row0 * s[2] + 32 * at.column) * 2, s[2] * 2, lane, p.S - at.row0);
+               to + (b * s[0] + hd * s[1] + at.row0 * s[2] + 32 * at.column) * sizeof(T), s[2] * sizeof(T), lane, p.S - at.row0);
 }
 
 dim3 combine_grid(const KParams& p, int outputs) {
@@ -141,10 +158,12 @@ int combine_backward(const KParams& p, int rows, hipStream_t st) {
 }  // namespace
 
 int launch_combine_forward(int dtype, const KParams& p, int rows, hipStream_t stream) {
+    if (dtype == TRI_ATTN_F32) return combine_forward<float>(p, rows, stream);
     return dtype == TRI_ATTN_BF16 ? combine_forward<bf16_t>(p, rows, stream) : combine_forward<f16_t>(p, rows, stream);
 }
 
 int launch_combine_backward(int dtype, const KParams& p, int rows, bool dkdv, hipStream_t stream) {
+    if (dtype == TRI_ATTN_F32) return dkdv ? combine_backward<float, 2>(p, rows, stream) : combine_backward<float, 1>(p, rows, stream);
     if (dtype == TRI_ATTN_BF16) return dkdv ? combine_backward<bf16_t, 2>(p, rows, stream) : combine_backward<bf16_t, 1>(p, rows, stream);
     return dkdv ? combine_backward<f16_t, 2>(p, rows, stream) : combine_backward<f16_t, 1>(p, rows, stream);
 }
@@ -155,17 +174,16 @@ int64_t plan_split(const SplitShape& shape, bool causal, KParams* p) {
     const int tiles = (p->S + 63) / 64, items = (p->S + shape.rows - 1) / shape.rows, step = shape.rows / 64;
     const int64_t slots = static_cast<int64_t>(persistent_grid(1 << 20)) * shape.slots_per_cu;
     // Microseconds, as measured at 21 to 94 tiles: a workgroup's start and end, the second launch, bytes of the workspace (mostly
-    // in the caches) that both launches move in one. Below kMinTiles tiles there is less to win than the second launch costs.
+    // in the caches) that both launches move in one.
     const double tile_us = shape.tile_us;
     constexpr double kFixed = 6, kCombine = 5, kBytesPerUs = 8e6;
-    constexpr int kMinTiles = 20;
     // A launch with a workgroup for every CU is worth it only where the workgroups are long.
-    if (tiles < kMinTiles || heads * items >= 2 * slots || (tiles < 64 && heads * items >= slots / shape.slots_per_cu)) return 0;
+    if (tiles < shape.min_tiles || heads * items >= 2 * slots || (tiles < 64 && heads * items >= slots / shape.slots_per_cu)) return 0;
     const double whole = causal ? std::max(tiles * tile_us + kFixed, static_cast<double>(heads) * items * ((tiles + step) / 2.0 * tile_us + kFixed) / slots)
                                 : static_cast<double>((heads * items + slots - 1) / slots) * (tiles * tile_us + kFixed);
     const int64_t unit_bytes = shape.rows * (static_cast<int64_t>(p->D) * shape.outputs + (shape.statistics ? 2 : 0)) * 4;
     double best = shape.gain * whole;
-    for (int c = std::max(4, step); c < tiles; c += causal ? step : 1) {
+    for (int c = std::max(shape.min_tiles / 5, step); c < tiles; c += causal ? step : 1) {  // (parts of at least a fifth of min_tiles)
         int64_t units;
         if (causal) {
             const int64_t group = c / step, full = items / group, rest = items % group;

@@ -9,10 +9,10 @@ bool dkdv_splits_phased(const KParams& p) {
     return p.D == 128 && (p.mask == nullptr || (p.ms[2] == 0 && (p.mask_binary || p.S % 128 == 0)));
 }
 SplitShape dkdv_split_shape(const KParams& p) {
-    if (dkdv_splits_phased(p)) return SplitShape{128, 1, 2, false, 1.5, split_gain(p)};
+    if (dkdv_splits_phased(p)) return SplitShape{128, 1, 2, false, 20, 1.5, split_gain(p)};
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = p.mask != nullptr && p.D == 64 && p.thr8 <= 0 ? 8 : 4;
-    return SplitShape{32 * waves, p.D == 128 || waves == 8 || (p.D == 64 && f32_mask) ? 1 : p.D == 64 || f32_mask ? 2 : 4, 2, false, 1.8, split_gain(p)};
+    return SplitShape{32 * waves, p.D == 128 || waves == 8 || (p.D == 64 && f32_mask) ? 1 : p.D == 64 || f32_mask ? 2 : 4, 2, false, 20, 1.8, split_gain(p)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>

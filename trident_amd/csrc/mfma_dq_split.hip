@@ -9,7 +9,7 @@ namespace {
 SplitShape dq_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = (p.D == 128 && p.mask == nullptr && p.thr8 <= 0) || (p.D == 64 && f32_mask) ? 8 : 4;
-    return SplitShape{32 * waves, p.D == 128 || waves == 8 ? 1 : p.D == 64 || f32_mask ? 2 : 4, 1, false, p.D == 128 ? 1.6 : 1.0, split_gain(p)};
+    return SplitShape{32 * waves, p.D == 128 || waves == 8 ? 1 : p.D == 64 || f32_mask ? 2 : 4, 1, false, 20, p.D == 128 ? 1.6 : 1.0, split_gain(p)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>

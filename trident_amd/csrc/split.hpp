@@ -80,6 +80,7 @@ struct SplitShape {
     int slots_per_cu;  // workgroups a CU holds
     int outputs;       // accumulators of D columns per row
     bool statistics;   // two more floats per row
+    int min_tiles;     // below so many there is less to win than the second launch costs
     double tile_us;    // a workgroup's time for one tile
     double gain;       // split where the plan's time is below this share of the whole launch's
 };
