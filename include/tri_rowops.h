@@ -65,6 +65,9 @@ typedef struct TriRowArgs {
     uint64_t seed;             /* dropout: Philox key */
     uint64_t offset;           /* dropout: Philox counter word 3 (low 32 bits used) */
     void* stream;              /* hipStream_t */
+    void* workspace;           /* softmax: NULL, or scratch memory (16-byte aligned, used until the stream has passed the call) of at
+                                  least tri_softmax_workspace_size bytes, with which long columns of narrow matrices run split */
+    int64_t workspace_size;    /* its bytes. A struct_size without these two fields (offsetof(TriRowArgs, workspace)) is taken too */
 } TriRowArgs;
 
 /* kernel.Softmax.forward and, with args->mask set, kernel.MaskedSoftmax.forward. Reads input[, mask]; writes output. */
@@ -73,6 +76,10 @@ int tri_softmax_fwd(const TriRowArgs* args);
 /* kernel.Softmax.backward_delta + kernel.Softmax.backward (and the MaskedSoftmax pair, which computes the same
  * thing: masked positions have output 0). Reads output, grad_output; writes grad_input. */
 int tri_softmax_bwd(const TriRowArgs* args);
+
+/* Bytes of args->workspace with which tri_softmax_fwd (backward = 0) or tri_softmax_bwd (1) on these arguments runs split along the
+ * columns, 0 where it never does, or a negative TRI_ATTN_E* code. Sums are then taken part by part in a fixed order. */
+int64_t tri_softmax_workspace_size(const TriRowArgs* args, int backward);
 
 /* kernel.Dropout.forward. Reads input; writes output. */
 int tri_dropout_fwd(const TriRowArgs* args);

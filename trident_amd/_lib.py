@@ -85,10 +85,12 @@ class TriRowArgs(ctypes.Structure):
         ("seed", ctypes.c_uint64),
         ("offset", ctypes.c_uint64),
         ("stream", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p),
+        ("workspace_size", ctypes.c_int64),
     ]
 
 
-ROW_EXPORTS = ("tri_softmax_fwd", "tri_softmax_bwd", "tri_dropout_fwd", "tri_dropout_bwd")
+ROW_EXPORTS = ("tri_softmax_fwd", "tri_softmax_bwd", "tri_softmax_workspace_size", "tri_dropout_fwd", "tri_dropout_bwd")
 
 EXPORTS = (
     "tri_attn_version",
@@ -150,6 +152,8 @@ def lib():
             fn = getattr(cdll, name)  # AttributeError if a declared symbol is not exported
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(TriRowArgs)]
+        cdll.tri_softmax_workspace_size.restype = ctypes.c_int64
+        cdll.tri_softmax_workspace_size.argtypes = [ctypes.POINTER(TriRowArgs), ctypes.c_int]
         if cdll.tri_attn_version() != ABI_VERSION:
             raise RuntimeError("libtrident_attn.so ABI version mismatch: rebuild it")
         _lib = cdll

@@ -1,8 +1,10 @@
 // Row softmax, masked row softmax and dropout: the HBM-bound sibling operations of the attention path
 // (C ABI in include/tri_rowops.h). Statistics are kept in fp32 in the log2 domain, as in the attention kernels.
 #include <math.h>
+#include <stddef.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -25,6 +27,12 @@ struct RowParams {
     uint32_t seed_lo, seed_hi, offset;
     int thr8;
     float zscale;
+    // columns split along their length: elements of a part and number of parts, and what the parts leave for each column
+    int64_t part_size;
+    int parts;
+    void* part_stats;
+    void* workspace;
+    int64_t workspace_bytes;
 };
 
 // M = element type of the mask (void: no mask). A position is masked where its mask value exceeds eps
@@ -460,9 +468,49 @@ constexpr int kColHeldBwd = 8;      // backward: of each of its two inputs
 struct ColPlace {
     int lane, group, groups;  // lane position in the panel, row group of this thread and their number
     int64_t first;            // the panel's first column
-    int64_t base;             // element offset of this thread's first column
+    int64_t base;             // element offset of this thread's first column (in its part)
+    int64_t x_size;           // length of the column (of the part)
     bool live;
 };
+// A column launch does all of a column's work in one workgroup (kWhole), or, where that leaves CUs idle and sweeps long columns
+// twice, in two launches of parts (blockIdx.y): one leaves each column's statistics in the workspace (kStatistics), the next
+// reads those of all parts and writes its own part (kOutput). Microseconds, forward and backward, one workgroup per panel ->
+// split: bf16 38122 x 424 with a uint8 mask 399 and 327 -> 61 and 57, fp16 29960 x 156 186 and 251 -> 34 and 39, bf16 9485 x 232
+// with mask 111 and 79 -> 25 and 15.
+enum ColWork { kWhole = 0, kStatistics = 1, kOutput = 2 };
+template <ColWork W>
+__device__ __forceinline__ void place_in_part(const RowParams& p, ColPlace* c) {
+    if constexpr (W != kWhole) {
+        const int64_t row0 = blockIdx.y * p.part_size;
+        c->x_size = min(p.part_size, p.x_size - row0);
+        if (c->live) c->base += row0 * p.x_stride;
+    }
+}
+template <ColWork W>
+__device__ __forceinline__ int64_t length(const RowParams& p, const ColPlace& c) {
+    return W == kWhole ? p.x_size : c.x_size;
+}
+// Columns of a panel's statistics over all parts, merged in their order by as many threads as there are: thread t takes column
+// t % columns and every (threads / columns)-th part, and `shared` takes what these leave.
+template <typename S, typename Merge>
+__device__ __forceinline__ void merge_parts(const RowParams& p, const ColPlace& c, int columns, S none, S* shared, Merge merge) {
+    const S* stats = static_cast<const S*>(p.part_stats);
+    const int chunks = max(1, static_cast<int>(blockDim.x) / columns);
+    for (int t = threadIdx.x; t < columns * chunks; t += blockDim.x) {
+        const int64_t col = c.first + t % columns;
+        S x = none;
+        if (col < p.y_size)
+            for (int i = t / columns; i < p.parts; i += chunks) x = merge(x, stats[i * p.y_size + col]);
+        shared[t] = x;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < columns; t += blockDim.x) {
+        S x = shared[t];
+        for (int i = 1; i < chunks; ++i) x = merge(x, shared[i * columns + t]);
+        shared[t] = x;
+    }
+    __syncthreads();
+}
 __device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int lanes_log2, int64_t panels, ColPlace* c) {
     const int64_t per_xcd = (panels + 7) / 8;
     const int64_t panel = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -483,9 +531,9 @@ __device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int la
 struct ColWalk {
     int64_t at, step;
     int left, groups;  // elements from this one to the column's end
-    __device__ __forceinline__ ColWalk(const RowParams& p, const ColPlace& c, int64_t r0)
+    __device__ __forceinline__ ColWalk(const RowParams& p, const ColPlace& c, int64_t length, int64_t r0)
         : at((r0 + c.group) * p.x_stride), step(c.groups * p.x_stride), left(0), groups(c.groups) {
-        const int64_t rest = p.x_size - r0 - c.group;
+        const int64_t rest = length - r0 - c.group;
         left = !c.live || rest < 0 ? 0 : (rest > 0x3fffffff ? 0x3fffffff : static_cast<int>(rest));
         asm volatile("" : "+v"(at), "+v"(left));
     }
@@ -497,18 +545,19 @@ struct ColWalk {
     }
 };
 
-template <typename T, int V, typename M>
+template <typename T, int V, typename M, ColWork W = kWhole>
 __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams p, int lanes_log2, int64_t panels) {
     extern __shared__ Stat part[];  // one per wave and column of the panel
     ColPlace c;
     if (!place_in_panel(p, V, lanes_log2, panels, &c)) return;
+    place_in_part<W>(p, &c);
     using VT = Vec<T, V>;
     const T* in = static_cast<const T*>(p.input) + c.base;
     T* out = static_cast<T*>(p.output) + c.base;
     const int64_t sweep = static_cast<int64_t>(kColHeld) * c.groups;  // elements of a column a sweep step covers
     Piece<T, V> held[kColHeld];
     auto load = [&](int64_t r0) {  // masked elements and those beyond the column's end: -inf
-        ColWalk w(p, c, r0);
+        ColWalk w(p, c, length<W>(p, c), r0);
 #pragma unroll
         for (int k = 0; k < kColHeld; ++k, w.next()) {
             if (w.exists()) {
@@ -518,8 +567,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
             }
         }
         if constexpr (!std::is_same<M, void>::value) {
-            ColWalk m(p, c, r0);
-            if constexpr (V == 8) {  // (bits, one piece at a time: there are no registers left for more)
+            ColWalk m(p, c, length<W>(p, c), r0);
+            if constexpr (V == 8 || sizeof(M) * V > 16) {  // (bits, one piece at a time: there are no registers left for more)
 #pragma unroll
                 for (int k = 0; k < kColHeld; ++k, m.next()) {
                     const uint32_t hit = m.exists() ? mask_bits<M, V>(p.mask, c.base + m.at) : 0u;
@@ -546,7 +595,7 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
     Stat s[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) s[e] = Stat{-INFINITY, 0.f};
-    for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
+    for (int64_t r0 = 0; W != kOutput && r0 < length<W>(p, c); r0 += sweep) {
         load(r0);
 #pragma unroll
         for (int e = 0; e < V; ++e) {
@@ -562,21 +611,31 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
         }
     }
     // the row groups of a wave, then the waves: one thread per column
-    for (int d = 1 << lanes_log2; d < 64; d <<= 1) {
+    if constexpr (W != kOutput) {
+        for (int d = 1 << lanes_log2; d < 64; d <<= 1) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) s[e] = merge(s[e], Stat{__shfl_xor(s[e].m, d), __shfl_xor(s[e].l, d)});
+            for (int e = 0; e < V; ++e) s[e] = merge(s[e], Stat{__shfl_xor(s[e].m, d), __shfl_xor(s[e].l, d)});
+        }
     }
     const int columns = V << lanes_log2, waves = blockDim.x / 64;
-    if ((threadIdx.x & 63) < (1 << lanes_log2)) {
+    if constexpr (W == kOutput) {
+        merge_parts(p, c, columns, Stat{-INFINITY, 0.f}, part, [](Stat x, Stat y) { return merge(x, y); });
+    } else {
+        if ((threadIdx.x & 63) < (1 << lanes_log2)) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) part[(threadIdx.x / 64) * columns + c.lane * V + e] = s[e];
+            for (int e = 0; e < V; ++e) part[(threadIdx.x / 64) * columns + c.lane * V + e] = s[e];
+        }
+        __syncthreads();
     }
-    __syncthreads();
     for (int i = threadIdx.x; i < columns; i += blockDim.x) {
         Stat t = part[i];
-        for (int w = 1; w < waves; ++w) t = merge(t, part[w * columns + i]);
+        for (int w = 1; W != kOutput && w < waves; ++w) t = merge(t, part[w * columns + i]);
+        if constexpr (W == kStatistics) {
+            if (c.first + i < p.y_size) static_cast<Stat*>(p.part_stats)[blockIdx.y * p.y_size + c.first + i] = t;
+        }
         part[i] = Stat{t.m, 1.f / t.l};  // a fully masked column: 0 * inf = NaN, as softmax gives
     }
+    if constexpr (W == kStatistics) return;
     __syncthreads();
     bool far = false;
 #pragma unroll
@@ -585,7 +644,8 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
         far |= far_from_zero(s[e].m);
         s[e].m = reference(s[e].m);
     }
-    if (__builtin_amdgcn_ballot_w64(far) != 0) {  // (a wave has all columns of the panel: the same in all waves)
+    if (__builtin_amdgcn_ballot_w64(far) != 0) {  // (a wave has all columns of the panel: the same in all waves, and in all parts)
+        if (W == kOutput && blockIdx.y > 0) return;
         float* const shared = &part[0].m;
         for (int i = 0; i < columns && c.first + i < p.y_size; ++i)
             softmax_far<T, M>(p, (c.first + i) * p.y_stride, p.x_stride, p.x_size, threadIdx.x, blockDim.x,
@@ -594,9 +654,9 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
         return;
     }
     if (!c.live) return;
-    for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
-        if (p.x_size > sweep) load(r0);
-        ColWalk w(p, c, r0);
+    for (int64_t r0 = 0; r0 < length<W>(p, c); r0 += sweep) {
+        if (W == kOutput || length<W>(p, c) > sweep) load(r0);
+        ColWalk w(p, c, length<W>(p, c), r0);
 #pragma unroll
         for (int k = 0; k < kColHeld; ++k, w.next()) {
             if (w.exists()) {
@@ -609,11 +669,12 @@ __global__ __launch_bounds__(1024) void softmax_fwd_cols_kernel(const RowParams 
     }
 }
 
-template <typename T, int V>
+template <typename T, int V, ColWork W = kWhole>
 __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams p, int lanes_log2, int64_t panels) {
     extern __shared__ float part_sums[];  // one per wave and column of the panel
     ColPlace c;
     if (!place_in_panel(p, V, lanes_log2, panels, &c)) return;
+    place_in_part<W>(p, &c);
     using VT = Vec<T, V>;
     const T* o = static_cast<const T*>(p.output) + c.base;
     const T* g = static_cast<const T*>(p.grad_output) + c.base;
@@ -621,7 +682,7 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
     const int64_t sweep = static_cast<int64_t>(kColHeldBwd) * c.groups;
     Piece<T, V> held_o[kColHeldBwd], held_g[kColHeldBwd];
     auto load = [&](int64_t r0) {
-        ColWalk w(p, c, r0);
+        ColWalk w(p, c, length<W>(p, c), r0);
 #pragma unroll
         for (int k = 0; k < kColHeldBwd; ++k, w.next()) {
             if (w.exists()) {
@@ -636,35 +697,45 @@ __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams 
     float delta[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) delta[e] = 0.f;
-    for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
+    for (int64_t r0 = 0; W != kOutput && r0 < length<W>(p, c); r0 += sweep) {
         load(r0);
 #pragma unroll
         for (int k = 0; k < kColHeldBwd; ++k)
 #pragma unroll
             for (int e = 0; e < V; ++e) delta[e] = fmaf(held_o[k].get(e), held_g[k].get(e), delta[e]);
     }
-    for (int d = 1 << lanes_log2; d < 64; d <<= 1) {
+    if constexpr (W != kOutput) {
+        for (int d = 1 << lanes_log2; d < 64; d <<= 1) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) delta[e] += __shfl_xor(delta[e], d);
+            for (int e = 0; e < V; ++e) delta[e] += __shfl_xor(delta[e], d);
+        }
     }
     const int columns = V << lanes_log2, waves = blockDim.x / 64;
-    if ((threadIdx.x & 63) < (1 << lanes_log2)) {
+    if constexpr (W == kOutput) {
+        merge_parts(p, c, columns, 0.f, part_sums, [](float x, float y) { return x + y; });
+    } else {
+        if ((threadIdx.x & 63) < (1 << lanes_log2)) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) part_sums[(threadIdx.x / 64) * columns + c.lane * V + e] = delta[e];
+            for (int e = 0; e < V; ++e) part_sums[(threadIdx.x / 64) * columns + c.lane * V + e] = delta[e];
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < columns; i += blockDim.x) {
+            float t = part_sums[i];
+            for (int w = 1; w < waves; ++w) t += part_sums[w * columns + i];
+            if constexpr (W == kStatistics) {
+                if (c.first + i < p.y_size) static_cast<float*>(p.part_stats)[blockIdx.y * p.y_size + c.first + i] = t;
+            }
+            part_sums[i] = t;
+        }
+        if constexpr (W == kStatistics) return;
+        __syncthreads();
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < columns; i += blockDim.x) {
-        float t = part_sums[i];
-        for (int w = 1; w < waves; ++w) t += part_sums[w * columns + i];
-        part_sums[i] = t;
-    }
-    __syncthreads();
     if (!c.live) return;
 #pragma unroll
     for (int e = 0; e < V; ++e) delta[e] = part_sums[c.lane * V + e];
-    for (int64_t r0 = 0; r0 < p.x_size; r0 += sweep) {
-        if (p.x_size > sweep) load(r0);
-        ColWalk w(p, c, r0);
+    for (int64_t r0 = 0; r0 < length<W>(p, c); r0 += sweep) {
+        if (W == kOutput || length<W>(p, c) > sweep) load(r0);
+        ColWalk w(p, c, length<W>(p, c), r0);
 #pragma unroll
         for (int k = 0; k < kColHeldBwd; ++k, w.next()) {
             if (w.exists()) {
@@ -842,7 +913,8 @@ __global__ __launch_bounds__(256) void dropout_kernel(const RowParams p, const T
 // ------------------------------------------------------------------ host side
 int make_row_params(const TriRowArgs* a, bool backward, bool dropout, RowParams* p) {
     if (a == nullptr) return TRI_ATTN_ENULL;
-    if (a->struct_size != sizeof(TriRowArgs)) return TRI_ATTN_ESIZE;
+    // (structures of callers built before the workspace fields were added end there)
+    if (a->struct_size != sizeof(TriRowArgs) && a->struct_size != offsetof(TriRowArgs, workspace)) return TRI_ATTN_ESIZE;
     if (a->dtype < TRI_ATTN_F32 || a->dtype > TRI_ATTN_BF16) return TRI_ATTN_EDTYPE;
     if (a->y_size <= 0 || a->x_size <= 0) return TRI_ATTN_ESHAPE;
     if (!dropout && (a->y_stride < 0 || a->x_stride < 0)) return TRI_ATTN_ESTRIDE;
@@ -854,6 +926,10 @@ int make_row_params(const TriRowArgs* a, bool backward, bool dropout, RowParams*
         return TRI_ATTN_ENULL;
     }
     memset(p, 0, sizeof(*p));
+    if (a->struct_size == sizeof(TriRowArgs)) {
+        p->workspace = a->workspace;
+        p->workspace_bytes = a->workspace_size;
+    }
     p->input = a->input;
     p->output = a->output;
     p->mask = a->mask;
@@ -878,7 +954,7 @@ bool aligned16(const void* ptr) { return ptr == nullptr || (reinterpret_cast<uin
 
 // Geometry of a column launch: panels as wide as leaves one for every CU, but no narrower than the 64 bytes HBM moves at
 // a time (16 lanes without vector accesses), and as many threads as give each kColHeld (kColHeldBwd) pieces of its column.
-// A column is never split: a matrix narrower than 256 such panels leaves CUs idle (bf16 65536 x 64: two workgroups, 0.25 ms).
+// A matrix narrower than 256 such panels leaves CUs idle; column_split is for the long ones among them.
 struct ColLaunch {
     int lanes_log2;
     int64_t panels;
@@ -902,6 +978,39 @@ ColLaunch column_launch(const RowParams& p, int v, int held) {
     c.stats = static_cast<unsigned>(threads / 64 * (v << c.lanes_log2));
     return c;
 }
+
+// Geometry of the split launches: workgroups of 256 threads, panels of 64 bytes, and as many parts as give two workgroups per CU,
+// each at least four pieces per thread and at most the forward's sixteen, kMaxParts of them at most, whose statistics every
+// workgroup of the second launch reads. (Panels of 256 bytes in workgroups of 1024 threads: 38122 x 424 bf16 with mask 107 and 76
+// us, so 61 and 57.) Returns the bytes of workspace, 0: the launch stays whole. That is where half the CUs and more have a panel, or
+// a panel's columns stay in its registers, which are then read once and not twice.
+constexpr int kMaxParts = 128;
+int64_t column_split(const RowParams& p, int v, int elem_bytes, int held, int stat_bytes, RowParams* split, ColLaunch* c) {
+    const ColLaunch whole = column_launch(p, v, held);
+    if (whole.panels > 128 || p.x_size <= static_cast<int64_t>(whole.block.x >> whole.lanes_log2) * held) return 0;
+    *c = whole;
+    c->lanes_log2 = v > 1 ? 2 : (elem_bytes == 4 ? 4 : 5);
+    const int64_t columns = static_cast<int64_t>(v) << c->lanes_log2, groups = 256 >> c->lanes_log2;
+    c->panels = (p.y_size + columns - 1) / columns;
+    c->block = dim3(256);
+    const auto parts_of = [&](int64_t rows) { return (p.x_size + rows - 1) / rows; };
+    const int64_t parts = std::min<int64_t>(kMaxParts, std::max(parts_of(groups * 16), std::min((512 + c->panels - 1) / c->panels, parts_of(groups * 4))));
+    *split = p;
+    split->part_size = parts_of(parts);
+    split->parts = static_cast<int>(parts_of(split->part_size));
+    c->grid = dim3(static_cast<unsigned>((c->panels + 7) / 8 * 8), static_cast<unsigned>(split->parts));
+    c->stats = static_cast<unsigned>(std::max<int64_t>(4 * columns, 256));  // (statistics of four waves, or of 256 threads' columns)
+    return split->parts * p.y_size * stat_bytes;
+}
+bool take_workspace(int64_t bytes, RowParams* split) {
+    if (bytes <= 0 || split->workspace == nullptr || split->workspace_bytes < bytes || reinterpret_cast<uintptr_t>(split->workspace) % 16 != 0) return false;
+    split->part_stats = split->workspace;
+    return true;
+}
+
+// whether a column launch takes whole vectors of neighbouring columns: every element row starts on a 16-byte boundary and holds
+// whole vectors
+bool columns_vec(const RowParams& p, int v, bool aligned) { return p.y_stride == 1 && p.y_size % v == 0 && p.x_stride % v == 0 && aligned; }
 
 dim3 few_rows_grid(const RowParams& p, int v) { return dim3(static_cast<unsigned>((p.y_size + 256 * v - 1) / (256 * v))); }
 
@@ -942,8 +1051,7 @@ int launch_softmax_fwd(const RowParams& p, hipStream_t st) {
     constexpr int kV = 16 / sizeof(T);
     const dim3 block(256);
     if (p.x_stride != 1 && p.x_size != 1) {
-        // 16-byte accesses across the columns when every element row starts on a 16-byte boundary and holds whole vectors
-        const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.input) && aligned16(p.output) && aligned16(p.mask);
+        const bool vec = columns_vec(p, kV, aligned16(p.input) && aligned16(p.output) && aligned16(p.mask));
         // Whole vectors where they leave two workgroups and more per CU: below, one column per thread is faster (forward, bf16 16 x
         // 16384 0.0094 -> 0.0057 ms, 262144 columns 0.0110 -> 0.0079; from 524288 columns on the vectors, 16 x 1048576 0.0180 to 0.0207).
         // 16-bit columns of up to 32 elements go one per thread, too, with a mask, which the panels work through piece by piece
@@ -956,6 +1064,21 @@ int launch_softmax_fwd(const RowParams& p, hipStream_t st) {
         if constexpr (sizeof(T) == 2) {
             if (p.x_size <= 32 && (!std::is_same<M, void>::value || p.y_size <= 1 << 18)) {
                 hipLaunchKernelGGL((softmax_fwd_few_rows_kernel<T, 1, M, 32>), few_rows_grid(p, 1), block, 0, st, p);
+                return static_cast<int>(hipGetLastError());
+            }
+        }
+        {
+            RowParams split;
+            ColLaunch c;
+            if (p.workspace != nullptr && take_workspace(column_split(p, vec ? kV : 1, sizeof(T), kColHeld, sizeof(Stat), &split, &c), &split)) {
+                const unsigned lds = c.stats * sizeof(Stat);
+                if (vec) {
+                    hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, kV, M, kStatistics>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                    hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, kV, M, kOutput>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                } else {
+                    hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, 1, M, kStatistics>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                    hipLaunchKernelGGL((softmax_fwd_cols_kernel<T, 1, M, kOutput>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                }
                 return static_cast<int>(hipGetLastError());
             }
         }
@@ -986,11 +1109,26 @@ int launch_softmax_bwd(const RowParams& p, hipStream_t st) {
     constexpr int kV = 16 / sizeof(T);
     const dim3 block(256);
     if (p.x_stride != 1 && p.x_size != 1) {
-        const bool vec = p.y_stride == 1 && p.y_size % kV == 0 && p.x_stride % kV == 0 && aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input);
+        const bool vec = columns_vec(p, kV, aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input));
         if (p.x_size <= kFewRowsBwd<T>) {
             if (vec) hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, kV>), few_rows_grid(p, kV), block, 0, st, p);
             else hipLaunchKernelGGL((softmax_bwd_few_rows_kernel<T, 1>), few_rows_grid(p, 1), block, 0, st, p);
             return static_cast<int>(hipGetLastError());
+        }
+        {
+            RowParams split;
+            ColLaunch c;
+            if (p.workspace != nullptr && take_workspace(column_split(p, vec ? kV : 1, sizeof(T), kColHeldBwd, sizeof(float), &split, &c), &split)) {
+                const unsigned lds = c.stats * sizeof(float);
+                if (vec) {
+                    hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, kV, kStatistics>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                    hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, kV, kOutput>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                } else {
+                    hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, 1, kStatistics>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                    hipLaunchKernelGGL((softmax_bwd_cols_kernel<T, 1, kOutput>), c.grid, c.block, lds, st, split, c.lanes_log2, c.panels);
+                }
+                return static_cast<int>(hipGetLastError());
+            }
         }
         const ColLaunch c = column_launch(p, vec ? kV : 1, kColHeldBwd);
         const unsigned lds = c.stats * sizeof(float);
@@ -1067,6 +1205,21 @@ int tri_softmax_bwd(const TriRowArgs* args) {
     if (rc) return rc;
     p.mask = nullptr;  // masked positions have output 0: the gradient needs no mask
     return launch_softmax_any(args->dtype, p, true, static_cast<hipStream_t>(args->stream));
+}
+
+int64_t tri_softmax_workspace_size(const TriRowArgs* args, int backward) {
+    RowParams p, split;
+    const int rc = make_row_params(args, backward != 0, false, &p);
+    if (rc) return rc;
+    const int v = args->dtype == TRI_ATTN_F32 ? 4 : 8;
+    if (p.x_stride == 1 || p.x_size <= 32) return 0;
+    ColLaunch c;
+    if (backward) {
+        const bool vec = columns_vec(p, v, aligned16(p.output) && aligned16(p.grad_output) && aligned16(p.grad_input));
+        return column_split(p, vec ? v : 1, 16 / v, kColHeldBwd, sizeof(float), &split, &c);
+    }
+    const bool vec = columns_vec(p, v, aligned16(p.input) && aligned16(p.output) && aligned16(p.mask));
+    return column_split(p, vec ? v : 1, 16 / v, kColHeld, sizeof(Stat), &split, &c);
 }
 
 int tri_dropout_fwd(const TriRowArgs* args) {

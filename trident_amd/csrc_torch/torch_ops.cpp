@@ -41,6 +41,7 @@ struct Library {
     decltype(&tri_attn_prepare_mask) prepare_mask = nullptr;
     decltype(&tri_softmax_fwd) softmax_fwd = nullptr;
     decltype(&tri_softmax_bwd) softmax_bwd = nullptr;
+    decltype(&tri_softmax_workspace_size) softmax_workspace_size = nullptr;
     decltype(&tri_dropout_fwd) dropout_fwd = nullptr;
     decltype(&tri_dropout_bwd) dropout_bwd = nullptr;
 } lib;
@@ -317,8 +318,8 @@ TriAttnArgs make_args(const Call& call, const Tensor& q, const Tensor& k, const 
 }
 
 // operation._take_workspace
-Tensor take_workspace(TriAttnArgs& a, int pass, const Tensor& q) {
-    const int64_t size = lib.workspace_size(&a, pass);
+template <typename Args>
+Tensor give_workspace(Args& a, int64_t size, const Tensor& q) {
     if (size <= 0) return Tensor();
     try {
         Tensor workspace = at::empty({size}, q.options().dtype(at::kByte).requires_grad(false));
@@ -329,6 +330,7 @@ Tensor take_workspace(TriAttnArgs& a, int pass, const Tensor& q) {
         return Tensor();
     }
 }
+Tensor take_workspace(TriAttnArgs& a, int pass, const Tensor& q) { return give_workspace(a, lib.workspace_size(&a, pass), q); }
 
 // operation.Attention._forward
 std::pair<Tensor, Tensor> attention_forward(Call& call, const Tensor& query, const Tensor& key, const Tensor& value) {
@@ -603,6 +605,7 @@ Tensor softmax_forward(const Tensor& given, const std::optional<Tensor>& given_m
         a.mask = mask.data_ptr();
         a.mask_dtype = row_mask_code(mask.scalar_type());
     }
+    const Tensor workspace = give_workspace(a, lib.softmax_workspace_size(&a, 0), input);  // (rowops._take_workspace)
     check(lib.softmax_fwd(&a));
     return output;
 }
@@ -623,6 +626,7 @@ struct SoftmaxBackward : torch::autograd::Function<SoftmaxBackward> {
         a.output = output.data_ptr();
         a.grad_output = grad_output.data_ptr();
         a.grad_input = grad_input.data_ptr();
+        const Tensor workspace = give_workspace(a, lib.softmax_workspace_size(&a, 1), output);
         check(lib.softmax_bwd(&a));
         return {grad_input, Tensor(), Tensor()};
     }
@@ -749,6 +753,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     entry("tri_attn_prepare_mask", lib.prepare_mask);
     entry("tri_softmax_fwd", lib.softmax_fwd);
     entry("tri_softmax_bwd", lib.softmax_bwd);
+    entry("tri_softmax_workspace_size", lib.softmax_workspace_size);
     entry("tri_dropout_fwd", lib.dropout_fwd);
     entry("tri_dropout_bwd", lib.dropout_bwd);
     Py_INCREF(args[0]);

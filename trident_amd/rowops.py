@@ -72,6 +72,20 @@ def _dense(input):
     return input.contiguous()
 
 
+def _take_workspace(args, backward, device):
+    """Gives a call the scratch memory with which it runs split along the columns, where it does and the GPU has that much left;
+    returns the tensor to keep alive until the call is enqueued."""
+    size = _lib.lib().tri_softmax_workspace_size(ctypes.byref(args), backward)
+    if size <= 0:
+        return None
+    try:
+        workspace = torch.empty(size, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+    args.workspace, args.workspace_size = workspace.data_ptr(), size
+    return workspace
+
+
 def _softmax_forward(input, mask, dim, trace):
     _require_gpu(input, mask=mask)
     input = _dense(input)
@@ -83,6 +97,7 @@ def _softmax_forward(input, mask, dim, trace):
             raise ValueError(f"Unable to convert the given input: '{mask.dtype}'.")
         mask = _same_layout(mask, input)
         args.mask, args.mask_dtype = mask.data_ptr(), _MASK_CODES[mask.dtype]
+    workspace = _take_workspace(args, 0, input.device)  # noqa: F841
     util.push_trace(trace)
     _lib.check(_lib.lib().tri_softmax_fwd(ctypes.byref(args)))
     util.pop_trace()
@@ -95,6 +110,7 @@ def _softmax_backward(grad_output, output, dim, trace):
     grad_input = torch.empty_like(output)
     args = _row_args(output, dim)
     args.output, args.grad_output, args.grad_input = output.data_ptr(), grad_output.data_ptr(), grad_input.data_ptr()
+    workspace = _take_workspace(args, 1, output.device)  # noqa: F841
     util.push_trace(trace)
     _lib.check(_lib.lib().tri_softmax_bwd(ctypes.byref(args)))
     util.pop_trace()
