@@ -156,3 +156,16 @@ def test_workspaces_that_do_not_do(device):
     many = torch.empty(64, 16, 1024, 64, dtype=torch.float16, device=device)
     args = operation._make_args(many, many, many, many, torch.empty(64, 16, 1024, device=device), None, 0.0, True, 0.125, 0, 0)
     assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 0) == 0
+
+
+def test_infinities_in_keys_without_weight_reach_the_output(device, monkeypatch):
+    """Probability 0 times an infinite value is NaN, also where the key's whole part of the sequence weighs nothing."""
+    S, D = 2048, 128
+    q = torch.ones(1, 2, S, D, dtype=torch.bfloat16, device=device)
+    k, v = q.clone(), q.clone()
+    k[:, :, S // 2:] = -20.0
+    v[:, 0, 3 * S // 4, 5] = math.inf
+    for split in (True, False):
+        (o, *_), used = _run(q, k, v, q, None, 0.0, False, 1.0, (0, 0), split, monkeypatch)
+        assert used[0] == split
+        assert o[0, 0, :, 5].isnan().all() and torch.equal(o[0, 0, :, :5], v[0, 0, :, :5]) and torch.equal(o[0, 1], v[0, 1])

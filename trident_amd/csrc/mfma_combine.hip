@@ -80,7 +80,8 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
     for (int i = 0; i < count; ++i) {
         const float2 ml = stats[static_cast<int64_t>(i) * rows];
         const float w = fast_exp2(ml.x - m);  // (a row without a visible key: -inf - -inf, NaN as in the kernel)
-        const bool none = w == 0.f;           // (a part without a visible key has left nothing there)
+        // (a part without a visible key has left nothing there; one whose keys weigh nothing still hands on a NaN or an infinity in V)
+        const bool none = w == 0.f && ml.x == -INFINITY;
         l += none ? 0.f : w * ml.y;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
