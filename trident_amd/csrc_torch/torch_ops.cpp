@@ -266,6 +266,12 @@ Tensor mask_classes(const Tensor& mask, TriAttnArgs& a, bool may_cache) {
         std::vector<Tensor> freed;  // (released outside the lock)
         std::lock_guard<std::mutex> guard(classes_lock);
         auto& cache = classes_cache();
+        // (also what this entry replaces: a tensor that Python has seen takes the interpreter's lock to go, which a thread
+        // waiting for this one may hold)
+        if (const auto old = cache.find(key); old != cache.end()) {
+            freed.push_back(std::move(old->second.classes));
+            cache.erase(old);
+        }
         for (auto it = cache.begin(); it != cache.end();) {  // entries of tensors that are gone; all of them when it is full
             if (it->second.owner.expired() || cache.size() >= kMaxClasses) {
                 freed.push_back(std::move(it->second.classes));
