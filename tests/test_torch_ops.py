@@ -130,3 +130,15 @@ def test_a_call_that_fails_raises_as_before(device):
         trident.function.scaled_dot_product_attention(x, x, x, torch.zeros(3, 64, device=device))
     with pytest.raises(RuntimeError, match="dropout_p must lie in"):
         trident.function.dropout(x[0, 0], 1.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unpack", [lambda t: t.cpu(), lambda t: t.double(), lambda t: t[..., :8]])
+def test_saved_tensors_that_come_back_changed_are_refused(unpack, device):
+    """A hook's unpack may return anything: what the kernels could not read raises, and nothing is launched."""
+    x = torch.zeros(1, 1, 64, 16, dtype=torch.float16, device=device, requires_grad=True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        outputs = [trident.function.scaled_dot_product_attention(x, x, x), trident.function.softmax(x[0, 0], 1)]
+    for out in outputs:
+        with pytest.raises(RuntimeError, match="trident_amd: .*(on the same GPU|another shape or dtype)"):
+            out.sum().backward()

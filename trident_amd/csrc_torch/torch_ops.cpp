@@ -18,6 +18,7 @@
 #include <torch/extension.h>
 
 #include <cmath>
+#include <limits>
 #include <mutex>
 #include <unordered_map>
 
@@ -368,10 +369,24 @@ std::pair<Tensor, Tensor> attention_forward(Call& call, const Tensor& query, con
     return {output, lse};
 }
 
+// operation._require_same_gpu and rowops._require_gpu, for what a backward finds: a saved tensor may come back from a hook of the
+// caller's as something else, and the kernels take raw pointers.
+void require_saved_as(const Tensor& saved, const char* name, const Tensor& like, at::IntArrayRef sizes, at::ScalarType dtype) {
+    TORCH_CHECK(on_gpu(saved) && saved.device() == like.device(), "trident_amd: ", name, " is on ", saved.device(), ", expected ", like.device(),
+                " (all tensors of a call must be on the same GPU)");
+    TORCH_CHECK(saved.sizes() == sizes && saved.scalar_type() == dtype, "trident_amd: the saved ", name, " has come back with another shape or dtype");
+}
+
 // operation.Attention._backward
 std::array<Tensor, 4> attention_backward(const Call& call, const Tensor& grad_out, const Tensor& query, const Tensor& key, const Tensor& value,
-                                         const Tensor& output, const Tensor& lse, bool want_grad_mask) {
+                                         const Tensor& output, const Tensor& saved_lse, bool want_grad_mask) {
+    require_saved_as(query, "query", grad_out, grad_out.sizes(), grad_out.scalar_type());
+    require_saved_as(key, "key", query, query.sizes(), query.scalar_type());
+    require_saved_as(value, "value", query, query.sizes(), query.scalar_type());
+    require_saved_as(output, "output", query, query.sizes(), query.scalar_type());
+    require_saved_as(saved_lse, "log_sum_exp", query, query.sizes().slice(0, 3), at::kFloat);
     const c10::DeviceGuard device(query.device());
+    const Tensor lse = saved_lse.contiguous();
     const Tensor q = dense_rows(query), k = dense_rows(key), v = dense_rows(value), grad_output = dense_rows(grad_out);
     const int64_t B = q.size(0), H = q.size(1), S = q.size(2);
     const std::array<int64_t, 4> full = {B, H, S, S};
@@ -484,6 +499,8 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int64_t S = q->size(2), D = q->size(3);
     if ((D != 16 && D != 32 && D != 64 && D != 128) || q->numel() == 0 || !plain_context()) Py_RETURN_NONE;
+    for (int i = 0; i < 3; ++i)
+        if (q->size(i) > std::numeric_limits<int32_t>::max()) Py_RETURN_NONE;
     if (!PyFloat_CheckExact(args[4]) && !PyLong_CheckExact(args[4])) Py_RETURN_NONE;
     if (!PyBool_Check(args[5]) || !PyFloat_CheckExact(args[6])) Py_RETURN_NONE;
     const bool limits = is_true(config_dict, name_reference_limits);
@@ -625,6 +642,7 @@ struct SoftmaxBackward : torch::autograd::Function<SoftmaxBackward> {
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
         const Tensor output = ctx->get_saved_variables()[0];
+        require_saved_as(output, "output", grads[0], grads[0].sizes(), grads[0].scalar_type());
         const c10::DeviceGuard device(output.device());
         const Tensor grad_output = same_layout(grads[0], output);
         const Tensor grad_input = at::empty_like(output);
