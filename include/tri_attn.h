@@ -159,8 +159,8 @@ int tri_attn_bwd_dkdv(const TriAttnArgs* args);
 int tri_attn_bwd_dq(const TriAttnArgs* args);
 
 /* bwd_delta and bwd_dq in one launch, for the problems whose dQ kernel can compute delta from the dO
- * rows it loads anyway (the 16-bit matrix-core kernels without a mask: fp16/bf16, D in {16,32,64,128}, 16-byte
- * aligned rows of o): reads q,k,v,o,d_o,lse; writes delta and dq. tri_attn_bwd_dkdv, which reads delta, has to
+ * rows it loads anyway (the 16-bit matrix-core kernels without a mask, or with one at D <= 64 and dmask NULL: fp16/bf16,
+ * 16-byte aligned rows of o): reads q,k,v,o,d_o,lse; writes delta and dq. tri_attn_bwd_dkdv, which reads delta, has to
  * follow it. Returns TRI_ATTN_ENOFUSE without launching anything where it does not apply (then call
  * tri_attn_bwd_delta, tri_attn_bwd_dkdv, tri_attn_bwd_dq). The reference has the two launches only
  * (trident/operation/attention.py:161-199); tri_attn_bwd picks between the two sequences itself. */
@@ -176,8 +176,7 @@ int tri_attn_bwd_dmask(const TriAttnArgs* args);
 
 /* The whole backward (trident/operation/attention.py:137-202): the results of bwd_delta, bwd_dkdv and
  * bwd_dq called in that order, written to delta, dk, dv, dq[, dmask]. The library may launch fewer
- * kernels and in another order: where tri_attn_bwd_dq_delta applies (16-bit matrix-core kernels
- * without a mask, any S) the dQ kernel computes delta on its way and runs before dK/dV. */
+ * kernels and in another order: where tri_attn_bwd_dq_delta applies the dQ kernel computes delta on its way and runs before dK/dV. */
 int tri_attn_bwd(const TriAttnArgs* args);
 
 /* tri_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving

@@ -27,7 +27,7 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
             if (with_delta) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
         } else {
-            if constexpr (MASK == kNoMask) {
+            if constexpr (MASK == kNoMask || D <= 64) {
                 if (with_delta) {
                     if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
                     else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, false, false, true>), grid, block, 0, stream, p);
@@ -66,6 +66,13 @@ template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
     const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
     if constexpr (MASK != kNoMask) {
+        if constexpr (D <= 64) {
+            if (with_delta) {
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true, false, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true, false, true>), grid, block, 0, stream, p);
+                return static_cast<int>(hipGetLastError());
+            }
+        }
         if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true>), grid, block, 0, stream, p);
         else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
         return static_cast<int>(hipGetLastError());
@@ -110,7 +117,7 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
             return launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta);
         }
     }
-    if (with_delta && MASK != kNoMask) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
+    if (with_delta && MASK != kNoMask && (D > 64 || p.dmask != nullptr)) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
     // 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows)
     if constexpr (D > 16) {  // (a D = 16 tile has four blocks in all: four waves)
         if (p.S % 256 == 0) return launch_dq_waves<T, D, 8, CAUSAL, MASK>(p, stream, with_delta);
@@ -120,7 +127,7 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     if constexpr (MASK == kNoMask && D < 128) return launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);  // any other length
     // a padded mask: at D = 64 one workgroup of 8 waves per CU beside an fp32 mask's staging regions, two of 4 beside a 16-bit
     // one's (as the forward); at D = 128 four waves with the whole register file (in 256 registers the kernel spills)
-    if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, D == 64 && MASK == kMaskF32 ? 8 : 4, CAUSAL, MASK>(p, stream, false);
+    if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, D == 64 && MASK == kMaskF32 ? 8 : 4, CAUSAL, MASK>(p, stream, with_delta);
     return TRI_ATTN_ESHAPE;
 }
 

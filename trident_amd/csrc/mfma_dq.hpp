@@ -37,7 +37,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // DMASK (with a mask): the kernel also writes the mask gradient dS (trident/kernel/attention.py:332-335), each lane four
 // consecutive keys of its row at a time; where the mask is broadcast over a dimension (dmask stride 0) the values are
 // added to the caller's zero-filled fp32 buffer with atomic adds instead.
-// DELTA (no mask): the kernel also computes delta = rowsum(dO * O) of its rows from the dO rows it loads anyway, instead
+// DELTA (no mask, or D <= 64 without a mask gradient): the kernel also computes delta = rowsum(dO * O) of its rows from the dO rows it loads anyway, instead
 // of reading it, and stores it for the dK/dV pass, which then runs after this one (tri_attn_bwd_dq_delta).
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from
 // key0; the first part stores delta.
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
-    static_assert(!DELTA || MASK == 0, "delta on the way: the variants without a mask");
+    static_assert(!DELTA || MASK == 0 || (D <= 64 && !DMASK), "delta on the way: no mask, or a small head without a mask gradient");
     using Tile = SwzTile<D>;
     constexpr int kRows = 32 * NW;
     constexpr int kStages = 4;

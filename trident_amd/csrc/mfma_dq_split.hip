@@ -15,19 +15,24 @@ SplitShape dq_split_shape(const KParams& p) {
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_split(const KParams& p, hipStream_t stream, bool with_delta) {
     constexpr int NW = D == 64 && MASK == kMaskF32 ? 8 : 4;
-    constexpr bool kDelta = MASK == kNoMask;
     const dim3 grid = split_grid(p);
-    if (kDelta && !with_delta) return TRI_ATTN_ESHAPE;  // (dq_splits)
+    if (MASK == kNoMask && !with_delta) return TRI_ATTN_ESHAPE;  // (dq_splits)
     if constexpr (D == 128 && MASK == kNoMask) {
         if (p.thr8 <= 0) {
             hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, true, true>), grid, dim3(512), 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
-    else if constexpr (!(D == 128 && MASK == kNoMask))
-        hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
-    return static_cast<int>(hipGetLastError());
+    const auto launch = [&](auto delta) {
+        constexpr bool kDelta = decltype(delta)::value;
+        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
+        else if constexpr (!(D == 128 && MASK == kNoMask))
+            hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, true, false, kDelta, true>), grid, dim3(64 * NW), 0, stream, p);
+        return static_cast<int>(hipGetLastError());
+    };
+    if constexpr (MASK == kNoMask) return launch(std::true_type{});
+    else if constexpr (D > 64) return launch(std::false_type{});
+    else return with_delta ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 template <typename T, int D>
@@ -39,8 +44,10 @@ int launch_dq_split_variant(int dtype, const KParams& p, hipStream_t stream, boo
     return TRI_ATTN_EDTYPE;
 }
 
-// (a mask gradient is written by whole items only; without a mask the parts bring delta along)
-bool dq_splits(const KParams& p, bool with_delta) { return p.dmask == nullptr && with_delta == (p.mask == nullptr); }
+// (a mask gradient is written by whole items only; without a mask the parts bring delta along, with one they may up to D = 64)
+bool dq_splits(const KParams& p, bool with_delta) {
+    return p.dmask == nullptr && (p.mask == nullptr ? with_delta : !with_delta || p.D <= 64);
+}
 
 template <typename T>
 int launch_dq_split_head(int dtype, const KParams& p, hipStream_t stream, bool with_delta) {

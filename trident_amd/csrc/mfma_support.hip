@@ -206,12 +206,15 @@ bool mfma_supported(int which, int dtype, const KParams& p) {
     }
 }
 
-// Without a mask the dQ kernels compute delta themselves, from the dO rows they load anyway and the O rows (16-byte
-// aligned like the others): the phased kernel through LDS (32-bit row offsets), the others with per-lane loads.
+// The dQ kernels compute delta themselves, from the dO rows they load anyway and the O rows (16-byte
+// aligned like the others): the phased kernel through LDS (32-bit row offsets), the others with per-lane loads. With a mask up to
+// D = 64 (us, the pre-pass of 9.5 and 10 against a dQ pass that reads O: training steps of bf16 B=8 H=12 S=2048 D=64, length mask,
+// 521 -> 511, fp16 B=16 H=12 S=777 D=64, key padding, 254 -> 245); not at D = 128, whose masked kernels fill their registers
+// (a row of O is 32 more in the prologue), and not where the pass writes a mask gradient, whose variants would double.
 bool mfma_dq_fuses_delta(const KParams& p) {
-    if (p.mask != nullptr) return false;
+    if (p.mask != nullptr && (p.D > 64 || p.dmask != nullptr)) return false;
     if (!aligned16(p.o) || !strides8(p.os)) return false;
-    const bool phased = p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0;  // (as the launcher decides)
+    const bool phased = p.mask == nullptr && (p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0);  // (as the launcher decides)
     return !phased || tile_offsets_fit(p.os);
 }
 
