@@ -159,8 +159,8 @@ int tri_attn_bwd_dkdv(const TriAttnArgs* args);
 int tri_attn_bwd_dq(const TriAttnArgs* args);
 
 /* bwd_delta and bwd_dq in one launch, for the problems whose dQ kernel can compute delta from the dO
- * rows it loads anyway (the 16-bit matrix-core kernels without a mask, or with one at D <= 64 and dmask NULL: fp16/bf16,
- * 16-byte aligned rows of o): reads q,k,v,o,d_o,lse; writes delta and dq. tri_attn_bwd_dkdv, which reads delta, has to
+ * rows it loads anyway (the 16-bit matrix-core kernels without a mask, or with one at D <= 64 and dmask NULL, with 16-byte
+ * aligned rows of o; whatever runs on the fp32 matrix instruction, with rows of o aligned to four elements): reads q,k,v,o,d_o,lse; writes delta and dq. tri_attn_bwd_dkdv, which reads delta, has to
  * follow it. Returns TRI_ATTN_ENOFUSE without launching anything where it does not apply (then call
  * tri_attn_bwd_delta, tri_attn_bwd_dkdv, tri_attn_bwd_dq). The reference has the two launches only
  * (trident/operation/attention.py:161-199); tri_attn_bwd picks between the two sequences itself. */

@@ -254,8 +254,10 @@ int tri_attn_bwd_dq_delta(const TriAttnArgs* args) {
     KParams p;
     int rc = make_params(args, 2 | 8, &p);
     if (rc) return rc;
-    if (!(mfma_supported(kMfmaDq, args->dtype, p) && mfma_dq_fuses_delta(p))) return TRI_ATTN_ENOFUSE;
-    return launch_mfma_dq(args->dtype, p, static_cast<hipStream_t>(args->stream), true);
+    hipStream_t st = static_cast<hipStream_t>(args->stream);
+    if (mfma_supported(kMfmaDq, args->dtype, p)) return mfma_dq_fuses_delta(p) ? launch_mfma_dq(args->dtype, p, st, true) : TRI_ATTN_ENOFUSE;
+    if (!(mfma32_supported(kMfmaDq, args->dtype, p) && mfma32_dq_fuses_delta(args->dtype, p))) return TRI_ATTN_ENOFUSE;
+    return launch_mfma32(kMfmaDq, args->dtype, p, st, true);
 }
 
 int tri_attn_bwd(const TriAttnArgs* args) {

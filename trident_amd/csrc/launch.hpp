@@ -36,7 +36,8 @@ int64_t mfma_dmask_workspace(const KParams& p);  // bytes with which it deals th
 // aligned to four elements. `which` is a MfmaKernel.
 bool mfma32_supported(int which, int dtype, const KParams& p);
 int64_t mfma32_workspace(int which, int dtype, const KParams& p);  // as mfma_fwd_workspace below
-int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream);
+int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream, bool with_delta = false);
+bool mfma32_dq_fuses_delta(int dtype, const KParams& p);  // (as mfma_dq_fuses_delta, where mfma32_supported)
 // Classes of the mask's 64 x 64 blocks (0 all zero, 1 all -inf, 2 mixed) into `out`, laid out as p.mcs says.
 int launch_classify_mask(const KParams& p, uint8_t* out, hipStream_t stream);
 // Source mask (additive, or bytes: TRI_ATTN_BOOL) -> padded additive mask `out` laid out as p.ms says, and its block classes

@@ -310,7 +310,9 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
 // ------------------------------------------------------------------------------------------------ dQ (and dMask)
 // Same data flow as the forward kernel: S^T = K Q^T and dP^T = V dO^T against the wave's Q and dO rows in registers,
 // P and dS on the vector ALU (this lane: its query, 16 keys), dQ^T += K^T dS^T walking the keys in accumulator order.
-template <typename T, int D, bool SPLIT>
+// DELTA: delta = rowsum(dO * O) of its rows is computed from the dO rows it loads anyway and stored for the dK/dV pass, which then
+// runs after this one (the first part of a split item stores it).
+template <typename T, int D, bool SPLIT, bool DELTA>
 __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const KParams p) {
     constexpr int LD = D + 4;
     constexpr int DB = D >= 32 ? D / 32 : 1;
@@ -340,17 +342,30 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
     const int64_t dmrow = p.dmask ? b * p.dms[0] + hd * p.dms[1] + qrow_c * p.dms[2] : 0;
 
     quad_t<T> qf[KJ], gf[KJ];
+    float dlt;
     {
         const T* qptr = static_cast<const T*>(p.q) + b * p.qs[0] + hd * p.qs[1] + qrow_c * p.qs[2];
         const T* gptr = static_cast<const T*>(p.d_o) + b * p.dos[0] + hd * p.dos[1] + qrow_c * p.dos[2];
+        [[maybe_unused]] const T* optr = static_cast<const T*>(p.o) + b * p.os[0] + hd * p.os[1] + qrow_c * p.os[2];
+        float4 sum{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < KJ; ++j) {
+            const float4 g4 = load4(gptr + 8 * j + 4 * h);
             qf[j] = quad<T>(load4(qptr + 8 * j + 4 * h));
-            gf[j] = quad<T>(load4(gptr + 8 * j + 4 * h));
+            gf[j] = quad<T>(g4);
+            if constexpr (DELTA) {  // (this lane has half of its row, the lane across the other half)
+                const float4 o4 = load4(optr + 8 * j + 4 * h);
+                sum = float4{fmaf(o4.x, g4.x, sum.x), fmaf(o4.y, g4.y, sum.y), fmaf(o4.z, g4.z, sum.z), fmaf(o4.w, g4.w, sum.w)};
+            }
+        }
+        if constexpr (DELTA) {
+            dlt = sum_xor32((sum.x + sum.y) + (sum.z + sum.w));
+            if (h == 0 && row_ok && (!SPLIT || part.index == 0)) p.delta[static_cast<int64_t>(bh) * p.S + qrow] = dlt;
+        } else {
+            dlt = p.delta[static_cast<int64_t>(bh) * p.S + qrow_c];
         }
     }
     const float lse = p.lse[static_cast<int64_t>(bh) * p.S + qrow_c];
-    const float dlt = p.delta[static_cast<int64_t>(bh) * p.S + qrow_c];
     f32x16 acc[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db) acc[db] = zero16();
@@ -868,10 +883,11 @@ SplitShape split_shape32(int which, const KParams& p) {
 bool splits32(int which, int dtype, const KParams& p) { return dtype == TRI_ATTN_F32 && !(which == kMfmaDq && p.dmask != nullptr); }
 
 template <int D>
-int launch32_split(int which, const KParams& p, int rows, hipStream_t stream) {
+int launch32_split(int which, const KParams& p, int rows, hipStream_t stream, bool with_delta) {
     const dim3 grid = split_grid(p), block(256);
     if (which == kMfmaFwd) hipLaunchKernelGGL((mfma32_fwd_kernel<float, D, true>), grid, block, 0, stream, p);
-    else if (which == kMfmaDq) hipLaunchKernelGGL((mfma32_dq_kernel<float, D, true>), grid, block, 0, stream, p);
+    else if (which == kMfmaDq && with_delta) hipLaunchKernelGGL((mfma32_dq_kernel<float, D, true, true>), grid, block, 0, stream, p);
+    else if (which == kMfmaDq) hipLaunchKernelGGL((mfma32_dq_kernel<float, D, true, false>), grid, block, 0, stream, p);
     else if constexpr (D == 128) hipLaunchKernelGGL((mfma32_dkdv_split_kernel<float, D, true>), grid, block, 0, stream, p);
     else hipLaunchKernelGGL((mfma32_dkdv_kernel<float, D, true>), grid, block, 0, stream, p);
     const int rc = static_cast<int>(hipGetLastError());
@@ -881,7 +897,7 @@ int launch32_split(int which, const KParams& p, int rows, hipStream_t stream) {
 }
 
 template <typename T, int D>
-int launch32(int which, const KParams& p, hipStream_t stream) {
+int launch32(int which, const KParams& p, hipStream_t stream, bool with_delta) {
     const int64_t groups = static_cast<int64_t>((p.S + kRowsPerGroup - 1) / kRowsPerGroup) * p.B * p.H;
     if (groups > 2147483647LL) return TRI_ATTN_ESHAPE;
     const dim3 grid(static_cast<unsigned>(groups)), block(256);
@@ -890,7 +906,8 @@ int launch32(int which, const KParams& p, hipStream_t stream) {
             hipLaunchKernelGGL((mfma32_fwd_kernel<T, D, false>), grid, block, 0, stream, p);
             break;
         case kMfmaDq:
-            hipLaunchKernelGGL((mfma32_dq_kernel<T, D, false>), grid, block, 0, stream, p);
+            if (with_delta) hipLaunchKernelGGL((mfma32_dq_kernel<T, D, false, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma32_dq_kernel<T, D, false, false>), grid, block, 0, stream, p);
             break;
         case kMfmaDkdv:
             if constexpr (D == 128) {
@@ -908,12 +925,12 @@ int launch32(int which, const KParams& p, hipStream_t stream) {
 }
 
 template <typename T>
-int launch32_d(int which, const KParams& p, hipStream_t stream) {
+int launch32_d(int which, const KParams& p, hipStream_t stream, bool with_delta) {
     switch (p.D) {
-        case 16: return launch32<T, 16>(which, p, stream);
-        case 32: return launch32<T, 32>(which, p, stream);
-        case 64: return launch32<T, 64>(which, p, stream);
-        case 128: return launch32<T, 128>(which, p, stream);
+        case 16: return launch32<T, 16>(which, p, stream, with_delta);
+        case 32: return launch32<T, 32>(which, p, stream, with_delta);
+        case 64: return launch32<T, 64>(which, p, stream, with_delta);
+        case 128: return launch32<T, 128>(which, p, stream, with_delta);
         default: return TRI_ATTN_ESHAPE;
     }
 }
@@ -944,20 +961,25 @@ int64_t mfma32_workspace(int which, int dtype, const KParams& p) {
     return splits32(which, dtype, p) ? plan_split(split_shape32(which, p), p.causal != 0, &plan) : 0;
 }
 
-int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream) {
+// The delta pre-pass is a launch that reads O and dO; here dO's rows are at hand, and O's are read four elements at a time like
+// the others (us, forward and backward, fp32: B=32 H=8 S=512 D=64 641 -> 634, causal 441 -> 430; B=16 H=16 S=256 D=16 68 -> 63; B=2
+// H=16 S=2048 D=128 1525 either way).
+bool mfma32_dq_fuses_delta(int dtype, const KParams& p) { return rows4(p.o, p.os, dtype == TRI_ATTN_F32 ? 4 : 2); }
+
+int launch_mfma32(int which, int dtype, const KParams& p, hipStream_t stream, bool with_delta) {
     if (p.workspace != nullptr && splits32(which, dtype, p)) {
         KParams plan = p;
         const SplitShape shape = split_shape32(which, p);
         if (take_workspace(plan_split(shape, p.causal != 0, &plan), &plan))
-            return p.D == 128  ? launch32_split<128>(which, plan, shape.rows, stream)
-                   : p.D == 64 ? launch32_split<64>(which, plan, shape.rows, stream)
-                   : p.D == 32 ? launch32_split<32>(which, plan, shape.rows, stream)
-                               : launch32_split<16>(which, plan, shape.rows, stream);
+            return p.D == 128  ? launch32_split<128>(which, plan, shape.rows, stream, with_delta)
+                   : p.D == 64 ? launch32_split<64>(which, plan, shape.rows, stream, with_delta)
+                   : p.D == 32 ? launch32_split<32>(which, plan, shape.rows, stream, with_delta)
+                               : launch32_split<16>(which, plan, shape.rows, stream, with_delta);
     }
     switch (dtype) {
-        case TRI_ATTN_F32: return launch32_d<float>(which, p, stream);
-        case TRI_ATTN_F16: return launch32_d<f16_t>(which, p, stream);
-        case TRI_ATTN_BF16: return launch32_d<bf16_t>(which, p, stream);
+        case TRI_ATTN_F32: return launch32_d<float>(which, p, stream, with_delta);
+        case TRI_ATTN_F16: return launch32_d<f16_t>(which, p, stream, with_delta);
+        case TRI_ATTN_BF16: return launch32_d<bf16_t>(which, p, stream, with_delta);
         default: return TRI_ATTN_EDTYPE;
     }
 }
