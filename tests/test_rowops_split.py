@@ -53,6 +53,25 @@ def test_split_columns(dtype, rows, cols, mask_dtype, device, monkeypatch):
         assert (a - e).abs().max() <= 1.5 * (b - e).abs().max() + 1e-7 * e.abs().max()
 
 
+@pytest.mark.parametrize("dtype,rows,cols", [(torch.float32, 2049, 512), (torch.float32, 4096, 500), (torch.bfloat16, 4000, 1024), (torch.float16, 2100, 1023),
+                                             (torch.float32, 4096, 2052)])
+def test_panels_of_32_bytes(dtype, rows, cols, device, monkeypatch):
+    """The backward's narrow panels, whose lines are dealt out in another order: numbers of them that are dealt, do not fill up the last
+    XCD, or stay in order. A panel's sums do not depend on its place: equal to those of the same columns in another matrix."""
+    g = torch.Generator(device=device).manual_seed(rows + cols)
+    x, grad = [torch.randn(rows, cols, generator=g, device=device).to(dtype) for _ in range(2)]
+    (out, dx), _ = _run(x, None, grad, False, monkeypatch)
+    exact = x.double().softmax(0)
+    want = exact * (grad.double() - (exact * grad.double()).sum(0))
+    limit = {torch.float32: 1e-6, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]  # (half an ulp of every element and of the output)
+    for a, e in ((out, exact), (dx, want)):
+        per_column = (a.double() - e).norm(dim=0) / e.norm(dim=0)
+        assert per_column.max() <= 1.5 * limit
+    if cols % 8 == 0:
+        (_, again), _ = _run(x.roll(cols // 2, 1), None, grad.roll(cols // 2, 1), False, monkeypatch)
+        assert torch.equal(again, dx.roll(cols // 2, 1))
+
+
 def test_columns_far_from_zero(device, monkeypatch):
     x = torch.randn(9000, 12, device=device)
     x[:, 3] -= 1e10

@@ -459,7 +459,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
 // panels go to the same XCD: where a panel row is narrower than a 128-byte line, the other half is then still in its L2.
 // The statistics' LDS is sized by the workgroup, so that single-wave ones fill a CU.
 // fp32 4096 x 4096 along dim 0, launches in a row: forward 0.0254 ms = 5.3 TB/s (what a large copy reaches), backward 0.0435 ms =
-// 4.6 TB/s (in a training step, whose four tensors fill the Infinity Cache, 0.031 and 0.068 ms). One
+// 4.6 TB/s (in a training step, whose four tensors fill the Infinity Cache, 0.031 and 0.059 ms). One
 // thread per column, which this replaces, took 2.1 and 2.4 ms: 64 waves in flight on the whole chip, each waiting for one
 // load at a time. (Its sums ran in plain order, too: at 65536 elements off by 7.5e-5, these by 1.8e-7.)
 constexpr int kColHeld = 16;        // forward: pieces a thread keeps (64 registers)
@@ -511,9 +511,17 @@ __device__ __forceinline__ void merge_parts(const RowParams& p, const ColPlace& 
     }
     __syncthreads();
 }
-__device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int lanes_log2, int64_t panels, ColPlace* c) {
+__device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int lanes_log2, int64_t panels, ColPlace* c, bool narrow = false) {
     const int64_t per_xcd = (panels + 7) / 8;
-    const int64_t panel = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    int64_t i = blockIdx.x >> 3;
+    // Panels of 32 bytes run in two rounds of the CUs. In order, a round covers every other KiB of the matrix's rows, which the HBM
+    // channels take badly; so the first round takes the even 128-byte lines and the second the odd ones (fp32 4096 x 4096, forward and
+    // backward, 102 -> 93.6 us; pieces of 64 bytes 100.7, of 256 bytes 94.8, the lines dealt to the XCDs in turn 95.5).
+    if (narrow && per_xcd % 8 == 0) {
+        const int64_t half = per_xcd / 8, u = i >> 2;
+        i = ((u < half ? 2 * u : 2 * (u - half) + 1) << 2) + (i & 3);
+    }
+    const int64_t panel = (blockIdx.x & 7) * per_xcd + i;
     if (panel >= panels) return false;  // (the whole workgroup)
     c->lane = threadIdx.x & ((1 << lanes_log2) - 1);
     c->group = threadIdx.x >> lanes_log2;
@@ -673,7 +681,7 @@ template <typename T, int V, ColWork W = kWhole>
 __global__ __launch_bounds__(1024) void softmax_bwd_cols_kernel(const RowParams p, int lanes_log2, int64_t panels) {
     extern __shared__ float part_sums[];  // one per wave and column of the panel
     ColPlace c;
-    if (!place_in_panel(p, V, lanes_log2, panels, &c)) return;
+    if (!place_in_panel(p, V, lanes_log2, panels, &c, (sizeof(T) * V << lanes_log2) == 32)) return;
     place_in_part<W>(p, &c);
     using VT = Vec<T, V>;
     const T* o = static_cast<const T*>(p.output) + c.base;
