@@ -43,7 +43,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions. The ring then has
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
     // phase before V of tile t, so with K(j + dist) and V(j + dist - 1) requested together every tile keeps the lead
-    // it has in the ring of four, and both fit three slots.
+    // it has in the ring of four, and both fit three slots. The first fragments of V wait for the barrier, though.
     constexpr bool kLeadK = D == 128 && MASK == 1 && NW == 8 && !DROPOUT;
     constexpr int kStages = kLeadK ? 3 : 4;  // LDS ring depth
     constexpr int kLag = kLeadK ? 1 : 0;     // how many tiles the V requests trail the K requests
@@ -546,7 +546,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 }
                 if constexpr (!DROPOUT) pb[ks] = pack8<T>(&x[8 * ks]);
                 if (ks < 2 && issued_v) issue_slice(j + dist, 2 + ks, issued, issued_v);
-                if (ks < 2) {
+                if (ks < 2 && !kLeadK) {
 #pragma unroll
                     for (int r = kRing / 2 * ks; r < kRing / 2 * (ks + 1); ++r) ring[r] = frag(Yes{}, st, r);
                 }
@@ -607,6 +607,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
             // them on whatever the next slot holds, the result is never used: the branch would cost registers
             // that variant does not have)
             if (with_s) load_mask(j + 1);
+            // (where the K tiles lead, group 0 has requested the V tile j in the step before this one and awaited it only now: no
+            // fragment of it can be read any earlier)
+            if constexpr (kLeadK) {
+#pragma unroll
+                for (int r = 0; r < kRing; ++r) ring[r] = frag(Yes{}, st, r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // the few instructions of this phase go first, so that the matrix pipe never waits for an
             // issue slot behind the partner's vector work
             __builtin_amdgcn_s_setprio(2);
