@@ -45,10 +45,12 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
                 return static_cast<int>(hipGetLastError());
             }
         }
-        // a padded mask: one workgroup of 8 waves per CU at D = 64 (LDS), 4 waves with the whole register file at D = 128
+        // a padded mask: at D = 64 beside an fp32 one's regions one workgroup of 8 waves per CU; beside a 16-bit one's the LDS holds two
+        // of 4 with a ring of three, whose 128 keys end closer to the sequence's end and wait at barriers of their own (fp16 B=16 H=12
+        // S=777 with key padding, forward and backward, 248 -> 218 us). 4 waves with the whole register file at D = 128
         if constexpr (MASK != kNoMask) {
             // (dropout beside mask and boundary handling does not fit 256 registers: four waves)
-            constexpr int NW = D == 64 ? 8 : 4;
+            constexpr int NW = D == 64 && MASK == kMaskF32 ? 8 : 4;
             const int nw = p.thr8 > 0 ? 4 : NW;
             const dim3 grid(p.B * p.H * ((p.S + 32 * nw - 1) / (32 * nw))), block(64 * nw);
             if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, false, MASK, true, true>), grid, block, 0, stream, p);

@@ -37,11 +37,13 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // are not stored.
 // SPLIT (with RAGGED): a workgroup streams one part of its item's row tiles (split.hpp).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
+__global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
     constexpr int kKeys = 32 * NW;
-    constexpr int kStages = 4;
+    // (a ring of three where it lets a second workgroup onto the CU beside the mask regions, as launch_dkdv_dropout says)
+    constexpr int kStages = MASK == kMaskT && D == 64 && NW == 4 && RAGGED && !DROPOUT ? 3 : 4;
+    constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes + 2 * kBN * 4;  // Q tile, dO tile, lse, delta
     constexpr int KK = D / 16;
     constexpr int DB = D >= 32 ? D / 32 : 1;  // (D = 16: one block of gradient columns, the upper 16 are not stored)
@@ -196,13 +198,13 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
                                               : static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
         }
     };
-    // issue order: mask block of the first tile, three tiles, then per tile j: mask j+1, tile j+3
+    // issue order: mask block of the first tile, kAhead tiles, then per tile j: mask j+1, tile j+kAhead
     if (t_begin < n_tiles) {
         issue_mask(t_begin);
         issue_tile(t_begin);
     }
     if (t_begin + 1 < n_tiles) issue_tile(t_begin + 1);
-    if (t_begin + 2 < n_tiles) issue_tile(t_begin + 2);
+    if (kAhead > 2 && t_begin + 2 < n_tiles) issue_tile(t_begin + 2);
     // (the K and V fragments were requested before the tiles, so both latencies overlap)
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
@@ -219,10 +221,10 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
 
     for (int j = t_begin; j < n_tiles; ++j) {
         {
-            // with a staged mask, block j must have landed too: only tile j+2 was issued after it
-            // (two tiles after the first block)
-            // (a block that is all zero was never requested: then the two youngest tiles are what may be in flight)
-            const int younger = kMaskViaLds && j > t_begin && !mask_is_zero(j) ? min(1, max(0, n_tiles - 2 - j)) : min(2, n_tiles - 1 - j);
+            // with a staged mask, block j must have landed too: only tile j + kAhead - 1 was issued after it
+            // (the kAhead first tiles after the first block)
+            // (a block that is all zero was never requested: then the kAhead - 1 youngest tiles are what may be in flight)
+            const int younger = kMaskViaLds && j > t_begin && !mask_is_zero(j) ? min(1, max(0, n_tiles - (kAhead - 1) - j)) : min(kAhead - 1, n_tiles - 1 - j);
             if (younger == 2) TRI_WAIT_VMCNT(2 * kLoadsPerTile);
             else if (younger == 1) TRI_WAIT_VMCNT(kLoadsPerTile);
             else TRI_WAIT_VMCNT(0);
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 ? 1 : 2) void mfma_dkdv_
             }
             if (j + 1 < n_tiles) issue_mask(j + 1);
         }
-        if (j + 3 < n_tiles) issue_tile(j + 3);
+        if (j + kAhead < n_tiles) issue_tile(j + kAhead);
         if (j < my_begin) continue;
 
         const char* sQ = smem + (j % kStages) * kStageBytes;
