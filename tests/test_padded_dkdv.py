@@ -1,4 +1,4 @@
-"""dK and dV of padded 16-bit masks at head size 64: 128 keys a workgroup, two of them on a CU, a ring of three row tiles."""
+"""dK and dV of 16-bit masks at head size 64: 128 keys a workgroup, two of them on a CU, a ring of three row tiles."""
 import math
 
 import pytest
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["keys", "length", "dense"])
-@pytest.mark.parametrize("S", [129, 191, 257, 777])
+@pytest.mark.parametrize("S", [128, 129, 191, 256, 257, 512, 777])
 def test_a_batch_does_not_depend_on_its_company(S, kind, dtype, device):
     """Two to thirteen row tiles, with and without tiles left out or of zeros only: every batch of a launch with several workgroups per
     CU gets bit for bit what it gets alone, and two heads match the oracle."""

@@ -63,7 +63,12 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
         // the two-waves-per-SIMD kernel fits its registers: 8 waves (256 keys) when the sequence
         // allows it, else 4 waves (128 keys)
         if constexpr (D > 16) {
-            if (p.S % 256 == 0) return launch_dkdv_waves<T, D, 8, CAUSAL, MASK>(p, stream);
+            // (beside a 16-bit mask two workgroups of 4 fit a CU, as above, and are faster wherever those of 8 leave CUs idle in
+            // their last round: bf16 training steps at D = 64, heads x S, 96 x 512 93.6 -> 91.9 us, 96 x 768 180 -> 167; in whole
+            // rounds 64 x 1024 127.5 either way against 128.3. 192 x 640, one of 4 before, 199 -> 161)
+            const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256);
+            const bool pairs = D == 64 && MASK == kMaskT && p.thr8 <= 0 && items % persistent_grid(1 << 20) != 0;
+            if (p.S % 256 == 0 && !pairs) return launch_dkdv_waves<T, D, 8, CAUSAL, MASK>(p, stream);
         }
         return launch_dkdv_waves<T, D, 4, CAUSAL, MASK>(p, stream);
     } else {

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
     using Tile = SwzTile<D>;
     constexpr int kKeys = 32 * NW;
     // (a ring of three where it lets a second workgroup onto the CU beside the mask regions, as launch_dkdv_dropout says)
-    constexpr int kStages = MASK == kMaskT && D == 64 && NW == 4 && RAGGED && !DROPOUT ? 3 : 4;
+    constexpr int kStages = MASK == kMaskT && D == 64 && NW == 4 && !DROPOUT ? 3 : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes + 2 * kBN * 4;  // Q tile, dO tile, lse, delta
     constexpr int KK = D / 16;
