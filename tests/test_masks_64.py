@@ -66,6 +66,36 @@ def test_learned_masks_at_lengths_that_are_no_multiple_of_128(S, D, shape, small
     parity.close(grads[3].reshape(full.shape), dm, torch.bfloat16, "dMask")
 
 
+@pytest.mark.parametrize("path", ["C++", "Python"])
+@pytest.mark.parametrize("moved", ["query", "key", "value", "grad"])
+@pytest.mark.parametrize("S,D,from_,pitch", [(64, 64, 4, 72), (192, 128, 0, 129), (260, 32, 4, 40)])
+def test_learned_full_masks_beside_rows_off_the_16_byte_boundaries(S, D, from_, pitch, moved, path, device, monkeypatch):
+    """tri_attn_bwd_dmask does not take such rows: the dQ pass writes the gradient of a [B,H,S,S] mask, as at multiples of 128. (Memory
+    freed before the backward holds NaN: a gradient that nobody writes shows.)"""
+    monkeypatch.setattr(operation, "_PADS_FROM", 0)
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(S)
+    given = {n: torch.randn(B, H, S, D, generator=g).to(torch.bfloat16) for n in ("query", "key", "value", "grad")}
+    mask = (0.5 * torch.randn(B, H, S, S, generator=g)).to(torch.bfloat16)
+    on_gpu = {n: x.to(device) for n, x in given.items()}
+    on_gpu[moved] = torch.zeros(B, H, S, pitch, dtype=torch.bfloat16, device=device)[..., from_:from_ + D].copy_(given[moved])
+    tq, tk, tv, tm = [x.requires_grad_() for x in (on_gpu["query"], on_gpu["key"], on_gpu["value"], mask.to(device))]
+    call = trident.function.scaled_dot_product_attention if path == "C++" else \
+        lambda q, k, v, m: operation.Attention.apply(q, k, v, m, 0.0, False, 1.0 / math.sqrt(D), False)
+    out = call(tq, tk, tv, tm)
+    assert (type(out.grad_fn).__name__ == "AttentionBackward") == (path == "Python")
+    stale = [torch.full_like(mask, math.nan, device=device) for _ in range(8)]
+    del stale
+    grads = torch.autograd.grad(out, (tq, tk, tv, tm), on_gpu["grad"])
+    q, k, v, d_o = given.values()
+    dq, dk, dv, dm, _ = parity.oracle_backward(q, k, v, d_o, mask=mask.float(), want_dmask=True, o=out.detach())
+    _, a_dq, a_dk, a_dv = parity.oracle_abs_sums(q, k, v, d_o, mask=mask.float(), o=out.detach())
+    for name, got, want, terms in (("dQ", grads[0], dq, a_dq), ("dK", grads[1], dk, a_dk), ("dV", grads[2], dv, a_dv)):
+        parity.close(got, want, torch.bfloat16, name, terms)
+    parity.close(grads[3], dm, torch.bfloat16, "dMask")
+
+
 @pytest.mark.parametrize("p", [0.0, 0.2])
 @pytest.mark.parametrize("shape", ["1HSS", "11SS"])
 @pytest.mark.parametrize("B,H,S,D,mask_dtype", [(40, 3, 70, 64, torch.bfloat16), (50, 2, 130, 128, torch.float32), (33, 4, 64, 32, torch.bfloat16),

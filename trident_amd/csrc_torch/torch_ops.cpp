@@ -433,8 +433,10 @@ std::array<Tensor, 4> attention_backward(const Call& call, const Tensor& grad_ou
     Tensor classes;  // (kept alive until the call is enqueued, as `prepared`)
     if (summed) {
         summed = lib.uses_matrix_cores(&a, 3) == 1;
-        a.dmask = nullptr;
-        if (summed) prepared = prepared_mask(call, q, switches.pads_from);
+        if (summed) {  // (else the dQ pass writes it: in place, or below, into what broadcast dimensions are added up in)
+            a.dmask = nullptr;
+            prepared = prepared_mask(call, q, switches.pads_from);
+        }
     }
     if (prepared) {
         prepared->describe(a);

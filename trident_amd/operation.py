@@ -403,8 +403,8 @@ class Attention(torch.autograd.Function):
         classes = None  # (kept alive until the call is enqueued, as ``prepared``)
         if summed:
             summed = lib.tri_attn_uses_matrix_cores(ctypes.byref(args), 3) == 1
-            args.dmask = None
-            if summed:
+            if summed:  # (else the dQ pass writes it: in place, or below, into what broadcast dimensions are added up in)
+                args.dmask = None
                 prepared = _prepared_mask(mask, query)
         if prepared is not None:
             prepared.describe(args)
