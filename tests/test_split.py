@@ -169,3 +169,21 @@ def test_infinities_in_keys_without_weight_reach_the_output(device, monkeypatch)
         (o, *_), used = _run(q, k, v, q, None, 0.0, False, 1.0, (0, 0), split, monkeypatch)
         assert used[0] == split
         assert o[0, 0, :, 5].isnan().all() and torch.equal(o[0, 0, :, :5], v[0, 0, :, :5]) and torch.equal(o[0, 1], v[0, 1])
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype,S,D", [(torch.float32, 640, 64), (torch.float32, 513, 128), (torch.bfloat16, 2048, 128), (torch.float16, 1300, 64)])
+def test_keys_of_nan_over_whole_parts_reach_the_output(dtype, S, D, causal, device, monkeypatch):
+    """NaN wherever the whole launch gives NaN, whichever part the first or the last key of NaN begins or ends (parts begin at multiples
+    of 64): a part with nothing but NaN scores has no maximum, and a sum that is NaN."""
+    g = torch.Generator(device=device).manual_seed(S)
+    q, k, v, d_o = [torch.randn(1, 2, S, D, generator=g, device=device).to(dtype) for _ in range(4)]
+    for first, last in [(n, S) for n in range(64, S, 64)] + [(0, n) for n in range(64, S, 64)]:
+        kk = k.clone()
+        kk[:, 0, first:last] = math.nan
+        whole, _ = _run(q, kk, v, d_o, None, 0.0, causal, 0.125, (0, 0), False, monkeypatch)
+        split, used = _run(q, kk, v, d_o, None, 0.0, causal, 0.125, (0, 0), True, monkeypatch)
+        assert all(used)
+        assert split[0][0, 0, first if causal else 0:].isnan().all(), ("O", first, last)
+        for name, a, b in zip(("O", "lse", "dQ", "dK", "dV"), split, whole):
+            assert torch.equal(a.isnan(), b.isnan()), (name, first, last)

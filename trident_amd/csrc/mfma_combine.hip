@@ -72,6 +72,7 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
         m = fmaxf(m, x);
     }
     if (nan) m = __builtin_nanf("");
+    const float ref = m == -INFINITY ? 0.f : m;  // (no score of any part has had a value: the sums are 0, or NaN where scores were)
     f32x16 acc[1] = {zero16()};
     float l = 0.f;
     const f32x4* src = reinterpret_cast<const f32x4*>(p.partial + (unit0 * rows + at.block * 32) * D) + at.column * 256 + lane;
@@ -79,9 +80,10 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
 #pragma unroll 4
     for (int i = 0; i < count; ++i) {
         const float2 ml = stats[static_cast<int64_t>(i) * rows];
-        const float w = fast_exp2(ml.x - m);  // (a row without a visible key: -inf - -inf, NaN as in the kernel)
-        // (a part without a visible key has left nothing there; one whose keys weigh nothing still hands on a NaN or an infinity in V)
-        const bool none = w == 0.f && ml.x == -INFINITY;
+        // (a part without a tile has left nothing but that; every other one takes part, also with weight 0: what its keys' scores
+        // and values have made NaN stays NaN)
+        const bool none = ml.y < 0.f;
+        const float w = fast_exp2(ml.x - ref);
         l += none ? 0.f : w * ml.y;
 #pragma unroll
         for (int g = 0; g < G; ++g) {
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(256) void combine_forward_kernel(const KParams p, i
     const int b = at.bh / p.H, hd = at.bh % p.H, rows_here = p.S - at.row0;
     char* o0 = static_cast<char*>(p.o) + (b * p.os[0] + hd * p.os[1] + at.row0 * p.os[2] + 32 * at.column) * sizeof(T);
     Store::run(acc, [inv](float x) { return x * inv; }, smem + (threadIdx.x >> 6) * Store::kPatchBytes, o0, p.os[2] * sizeof(T), lane, rows_here);
-    if (at.column == 0 && h == 0 && l32 < rows_here) p.lse[static_cast<int64_t>(at.bh) * p.S + at.row0 + l32] = m == -INFINITY ? m : m + fast_log2(l);
+    if (at.column == 0 && h == 0 && l32 < rows_here) p.lse[static_cast<int64_t>(at.bh) * p.S + at.row0 + l32] = m + fast_log2(l);
 }
 
 // OUTPUTS = 2: dK (blockIdx.y = 0) and dV (1); the accumulators of a unit's rows for the first come before those for the second.

@@ -416,8 +416,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     using No = std::integral_constant<bool, false>;
 
     if constexpr (SPLIT) {
-        if (n_tiles == 0) {  // nothing to see for anybody: no score was as much as -inf
-            if (lane < 32) reinterpret_cast<float2*>(p.partial + static_cast<int64_t>(p.B) * p.H * p.part_units * kBM * D)[static_cast<int64_t>(part.unit) * kBM + 32 * wave + lane] = make_float2(-INFINITY, 0.f);
+        if (n_tiles == 0) {  // nothing to see for anybody: no accumulators (a sum below 0 says so)
+            if (lane < 32) reinterpret_cast<float2*>(p.partial + static_cast<int64_t>(p.B) * p.H * p.part_units * kBM * D)[static_cast<int64_t>(part.unit) * kBM + 32 * wave + lane] = make_float2(-INFINITY, -1.f);
             return;
         }
     }
