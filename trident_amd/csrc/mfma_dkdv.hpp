@@ -132,29 +132,25 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
     uint64_t zero_tiles = 0;
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles - t_first <= 64) {
-            const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + k0 / 64 + t_first * p.mcs[2], p.mcs[2], n_tiles - t_first,
-                                                RAGGED ? min(kKeys / 64, (p.S + kBN - 1) / kBN - k0 / 64) : kKeys / 64, 1, lane);
+            const uint8_t* const classes = p.mcls + b * p.mcs[0] + hd * p.mcs[1] + k0 / 64;
+            const int all_tiles = (p.S + kBN - 1) / kBN, across = RAGGED ? min(kKeys / 64, all_tiles - k0 / 64) : kKeys / 64;
+            const TileClasses tc = tile_classes(classes + t_first * p.mcs[2], p.mcs[2], n_tiles - t_first, across, 1, lane);
             zero_tiles = tc.zero;
-            if (tc.active) {
-                n_tiles = t_first + 64 - __builtin_clzll(tc.active);
-                t_begin = t_first + __builtin_ctzll(tc.active);
+            if constexpr (SPLIT) {
+                const int2 on = active_range(classes, p.mcs[2], all_tiles, across, 1, lane);
+                t_begin = max(t_first, min(on.x, n_tiles));
+                n_tiles = max(t_begin, min(on.y, n_tiles));
+            } else if (tc.active) {
+                n_tiles = 64 - __builtin_clzll(tc.active);
+                t_begin = __builtin_ctzll(tc.active);
             } else {
-                n_tiles = t_begin = t_first;
+                n_tiles = t_begin = 0;
             }
-            if constexpr (RAGGED) {
+            // (whole items at multiples of 128 with classes leave them out unlooked; those of the paired kernel, D = 128, leave out none)
+            if (RAGGED && !(SPLIT && D < 128 && p.S % 128 == 0 && all_tiles <= 64)) {
                 bool lost = false;
-                int from = 0, to = p.S;
-                if constexpr (SPLIT && D < 128) {
-                    // (whole items at multiples of 128 leave out the row tiles before the first and behind the last active one
-                    // unlooked; those of the paired kernel, D = 128, leave out none)
-                    if (p.S % 128 == 0 && p.S <= 64 * kBN) {
-                        const uint64_t on = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + k0 / 64, p.mcs[2], p.S / kBN, min(kKeys / 64, p.S / kBN - k0 / 64), 1, lane).active;
-                        from = on ? __builtin_ctzll(on) * kBN : 0;
-                        to = on ? (64 - __builtin_clzll(on)) * kBN : 0;
-                    }
-                }
-                for (int r = max(t_first * kBN, from) + lane; r < min(t_begin * kBN, to); r += 64) lost |= !(lse_base[r] > -INFINITY);
-                for (int r = max(n_tiles * kBN, from) + lane; r < min(rows_end, to); r += 64) lost |= !(lse_base[r] > -INFINITY);
+                for (int r = t_first * kBN + lane; r < t_begin * kBN; r += 64) lost |= !(lse_base[r] > -INFINITY);
+                for (int r = n_tiles * kBN + lane; r < rows_end; r += 64) lost |= !(lse_base[r] > -INFINITY);
                 if (__builtin_amdgcn_ballot_w64(lost) != 0) left_out = __builtin_nanf("");
             }
         }

@@ -134,13 +134,15 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     uint64_t zero_tiles = 0;
     if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
-            const TileClasses tc = tile_classes(p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (q0 / 64) * p.mcs[2] + key0 / kBN, 1, n_tiles,
-                                                RAGGED ? min(kRows / 64, num_key_tiles - q0 / 64) : kRows / 64, p.mcs[2], lane);
+            const uint8_t* const classes = p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (q0 / 64) * p.mcs[2] + key0 / kBN;
+            const int across = RAGGED ? min(kRows / 64, num_key_tiles - q0 / 64) : kRows / 64;
+            const TileClasses tc = tile_classes(classes, 1, n_tiles, across, p.mcs[2], lane);
             zero_tiles = tc.zero;
             // (a mask gradient written in place covers every tile: the tiles behind the last active one get their
             // zeros from the loop; an accumulated one adds into a buffer the caller has zero-filled)
             if (!DMASK || p.dmask_acc) {
-                n_tiles = tc.active ? 64 - __builtin_clzll(tc.active) : SPLIT && part.index > 0 ? 0 : 1;
+                if (!(SPLIT && any_active(classes + n_tiles, 1, num_key_tiles - key0 / kBN - n_tiles, across, p.mcs[2], lane)))
+                    n_tiles = tc.active ? 64 - __builtin_clzll(tc.active) : SPLIT && part.index > 0 ? 0 : 1;
                 my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
             }
         }

@@ -61,6 +61,25 @@ __device__ __forceinline__ bool map_part(const KParams& p, int bid, int grid, in
     return true;
 }
 
+// Whole items leave out only tiles before the first and behind the last one that is not masked out altogether: in between, probability 0
+// times a NaN or an infinity of a hidden key or row reaches the result. So it does from parts, which ask for all of the item's `n` tiles
+// (as tile_classes, any n): whether one of them is active, and the first and the end of those that are.
+__device__ __forceinline__ bool any_active(const uint8_t* first, int64_t tile_step, int n, int across, int64_t step, int lane) {
+    for (int t = 0; t < n; t += 64)
+        if (tile_classes(first + t * tile_step, tile_step, min(64, n - t), across, step, lane).active != 0) return true;
+    return false;
+}
+__device__ __forceinline__ int2 active_range(const uint8_t* first, int64_t tile_step, int n, int across, int64_t step, int lane) {
+    int2 range = make_int2(0, 0);
+    for (int t = 0; t < n; t += 64) {
+        const uint64_t active = tile_classes(first + t * tile_step, tile_step, min(64, n - t), across, step, lane).active;
+        if (active == 0) continue;
+        if (range.y == 0) range.x = t + __builtin_ctzll(active);
+        range.y = t + 64 - __builtin_clzll(active);
+    }
+    return range;
+}
+
 // Accumulators of a wave's NB blocks of 32 rows (this lane: row l32) x 32 columns as they are, whole lines per store. `base`: of
 // the wave's 32 rows (all columns) in the workspace; first: the wave's first column block. D = 16 has half a block.
 template <int NB, int D>
