@@ -142,3 +142,38 @@ def test_saved_tensors_that_come_back_changed_are_refused(unpack, device):
     for out in outputs:
         with pytest.raises(RuntimeError, match="trident_amd: .*(on the same GPU|another shape or dtype)"):
             out.sum().backward()
+
+
+def _wider(t):
+    """The same values in rows of a wider buffer."""
+    return torch.zeros(t.shape[:-1] + (t.shape[-1] + 8,), dtype=t.dtype, device=t.device)[..., : t.shape[-1]].copy_(t)
+
+
+def _turned(t):
+    """The same values with the first and the last dimension exchanged in memory."""
+    return t.transpose(0, -1).contiguous().transpose(0, -1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("path", ["C++", "Python"])
+@pytest.mark.parametrize("unpack", [_wider, _turned, lambda t: t.clone()])
+@pytest.mark.parametrize("operation_of", ["rows", "columns", "3-d", "attention"])
+def test_saved_tensors_that_come_back_in_another_layout(operation_of, unpack, path, device):
+    """Equal values, other strides: the gradients of a call without the hook, bit for bit."""
+    g = torch.Generator(device=device).manual_seed(3)
+    shape, dim = {"rows": ((40, 60), 1), "columns": ((40, 60), 0), "3-d": ((3, 5, 60), -1), "attention": ((2, 3, 64, 32), None)}[operation_of]
+    x = torch.randn(shape, generator=g, device=device).half().requires_grad_()
+    grad = torch.randn(shape, generator=g, device=device).half()
+
+    def call():
+        if dim is None:
+            return operation.Attention.apply(x, x, x, None, 0.0, False, 0.25, False) if path == "Python" else trident.function.attention(x, x, x, softmax_scale=0.25)
+        return operation.Softmax.apply(x, dim) if path == "Python" else trident.function.softmax(x, dim)
+
+    want = torch.autograd.grad(call(), x, grad)[0]
+    if dim is None and unpack is _turned:
+        # (lse only: rows of q, k, v and o of another stride are copied or refused)
+        unpack = lambda t: _turned(t) if t.dim() == 3 else t
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        out = call()
+    assert torch.equal(torch.autograd.grad(out, x, grad)[0], want)

@@ -643,9 +643,10 @@ struct SoftmaxBackward : torch::autograd::Function<SoftmaxBackward> {
         return output;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
-        const Tensor output = ctx->get_saved_variables()[0];
-        require_saved_as(output, "output", grads[0], grads[0].sizes(), grads[0].scalar_type());
-        const c10::DeviceGuard device(output.device());
+        const Tensor saved = ctx->get_saved_variables()[0];
+        require_saved_as(saved, "output", grads[0], grads[0].sizes(), grads[0].scalar_type());
+        const c10::DeviceGuard device(saved.device());
+        const Tensor output = dense_matrix(saved);  // (a hook may have laid it out anew)
         const Tensor grad_output = same_layout(grads[0], output);
         const Tensor grad_input = at::empty_like(output);
         TriRowArgs a = row_args(output, ctx->saved_data["columns"].toBool());

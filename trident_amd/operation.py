@@ -377,6 +377,7 @@ class Attention(torch.autograd.Function):
         lib = _lib.lib()
         query, key, value = _dense_rows(query), _dense_rows(key), _dense_rows(value)
         grad_output = _dense_rows(grad_output)
+        log2sum = log2sum.contiguous()  # (a saved-tensor hook may have laid it out anew)
         num_batches, num_heads, y_size, x_size = output.shape
         grad_query = torch.empty(query.shape, device=query.device, dtype=query.dtype)
         grad_key = torch.empty(key.shape, device=key.device, dtype=key.dtype)

@@ -106,6 +106,7 @@ def _softmax_forward(input, mask, dim, trace):
 
 def _softmax_backward(grad_output, output, dim, trace):
     _require_gpu(output, grad_output=grad_output)
+    output = _dense(output)  # (a saved-tensor hook may have laid it out anew)
     grad_output = _same_layout(grad_output, output)
     grad_input = torch.empty_like(output)
     args = _row_args(output, dim)
