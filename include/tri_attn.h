@@ -126,7 +126,8 @@ typedef struct TriAttnArgs {
                                   read by tri_attn_fwd / tri_attn_bwd*: dense [MB][MH][RB][S/64] bytes with MB = B (1 if
                                   mask_stride[0] == 0), MH = H (1 if mask_stride[1] == 0), RB = S/64 (1 if mask_stride[2] == 0);
                                   0 = every entry of the block is 0, 1 = every entry is -inf, 2 = anything else.
-                                  Only used where S is a multiple of 64, or with TRI_ATTN_MASK_PADDED (S/64 rounded up). */
+                                  Only used where S is a multiple of 64, or with TRI_ATTN_MASK_PADDED (S/64 rounded up), and not by
+                                  fp32 problems. */
 
     void* workspace;           /* NULL, or scratch memory for this call (16-byte aligned, used until the stream has passed it): with at
                                   least tri_attn_workspace_size bytes of it, calls of few heads run split along the sequence */
@@ -209,8 +210,8 @@ int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass);
  * to within an ulp of the 16-bit outputs, not bit for bit. Reads mask; writes mask_classes.
  * Returns TRI_ATTN_ENOFUSE (nothing launched) where the classes would not be used: S not a multiple of 64. */
 int tri_attn_classify_mask(const TriAttnArgs* args);
-/* Bytes of mask_classes for these arguments (MB * MH * RB * S/64), 0 where tri_attn_classify_mask does not apply, or a
- * negative TRI_ATTN_E* code. */
+/* Bytes of mask_classes for these arguments (MB * MH * RB * S/64; whatever the dtype), 0 where tri_attn_classify_mask does not
+ * apply, or a negative TRI_ATTN_E* code. */
 int64_t tri_attn_mask_classes_size(const TriAttnArgs* args);
 
 /* Writes an additive padded mask for the kernels: args->mask is the destination (mask_dtype with TRI_ATTN_MASK_PADDED,

@@ -44,6 +44,17 @@ def test_multiples_of_64(dtype, B, H, S, D, kind, device):
     parity.close(dv, dv_r, dtype, f"{kind} dV", a_dv)
 
 
+@pytest.mark.parametrize("S", [128, 192])
+def test_masks_of_fp32_calls_are_not_classified(S, device, monkeypatch):
+    """No fp32 kernel looks at classes: a pass over the mask, and memory, for nothing. (The first call with a mask: nothing is cached.)"""
+    q = torch.randn(1, 2, S, 64, device=device)
+    mask = torch.randn(1, 1, S, S, device=device)
+    for dtype, wanted in ((torch.float32, False), (torch.float16, True)):
+        x = q.to(dtype)
+        args = operation._make_args(x, x, x, x, torch.empty(1, 2, S, device=device), operation._expand_mask(mask, (1, 2, S, S)), 0.0, False, 0.125, 0, 0)
+        assert (operation._mask_classes(mask, args) is not None) == wanted and bool(args.mask_classes) == wanted
+
+
 @pytest.mark.parametrize("S,D", [(1, 64), (63, 32), (64, 64), (130, 128), (192, 16), (260, 64)])
 @pytest.mark.parametrize("shape", ["BHSS", "1HSS", "SS"])
 @pytest.mark.parametrize("small", [False, True])

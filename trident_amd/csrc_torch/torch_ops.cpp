@@ -239,6 +239,7 @@ std::vector<int64_t> classes_signature(const Tensor& mask, const TriAttnArgs& a)
 }
 
 Tensor mask_classes(const Tensor& mask, TriAttnArgs& a, bool may_cache) {
+    if (a.dtype == TRI_ATTN_F32) return Tensor();  // (no fp32 kernel looks at them)
     const int64_t size = lib.mask_classes_size(&a);
     if (size <= 0) return Tensor();
     const bool use_cache = may_cache && !stream_is_capturing() && !mask.is_inference();

@@ -112,8 +112,8 @@ def forget_mask_classes():
 
 def _mask_classes(mask: torch.Tensor, args):
     """Sets args.mask_classes for the mask already described in ``args``; returns the tensor to keep alive, or None
-    where the library has no use for classes (nothing is launched then; padded masks bring theirs along, and the kernels use
-    no others at lengths that are no multiple of 64)."""
+    where the library has no use for classes (nothing is launched then; padded masks bring theirs along, the kernels use no others at
+    lengths that are no multiple of 64, and those of fp32 calls use none)."""
     return _lib.torch_ops().mask_classes(mask, ctypes.addressof(args), bool(config.cache_mask_classes))
 
 
