@@ -215,3 +215,24 @@ def test_what_a_mask_hides_over_whole_parts_is_not_left_out(what, hidden, S, D, 
         # (beyond 64 tiles, and in dK/dV at D = 128, whole items leave out nothing, parts what whole ones leave out elsewhere)
         ends = name in ("dK", "dV") and (S > 4096 or S % 128 == 0 and D == 128) or S > 4096 and (hidden[0] == 0 or hidden[1] is None)
         assert not (a.isnan() & ~b.isnan()).any() if ends else torch.equal(a.isnan(), b.isnan()), name
+
+
+@pytest.mark.parametrize("dtype,heads,S,D,causal,which,split", [
+    # whole launch -> split one as it was planned before (us): the plan took a CU for one that holds more workgroups than it does, and a
+    # tile for as long beside three other workgroups as alone
+    (torch.bfloat16, 25, 1280, 32, False, 0, False),   # forward 16.1 -> 23.7
+    (torch.bfloat16, 20, 1237, 32, False, 0, False),   # forward 17.1 -> 23.7
+    (torch.float16, 22, 1408, 32, True, 0, False),     # forward 17.6 -> 22.2
+    (torch.float16, 21, 4096, 16, True, 1, False),     # dK/dV 70.3 -> 112.3
+    (torch.bfloat16, 18, 4224, 32, True, 1, False),    # dK/dV 79.6 -> 115.7
+    (torch.float16, 12, 4992, 32, False, 1, False),    # dK/dV 102.3 -> 133.1
+    # launches that take half as long split
+    (torch.float32, 5, 193, 128, False, 1, True),      # dK/dV 43.3 -> 21.3
+    (torch.float32, 9, 768, 128, True, 0, True),       # forward 116.5 -> 38.8
+    (torch.bfloat16, 6, 1984, 64, True, 1, True),      # dK/dV 57.9 -> 28.9
+    (torch.bfloat16, 6, 3392, 32, True, 1, True)])     # dK/dV 79.4 -> 36.7
+def test_launches_that_split(dtype, heads, S, D, causal, which, split, device):
+    q = torch.empty(1, heads, S, D, dtype=dtype, device=device)
+    lse = torch.empty(1, heads, S, device=device)
+    args = operation._make_args(q, q, q, q, lse, None, 0.0, causal, 0.125, 0, 0, q, q, q, q, None, lse)
+    assert (_lib.lib().tri_attn_workspace_size(ctypes.byref(args), which) > 0) == split

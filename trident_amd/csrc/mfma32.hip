@@ -874,10 +874,9 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
 // fp32 launches of few heads, split along the streamed rows (split.hpp). A tile of 64 rows takes a workgroup its products at about
 // 70 % of the fp32 matrix rate of a CU, so that parts pay from a few tiles on; a second workgroup on a CU adds little.
 SplitShape split_shape32(int which, const KParams& p) {
-    const double fwd_us = p.D == 128 ? 9.5 : p.D == 64 ? 4.9 : p.D == 32 ? 2.6 : 2.0;
-    if (which == kMfmaFwd) return SplitShape{kRowsPerGroup, 1, 1, true, 4, fwd_us, 0.85};
-    if (which == kMfmaDq) return SplitShape{kRowsPerGroup, 1, 1, false, 4, 1.5 * fwd_us, 0.85};
-    return SplitShape{p.D == 128 ? 64 : kRowsPerGroup, 1, 2, false, 4, p.D == 128 ? 10.0 : 2 * fwd_us, 0.85};
+    const double fwd_us = (p.mask != nullptr ? 1.6 : 1.0) * (p.D == 128 ? 8.9 : p.D == 64 ? 5.4 : p.D == 32 ? 3.3 : 3.0);
+    const double us = fwd_us * (which == kMfmaFwd ? 1.0 : which == kMfmaDq ? 1.25 : p.D == 128 ? 0.95 : 1.6);
+    return SplitShape{which == kMfmaDkdv && p.D == 128 ? 64 : kRowsPerGroup, 1, which == kMfmaDkdv ? 2 : 1, which == kMfmaFwd, 4, us, us, 0.95};
 }
 // (a mask gradient is written by whole items only)
 bool splits32(int which, int dtype, const KParams& p) { return dtype == TRI_ATTN_F32 && !(which == kMfmaDq && p.dmask != nullptr); }

@@ -175,15 +175,19 @@ int64_t plan_split(const SplitShape& shape, bool causal, KParams* p) {
     p->part_units = 0;
     const int64_t heads = static_cast<int64_t>(p->B) * p->H;
     const int tiles = (p->S + 63) / 64, items = (p->S + shape.rows - 1) / shape.rows, step = shape.rows / 64;
-    const int64_t slots = static_cast<int64_t>(persistent_grid(1 << 20)) * shape.slots_per_cu;
-    // Microseconds, as measured at 21 to 94 tiles: a workgroup's start and end, the second launch, bytes of the workspace (mostly
-    // in the caches) that both launches move in one.
-    const double tile_us = shape.tile_us;
-    constexpr double kFixed = 6, kCombine = 5, kBytesPerUs = 8e6;
+    const int64_t cus = static_cast<int64_t>(persistent_grid(1 << 20)), slots = cus * shape.slots_per_cu;
+    // Microseconds, as measured over 2700 passes of 1 to 40 heads and 193 to 8000 rows: a workgroup's start and end, the second launch,
+    // bytes of the workspace (mostly in the caches) that both launches move in one. A CU with several workgroups takes longer for a
+    // tile of each than one workgroup alone on it, but less than for that many one after the other.
+    constexpr double kFixed = 4, kCombine = 7, kBytesPerUs = 5e6;
+    const auto time = [&](int64_t units, int each) {
+        const int64_t on_cu = (units + cus - 1) / cus, rounds = (on_cu + shape.slots_per_cu - 1) / shape.slots_per_cu;
+        return static_cast<double>(rounds) * kFixed + each * std::max(static_cast<double>(rounds) * shape.tile_us, static_cast<double>(on_cu) * shape.cu_us);
+    };
     // A launch with a workgroup for every CU is worth it only where the workgroups are long.
-    if (tiles < shape.min_tiles || heads * items >= 2 * slots || (tiles < 64 && heads * items >= slots / shape.slots_per_cu)) return 0;
-    const double whole = causal ? std::max(tiles * tile_us + kFixed, static_cast<double>(heads) * items * ((tiles + step) / 2.0 * tile_us + kFixed) / slots)
-                                : static_cast<double>((heads * items + slots - 1) / slots) * (tiles * tile_us + kFixed);
+    if (tiles < shape.min_tiles || heads * items >= 2 * slots || (tiles < 64 && heads * items >= cus)) return 0;
+    const double whole = causal ? kFixed + std::max(tiles * shape.tile_us, static_cast<double>(heads) * items * (tiles + step) / 2.0 * shape.cu_us / cus)
+                                : time(heads * items, tiles);
     const int64_t unit_bytes = shape.rows * (static_cast<int64_t>(p->D) * shape.outputs + (shape.statistics ? 2 : 0)) * 4;
     double best = shape.gain * whole;
     for (int c = std::max(shape.min_tiles / 5, step); c < tiles; c += causal ? step : 1) {  // (parts of at least a fifth of min_tiles)
@@ -194,8 +198,7 @@ int64_t plan_split(const SplitShape& shape, bool causal, KParams* p) {
         } else {
             units = static_cast<int64_t>(items) * ((tiles + c - 1) / c);
         }
-        const double rounds = static_cast<double>((heads * units + slots - 1) / slots);
-        const double t = rounds * (c * tile_us + kFixed) + kCombine + 2.0 * heads * units * unit_bytes / kBytesPerUs;
+        const double t = time(heads * units, c) + kCombine + 2.0 * heads * units * unit_bytes / kBytesPerUs;
         if (t < best) {
             best = t;
             p->part_units = static_cast<int>(units);

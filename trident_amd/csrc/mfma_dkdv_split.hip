@@ -9,10 +9,14 @@ bool dkdv_splits_phased(const KParams& p) {
     return p.D == 128 && (p.mask == nullptr || (p.ms[2] == 0 && (p.mask_binary || p.S % 128 == 0)));
 }
 SplitShape dkdv_split_shape(const KParams& p) {
-    if (dkdv_splits_phased(p)) return SplitShape{128, 1, 2, false, 20, 1.5, split_gain(p)};
-    const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
+    if (dkdv_splits_phased(p)) {
+        const double us = split_work(p) * 1.35;
+        return SplitShape{128, 1, 2, false, 20, us, us, split_gain(p)};
+    }
     const int waves = p.mask != nullptr && p.D == 64 && p.thr8 <= 0 ? 8 : 4;
-    return SplitShape{32 * waves, p.D == 128 || waves == 8 || (p.D == 64 && f32_mask) ? 1 : p.D == 64 || f32_mask ? 2 : 4, 2, false, 20, 1.8, split_gain(p)};
+    const int slots = p.D == 128 || (p.D == 64 && p.mask != nullptr) ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 3;
+    const double us = split_work(p) * (p.D >= 64 ? 1.65 : p.D == 32 ? 1.22 : 1.05);
+    return SplitShape{32 * waves, slots, 2, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.58 : 0.52) * us, split_gain(p) - (p.D < 64 ? 0.04 : 0.0)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>

@@ -9,7 +9,9 @@ namespace {
 SplitShape dq_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = (p.D == 128 && p.mask == nullptr && p.thr8 <= 0) || (p.D == 64 && f32_mask) ? 8 : 4;
-    return SplitShape{32 * waves, p.D == 128 || waves == 8 ? 1 : p.D == 64 || f32_mask ? 2 : 4, 1, false, 20, p.D == 128 ? 1.6 : 1.0, split_gain(p)};
+    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 4;
+    const double us = split_work(p) * (p.D == 128 ? 1.55 : p.D == 64 ? 0.96 : p.D == 32 ? 0.68 : 0.53);
+    return SplitShape{32 * waves, slots, 1, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.65 : 0.59) * us, split_gain(p)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>
@@ -45,7 +47,11 @@ int launch_dq_split_variant(int dtype, const KParams& p, hipStream_t stream, boo
 }
 
 // (a mask gradient is written by whole items only; without a mask the parts bring delta along, with one they may up to D = 64)
+// Beside dropout at D = 128 a workgroup's start, with one wave per SIMD, costs more than the last round of a launch that fills the GPU
+// saves (bf16 S=4352, 11 heads: 209 -> 286 us).
 bool dq_splits(const KParams& p, bool with_delta) {
+    const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
+    if (p.D == 128 && p.thr8 > 0 && !p.causal && items >= persistent_grid(1 << 20)) return false;
     return p.dmask == nullptr && (p.mask == nullptr ? with_delta : !with_delta || p.D <= 64);
 }
 

@@ -32,7 +32,9 @@ int launch_fwd_split_variant(int dtype, const KParams& p, int waves, hipStream_t
 SplitShape fwd_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = p.D == 128 ? (p.mask != nullptr && p.thr8 > 0 ? 4 : 8) : p.D == 64 && f32_mask ? 8 : 4;
-    return SplitShape{32 * waves, p.D == 128 || waves == 8 ? 1 : p.D == 64 || f32_mask ? 2 : 4, 1, true, 20, p.D == 128 ? 1.4 : 0.9, split_gain(p)};
+    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 ? 2 : p.mask == nullptr ? 4 : p.thr8 > 0 || (f32_mask && p.D == 32) ? 2 : 3;
+    const double us = split_work(p) * (p.D == 128 ? 1.4 : p.D == 64 ? 0.9 : 0.62);
+    return SplitShape{32 * waves, slots, 1, true, 20, us, slots == 1 ? us : 0.6 * us, split_gain(p)};
 }
 
 template <typename T>

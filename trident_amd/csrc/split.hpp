@@ -96,16 +96,20 @@ __device__ __forceinline__ void store_partial(const f32x16 (&acc)[NB], float* ba
 // ceil(S / 64) tiles (`causal`: as many as the diagonal leaves).
 struct SplitShape {
     int rows;          // stationary rows of a workgroup
-    int slots_per_cu;  // workgroups a CU holds
+    int slots_per_cu;  // workgroups a CU holds (registers and LDS)
     int outputs;       // accumulators of D columns per row
     bool statistics;   // two more floats per row
     int min_tiles;     // below so many there is less to win than the second launch costs
-    double tile_us;    // a workgroup's time for one tile
+    double tile_us;    // a workgroup's time for one tile, alone on its CU
+    double cu_us;      // a full CU's time for one tile of one workgroup
     double gain;       // split where the plan's time is below this share of the whole launch's
 };
-// Masked lengths that are multiples of 128 have faster kernels (a mask value joins its score before the scale, row sums on the
-// matrix pipe) than the parts, which have boundary handling.
-inline double split_gain(const KParams& p) { return p.mask != nullptr && p.S % 128 == 0 ? 0.65 : 0.9; }
+// What masks and dropout add to a tile's time (a mask of keys is read once, or not at all where it is zero).
+inline double split_work(const KParams& p) { return (p.mask == nullptr ? 1.0 : p.ms[2] == 0 ? 1.3 : 1.6) * (p.thr8 > 0 ? 1.7 : 1.0); }
+// Lengths that are multiples of 128 have faster kernels than the parts, which have boundary handling, most of all beside a mask (a value
+// joins its score before the scale, row sums on the matrix pipe). Causal plans turn out faster than they promise: what they cut
+// are the long items.
+inline double split_gain(const KParams& p) { return (p.S % 128 != 0 ? 0.98 : p.mask != nullptr ? 0.84 : 0.93) + (p.causal ? 0.08 : 0.0); }
 // Fills p->part_* and returns the bytes of workspace the split launch needs; 0: the launch stays whole.
 int64_t plan_split(const SplitShape& shape, bool causal, KParams* p);
 // Whether the caller's workspace holds what plan_split asked for; sets p->partial.
