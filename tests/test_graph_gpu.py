@@ -8,6 +8,7 @@ import math
 import pytest
 import torch
 
+import trident_amd as trident
 from trident_amd import _lib, operation
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,65 @@ def test_forward_and_backward_replay_from_a_graph(dtype, shape, causal, p, devic
         for name, a, b in zip(("O", "LSE", "dQ", "dK", "dV"), held[4:], eager[4:]):
             assert not torch.isnan(a.float()).any(), f"{name}, replay {replay}"
             assert torch.equal(a, b), f"{name} differs in replay {replay}"
+
+
+def _replays(step, inputs, names, seed):
+    """``step()`` recorded once and replayed on new values of ``inputs``: every replay against the eager call, bit for bit."""
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # (first use outside the capture)
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = step()
+    for replay in range(3):
+        for n, t in enumerate(inputs):
+            g = torch.Generator().manual_seed(1000 * seed + 10 * replay + n)
+            with torch.no_grad():
+                t.copy_(torch.randn(t.shape, generator=g).to(t.dtype))
+        for t in held:
+            t.fill_(float("nan"))
+        eager = [t.clone() for t in step()]
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, a, b in zip(names, held, eager):
+            assert not torch.isnan(a.float()).any(), f"{name}, replay {replay}"
+            assert torch.equal(a, b), f"{name} differs in replay {replay}"
+
+
+@pytest.mark.parametrize("dtype,B,H,S,D,kind,causal", [
+    (torch.bfloat16, 2, 4, 512, 128, "none", True),
+    (torch.bfloat16, 1, 2, 2048, 128, "none", True),    # split: the workspace and the second launch are part of the graph
+    (torch.float16, 1, 3, 1300, 64, "padding", False),  # split, boolean mask made additive inside the graph
+    (torch.float32, 1, 3, 513, 64, "none", False),      # split, fp32
+    (torch.bfloat16, 8, 2, 320, 64, "bias", False)])    # gradient of a learned mask, its pairs dealt to several workgroups
+def test_operator_replays_from_a_graph(dtype, B, H, S, D, kind, causal, device, monkeypatch):
+    """The operator with its allocations, forward and backward through autograd, as a training step records it."""
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    q, k, v, grad = [t.requires_grad_(n < 3) for n, t in enumerate(_fresh((B, H, S, D), dtype, device, 1))]
+    inputs, mask = [q, k, v], None
+    if kind == "padding":
+        mask = (torch.arange(S, device=device) < S - 70).expand(B, 1, 1, S).contiguous()
+    elif kind == "bias":
+        mask = torch.zeros(1, H, S, S, dtype=dtype, device=device, requires_grad=True)
+        inputs.append(mask)
+
+    def step():
+        out = trident.function.scaled_dot_product_attention(q, k, v, mask, 0.0, causal)
+        return [out.detach(), *torch.autograd.grad(out, inputs, grad)]
+
+    _replays(step, inputs + [grad], ("O", "dQ", "dK", "dV", "dMask"), S)
+
+
+@pytest.mark.parametrize("rows,cols", [(9000, 132), (300, 77)])  # (columns split along their length, and whole)
+def test_column_softmax_replays_from_a_graph(rows, cols, device):
+    x = torch.randn(rows, cols, device=device).requires_grad_()
+    grad = torch.randn(rows, cols, device=device)
+
+    def step():
+        out = trident.function.softmax(x, 0)
+        return [out.detach(), *torch.autograd.grad(out, [x], grad)]
+
+    _replays(step, [x, grad], ("output", "gradient"), rows)

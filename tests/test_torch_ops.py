@@ -98,6 +98,44 @@ def test_attention_is_the_function_it_stands_in_for(kind, dtype, S, D, p, layout
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,B,H,S,D,kind,causal,p", [
+    (torch.bfloat16, 1, 2, 2048, 128, "none", True, 0.0), (torch.float16, 1, 3, 1300, 64, "bool", False, 0.0),
+    (torch.bfloat16, 2, 1, 1408, 32, "length", False, 0.2), (torch.bfloat16, 1, 2, 1300, 64, "shared grad", False, 0.0),
+    (torch.float32, 1, 3, 513, 64, "none", True, 0.0), (torch.float32, 2, 1, 640, 128, "matrix", False, 0.2)])
+def test_split_attention_is_the_function_it_stands_in_for(dtype, B, H, S, D, kind, causal, p, device, monkeypatch):
+    """Both host paths give a call of few heads the workspace with which it runs split, in both directions: the same bits, and other
+    ones than without a workspace (parts add their sums up in another order)."""
+    monkeypatch.setattr(trident.config, "reference_limits", False)
+    g = torch.Generator(device=device).manual_seed(S + D)
+    q, k, v, grad = [torch.randn(B, H, S, D, generator=g, device=device).to(dtype) for _ in range(4)]
+    q, k, v = [t.requires_grad_() for t in (q, k, v)]
+    mask = _mask(kind, B, H, S, dtype, device)
+    inputs = [q, k, v] + ([mask] if "grad" in kind else [])
+    take, used = operation._take_workspace, []
+
+    def spy(args, which, gpu):
+        workspace = take(args, which, gpu)
+        used.append(workspace is not None)
+        return workspace
+
+    def run(f):
+        monkeypatch.setattr(trident.config, "dropout_seed", (5, 1))
+        out = f(q, k, v, mask, p, causal, 0.125, False)
+        return [out.detach(), *torch.autograd.grad(out, inputs, grad)]
+
+    got = run(operation.Attention.call)
+    monkeypatch.setattr(operation, "_take_workspace", spy)
+    want = run(operation.Attention.apply)
+    assert len(used) >= 2 and all(used[:2])
+    monkeypatch.setattr(operation, "_take_workspace", lambda *_: None)
+    whole = run(operation.Attention.apply)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    for a, b in zip(got[:4], whole):
+        assert not torch.equal(a, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shape,dim", [((40, 33), 0), ((40, 33), 1), ((40, 33), None), ((3, 5, 16), -1)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_row_operations_are_the_functions_they_stand_in_for(shape, dim, masked, device, monkeypatch):
