@@ -192,10 +192,10 @@ int tri_attn_bwd(const TriAttnArgs* args);
 int tri_attn_bwd_noalloc(const TriAttnArgs* args);
 
 /* Bytes of args->workspace with which a call on these arguments runs split along the streamed dimension, 0 where it never does
- * (enough heads to fill the GPU, fewer than 20 tiles of 64, kernels other than the 16-bit matrix-core ones), or a negative
- * TRI_ATTN_E* code. pass 0 = tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq, 3 = tri_attn_bwd (its passes share the
+ * (enough heads to fill the GPU; lengths below 1217 in the 16-bit matrix-core kernels and below 193 in the fp32 ones; 16-bit problems on
+ * the 32-row-tile kernels and all problems on the element-wise ones), or a negative TRI_ATTN_E* code. pass 0 = tri_attn_fwd, 1 = tri_attn_bwd_dkdv, 2 = tri_attn_bwd_dq, 3 = tri_attn_bwd (its passes share the
  * workspace, one after the other), 4 = tri_attn_bwd_dmask (which then deals the batches and heads that share a mask to several
- * workgroups). A split call adds the parts' fp32 sums up in a fixed order: its results differ from an
+ * workgroups, at any length). A split call adds the parts' fp32 sums up in a fixed order: its results differ from an
  * unsplit call's by fp32 rounding, and do not depend on how the GPU schedules it. The reference launches one program per
  * row or key tile whatever the number of heads (trident/operation/attention.py:106-108). */
 int64_t tri_attn_workspace_size(const TriAttnArgs* args, int pass);
