@@ -54,7 +54,8 @@ def test_split_columns(dtype, rows, cols, mask_dtype, device, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype,rows,cols", [(torch.float32, 2049, 512), (torch.float32, 4096, 500), (torch.bfloat16, 4000, 1024), (torch.float16, 2100, 1023),
-                                             (torch.float32, 4096, 2052)])
+                                             (torch.float32, 4096, 2052), (torch.float32, 2049, 3072), (torch.bfloat16, 2100, 8192), (torch.float32, 2049, 7672),
+                                             (torch.float32, 2300, 4608)])
 def test_panels_of_32_bytes(dtype, rows, cols, device, monkeypatch):
     """The backward's narrow panels, whose lines are dealt out in another order: numbers of them that are dealt, do not fill up the last
     XCD, or stay in order. A panel's sums do not depend on its place: equal to those of the same columns in another matrix."""

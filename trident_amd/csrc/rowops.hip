@@ -514,9 +514,13 @@ __device__ __forceinline__ void merge_parts(const RowParams& p, const ColPlace& 
 __device__ __forceinline__ bool place_in_panel(const RowParams& p, int v, int lanes_log2, int64_t panels, ColPlace* c, bool narrow = false) {
     const int64_t per_xcd = (panels + 7) / 8;
     int64_t i = blockIdx.x >> 3;
-    // Panels of 32 bytes run in two rounds of the CUs. In order, a round covers every other KiB of the matrix's rows, which the HBM
-    // channels take badly; so the first round takes the even 128-byte lines and the second the odd ones (fp32 4096 x 4096, forward and
-    // backward, 102 -> 93.6 us; pieces of 64 bytes 100.7, of 256 bytes 94.8, the lines dealt to the XCDs in turn 95.5).
+    // Panels of 32 bytes, one workgroup per CU, run in up to four rounds of an XCD's 32 CUs. In order, a round covers every other KiB of
+    // the matrix's rows, which the HBM channels take badly; so the first half takes the even 128-byte lines and the second the odd ones
+    // (fp32 4096 x 4096, forward and backward, 102 -> 93.6 us; pieces of 64 bytes 100.7, of 256 bytes 94.8, the lines dealt to the XCDs
+    // in turn 95.5). Forward and backward, in order -> dealt, us: two rounds, fp32 2304 x 4096 58.6 -> 56.6, 4096 x 3072 93.0 -> 90.6,
+    // bf16 4096 x 8192 106 -> 97.5; three, fp32 4096 x 5120 146 -> 142.6, 4096 x 6144 153 -> 151, 4096 x 4608 138.5 -> 138.2; four, 4096 x
+    // 7680 206 -> 200. One round (4096 x 2048) and numbers of panels that do not divide (2304 columns) are as they were. The backward
+    // alone gains up to 16 % in two and four full rounds; in between it is from 1.5 % faster to 3 % slower (2304 x 6144 58.6 -> 60.3).
     if (narrow && per_xcd % 8 == 0) {
         const int64_t half = per_xcd / 8, u = i >> 2;
         i = ((u < half ? 2 * u : 2 * (u - half) + 1) << 2) + (i & 3);
