@@ -92,6 +92,8 @@ def _demangle(names):
             rest = rest[1:]
             while rest and not rest.startswith("E"):
                 for pat, fn in ((r"DF16_", lambda g: "_Float16"), (r"DF16b", lambda g: "__bf16"), (r"f", lambda g: "float"),
+                                (r"h", lambda g: "uint8"), (r"i", lambda g: "int"), (r"l", lambda g: "int64"), (r"v", lambda g: "void"),
+                                (r"LNS\d*_\d+[A-Za-z]+E(\d+)E", lambda g: g.group(1)),
                                 (r"Li(\d+)E", lambda g: g.group(1)), (r"Lb([01])E", lambda g: "true" if g.group(1) == "1" else "false")):
                     g = re.match(pat, rest)
                     if g:
