@@ -40,10 +40,11 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // DELTA (no mask, or D <= 64 without a mask gradient): the kernel also computes delta = rowsum(dO * O) of its rows from the dO rows it loads anyway, instead
 // of reading it, and stores it for the dK/dV pass, which then runs after this one (tri_attn_bwd_dq_delta).
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from
-// key0; the first part stores delta.
+// key0; the first part stores delta. Parts beside a mask at D = 16 are held to 168 registers: at 169, with two workgroups per CU instead
+// of three, they took a quarter longer (bf16 key mask, 4 heads, S=10368, with the second launch: 77 -> 96 us).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool DMASK = false, bool DELTA = false,
           bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) void mfma_dq_kernel(const KParams p) {
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 16 && SPLIT && MASK != kNoMask ? 3 : 2) void mfma_dq_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
