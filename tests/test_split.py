@@ -236,3 +236,51 @@ def test_launches_that_split(dtype, heads, S, D, causal, which, split, device):
     lse = torch.empty(1, heads, S, device=device)
     args = operation._make_args(q, q, q, q, lse, None, 0.0, causal, 0.125, 0, 0, q, q, q, q, None, lse)
     assert (_lib.lib().tri_attn_workspace_size(ctypes.byref(args), which) > 0) == split
+
+
+@pytest.mark.parametrize("dtype,heads,S,D,p,which", [
+    # whole launch -> parts (us)
+    (torch.bfloat16, 4, 11776, 16, 0.0, 3),   # dQ 255 -> 123
+    (torch.bfloat16, 16, 9108, 32, 0.1, 0),   # forward 827 -> 409
+    (torch.bfloat16, 16, 9108, 32, 0.1, 1),   # dK/dV 1275 -> 632
+    (torch.float16, 24, 6995, 32, 0.0, 0),    # forward 418 -> 189
+    (torch.bfloat16, 6, 5694, 128, 0.1, 3)])  # dQ 530 -> 281
+def test_key_masks_beyond_64_tiles_split(dtype, heads, S, D, p, which, device):
+    """Workgroups of more than 64 tiles do without the mask's classes, which costs them more than many heads make up for. (One part of
+    up to 64 tiles has them.)"""
+    q = torch.empty(1, heads, S, D, dtype=dtype, device=device)
+    lse = torch.empty(1, heads, S, device=device)
+    mask = operation._PreparedMask(torch.ones(1, 1, 1, S, dtype=torch.bool, device=device), q)
+    args = operation._make_args(q, q, q, q, lse, None, p, False, 0.125, 0, 0, q, q, q, q, None, lse)
+    mask.describe(args)
+    assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), which) > 0
+    if which != 1 and D < 128:
+        args.mask_classes = None  # (nothing to make use of: as a launch that fills the GPU)
+        assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), which) == 0 or heads < 16
+
+
+@pytest.mark.parametrize("S", [16384, 65536, 262144])
+@pytest.mark.parametrize("D,masked", [(16, True), (32, True), (128, False)])
+def test_workspaces_are_bounded(S, D, masked, device):
+    q = torch.empty(1, 2, S, D, dtype=torch.bfloat16, device=device)
+    lse = torch.empty(1, 2, S, device=device)
+    args = operation._make_args(q, q, q, q, lse, None, 0.0, False, 0.125, 0, 0, q, q, q, q, None, lse)
+    if masked:
+        mask = operation._PreparedMask(torch.ones(1, 1, 1, S, dtype=torch.bool, device=device), q)
+        mask.describe(args)
+    for which in (0, 1, 2, 3):
+        assert 0 <= _lib.lib().tri_attn_workspace_size(ctypes.byref(args), which) <= 1 << 28
+
+
+def test_whole_launches_of_eight_waves_beside_masks_do_not_split(device):
+    q = torch.empty(1, 10, 4096, 128, dtype=torch.bfloat16, device=device)
+    lse = torch.empty(1, 10, 4096, device=device)
+    mask = torch.zeros(1, 10, 4096, 4096, device=device)
+    args = operation._make_args(q, q, q, q, lse, mask, 0.1, False, 0.125, 0, 0)
+    assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 0) == 0  # (forward 90 us, split 213)
+    q = torch.empty(1, 8, 6400, 128, dtype=torch.bfloat16, device=device)
+    lse = torch.empty(1, 8, 6400, device=device)
+    mask = operation._PreparedMask(torch.ones(1, 1, 1, 6400, dtype=torch.bool, device=device), q)
+    args = operation._make_args(q, q, q, q, lse, None, 0.0, False, 0.125, 0, 0, q, q, q, q, None, lse)
+    mask.describe(args)
+    assert _lib.lib().tri_attn_workspace_size(ctypes.byref(args), 2) == 0  # (dQ 287 us, split 400)

@@ -176,18 +176,25 @@ int64_t plan_split(const SplitShape& shape, bool causal, KParams* p) {
     const int64_t heads = static_cast<int64_t>(p->B) * p->H;
     const int tiles = (p->S + 63) / 64, items = (p->S + shape.rows - 1) / shape.rows, step = shape.rows / 64;
     const int64_t cus = static_cast<int64_t>(persistent_grid(1 << 20)), slots = cus * shape.slots_per_cu;
-    // Microseconds, as measured over 2700 passes of 1 to 40 heads and 193 to 8000 rows: a workgroup's start and end, the second launch,
+    // Microseconds, as measured over 9000 passes of 1 to 40 heads and 193 to 12000 rows: a workgroup's start and end, the second launch,
     // bytes of the workspace (mostly in the caches) that both launches move in one. A CU with several workgroups takes longer for a
     // tile of each than one workgroup alone on it, but less than for that many one after the other.
     constexpr double kFixed = 4, kCombine = 7, kBytesPerUs = 5e6;
+    constexpr int64_t kMostBytes = int64_t{1} << 28;  // (what a call may ask its caller for; reached beyond 16384 rows)
     const auto time = [&](int64_t units, int each) {
         const int64_t on_cu = (units + cus - 1) / cus, rounds = (on_cu + shape.slots_per_cu - 1) / shape.slots_per_cu;
-        return static_cast<double>(rounds) * kFixed + each * std::max(static_cast<double>(rounds) * shape.tile_us, static_cast<double>(on_cu) * shape.cu_us);
+        return static_cast<double>(rounds) * kFixed +
+               (each > 64 ? shape.unclassed : 1.0) * each * std::max(static_cast<double>(rounds) * shape.tile_us, static_cast<double>(on_cu) * shape.cu_us);
     };
-    // A launch with a workgroup for every CU is worth it only where the workgroups are long.
-    if (tiles < shape.min_tiles || heads * items >= 2 * slots || (tiles < 64 && heads * items >= cus)) return 0;
-    const double whole = causal ? kFixed + std::max(tiles * shape.tile_us, static_cast<double>(heads) * items * (tiles + step) / 2.0 * shape.cu_us / cus)
-                                : time(heads * items, tiles);
+    // A launch with a workgroup for every CU is worth it only where the workgroups are long. One of two full rounds has little to win, unless
+    // its parts are what makes use of the mask's classes.
+    const int64_t most = shape.unclassed > 1.0 && tiles > 64 ? cus * 256 / std::max(p->D, 32) : 2 * slots;
+    if (tiles < shape.min_tiles || heads * items >= most || (tiles < 64 && heads * items >= cus)) return 0;
+    // (causal: the longest item shares its CU with others that are half as long on average)
+    const int64_t beside = std::min<int64_t>((heads * items + cus - 1) / cus, shape.slots_per_cu) - 1;
+    const double whole = causal ? kFixed + std::max(tiles * std::max(shape.tile_us, shape.cu_us * (1.0 + 0.5 * static_cast<double>(beside))),
+                                                    static_cast<double>(heads) * items * (tiles + step) / 2.0 * shape.cu_us / cus)
+                                : time(heads * (shape.whole_rows > 0 ? (p->S + shape.whole_rows - 1) / shape.whole_rows : items), tiles);
     const int64_t unit_bytes = shape.rows * (static_cast<int64_t>(p->D) * shape.outputs + (shape.statistics ? 2 : 0)) * 4;
     double best = shape.gain * whole;
     for (int c = std::max(shape.min_tiles / 5, step); c < tiles; c += causal ? step : 1) {  // (parts of at least a fifth of min_tiles)
@@ -198,6 +205,7 @@ int64_t plan_split(const SplitShape& shape, bool causal, KParams* p) {
         } else {
             units = static_cast<int64_t>(items) * ((tiles + c - 1) / c);
         }
+        if (heads * units * unit_bytes > kMostBytes) continue;
         const double t = time(heads * units, c) + kCombine + 2.0 * heads * units * unit_bytes / kBytesPerUs;
         if (t < best) {
             best = t;

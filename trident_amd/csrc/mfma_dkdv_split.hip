@@ -16,7 +16,7 @@ SplitShape dkdv_split_shape(const KParams& p) {
     const int waves = p.mask != nullptr && p.D == 64 && p.thr8 <= 0 ? 8 : 4;
     const int slots = p.D == 128 || (p.D == 64 && p.mask != nullptr) ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 3;
     const double us = split_work(p) * (p.D >= 64 ? 1.65 : p.D == 32 ? 1.22 : 1.05);
-    return SplitShape{32 * waves, slots, 2, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.58 : 0.52) * us, split_gain(p) - (p.D < 64 ? 0.04 : 0.0)};
+    return SplitShape{32 * waves, slots, 2, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.58 : 0.52) * us, split_gain(p) - (p.D < 64 ? 0.04 : 0.0), split_unclassed(p)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>

@@ -9,9 +9,13 @@ namespace {
 SplitShape dq_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = (p.D == 128 && p.mask == nullptr && p.thr8 <= 0) || (p.D == 64 && f32_mask) ? 8 : 4;
-    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 4;
+    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 || (p.D == 32 && p.mask != nullptr) ? 2 : p.mask != nullptr ? 3 : 4;
+    // Beside a mask at D = 128 parts have four waves, one per SIMD, and take longer than they promise (bf16 key mask with dropout, 12
+    // heads, S=1489, whole 45 us, split 59); whole launches of multiples of 256 have eight, half the items (8 heads, S=6400, 287 and 400).
+    const int whole_rows = p.D == 128 && p.mask != nullptr && p.thr8 <= 0 && p.S % 256 == 0 ? 256 : 32 * waves;
+    const double gain = split_gain(p) * (p.D == 128 && p.mask != nullptr ? 0.85 : 1.0);
     const double us = split_work(p) * (p.D == 128 ? 1.55 : p.D == 64 ? 0.96 : p.D == 32 ? 0.68 : 0.53);
-    return SplitShape{32 * waves, slots, 1, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.65 : 0.59) * us, split_gain(p)};
+    return SplitShape{32 * waves, slots, 1, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.65 : 0.59) * us, gain, split_unclassed(p), whole_rows};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>
@@ -48,10 +52,10 @@ int launch_dq_split_variant(int dtype, const KParams& p, hipStream_t stream, boo
 
 // (a mask gradient is written by whole items only; without a mask the parts bring delta along, with one they may up to D = 64)
 // Beside dropout at D = 128 a workgroup's start, with one wave per SIMD, costs more than the last round of a launch that fills the GPU
-// saves (bf16 S=4352, 11 heads: 209 -> 286 us).
+// saves (bf16 S=4352, 11 heads: 209 -> 286 us), except where parts are what makes use of a mask's classes (6 heads, S=5694: 530 -> 281).
 bool dq_splits(const KParams& p, bool with_delta) {
     const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
-    if (p.D == 128 && p.thr8 > 0 && !p.causal && items >= persistent_grid(1 << 20)) return false;
+    if (p.D == 128 && p.thr8 > 0 && !p.causal && items >= persistent_grid(1 << 20) && !(split_unclassed(p) > 1.0 && p.S > 64 * 64)) return false;
     return p.dmask == nullptr && (p.mask == nullptr ? with_delta : !with_delta || p.D <= 64);
 }
 

@@ -33,8 +33,11 @@ SplitShape fwd_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
     const int waves = p.D == 128 ? (p.mask != nullptr && p.thr8 > 0 ? 4 : 8) : p.D == 64 && f32_mask ? 8 : 4;
     const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 ? 2 : p.mask == nullptr ? 4 : p.thr8 > 0 || (f32_mask && p.D == 32) ? 2 : 3;
+    // (beside mask and dropout at D = 128 whole launches of multiples of 256 have eight waves, half the items: bf16 fp32 mask, 10 heads,
+    // S=4096, whole 90 us, split 213)
+    const int whole_rows = p.D == 128 && waves == 4 && p.S % 256 == 0 ? 256 : 32 * waves;
     const double us = split_work(p) * (p.D == 128 ? 1.4 : p.D == 64 ? 0.9 : 0.62);
-    return SplitShape{32 * waves, slots, 1, true, 20, us, slots == 1 ? us : 0.6 * us, split_gain(p)};
+    return SplitShape{32 * waves, slots, 1, true, 20, us, slots == 1 ? us : 0.6 * us, split_gain(p), split_unclassed(p), whole_rows};
 }
 
 template <typename T>
