@@ -79,12 +79,15 @@ __device__ __forceinline__ void store_mask_elem(void* base, int dtype, int64_t o
 struct Philox4 {
     uint32_t w[4];
 };
-// One of the ten rounds (r = 0 .. 9), for callers that spread them over other work.
+constexpr uint32_t kPhiloxM0 = 0xD2511F53u, kPhiloxM1 = 0xCD9E8D57u;  // multipliers
+constexpr uint32_t kPhiloxW0 = 0x9E3779B9u, kPhiloxW1 = 0xBB67AE85u;  // key increments
+// One of the ten rounds (r = 0 .. 9), for callers that spread them over other work or have folded the first ones. (The exclusive or of
+// three words is one instruction, which the compiler does not find by itself.)
 __device__ __forceinline__ void philox_round(Philox4& s, int r, uint32_t k0, uint32_t k1) {
-    const uint64_t p0 = static_cast<uint64_t>(0xD2511F53u) * s.w[0];
-    const uint64_t p1 = static_cast<uint64_t>(0xCD9E8D57u) * s.w[2];
-    s.w[0] = static_cast<uint32_t>(p1 >> 32) ^ s.w[1] ^ (k0 + r * 0x9E3779B9u);
-    s.w[2] = static_cast<uint32_t>(p0 >> 32) ^ s.w[3] ^ (k1 + r * 0xBB67AE85u);
+    const uint64_t p0 = static_cast<uint64_t>(kPhiloxM0) * s.w[0];
+    const uint64_t p1 = static_cast<uint64_t>(kPhiloxM1) * s.w[2];
+    s.w[0] = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(p1 >> 32), s.w[1], k0 + r * kPhiloxW0, 0x96);
+    s.w[2] = __builtin_amdgcn_bitop3_b32(static_cast<uint32_t>(p0 >> 32), s.w[3], k1 + r * kPhiloxW1, 0x96);
     s.w[1] = static_cast<uint32_t>(p1);
     s.w[3] = static_cast<uint32_t>(p0);
 }

@@ -132,10 +132,6 @@ struct Stage32 {
     }
 };
 
-__device__ __forceinline__ uint32_t pick_word(const Philox4& r, int s) {
-    return s == 0 ? r.w[0] : (s == 1 ? r.w[1] : (s == 2 ? r.w[2] : r.w[3]));
-}
-
 // ------------------------------------------------------------------------------------------------ forward
 // SPLIT (here and below): a workgroup streams one part of its item's rows (split.hpp).
 template <typename T, int D, bool SPLIT>
@@ -248,15 +244,16 @@ __global__ __launch_bounds__(256, 2) void mfma32_fwd_kernel(const KParams p) {
                 x[i] = fast_exp2(fmaf(x[i], xs, -m_use));
                 l += x[i];
             }
-            if (p.thr8 > 0) {
+            if (p.thr8 > 0) {  // keys k0 + 8 g + 4 h + 0..3 of row qrow: one word of one generator block (shared inside the quad)
+                uint32_t w[4];
+                DropoutRows drop;
+                drop.init(p, bh, qrow >> 2);
+                DropoutRows::words(drop.block(p, (k0 + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    // keys k0 + 8 g + 4 h + 0..3 of row qrow: one word of one generator block
-                    const Philox4 r = dropout_block(p, bh, qrow >> 2, (k0 + 8 * g + 4 * h) >> 2);
-                    const uint32_t word = pick_word(r, qrow & 3);
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
-                        const bool keep = static_cast<int>((word >> (8 * bb)) & 0xffu) >= p.thr8;
+                        const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
                         x[4 * g + bb] = keep ? x[4 * g + bb] * p.zscale : 0.f;
                     }
                 }
@@ -417,14 +414,16 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void mfma32_dq_kernel(const 
                     ds[i] = visible ? ds[i] : 0.f;
                 }
             }
-            if (p.thr8 > 0) {
+            if (p.thr8 > 0) {  // (as the forward)
+                uint32_t w[4];
+                DropoutRows drop;
+                drop.init(p, bh, qrow >> 2);
+                DropoutRows::words(drop.block(p, (k0 + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    const Philox4 r = dropout_block(p, bh, qrow >> 2, (k0 + 8 * g + 4 * h) >> 2);
-                    const uint32_t word = pick_word(r, qrow & 3);
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
-                        const bool keep = static_cast<int>((word >> (8 * bb)) & 0xffu) >= p.thr8;
+                        const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
                         dp[4 * g + bb] = keep ? dp[4 * g + bb] * p.zscale : 0.f;
                     }
                 }
@@ -591,14 +590,16 @@ __global__ __launch_bounds__(256, 2) void mfma32_dkdv_kernel(const KParams p) {
                     pr[i] = visible ? pr[i] : 0.f;
                 }
             }
-            if (p.thr8 > 0) {
+            if (p.thr8 > 0) {  // rows r0 + 8 g + 4 h + 0..3 of this key: one byte of each word of one generator block (shared inside the quad)
+                uint32_t w[4];
+                DropoutKeys drop;
+                drop.init(p, bh, key >> 2);
+                DropoutKeys::words(drop.block(p, (r0 + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    // rows r0 + 8 g + 4 h + 0..3 of this key: one byte of each word of one generator block
-                    const Philox4 r = dropout_block(p, bh, (r0 + 8 * g + 4 * h) >> 2, key >> 2);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const bool keep = static_cast<int>((r.w[e] >> (8 * (key & 3))) & 0xffu) >= p.thr8;
+                        const bool keep = static_cast<int>((w[g] >> (8 * e)) & 0xffu) >= p.thr8;
                         const int i = 4 * g + e;
                         ds[i] = pr[i] * ((keep ? dp[i] * p.zscale : 0.f) - sDelta[c_row(i, h)]);
                         pr[i] = keep ? pr[i] * p.zscale : 0.f;
@@ -783,13 +784,16 @@ __global__ __launch_bounds__(256, 1) void mfma32_dkdv_split_kernel(const KParams
                     pr[i] = visible ? pr[i] : 0.f;
                 }
             }
-            if (p.thr8 > 0) {
+            if (p.thr8 > 0) {  // rows r0 + 8 g + 4 h + 0..3 of this key: one byte of each word of one generator block (shared inside the quad)
+                uint32_t w[4];
+                DropoutKeys drop;
+                drop.init(p, bh, key >> 2);
+                DropoutKeys::words(drop.block(p, (r0 + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    const Philox4 r = dropout_block(p, bh, (r0 + 8 * g + 4 * h) >> 2, key >> 2);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const bool keep = static_cast<int>((r.w[e] >> (8 * (key & 3))) & 0xffu) >= p.thr8;
+                        const bool keep = static_cast<int>((w[g] >> (8 * e)) & 0xffu) >= p.thr8;
                         const int i = 4 * g + e;
                         ds[i] = pr[i] * ((keep ? dp[i] * p.zscale : 0.f) - sDelta[kTile32 * rh + c_row(i, h)]);
                         pr[i] = keep ? pr[i] * p.zscale : 0.f;

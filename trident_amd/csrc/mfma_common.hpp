@@ -375,45 +375,108 @@ struct RowBlockStore {
 // A Philox call yields the 16 keep-bytes of a 4x4 block of P. In the MFMA register layouts the four
 // lanes of a quad (lanes 4n..4n+3) own four consecutive rows (forward, dQ) or four consecutive
 // columns (dK/dV) of the same blocks, so each of them would generate every block itself. Instead
-// lane q of the quad generates only the blocks of group q (mod 4) and the others fetch them with
-// quad-broadcast DPP moves: a quarter of the Philox work for 4 moves per block.
-template <int G>
-__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), G * 0x55, 0xf, 0xf, true));
+// lane q of the quad generates only the blocks of group q (mod 4), and a 4 x 4 transposition inside the quad hands
+// every lane its own word of each of the four.
+// The vector ALU is what dropout costs (a block is 18 or 16 multiplications and 19 logic operations for 16 scores, beside 32 fma and exp2),
+// so nothing is computed twice: of a block's counter (j >> 2, i >> 2, head, offset) a lane keeps one of the first two words for all its
+// tiles, and what follows from that word and the uniform ones in the first rounds is made once per item (DropoutRows, DropoutKeys); the
+// transposition selects while it moves (8 instructions where moves and selections apart took 16, or 32 with the shifts of the
+// key-owner form). Training steps with p = 0.1, us, before -> with all of this: bf16 causal B=4 H=16 S=2048 D=64 295 -> 273, D=32
+// without the causal mask 354 -> 312, bf16 causal B=2 H=16 S=4096 D=128 708 -> 692 (the power limit holds those), B=1 H=32 S=16384
+// 10310 -> 10111; fp32 causal B=2 H=32 S=1024 D=16 274 -> 239 (the fp32 kernels had not shared blocks inside the quad).
+
+// Lane g's word q goes to lane q's word g (within the quad): exchanges with lane ^ 1, then with lane ^ 2. v_cndmask takes one
+// side from the neighbour (DPP), the other from the lane itself; the two scalar moves in front of each group are the wait states that a
+// DPP operand written by a vector instruction needs.
+__device__ __forceinline__ void quad_transpose(uint32_t (&w)[4]) {
+    uint32_t n0, n1, n2, n3;
+    asm("s_mov_b32 vcc_lo, 0x55555555\n\ts_mov_b32 vcc_hi, 0x55555555\n\ts_nop 0\n\t"
+        "v_cndmask_b32_dpp %0, %5, %4, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %2, %7, %6, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_not_b64 vcc, vcc\n\t"
+        "v_cndmask_b32_dpp %1, %4, %5, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %3, %6, %7, vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+        : "=&v"(n0), "=&v"(n1), "=&v"(n2), "=&v"(n3) : "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]) : "vcc", "scc");
+    asm("s_mov_b32 vcc_lo, 0x33333333\n\ts_mov_b32 vcc_hi, 0x33333333\n\ts_nop 0\n\t"
+        "v_cndmask_b32_dpp %0, %6, %4, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %1, %7, %5, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_not_b64 vcc, vcc\n\t"
+        "v_cndmask_b32_dpp %2, %4, %6, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_cndmask_b32_dpp %3, %5, %7, vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]) : "v"(n0), "v"(n1), "v"(n2), "v"(n3) : "vcc", "scc");
 }
-// The block lane G of the quad holds, for every lane of the quad.
-template <int G>
-__device__ __forceinline__ Philox4 quad_bcast(const Philox4& r) {
-    Philox4 o;
+
+// Row-owner form (forward, dQ): this lane owns row i (i % 4 == lane % 4). Rounds 0 and 1 of Philox with i >> 2, the head and the offset folded:
+// round 0 takes w0 and w1 from the head's product alone, so that round 1's product of w0 is the lane's for all its tiles.
+struct DropoutRows {
+    uint32_t u0, u2;    // uniform: what joins w0 of round 1 and w2 of round 0
+    uint32_t a, b;      // of this lane: what joins w2 of round 1, and w3 of it
+    __device__ __forceinline__ void init(const KParams& p, uint32_t bh, uint32_t ib) {
+        const uint64_t p1 = static_cast<uint64_t>(kPhiloxM1) * bh;
+        u2 = p.offset ^ p.seed_hi;
+        u0 = static_cast<uint32_t>(p1) ^ (p.seed_lo + kPhiloxW0);
+        const uint64_t q = static_cast<uint64_t>(kPhiloxM0) * (static_cast<uint32_t>(p1 >> 32) ^ p.seed_lo ^ ib);
+        a = static_cast<uint32_t>(q >> 32) ^ (p.seed_hi + kPhiloxW1);
+        b = static_cast<uint32_t>(q);
+    }
+    static constexpr int kFirstRound = 2;  // rounds that start() leaves to do: kFirstRound .. 9
+    __device__ __forceinline__ Philox4 start(uint32_t jb) const {
+        const uint64_t p0 = static_cast<uint64_t>(kPhiloxM0) * jb;
+        const uint64_t p1 = static_cast<uint64_t>(kPhiloxM1) * (static_cast<uint32_t>(p0 >> 32) ^ u2);
+        return Philox4{{static_cast<uint32_t>(p1 >> 32) ^ u0, static_cast<uint32_t>(p1), a ^ static_cast<uint32_t>(p0), b}};
+    }
+    // The block of columns 4 jb .. +3 (dropout_block(p, bh, ib, jb)).
+    __device__ __forceinline__ Philox4 block(const KParams& p, uint32_t jb) const {
+        Philox4 s = start(jb);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o.w[k] = quad_bcast<G>(r.w[k]);
-    return o;
-}
-// Same with the source lane as an argument (a constant once the caller's loop is unrolled).
-__device__ __forceinline__ Philox4 quad_bcast_from(int g, const Philox4& r) {
-    return g == 0 ? quad_bcast<0>(r) : (g == 1 ? quad_bcast<1>(r) : (g == 2 ? quad_bcast<2>(r) : quad_bcast<3>(r)));
-}
-// Row-owner form: this lane owns row i (i % 4 == lane % 4) and wants, for groups g = 0..3, the word
-// (4 key bytes) of keys key0 + gstride*g .. +3. `mine` is the block this lane generated for group
-// lane % 4, i.e. dropout_block(p, bh, i >> 2, (key0 + gstride * (lane % 4)) >> 2).
-// A 4 x 4 transposition inside the quad (lane g's word q goes to lane q's word g) by two exchanges, with lane ^ 1 and with
-// lane ^ 2: 4 moves and 12 selections (broadcasting the four blocks and picking words took 16 and 12).
-__device__ __forceinline__ void quad_row_words(const Philox4& mine, int lane, uint32_t (&w)[4]) {
-    const bool odd = (lane & 1) != 0, high = (lane & 2) != 0;
-    auto exchange = [](uint32_t& a, uint32_t& b, bool second, auto ctrl) {  // a of the second lane <-> b of the first
-        const uint32_t out = second ? a : b;
-        const uint32_t in = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(out), decltype(ctrl)::value, 0xf, 0xf, true));
-        a = second ? in : a;
-        b = second ? b : in;
-    };
-    using Xor1 = std::integral_constant<int, 0xB1>;  // quad_perm [1, 0, 3, 2]
-    using Xor2 = std::integral_constant<int, 0x4E>;  // quad_perm [2, 3, 0, 1]
+        for (int r = kFirstRound; r < 10; ++r) philox_round(s, r, p.seed_lo, p.seed_hi);
+        return s;
+    }
+    // w[g]: the four key bytes of this lane's row in the group of keys key0 + gstride * g .. +3, `mine` being the block of the group
+    // lane % 4, i.e. block(p, (key0 + gstride * (lane % 4)) >> 2).
+    static __device__ __forceinline__ void words(const Philox4& mine, uint32_t (&w)[4]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = mine.w[i];
-    exchange(w[0], w[1], odd, Xor1{});
-    exchange(w[2], w[3], odd, Xor1{});
-    exchange(w[0], w[2], high, Xor2{});
-    exchange(w[1], w[3], high, Xor2{});
-}
+        for (int i = 0; i < 4; ++i) w[i] = mine.w[i];
+        quad_transpose(w);
+    }
+};
+
+// Key-owner form (dK/dV): this lane owns key j (j % 4 == lane % 4). Rounds 0 to 2 with j >> 2, the head and the offset folded: of the six
+// products four are the lane's or the head's.
+struct DropoutKeys {
+    uint32_t u;               // uniform: what joins w0 of round 0
+    uint32_t c1, c3, h2, l2;  // of this lane: what joins w2 of round 1, w0 of round 2 and w2 of round 2, and w3 of it
+    __device__ __forceinline__ void init(const KParams& p, uint32_t bh, uint32_t jb) {
+        const uint64_t p1 = static_cast<uint64_t>(kPhiloxM1) * bh, p0 = static_cast<uint64_t>(kPhiloxM0) * jb;
+        u = static_cast<uint32_t>(p1 >> 32) ^ p.seed_lo;
+        c1 = static_cast<uint32_t>(p0) ^ (p.seed_hi + kPhiloxW1);
+        const uint64_t q1 = static_cast<uint64_t>(kPhiloxM1) * (static_cast<uint32_t>(p0 >> 32) ^ p.offset ^ p.seed_hi);
+        const uint32_t w0 = static_cast<uint32_t>(q1 >> 32) ^ static_cast<uint32_t>(p1) ^ (p.seed_lo + kPhiloxW0);
+        c3 = static_cast<uint32_t>(q1) ^ (p.seed_lo + 2 * kPhiloxW0);
+        const uint64_t r0 = static_cast<uint64_t>(kPhiloxM0) * w0;
+        h2 = static_cast<uint32_t>(r0 >> 32) ^ (p.seed_hi + 2 * kPhiloxW1);
+        l2 = static_cast<uint32_t>(r0);
+    }
+    // The block of rows 4 ib .. +3 (dropout_block(p, bh, ib, jb)).
+    __device__ __forceinline__ Philox4 block(const KParams& p, uint32_t ib) const {
+        const uint64_t p0 = static_cast<uint64_t>(kPhiloxM0) * (ib ^ u);
+        const uint64_t p1 = static_cast<uint64_t>(kPhiloxM1) * (static_cast<uint32_t>(p0 >> 32) ^ c1);
+        Philox4 s{{static_cast<uint32_t>(p1 >> 32) ^ c3, static_cast<uint32_t>(p1), h2 ^ static_cast<uint32_t>(p0), l2}};
+#pragma unroll
+        for (int r = 3; r < 10; ++r) philox_round(s, r, p.seed_lo, p.seed_hi);
+        return s;
+    }
+    // w[g]: the four row bytes at this lane's key in the group of rows row0 + gstride * g .. +3, `mine` being the block of the group
+    // lane % 4. A block's words are rows and its bytes keys: transposed in the lane first, then in the quad.
+    static __device__ __forceinline__ void words(const Philox4& mine, uint32_t (&w)[4]) {
+        const uint32_t a = __builtin_amdgcn_perm(mine.w[1], mine.w[0], 0x05010400u), b = __builtin_amdgcn_perm(mine.w[1], mine.w[0], 0x07030602u);
+        const uint32_t c = __builtin_amdgcn_perm(mine.w[3], mine.w[2], 0x05010400u), d = __builtin_amdgcn_perm(mine.w[3], mine.w[2], 0x07030602u);
+        w[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+        w[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+        w[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+        w[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+        quad_transpose(w);
+    }
+};
 
 }  // namespace tri

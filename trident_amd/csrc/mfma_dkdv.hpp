@@ -212,6 +212,8 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
         }
     }
 
+    [[maybe_unused]] DropoutKeys drop;
+    if constexpr (DROPOUT) drop.init(p, bh, key >> 2);
     const int row_off0 = Tile::off(l32, h);
     const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
@@ -326,31 +328,25 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
                         for (int bb = 0; bb < 4; ++bb) pexp[4 * g + bb] = fast_exp2(fmaf(s[4 * g + bb], c, -l4[bb]));
                     }
                 }
-                Philox4 mine;  // the block of rows rb + 8 (lane % 4) + 4 h .. +3: this lane's share of the quad's four
-                if constexpr (DROPOUT) mine = dropout_block(p, bh, (rb + 8 * (lane & 3) + 4 * h) >> 2, key >> 2);
+                uint32_t w[4];  // (this lane's share of the quad's four blocks: rows rb + 8 (lane % 4) + 4 h .. +3)
+                if constexpr (DROPOUT) DropoutKeys::words(drop.block(p, (rb + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
                     if constexpr (!kDeltaInAcc) d4 = *reinterpret_cast<const f32x4*>(sDelta + 32 * qb + 8 * g + 4 * h);
-                    uint32_t dw[4];
-                    if constexpr (DROPOUT) {
-                        const Philox4 r = quad_bcast_from(g, mine);  // lane g of the quad generated rows rb + 8 g + 4 h .. +3
-#pragma unroll
-                        for (int bb = 0; bb < 4; ++bb) dw[bb] = (r.w[bb] >> (8 * (key & 3))) & 0xffu;
-                    }
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
                         const int i = 4 * g + bb;
                         const float pv = pexp[i];
                         float dpv = dp[i];
                         if constexpr (DROPOUT) {
-                            const bool keep = static_cast<int>(dw[bb]) >= p.thr8;
-                            dpv = keep ? dpv * p.zscale : 0.f;
-                            pr[i] = keep ? pv * p.zscale : 0.f;
+                            const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
+                            dpv = keep ? dpv : 0.f;
+                            pr[i] = keep ? pv : 0.f;  // (the 1 / (1 - p) factor: at the end)
                         } else {
                             pr[i] = pv;
                         }
-                        ds[i] = kDeltaInAcc ? pv * dpv : pv * (dpv - d4[bb]);
+                        ds[i] = kDeltaInAcc ? pv * dpv : pv * fmaf(dpv, p.zscale, -d4[bb]);
                     }
                 }
 #pragma unroll
@@ -383,7 +379,7 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
         if (part.count > 1) {
             float* const sums = p.partial + (static_cast<int64_t>(part.unit) * 2 * kKeys + 32 * wave) * D;
             store_partial<DB, D>(dk, sums, 0, lane, (kDeltaInAcc ? -1.f : 1.f) * (kLeftOut ? left_out : 1.f));
-            store_partial<DB, D>(dv, sums + static_cast<int64_t>(kKeys) * D, 0, lane, kLeftOut ? left_out : 1.f);
+            store_partial<DB, D>(dv, sums + static_cast<int64_t>(kKeys) * D, 0, lane, (DROPOUT ? p.zscale : 1.f) * (kLeftOut ? left_out : 1.f));
             return;
         }
     }
@@ -399,7 +395,8 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
         const int keys_here = RAGGED ? p.S - wkey0 : 32;
         Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, lane, keys_here);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
-        Store::run(dv, [left_out](float x) { return kLeftOut ? x * left_out : x; }, patch, dv0, p.dvs[2] * 2, lane, keys_here);
+        const float dv_sc = (DROPOUT ? p.zscale : 1.f) * (kLeftOut ? left_out : 1.f);
+        Store::run(dv, [dv_sc](float x) { return DROPOUT || kLeftOut ? x * dv_sc : x; }, patch, dv0, p.dvs[2] * 2, lane, keys_here);
     }
 }
 
@@ -532,6 +529,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
     // step 2t+3; by then it has scored tile t+1, so it takes its own P and dS of tile t back from
     // its slot just before it overwrites them.
     const int n_local = n_tiles - t_begin;
+    [[maybe_unused]] DropoutKeys drop;
+    if constexpr (DROPOUT) drop.init(p, bh, key >> 2);
     u32x4 cur_p[2], cur_s[2];
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
@@ -660,8 +659,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) mk[i] = sc_mk[i];
             }
-            Philox4 mine;  // the block of rows rb + 8 (lane % 4) + 4 h .. +3: this lane's share of the quad's four
-            if constexpr (DROPOUT) mine = dropout_block(p, bh, (rb + 8 * (lane & 3) + 4 * h) >> 2, key >> 2);
+            uint32_t w[4];  // (this lane's share of the quad's four blocks: rows rb + 8 (lane % 4) + 4 h .. +3)
+            if constexpr (DROPOUT) DropoutKeys::words(drop.block(p, (rb + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
             for (int gg = 0; gg < 2; ++gg) {  // eight rows at a time, packed as soon as they are done
                 float pr[8], ds[8];
@@ -676,12 +675,6 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
                     const int g = 2 * gg + g2;
                     f32x4 l4 = sc_lse[g];
                     const f32x4 d4 = dlt4[g2];
-                    uint32_t dw[4];
-                    if constexpr (DROPOUT) {
-                        const Philox4 r = quad_bcast_from(g, mine);  // lane g of the quad generated rows rb + 8 g + 4 h .. +3
-#pragma unroll
-                        for (int bb = 0; bb < 4; ++bb) dw[bb] = (r.w[bb] >> (8 * (key & 3))) & 0xffu;
-                    }
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
                         const int i = 4 * g + bb;
@@ -690,13 +683,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
                         else pv = fast_exp2(fmaf(s[i], c, -l4[bb]));
                         float dpv = dp[i];
                         if constexpr (DROPOUT) {
-                            const bool keep = static_cast<int>(dw[bb]) >= p.thr8;
-                            dpv = keep ? dpv * p.zscale : 0.f;
-                            pr[4 * g2 + bb] = keep ? pv * p.zscale : 0.f;
+                            const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
+                            dpv = keep ? dpv : 0.f;
+                            pr[4 * g2 + bb] = keep ? pv : 0.f;  // (the 1 / (1 - p) factor: at the end)
                         } else {
                             pr[4 * g2 + bb] = pv;
                         }
-                        ds[4 * g2 + bb] = pv * (dpv - d4[bb]);
+                        ds[4 * g2 + bb] = pv * (DROPOUT ? fmaf(dpv, p.zscale, -d4[bb]) : dpv - d4[bb]);
                     }
                 }
                 cur_p[gg] = pack8<T>(pr);
@@ -807,7 +800,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_pair_kernel(const KParams p)
         asm volatile("" : "+v"(elane));
         Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, elane);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
-        Store::run(dv, [](float x) { return x; }, patch, dv0, p.dvs[2] * 2, elane);
+        const float dv_sc = DROPOUT ? p.zscale : 1.f;
+        Store::run(dv, [dv_sc](float x) { return DROPOUT ? x * dv_sc : x; }, patch, dv0, p.dvs[2] * 2, elane);
     }
 }
 
@@ -1010,6 +1004,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
     // whether this pair has anything in block r (under the causal mask: rows at or below its first key)
     auto block_on = [&](int r) { return r >= 0 && r < n_blocks && (!CAUSAL || r >= first_on); };
 
+    [[maybe_unused]] DropoutKeys drop;
+    if constexpr (DROPOUT) drop.init(p, bh, key >> 2);
     constexpr float kFoldUnit = 256.f;  // the constant the first of the split terms multiplies (keeps f16 terms in range)
     const float neg_inv_c = -1.f / c;
     f32x16 sc_s, sc_dp;  // S - lse / c and dP - delta of this member's next block
@@ -1098,8 +1094,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
         }
         const f32x16 s = sc_s, dp = sc_dp;
         const float* sDelta = reinterpret_cast<const float*>(smem + so + 2 * kHalfBytes) + 64;
-        Philox4 mine;  // the block of rows rb + 8 (lane % 4) + 4 h .. +3: this lane's share of the quad's four
-        if constexpr (DROPOUT) mine = dropout_block(p, bh, (rb + 8 * (lane & 3) + 4 * h) >> 2, key >> 2);
+        uint32_t w[4];  // (this lane's share of the quad's four blocks: rows rb + 8 (lane % 4) + 4 h .. +3)
+        if constexpr (DROPOUT) DropoutKeys::words(drop.block(p, (rb + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
         for (int gg = 0; gg < 2; ++gg) {
             float pr[8], ds[8];
@@ -1107,21 +1103,15 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
             for (int g2 = 0; g2 < 2; ++g2) {
                 const int g = 2 * gg + g2;
                 f32x4 d4 = {0.f, 0.f, 0.f, 0.f};
-                uint32_t dw[4] = {0, 0, 0, 0};
-                if constexpr (DROPOUT) {
-                    d4 = *reinterpret_cast<const f32x4*>(sDelta + 8 * g + 4 * h);
-                    const Philox4 rr = quad_bcast_from(g, mine);  // lane g of the quad generated rows rb + 8 g + 4 h .. +3
-#pragma unroll
-                    for (int bb = 0; bb < 4; ++bb) dw[bb] = (rr.w[bb] >> (8 * (key & 3))) & 0xffu;
-                }
+                if constexpr (DROPOUT) d4 = *reinterpret_cast<const f32x4*>(sDelta + 8 * g + 4 * h);
 #pragma unroll
                 for (int bb = 0; bb < 4; ++bb) {
                     const int i = 4 * g + bb, j = 4 * g2 + bb;
                     const float pv = KEYMASK != kNoMask ? fast_exp2(fmaf(s[i], c, key_bias)) : fast_exp2(s[i] * c);
                     if constexpr (DROPOUT) {
-                        const bool keep = static_cast<int>(dw[bb]) >= p.thr8;
-                        pr[j] = keep ? pv * p.zscale : 0.f;
-                        ds[j] = pv * ((keep ? dp[i] * p.zscale : 0.f) - d4[bb]);
+                        const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
+                        pr[j] = keep ? pv : 0.f;  // (the 1 / (1 - p) factor: at the end)
+                        ds[j] = pv * fmaf(keep ? dp[i] : 0.f, p.zscale, -d4[bb]);
                     } else {
                         pr[j] = pv;
                         ds[j] = pv * dp[i];
@@ -1242,7 +1232,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
             asm volatile("" : "+v"(elane));
             float* const sums = p.partial + (static_cast<int64_t>(part.unit) * 2 * kKeys + 32 * kb) * D;
             store_partial<DH, D>(dk, sums, DH * member, elane, 1.f);
-            store_partial<DH, D>(dv, sums + static_cast<int64_t>(kKeys) * D, DH * member, elane, 1.f);
+            store_partial<DH, D>(dv, sums + static_cast<int64_t>(kKeys) * D, DH * member, elane, DROPOUT ? p.zscale : 1.f);
             return;
         }
     }
@@ -1261,7 +1251,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dkdv_phased_kernel(const KParams 
         asm volatile("" : "+v"(elane));
         Store::run(dk, [sc](float x) { return x * sc; }, patch, dk0, p.dks[2] * 2, elane, RAGGED ? p.S - wkey0 : 32);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // patch read before it is rewritten
-        Store::run(dv, [](float x) { return x; }, patch, dv0, p.dvs[2] * 2, elane, RAGGED ? p.S - wkey0 : 32);
+        const float dv_sc = DROPOUT ? p.zscale : 1.f;
+        Store::run(dv, [dv_sc](float x) { return DROPOUT ? x * dv_sc : x; }, patch, dv0, p.dvs[2] * 2, elane, RAGGED ? p.S - wkey0 : 32);
     }
 }
 

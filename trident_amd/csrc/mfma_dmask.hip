@@ -188,7 +188,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dmask_kernel(const KParams p, con
             for (int kb = 0; kb < 2; ++kb) {
                 const Philox4 mine = dropout_block(p, static_cast<uint32_t>(bh), qrow >> 2, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
                 uint32_t w[4];
-                quad_row_words(mine, lane, w);
+                DropoutRows::words(mine, w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
 #pragma unroll

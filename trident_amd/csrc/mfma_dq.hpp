@@ -232,6 +232,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
         asm volatile("" : "+v"(dlt16));  // (kept in registers: as a splat it would be made anew for every block)
     }
 
+    [[maybe_unused]] DropoutRows drop;
+    if constexpr (DROPOUT) drop.init(p, bh, qrow >> 2);
     const int row_off0 = Tile::off(l32, h);
     const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
@@ -335,19 +337,18 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
                 for (int i = 0; i < 16; ++i) ds[i] = fast_exp2(fmaf(st[i], c, -lse));
             }
             if constexpr (DROPOUT) {
-                const Philox4 mine = dropout_block(p, bh, qrow >> 2, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
                 uint32_t w[4];
-                quad_row_words(mine, lane, w);
+                DropoutRows::words(drop.block(p, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
                         const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
-                        dpt[4 * g + bb] = keep ? dpt[4 * g + bb] * p.zscale : 0.f;
+                        dpt[4 * g + bb] = keep ? dpt[4 * g + bb] : 0.f;
                     }
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ds[i] *= kDeltaInAcc ? dpt[i] : dpt[i] - dlt;
+            for (int i = 0; i < 16; ++i) ds[i] *= kDeltaInAcc ? dpt[i] : DROPOUT ? fmaf(dpt[i], p.zscale, -dlt) : dpt[i] - dlt;
             if constexpr (DMASK) {
                 const int64_t at = b * p.dms[0] + hd * p.dms[1] + static_cast<int64_t>(qrow) * p.dms[2] + t0 + 32 * kb + 4 * h;
                 if (p.dmask_acc) {
@@ -582,6 +583,8 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         for (int i = 0; i < 16; ++i) dlt16[i] = dlt;
         asm volatile("" : "+v"(dlt16));  // (kept in registers: as a splat it would be made anew for every tile)
     }
+    [[maybe_unused]] DropoutRows drop;
+    if constexpr (DROPOUT) drop.init(p, bh, qrow >> 2);
     const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
     // fragment n of the matrix phase of tile t: n < kDqSteps: K^T of tile t (column block n % DB, K-step
@@ -668,19 +671,18 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
             }
             f32x16 dpv = dpt[kb];
             if constexpr (DROPOUT) {
-                const Philox4 mine = dropout_block(p, bh, qrow >> 2, (first_key + 8 * (lane & 3) + 4 * h) >> 2);
                 uint32_t w[4];
-                quad_row_words(mine, lane, w);
+                DropoutRows::words(drop.block(p, (first_key + 8 * (lane & 3) + 4 * h) >> 2), w);
 #pragma unroll
                 for (int g = 0; g < 4; ++g)
 #pragma unroll
                     for (int bb = 0; bb < 4; ++bb) {
                         const bool keep = static_cast<int>((w[g] >> (8 * bb)) & 0xffu) >= p.thr8;
-                        dpv[4 * g + bb] = keep ? dpv[4 * g + bb] * p.zscale : 0.f;
+                        dpv[4 * g + bb] = keep ? dpv[4 * g + bb] : 0.f;
                     }
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ds[i] *= kDeltaInAcc ? dpv[i] : dpv[i] - dlt;
+            for (int i = 0; i < 16; ++i) ds[i] *= kDeltaInAcc ? dpv[i] : DROPOUT ? fmaf(dpv[i], p.zscale, -dlt) : dpv[i] - dlt;
             bop[2 * kb + 0] = pack8<T>(&ds[0]);
             bop[2 * kb + 1] = pack8<T>(&ds[8]);
         };

@@ -358,10 +358,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
     // matrix phase is as long there, and the clock gives under the power limit), so that the rounds stay where they are.
     constexpr bool kEarlyBits = DROPOUT && kPingPong && D == 64;
     Philox4 bits[kEarlyBits ? 2 : 1];  // of the next tile's two key blocks
-    auto start_bits = [&](int kb, int t) {
-        return Philox4{{static_cast<uint32_t>((key0 + t * kBN + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2), static_cast<uint32_t>(qrow >> 2),
-                        static_cast<uint32_t>(bh), p.offset}};
-    };
+    [[maybe_unused]] DropoutRows drop;
+    auto block_column = [&](int kb, int t) { return static_cast<uint32_t>((key0 + t * kBN + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2); };
     auto matrix_phase = [&](auto with_pv, auto with_s, int st, bool do_s = true, int next_tile = 0) __attribute__((always_inline)) {
         constexpr int pv = decltype(with_pv)::value ? kPvSteps : 0;
         constexpr int total = pv + (decltype(with_s)::value ? kSteps : 0);
@@ -404,11 +402,12 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                 }
             }
             if constexpr (kEarlyBits && pv > 0) {
-                constexpr int per_step = (20 + total - 1) / total;
+                constexpr int left = 10 - DropoutRows::kFirstRound;  // rounds of a block behind its start
+                constexpr int per_step = (2 * left + total - 1) / total;
 #pragma unroll
-                for (int n = s * per_step; n < (s + 1) * per_step && n < 20; ++n) {
-                    if (n % 10 == 0) bits[n / 10] = start_bits(n / 10, next_tile);
-                    philox_round(bits[n / 10], n % 10, p.seed_lo, p.seed_hi);
+                for (int n = s * per_step; n < (s + 1) * per_step && n < 2 * left; ++n) {
+                    if (n % left == 0) bits[n / left] = drop.start(block_column(n / left, next_tile));
+                    philox_round(bits[n / left], DropoutRows::kFirstRound + n % left, p.seed_lo, p.seed_hi);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -429,6 +428,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
 #pragma unroll
     for (int db = 0; db < DB; ++db) oacc[db] = zero16();
     lacc = zero16();
+    if constexpr (DROPOUT) drop.init(p, bh, qrow >> 2);
     m = -INFINITY;
     m_use = 0.f;
     l = 0.f;
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
         matrix_phase(No{}, Yes{}, kStages - 1);
         if constexpr (kEarlyBits) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) bits[kb] = dropout_block(p, bh, qrow >> 2, (key0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
+            for (int kb = 0; kb < 2; ++kb) bits[kb] = drop.block(p, block_column(kb, 0));
         }
         take_mask_block(0, true, false);
     }
@@ -574,9 +574,9 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
                     // group g of key block kb: keys t0 + 32 kb + 8 g + 4 h .. +3; this lane generates g = lane % 4
                     Philox4 mine;
                     if constexpr (kEarlyBits) mine = bits[kb];
-                    else mine = dropout_block(p, bh, qrow >> 2, (t0 + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2);
+                    else mine = drop.block(p, block_column(kb, j));
                     uint32_t w[4];
-                    quad_row_words(mine, lane, w);
+                    DropoutRows::words(mine, w);
 #pragma unroll
                     for (int g = 0; g < 4; ++g)
 #pragma unroll
