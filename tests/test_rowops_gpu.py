@@ -104,6 +104,30 @@ def test_softmax_of_rows_off_the_16_byte_boundaries(x_size, offset, dtype, devic
     parity.close(grad, rowops.softmax_backward(parity.to64(out), parity.to64(tg), 1), dtype, f"rows {x_size} + {offset} grad")
 
 
+# Pieces of a row on the edges of what a thread holds: the last piece falls to thread 0 again (129, 513, 2049, 4097, 20481 + the shift), a row
+# is two pieces or one more than the threads; the tensor ends inside a piece or on its boundary.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("rows", [5, 8])
+@pytest.mark.parametrize("x_size", [65, 129, 130, 257, 259, 511, 513, 633, 1027, 2049, 2050, 2555, 4097, 4099, 20483])
+def test_rows_keep_to_their_own_elements(x_size, rows, masked, dtype, device):
+    """Rows that share 16-byte pieces with their neighbours: every other row is nothing but NaN and infinities (in the gradient, too), which
+    the rows between them must neither read as theirs nor overwrite."""
+    x, g = _pair((rows, x_size), 4000 + x_size + rows, dtype)
+    mask = _build_mask((rows, x_size), x_size).to(torch.uint8) if masked else None
+    if masked:
+        mask[:, -1] = mask[:, 0] = 0
+    clean = slice(0, rows, 2)
+    x[1::2], g[1::2] = float("nan"), float("inf")
+    tx = x.to(device).requires_grad_(True)
+    out = trident.function.masked_softmax(tx, mask.to(device), 1) if masked else trident.function.softmax(tx, 1)
+    (grad,) = torch.autograd.grad(out, tx, g.to(device))
+    want = rowops.softmax_forward(parity.to64(x[clean]), 1, mask[clean].numpy() if masked else None)
+    parity.close(out[clean], want, dtype, "out")
+    parity.close(grad[clean], rowops.softmax_backward(parity.to64(out[clean]), parity.to64(g[clean]), 1), dtype, "grad")
+    assert out[1::2].isnan().all() and grad[1::2].isnan().all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("mask_dtype", [torch.uint8, torch.float16, torch.int64])
 @pytest.mark.parametrize("x_size", [8, 63, 64, 65, 97, 256, 257, 512, 1000, 1001, 1024, 1025])

@@ -114,6 +114,23 @@ struct Piece {
         uint32_t& word = w[sizeof(T) == 4 ? e : e >> 1];
         word = (word & ~half) | (bits(x) & half);
     }
+    // elements outside [lo, hi): x
+    __device__ __forceinline__ void trim(int lo, int hi, float x) {
+        const uint32_t b = bits(x);
+        constexpr int kPer = sizeof(T) == 4 ? 1 : 2;  // elements of a word
+#pragma unroll
+        for (int i = 0; i < kWords; ++i) {
+            uint32_t keep = i * kPer >= lo && i * kPer < hi ? (kPer == 1 ? 0xffffffffu : 0xffffu) : 0u;
+            if constexpr (kPer == 2) keep |= i * kPer + 1 >= lo && i * kPer + 1 < hi ? 0xffff0000u : 0u;
+            w[i] = (w[i] & keep) | (b & ~keep);
+        }
+    }
+    // element e (not known to the compiler) := the element whose bits() are b, as far as it lies in word i
+    __device__ __forceinline__ void put(int i, int e, uint32_t b) {
+        constexpr int kPer = sizeof(T) == 4 ? 1 : 2;
+        const uint32_t half = kPer == 1 ? 0xffffffffu : 0xffffu << (16 * (e & 1));
+        w[i] = e / kPer == i ? (w[i] & ~half) | (b & half) : w[i];
+    }
     // converted anew by the next reader: values kept across would take twice the registers of the words
     __device__ __forceinline__ void hide() {
 #pragma unroll
@@ -187,8 +204,11 @@ private:
 // time, all loaded together. A row of up to G * V * kHeld elements stays in registers between the statistics and the
 // output; a longer one takes two sweeps, the second of which finds the row in the L2 it was just read through.
 // SHIFT: rows that do not start on 16-byte boundaries (an odd row length): the pieces are those of the tensor, not of the
-// row, and only a row's first and last piece, which it shares with its neighbours, are read and written element by
-// element. Launches in a row, bf16 12288 x 2047 with a uint8 mask: forward 0.0336 ms = 3.7 TB/s, backward 0.0333 ms = 4.5 TB/s; with one element
+// row. A row's first and last piece, which it shares with its neighbours, are read whole, too, and trimmed in registers, so that all
+// of a thread's loads are in flight before the first is looked at; only what lies behind the tensor's last whole piece is read element by
+// element, and the two pieces are written so. (Read element by element, a branch each, they held up the loads behind them and were
+// most of the vector work. Launches in a row, us, bf16 12288 x 2047 with a uint8 mask: forward 37 -> 27 = 4.6 TB/s, backward 33 -> 26; fp16
+// 17740 x 2589 with the mask 113 -> 73, backward 86 -> 62; bf16 65536 x 197 24 -> 18; fp32 23855 x 477, backward, 28 -> 24.) One element
 // per load, which still serves short odd rows and tensors that are not 16-byte aligned themselves, 0.0545 and 0.0493 ms. Rows on 16-byte
 // boundaries: bf16 65536 x 64 forward 0.0092 ms (a wave per row, most of it idle: 0.0265), fp32 8192 x 1536 backward 0.0226
 // (two sweeps: 0.0362), bf16 16384 x 8192 forward 0.1027 (5.2 TB/s), with the mask 0.134 (one mask byte per load: 0.139).
@@ -201,63 +221,113 @@ struct RowPlace {
     int64_t at0;      // element offset of the row's piece 0
     int shift;        // where in piece 0 the row starts
     int64_t pieces;   // number of pieces of the row
+    int64_t readable; // pieces from the row's first on that end within the tensor
     int64_t x_size;
     __device__ __forceinline__ explicit RowPlace(const RowParams& p) : x_size(p.x_size) {
         t = threadIdx.x % G;
-        const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / G) + threadIdx.x / G;
+        // (a wave has one row from G == 64 on: what follows from its number stays in scalar registers)
+        const int in_group = threadIdx.x / G;
+        const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / G) + (G >= 64 ? __builtin_amdgcn_readfirstlane(in_group) : in_group);
         live = row < p.y_size;  // (G == 256: always)
         at0 = (live ? row : 0) * p.y_stride;
         shift = SHIFT ? static_cast<int>(at0 % V) : 0;
         at0 -= shift;
         pieces = live ? (x_size + shift + V - 1) / V : 0;
+        readable = ((p.y_size - 1) * p.y_stride + x_size - at0) / V;
     }
-    // the row's elements [lo, hi) of piece i (V > 1 without SHIFT: always the whole piece)
-    __device__ __forceinline__ void range(int64_t i, int* lo, int* hi) const {
-        const int64_t end = x_size + shift - i * V;
-        *lo = i == 0 ? shift : 0;
-        *hi = end < V ? static_cast<int>(end) : V;
+    // G pieces of the row from piece `first` on, one per thread.
+    struct Step {
+        int64_t at;     // element offset of the first one
+        bool head;      // it is the row's first piece
+        int count, end; // how many pieces there are of the row, and the number of the row's elements from `at` on
+        int readable;   // how many end within the tensor
+    };
+    static __device__ __forceinline__ int bounded(int64_t x) { return static_cast<int>(min(x, static_cast<int64_t>(1) << 20)); }
+    __device__ __forceinline__ Step step(int64_t first) const {
+        return Step{at0 + first * V, first == 0, bounded(pieces - first), bounded(live ? x_size + shift - first * V : 0), bounded(readable - first)};
     }
-    __device__ __forceinline__ bool whole(int64_t i) const { return !SHIFT || ((i > 0 || shift == 0) && (i + 1) * V <= x_size + shift); }
-    __device__ __forceinline__ Piece<T, V> load(const T* base, int64_t i, float outside) const {
-        Piece<T, V> r;
-        const T* from = base + at0 + i * V;
-        if (whole(i)) {
-            r.load(from);
-        } else {
+    // the row's elements [lo, hi) of this thread's piece (V > 1 without SHIFT: always the whole piece); hi < 1: it is not a piece of the row
+    __device__ __forceinline__ void range(const Step& s, int* lo, int* hi) const {
+        *lo = s.head && t == 0 ? shift : 0;
+        *hi = min(s.end - t * V, V);
+    }
+    __device__ __forceinline__ bool whole(const Step& s) const { return !SHIFT || (!(s.head && t == 0 && shift != 0) && (t + 1) * V <= s.end); }
+    // where this thread reads its piece: with SHIFT one that ends within the tensor, whatever it is
+    __device__ __forceinline__ int read_at(const Step& s) const { return (SHIFT ? min(t, s.readable - 1) : t) * V; }
+    // Pieces c0 + k * G + t of the row. All of them are requested before the first is looked at. With SHIFT a row's first and last
+    // piece come whole, with their neighbours' elements, and are trimmed in registers (trim); only a piece behind the last one that ends
+    // within the tensor is read element by element. (Pieces whose number is beyond every thread's share are skipped by a branch the
+    // whole row takes.)
+    __device__ __forceinline__ void load(const T* base, const Step& s, Piece<T, V>& held, float outside) const {
+        if (SHIFT ? s.count > 0 : t < s.count) held.load(base + s.at + read_at(s));
+        else held.fill(outside);
+    }
+    // (once all loads are on their way; element(offset): the value of one element)
+    template <typename Element>
+    __device__ __forceinline__ void trim(const Step& s, Piece<T, V>& held, float outside, Element element) const {
+        if constexpr (SHIFT) {
+            if (s.count <= 0 || whole(s)) return;
             int lo, hi;
-            range(i, &lo, &hi);
-            r.fill(outside);
+            range(s, &lo, &hi);
+            asm volatile("" : "+v"(lo), "+v"(hi));  // (comparisons made where they are needed, not kept as lane masks)
+            held.trim(lo, hi, outside);
+            if (t >= s.readable && t < s.count) {
+#pragma unroll 1
+                for (int e = lo; e < hi; ++e) {
+                    const uint32_t b = Piece<T, V>::bits(element(s.at + t * V + e));
 #pragma unroll
-            for (int e = 0; e < V; ++e)
-                if (e >= lo && e < hi) r.set(e, to_f32(from[e]));
+                    for (int w = 0; w < Piece<T, V>::kWords; ++w) held.put(w, e, b);
+                }
+            }
         }
-        return r;
     }
+    // The mask's piece beside one. (What it says of elements that are not the row's does not matter: they are trimmed behind it.)
     template <typename M, bool PIECES>
-    __device__ __forceinline__ MaskPiece<M, V> mask(const void* base, int64_t i) const {
-        MaskPiece<M, V> r;
-        const int64_t at = at0 + i * V;
-        if (whole(i)) {
-            if constexpr (PIECES) r.load(base, at);
-            else r.load(base, at, 0, V);
+    __device__ __forceinline__ void mask(const void* base, const Step& s, MaskPiece<M, V>& r) const {
+        if constexpr (PIECES) {
+            r.load(base, s.at + read_at(s));
         } else {
-            int lo, hi;
-            range(i, &lo, &hi);
-            r.load(base, at, lo, hi);
+            int lo = 0, hi = V;
+            if (!whole(s)) range(s, &lo, &hi);
+            r.load(base, s.at + t * V, lo, hi);
         }
-        return r;
     }
-    __device__ __forceinline__ void store(T* base, int64_t i, const Vec<T, V>& v) const {
-        T* to = base + at0 + i * V;
-        if (whole(i)) {
-            *reinterpret_cast<Vec<T, V>*>(to) = v;
-        } else {
-            int lo, hi;
-            range(i, &lo, &hi);
+    // Output of the held pieces c0 + k * G + t, value(k, e) each: whole pieces at once; a row's first and last, of which a thread has at most
+    // one unless the last falls to thread 0, element by element in one pass behind the others.
+    template <int N, typename Value>
+    __device__ __forceinline__ void store(T* base, int64_t c0, Value value) const {
+        [[maybe_unused]] Vec<T, V> rest;
+        [[maybe_unused]] int lo = 0, hi = 0;
+        [[maybe_unused]] T* rest_to = base;
+        [[maybe_unused]] auto store_rest = [&]() {
+            if (lo < hi) {
 #pragma unroll
-            for (int e = 0; e < V; ++e)
-                if (e >= lo && e < hi) to[e] = v.e[e];
+                for (int e = 0; e < V; ++e)
+                    if (e >= lo && e < hi) rest_to[e] = rest.e[e];
+                hi = 0;
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const Step s = step(c0 + k * G);
+            if (t < s.count) {
+                Vec<T, V> v;
+#pragma unroll
+                for (int e = 0; e < V; ++e) v.e[e] = from_f32<T>(value(k, e));
+                T* to = base + s.at + t * V;
+                if (whole(s)) {
+                    *reinterpret_cast<Vec<T, V>*>(to) = v;
+                } else if constexpr (SHIFT) {
+                    range(s, &lo, &hi);
+                    rest = v;
+                    rest_to = to;
+                }
+            }
+            if constexpr (SHIFT) {
+                if (k == 0 && (pieces - 1) % G == 0) store_rest();
+            }
         }
+        if constexpr (SHIFT) store_rest();
     }
 };
 
@@ -314,25 +384,23 @@ __global__ __launch_bounds__(256) void softmax_fwd_rows_kernel(const RowParams p
     const T* in = static_cast<const T*>(p.input);
     T* out = static_cast<T*>(p.output);
     Piece<T, V> held[kHeld];
-    // (pieces whose number is beyond every thread's share are skipped by a branch the whole row takes)
     auto load = [&](int64_t c0) {  // masked elements and those that are not the row's: -inf
 #pragma unroll
-        for (int k = 0; k < kHeld; ++k) {
-            const int64_t i = c0 + k * G + row.t;
-            if (i < row.pieces) held[k] = row.load(in, i, -INFINITY);
-            else held[k].fill(-INFINITY);
-        }
+        for (int k = 0; k < kHeld; ++k) row.load(in, row.step(c0 + k * G), held[k], -INFINITY);
         if constexpr (!std::is_same<M, void>::value) {
             MaskPiece<M, V> masks[kHeld];
 #pragma unroll
             for (int k = 0; k < kHeld; ++k) {
-                const int64_t i = c0 + k * G + row.t;
-                if (i < row.pieces) masks[k] = row.template mask<M, PIECES>(p.mask, i);
+                const auto step = row.step(c0 + k * G);
+                if (row.t < step.count) row.template mask<M, PIECES>(p.mask, step, masks[k]);
             }
 #pragma unroll
             for (int k = 0; k < kHeld; ++k)
-                if (c0 + k * G + row.t < row.pieces) masks[k].apply(held[k]);
+                if (row.t < row.step(c0 + k * G).count) masks[k].apply(held[k]);
         }
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k)
+            row.trim(row.step(c0 + k * G), held[k], -INFINITY, [&](int64_t at) { return mask_hit<M>(p.mask, at) ? -INFINITY : to_f32(in[at]); });
     };
     Stat s{-INFINITY, 0.f};
     int64_t last = 0;
@@ -378,16 +446,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_rows_kernel(const RowParams p
     // like the other 0.0130 before masks went as they do now; fp32 4096 x 8192 0.0575 -> 0.0488)
     for (int64_t c0 = kOnce ? 0 : last; c0 >= 0; c0 -= G * kHeld) {
         if (!kOnce && c0 != last) load(c0);
-#pragma unroll
-        for (int k = 0; k < kHeld; ++k) {
-            const int64_t i = c0 + k * G + row.t;
-            if (i < row.pieces) {
-                Vec<T, V> o;
-#pragma unroll
-                for (int e = 0; e < V; ++e) o.e[e] = from_f32<T>(fast_exp2(fmaf(held[k].get(e), kLog2e, -ms)) * inv);
-                row.store(out, i, o);
-            }
-        }
+        row.template store<kHeld>(out, c0, [&](int k, int e) { return fast_exp2(fmaf(held[k].get(e), kLog2e, -ms)) * inv; });
     }
 }
 
@@ -404,14 +463,19 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
     auto load = [&](int64_t c0) {
 #pragma unroll
         for (int k = 0; k < kHeld; ++k) {
-            const int64_t i = c0 + k * G + row.t;
-            if (i < row.pieces) {
-                held_o[k] = row.load(o, i, 0.f);
-                held_g[k] = row.load(g, i, 0.f);
+            const auto step = row.step(c0 + k * G);
+            if (SHIFT ? step.count > 0 : row.t < step.count) {  // (one branch for both)
+                held_o[k].load(o + step.at + row.read_at(step));
+                held_g[k].load(g + step.at + row.read_at(step));
             } else {
                 held_o[k].fill(0.f);
                 held_g[k].fill(0.f);
             }
+        }
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            row.trim(row.step(c0 + k * G), held_o[k], 0.f, [&](int64_t at) { return to_f32(o[at]); });
+            row.trim(row.step(c0 + k * G), held_g[k], 0.f, [&](int64_t at) { return to_f32(g[at]); });
         }
     };
     float delta = 0.f;
@@ -424,6 +488,8 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
             if (c0 + k * G < row.pieces) {
 #pragma unroll
                 for (int e = 0; e < V; ++e) delta = fmaf(held_o[k].get(e), held_g[k].get(e), delta);
+                held_o[k].hide();
+                held_g[k].hide();
             }
     }
 #pragma unroll
@@ -436,16 +502,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_rows_kernel(const RowParams p
     // the other way round, as in the forward (fp32 4096 x 8192 0.0964 -> 0.0774 ms, bf16 1024 x 12288 0.0186 -> 0.0154)
     for (int64_t c0 = kOnce ? 0 : last; c0 >= 0; c0 -= G * kHeld) {
         if (!kOnce && c0 != last) load(c0);
-#pragma unroll
-        for (int k = 0; k < kHeld; ++k) {
-            const int64_t i = c0 + k * G + row.t;
-            if (i < row.pieces) {
-                Vec<T, V> r;
-#pragma unroll
-                for (int e = 0; e < V; ++e) r.e[e] = from_f32<T>(held_o[k].get(e) * (held_g[k].get(e) - delta));
-                row.store(gi, i, r);
-            }
-        }
+        row.template store<kHeld>(gi, c0, [&](int k, int e) { return held_o[k].get(e) * (held_g[k].get(e) - delta); });
     }
 }
 
@@ -1045,12 +1102,11 @@ int launch_rows(const RowParams& p, bool base16, bool backward, Launch launch) {
         else if (worst <= (decltype(v)::value == 1 ? 1024 : 64 * held)) launch(v, integral_constant<int, 64>{}, shift);
         else launch(v, integral_constant<int, 256>{}, shift);
     };
-    // 16-byte accesses when the tensors start on 16-byte boundaries; shifted ones when the rows do not, but for short rows,
-    // which are little more than their first and last pieces (bf16, 16.7 M elements, shifted -> element by element: 17 per row
-    // forward 0.148 -> 0.061 ms, backward 0.161 -> 0.043; 63: 0.045 -> 0.024 and 0.050 -> 0.020; forward at 65 0.044 -> 0.074).
-    // The backward, with two inputs to read so, turns later: bf16 255 0.030 -> 0.021, 511 0.027 -> 0.022, 1001 0.024 -> 0.029;
-    // fp32 65 0.043 -> 0.049, 255 0.037 -> 0.031, 257 0.033 -> 0.039.
-    const bool by_element = p.x_size <= 64 || (backward && p.x_size > 96 && p.x_size <= (sizeof(T) == 2 ? 512 : 256));
+    // 16-byte accesses when the tensors start on 16-byte boundaries; shifted ones when the rows do not, but for short rows, of which
+    // one element per load is less work (16.7 M elements, us, shifted and by elements: forward bf16 33 per row 72 and 43, 49 49 and 32, 65
+    // 38 and 76, 255 20 and 25; fp32 49 43 and 34, 65 42 and 76. Backward bf16 49 42 and 23, 65 34 and 51, 197 19.6 and 20.8, 255 20.5 and 19.3;
+    // fp32 49 38 and 39, 65 40 and 59, 110 34 and 39, 150 36 and 33, 197 37 and 32, 255 37 and 33, 301 36 and 42).
+    const bool by_element = p.x_size <= 64 || (backward && sizeof(T) == 4 && p.x_size > 128 && p.x_size <= 256);
     if (!base16) with_group(One{}, No{});
     else if (p.x_size % kV == 0 && p.y_stride % kV == 0) with_group(Full{}, No{});
     else if (by_element) with_group(One{}, No{});
