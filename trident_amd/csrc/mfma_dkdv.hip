@@ -5,14 +5,6 @@
 namespace tri {
 namespace {
 
-template <typename T, int D, int NW, bool CAUSAL, int MASK>
-int launch_dkdv_waves(const KParams& p, hipStream_t stream) {
-    const dim3 grid(p.B * p.H * (p.S / (32 * NW))), block(64 * NW);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
-    return static_cast<int>(hipGetLastError());
-}
-
 // D = 128 without a mask, S no multiple of 128: 32 keys per wave instead of the phased pairs where the rows are one tile, which
 // the pairs pad to four blocks: time over theirs 0.75-0.91, with dropout 0.68-0.81 (S = 65: 1.01-1.19).
 bool dkdv_runs_four_waves(const KParams& p) { return p.S <= 64; }
@@ -24,8 +16,8 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
         if constexpr (MASK == kNoMask) {
             if (D < 128 || dkdv_runs_four_waves(p)) {
                 const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
-                else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
+                if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, kNoMask, true, true>), grid, block, 0, stream, p);
+                else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, kNoMask, false, true>), grid, block, 0, stream, p);
                 return static_cast<int>(hipGetLastError());
             }
             if constexpr (D == 128) {
@@ -45,32 +37,25 @@ int launch_dkdv_dropout(const KParams& p, hipStream_t stream) {
                 return static_cast<int>(hipGetLastError());
             }
         }
-        // a padded mask: at D = 64 beside an fp32 one's regions one workgroup of 8 waves per CU; beside a 16-bit one's the LDS holds two
-        // of 4 with a ring of three, whose 128 keys end closer to the sequence's end and wait at barriers of their own (fp16 B=16 H=12
-        // S=777 with key padding, forward and backward, 248 -> 218 us). 4 waves with the whole register file at D = 128
+        // a padded mask: 4 waves, of which two workgroups share a CU at D = 64 (time over that of one of 8 waves: beside a 16-bit mask 0.88 of
+        // a training step, beside an fp32 one 0.76-0.98), but for dropout, beside which it takes the whole register file, as at D = 128
         if constexpr (MASK != kNoMask) {
-            // (dropout beside mask and boundary handling does not fit 256 registers: four waves)
-            constexpr int NW = D == 64 && MASK == kMaskF32 ? 8 : 4;
-            const int nw = p.thr8 > 0 ? 4 : NW;
-            const dim3 grid(p.B * p.H * ((p.S + 32 * nw - 1) / (32 * nw))), block(64 * nw);
-            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, false, MASK, true, true>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, NW, false, MASK, false, true>), grid, block, 0, stream, p);
+            const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
+            if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, false, MASK, true, true>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, false, MASK, false, true>), grid, block, 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
         return TRI_ATTN_ESHAPE;
     }
     if constexpr (D <= 64) {
-        // the two-waves-per-SIMD kernel fits its registers: 8 waves (256 keys) when the sequence
-        // allows it, else 4 waves (128 keys)
-        if constexpr (D > 16) {
-            // (beside a 16-bit mask two workgroups of 4 fit a CU, as above, and are faster wherever those of 8 leave CUs idle in
-            // their last round: bf16 training steps at D = 64, heads x S, 96 x 512 93.6 -> 91.9 us, 96 x 768 180 -> 167; in whole
-            // rounds 64 x 1024 127.5 either way against 128.3. 192 x 640, one of 4 before, 199 -> 161)
-            const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256);
-            const bool pairs = D == 64 && MASK == kMaskT && p.thr8 <= 0 && items % persistent_grid(1 << 20) != 0;
-            if (p.S % 256 == 0 && !pairs) return launch_dkdv_waves<T, D, 8, CAUSAL, MASK>(p, stream);
-        }
-        return launch_dkdv_waves<T, D, 4, CAUSAL, MASK>(p, stream);
+        // 128 keys to a workgroup of four waves; two and more share a CU. One of eight waves, which every wave of a SIMD's pair waits for at
+        // its barriers and whose 256 keys leave more CUs idle in the last round, takes (time of the four over its): without a mask 0.74-0.77 at
+        // half as many items of 256 keys as CUs, 0.82-1.07 at as many, 0.94-1.03 beyond; with dropout 0.68-1.00; beside masks 0.88-0.98, few items 0.73;
+        // D = 32 0.85-0.95.
+        const dim3 grid(p.B * p.H * (p.S / 128)), block(256);
+        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, MASK, false>), grid, block, 0, stream, p);
+        return static_cast<int>(hipGetLastError());
     } else {
         // D = 128: K, V and both gradient accumulators of a 32-key block take 192 registers, too many
         // for two waves per SIMD, so two waves are paired on each key block of a 128-key workgroup

@@ -25,10 +25,10 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
     else return static_cast<float>(static_cast<const T*>(mask)[off]);
 }
 
-// ------------------------------------------------------------------ dK, dV (8 waves)
+// ------------------------------------------------------------------ dK, dV (4 waves)
 // Same data flow as the dQ kernel with the roles of queries and keys exchanged: a workgroup of
-// NW waves owns 32*NW keys, one wave 32 of them with its K and V rows in registers (B operands)
-// and dK^T, dV^T in fp32 accumulators; two waves per SIMD. Q and dO stream as 64-row swizzled LDS
+// 4 waves owns 128 keys, one wave 32 of them with its K and V rows in registers (B operands)
+// and dK^T, dV^T in fp32 accumulators; two workgroups and more per CU. Q and dO stream as 64-row swizzled LDS
 // tiles (plus their lse and delta) in a ring of 4 filled by LDS-direct loads three tiles ahead.
 // Per 32-row query block: S = Q K^T and dP = dO V^T from row fragments, P and dS on the vector
 // ALU, dV^T += dO^T P and dK^T += Q^T dS with the transposed LDS reads of the same tiles.
@@ -36,13 +36,15 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // row index to S - 1, query rows >= S get probability 0 (they would otherwise add the last row once more), keys >= S
 // are not stored.
 // SPLIT (with RAGGED): a workgroup streams one part of its item's row tiles (split.hpp).
-template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
+template <typename T, int D, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
+__global__ __launch_bounds__(256, RAGGED && !(MASK != kNoMask && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
+    constexpr int NW = 4;
     constexpr int kKeys = 32 * NW;
-    // (a ring of three where it lets a second workgroup onto the CU beside the mask regions, as launch_dkdv_dropout says)
-    constexpr int kStages = MASK == kMaskT && D == 64 && NW == 4 && !DROPOUT ? 3 : 4;
+    // (a ring of three, or two beside an fp32 mask, where it lets a second workgroup onto the CU beside the mask regions, whose tiles hide what
+    // the shorter lead leaves of the loads' latency: launch_dkdv_dropout says what that gives)
+    constexpr int kStages = MASK != kNoMask && D == 64 && !(DROPOUT && RAGGED) ? (MASK == kMaskT ? 3 : 2) : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes + 2 * kBN * 4;  // Q tile, dO tile, lse, delta
     constexpr int KK = D / 16;
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(NW * 64, RAGGED && NW == 4 && !(MASK == kMaskT && D
         issue_mask(t_begin);
         issue_tile(t_begin);
     }
-    if (t_begin + 1 < n_tiles) issue_tile(t_begin + 1);
+    if (kAhead > 1 && t_begin + 1 < n_tiles) issue_tile(t_begin + 1);
     if (kAhead > 2 && t_begin + 2 < n_tiles) issue_tile(t_begin + 2);
     // (the K and V fragments were requested before the tiles, so both latencies overlap)
 #pragma unroll

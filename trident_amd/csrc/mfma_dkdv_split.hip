@@ -13,10 +13,9 @@ SplitShape dkdv_split_shape(const KParams& p) {
         const double us = split_work(p) * 1.35;
         return SplitShape{128, 1, 2, false, 20, us, us, split_gain(p)};
     }
-    const int waves = p.mask != nullptr && p.D == 64 && p.thr8 <= 0 ? 8 : 4;
-    const int slots = p.D == 128 || (p.D == 64 && p.mask != nullptr) ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 3;
+    const int slots = p.D == 128 || (p.D == 64 && p.mask != nullptr && p.thr8 > 0) ? 1 : p.D == 64 || p.mask != nullptr ? 2 : 3;
     const double us = split_work(p) * (p.D >= 64 ? 1.65 : p.D == 32 ? 1.22 : 1.05);
-    return SplitShape{32 * waves, slots, 2, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.58 : 0.52) * us, split_gain(p) - (p.D < 64 ? 0.04 : 0.0), split_unclassed(p)};
+    return SplitShape{128, slots, 2, false, 20, us, slots == 1 ? us : (p.D == 64 ? 0.58 : 0.52) * us, split_gain(p) - (p.D < 64 ? 0.04 : 0.0), split_unclassed(p)};
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>
@@ -30,9 +29,8 @@ int launch_dkdv_split(const KParams& p, hipStream_t stream) {
         }
     }
     if constexpr (D < 128 || MASK != kNoMask) {
-        constexpr int NW = D == 64 && MASK != kNoMask ? 8 : 4;
-        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, 4, CAUSAL, MASK, true, true, true>), grid, dim3(256), 0, stream, p);
-        else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, NW, CAUSAL, MASK, false, true, true>), grid, dim3(64 * NW), 0, stream, p);
+        if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, MASK, true, true, true>), grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dkdv_wide_kernel<T, D, CAUSAL, MASK, false, true, true>), grid, dim3(256), 0, stream, p);
     }
     return static_cast<int>(hipGetLastError());
 }

@@ -43,14 +43,21 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
 
 // whether the phased dQ kernel serves this problem (no mask, 256-row workgroups, D >= 64; with dropout at D = 128 it
 // fits its registers only under the causal mask, without boundary handling and with a fragment ring of 4). At D = 32 the
-// kernel above needs 96 registers, two of its workgroups share a CU, and that measured 27 % faster than the phased pairs.
+// kernel above needs 112 registers, and four of its workgroups that share a CU measured 27 % faster than the phased pairs.
+// At D = 64 with S a multiple of 256 only launches that fill the chip with 256-row workgroups several times over: time of two unphased
+// workgroups of four waves per CU over that of the phased one, at half as many items of 256 rows as CUs 0.80-0.90, at as many 1.03-1.09,
+// beyond 1.00-1.09 (causal 0.78-0.84, 0.83-0.95, and 0.97-1.07 from twice as many on); with dropout 0.69-0.98.
 // Lengths that are no multiple of 256: at D = 128 the phased kernel with boundary handling (against 4 unphased waves, bf16
 // causal, heads x S: 768 x 130 0.071 -> 0.044 ms, 768 x 450 0.216 -> 0.152, 136 x 1531 0.216 -> 0.145; 768 x 65 equal); at
 // D = 64 two 128-row workgroups share a CU, which is 5-30 % faster than the phased kernel up to S = 3000.
 template <int D, int MASK>
 bool dq_is_phased(const KParams& p) {
     if (MASK != kNoMask) return false;
-    return D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : D == 64 && p.S % 256 == 0;
+    if (D == 64) {
+        const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256), cus = persistent_grid(1 << 20);
+        return p.S % 256 == 0 && p.thr8 <= 0 && (p.causal ? items > cus : 2 * items > cus);
+    }
+    return D == 128 && (p.thr8 <= 0 || (p.causal && p.S % 256 == 0));
 }
 
 // D = 128 without a mask, S no multiple of 256: the unphased kernel in workgroups of four waves. One key tile (S <= 64) is over
@@ -91,7 +98,7 @@ int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
 template <typename T, int D, bool CAUSAL, bool RAGGED>
 int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
     const dim3 grid(p.B * p.H * ((p.S + 255) / 256)), block(512);
-    if constexpr (D == 64 || (CAUSAL && !RAGGED)) {
+    if constexpr (D == 128 && CAUSAL && !RAGGED) {
         if (p.thr8 > 0) {
             if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true, RAGGED>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, false, RAGGED>), grid, block, 0, stream, p);
@@ -118,16 +125,17 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
         }
     }
     if (with_delta && MASK != kNoMask && (D > 64 || p.dmask != nullptr)) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
-    // 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows)
-    if constexpr (D > 16) {  // (a D = 16 tile has four blocks in all: four waves)
+    // D = 128: 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows). Up to D = 64 always 4: several such workgroups
+    // share a CU (time over that of 8 waves at multiples of 256: D = 32 0.92-1.00; D = 64 beside 16-bit masks 0.90-1.02, beside fp32 ones with a
+    // ring of three 0.78-1.05, in most cases 0.95-0.98)
+    if constexpr (D == 128) {
         if (p.S % 256 == 0) return launch_dq_waves<T, D, 8, CAUSAL, MASK>(p, stream, with_delta);
     }
     if constexpr (D == 128 && MASK == kNoMask) return launch_dq_ragged<T, D, 8, CAUSAL>(p, stream, with_delta);  // (dropout)
     if (p.S % 128 == 0) return launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
     if constexpr (MASK == kNoMask && D < 128) return launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);  // any other length
-    // a padded mask: at D = 64 one workgroup of 8 waves per CU beside an fp32 mask's staging regions, two of 4 beside a 16-bit
-    // one's (as the forward); at D = 128 four waves with the whole register file (in 256 registers the kernel spills)
-    if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, D == 64 && MASK == kMaskF32 ? 8 : 4, CAUSAL, MASK>(p, stream, with_delta);
+    // a padded mask: four waves; at D = 128 with the whole register file (in 256 registers the kernel spills)
+    if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
     return TRI_ATTN_ESHAPE;
 }
 

@@ -51,7 +51,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
     static_assert(!DELTA || MASK == 0 || (D <= 64 && !DMASK), "delta on the way: no mask, or a small head without a mask gradient");
     using Tile = SwzTile<D>;
     constexpr int kRows = 32 * NW;
-    constexpr int kStages = 4;
+    constexpr int kStages = MASK == kMaskF32 && D == 64 && NW == 4 ? 3 : 4;
+    constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes;  // K tile, V tile
     constexpr int KK = D / 16;
     constexpr int DB = D >= 32 ? D / 32 : 1;  // (D = 16: one block of gradient columns, the upper 16 are not stored)
@@ -191,13 +192,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
                                               : static_cast<uint32_t>(MaskTile::src_off(blk, l, p.ms[2] * kMaskElt)), mask_lds + blk * 1024);
         }
     };
-    // issue order: mask 0, tiles 0 1 2, then per tile j: mask j+1, tile j+3
+    // issue order: mask 0, kAhead tiles, then per tile j: mask j+1, tile j+kAhead
     if (!SPLIT || n_tiles > 0) {
         issue_mask(0);
         issue_tile(0);
     }
     if (1 < n_tiles) issue_tile(1);
-    if (2 < n_tiles) issue_tile(2);
+    if (kAhead > 2 && 2 < n_tiles) issue_tile(2);
     // (the row fragments were requested before the tiles, so both latencies overlap)
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
@@ -241,10 +242,10 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
         // tile j has landed (up to two younger tiles may still be in flight) and is visible to all
         // waves; every wave is done with tile j-1, whose slot takes the load of tile j+3
         {
-            // with a staged mask, block j must have landed too: only tile j+2 was issued after it
-            // (tiles 1 and 2 for j = 0)
-            // (a block that is all zero was never requested: then the two youngest tiles are what may be in flight)
-            const int younger = kMaskViaLds && j > 0 && !mask_is_zero(j) ? min(1, max(0, n_tiles - 2 - j)) : min(2, n_tiles - 1 - j);
+            // with a staged mask, block j must have landed too: only tile j + kAhead - 1 was issued after it
+            // (the kAhead first tiles after the first block)
+            // (a block that is all zero was never requested: then the kAhead - 1 youngest tiles are what may be in flight)
+            const int younger = kMaskViaLds && j > 0 && !mask_is_zero(j) ? min(1, max(0, n_tiles - (kAhead - 1) - j)) : min(kAhead - 1, n_tiles - 1 - j);
             if (younger == 2) TRI_WAIT_VMCNT(2 * kBlocksPerWave);
             else if (younger == 1) TRI_WAIT_VMCNT(kBlocksPerWave);
             else TRI_WAIT_VMCNT(0);
@@ -269,7 +270,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
             }
             if (j + 1 < n_tiles) issue_mask(j + 1);
         }
-        if (j + 3 < n_tiles) issue_tile(j + 3);
+        if (j + kAhead < n_tiles) issue_tile(j + kAhead);
         if (j >= my_tiles) continue;
 
         const char* sK = smem + (j % kStages) * kStageBytes;

@@ -7,9 +7,8 @@ namespace {
 // Few heads: items split along the keys, in workgroups with boundary handling: at D = 128 without mask and dropout the phased
 // kernel, else the one above with as many waves as a ragged length has.
 SplitShape dq_split_shape(const KParams& p) {
-    const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
-    const int waves = (p.D == 128 && p.mask == nullptr && p.thr8 <= 0) || (p.D == 64 && f32_mask) ? 8 : 4;
-    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 || (p.D == 32 && p.mask != nullptr) ? 2 : p.mask != nullptr ? 3 : 4;
+    const int waves = p.D == 128 && p.mask == nullptr && p.thr8 <= 0 ? 8 : 4;
+    const int slots = p.D == 128 ? 1 : p.D == 64 || (p.D == 32 && p.mask != nullptr) ? 2 : p.mask != nullptr ? 3 : 4;
     // Beside a mask at D = 128 parts have four waves, one per SIMD, and take longer than they promise (bf16 key mask with dropout, 12
     // heads, S=1489, whole 45 us, split 59); whole launches of multiples of 256 have eight, half the items (8 heads, S=6400, 287 and 400).
     const int whole_rows = p.D == 128 && p.mask != nullptr && p.thr8 <= 0 && p.S % 256 == 0 ? 256 : 32 * waves;
@@ -20,7 +19,7 @@ SplitShape dq_split_shape(const KParams& p) {
 
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_split(const KParams& p, hipStream_t stream, bool with_delta) {
-    constexpr int NW = D == 64 && MASK == kMaskF32 ? 8 : 4;
+    constexpr int NW = 4;
     const dim3 grid = split_grid(p);
     if (MASK == kNoMask && !with_delta) return TRI_ATTN_ESHAPE;  // (dq_splits)
     if constexpr (D == 128 && MASK == kNoMask) {

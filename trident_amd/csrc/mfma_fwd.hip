@@ -35,8 +35,11 @@ int launch_fwd_dropout(const KParams& p, hipStream_t stream) {
     const int items = p.B * p.H * (p.S / (32 * NW));
     // (the kernel's kPersistent: one workgroup per CU walks the items)
     const dim3 grid(NW == 8 && MASK == kNoMask ? persistent_grid(items) : items), block(64 * NW);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
+    if (p.thr8 > 0) {
+        if constexpr (!(D == 64 && NW == 8)) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
+    }
     return static_cast<int>(hipGetLastError());
 }
 
@@ -63,13 +66,27 @@ bool fwd_runs_four_waves(const KParams& p) {
     return p.S > 128 && (whole ? !p.causal : p.S <= 512);
 }
 
+// D = 64, S a multiple of 256: eight waves in two opposite phases, one workgroup per CU, or two workgroups of four waves, whose starts and
+// ends pass behind one another's tiles and which leave less of the chip idle in the last round. Time of the four over that of the
+// eight: without a mask 0.82-0.86 at half as many items of 256 rows as CUs, 0.93-0.99 at as many, 0.99-1.03 beyond (causal 0.77-0.86, 0.88-0.91
+// and at twice as many 0.95-1.00, beyond 1.00-1.03); with dropout 0.70-0.99; beside 16-bit masks 0.90-1.01; beside fp32 ones, whose ring of three
+// lets two workgroups onto a CU, 0.88-0.96, length masks 0.84-1.00 (dense ones in whole rounds of S = 2048 1.04-1.06).
+bool fwd_runs_eight_waves(const KParams& p) {
+    const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256);
+    return p.mask == nullptr && p.thr8 <= 0 && items > (p.causal ? 2 : 1) * static_cast<int64_t>(persistent_grid(1 << 20));
+}
+
 template <typename T, int D>
 int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
-    // 8 waves (256 query rows) when the sequence allows it: two waves per SIMD out of phase. At D = 32 the vector ALU
+    // 8 waves (256 query rows) at D = 128 when the sequence allows it: two waves per SIMD out of phase. At D = 32 the vector ALU
     // is the busy unit and a workgroup's phases are short: four independent 4-wave workgroups per CU (the kernel then
     // fits 128 registers) measured 28 % faster than the 8-wave pairs.
-    if constexpr (D > 32) {
+    if constexpr (D == 128) {
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
+    }
+    if constexpr (D == 64) {
+        if (p.S % 256 == 0 && fwd_runs_eight_waves(p))
+            return p.causal ? launch_fwd_dropout<T, D, 8, true, kNoMask>(p, stream) : launch_fwd_dropout<T, D, 8, false, kNoMask>(p, stream);
     }
     // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
     // one workgroup per CU, so that four waves are one per SIMD. bf16 causal, heads x S: 768 x 130 0.057 -> 0.034 ms,
@@ -83,9 +100,9 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     }
     if (p.S % 128 == 0) return launch_fwd_variant<T, D, 4>(dtype, p, stream);
     if (p.mask != nullptr) {
-        // A padded mask: as many waves as share a CU's LDS with the mask's staging regions. At D = 64 an fp32 mask leaves room
-        // for one workgroup per CU (8 waves), a 16-bit one for two of 4 waves.
-        if (p.mask_dtype == TRI_ATTN_F32) return launch_fwd_ragged<T, D, D >= 64 ? 8 : 4, false, kMaskF32>(p, stream);
+        // A padded mask: at D = 64 two workgroups of 4 waves share a CU's LDS with the mask's staging regions (beside an fp32 mask one of 8
+        // waves was 1-19 % slower)
+        if (p.mask_dtype == TRI_ATTN_F32) return launch_fwd_ragged<T, D, D == 128 ? 8 : 4, false, kMaskF32>(p, stream);
         if (p.mask_dtype == dtype) return launch_fwd_ragged<T, D, D == 128 ? 8 : 4, false, kMaskT>(p, stream);
         return TRI_ATTN_EDTYPE;
     }

@@ -40,11 +40,12 @@ template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool R
 __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) void mfma_fwd_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
-    // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions. The ring then has
+    // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions, at D = 64 32 KiB of the 80 with which
+    // two workgroups of 4 waves share a CU. The ring then has
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
     // phase before V of tile t, so with K(j + dist) and V(j + dist - 1) requested together every tile keeps the lead
     // it has in the ring of four, and both fit three slots. The first fragments of V wait for the barrier, though.
-    constexpr bool kLeadK = D == 128 && MASK == 1 && NW == 8 && !DROPOUT;
+    constexpr bool kLeadK = MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4));
     constexpr int kStages = kLeadK ? 3 : 4;  // LDS ring depth
     constexpr int kLag = kLeadK ? 1 : 0;     // how many tiles the V requests trail the K requests
     constexpr int kBM = 32 * NW;
@@ -351,12 +352,12 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) voi
         constexpr int pv = decltype(with_pv)::value ? kPvSteps : 0;
         return s < pv ? v_frag(smem + st * kKBytes, s) : k_frag(smem + ((st + 1) % kStages) * kKBytes, s - pv);
     };
-    // With dropout the softmax phase, where the partner waits, is far longer than the matrix phase. The generator does not
-    // depend on the scores: its rounds for the next tile (two blocks of ten, each lane its share of the quad's) run between
-    // the MFMAs of the matrix phase, two per step, and the softmax phase starts from their result. D = 64 forward, B=1 H=32
-    // S=8192: 1.21 -> 1.13 ms, causal 0.61 -> 0.56. At D = 128 the same move changed nothing (0.69 ms causal either way: the
-    // matrix phase is as long there, and the clock gives under the power limit), so that the rounds stay where they are.
-    constexpr bool kEarlyBits = DROPOUT && kPingPong && D == 64;
+    // With dropout the softmax phase is far longer than the matrix phase. The generator does not
+    // depend on the scores: its rounds for the next tile (two blocks of ten, the first two of each folded) run between
+    // the MFMAs of the matrix phase, one or two per step, and the softmax phase starts from their result. D = 64, bf16 causal, heads x S: 16 x
+    // 1024 25.6 -> 22.4 us, 16 x 8192 245 -> 235, not causal 64 x 1024 35.7 -> 34.9. At D = 128 the same move changed nothing (0.69 ms causal
+    // either way: the matrix phase is as long there, and the clock gives under the power limit), so that the rounds stay where they are.
+    constexpr bool kEarlyBits = DROPOUT && D == 64 && MASK == kNoMask;
     Philox4 bits[kEarlyBits ? 2 : 1];  // of the next tile's two key blocks
     [[maybe_unused]] DropoutRows drop;
     auto block_column = [&](int kb, int t) { return static_cast<uint32_t>((key0 + t * kBN + 32 * kb + 8 * (lane & 3) + 4 * h) >> 2); };

@@ -8,7 +8,7 @@ namespace {
 // length, at D = 128 eight (four beside a mask and dropout, which need the whole register file).
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_fwd_split(const KParams& p, int waves, hipStream_t stream) {
-    constexpr int NW = D == 128 || (D == 64 && MASK == kMaskF32) ? 8 : 4;
+    constexpr int NW = D == 128 ? 8 : 4;
     const dim3 grid = split_grid(p);
     if (waves != NW) {
         if constexpr (D == 128 && MASK != kNoMask) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, 4, CAUSAL, MASK, true, true, true>), grid, dim3(256), 0, stream, p);
@@ -31,8 +31,8 @@ int launch_fwd_split_variant(int dtype, const KParams& p, int waves, hipStream_t
 
 SplitShape fwd_split_shape(const KParams& p) {
     const bool f32_mask = p.mask != nullptr && p.mask_dtype == TRI_ATTN_F32;
-    const int waves = p.D == 128 ? (p.mask != nullptr && p.thr8 > 0 ? 4 : 8) : p.D == 64 && f32_mask ? 8 : 4;
-    const int slots = p.D == 128 || waves == 8 ? 1 : p.D == 64 ? 2 : p.mask == nullptr ? 4 : p.thr8 > 0 || (f32_mask && p.D == 32) ? 2 : 3;
+    const int waves = p.D == 128 && !(p.mask != nullptr && p.thr8 > 0) ? 8 : 4;
+    const int slots = p.D == 128 ? 1 : p.D == 64 ? 2 : p.mask == nullptr ? 4 : p.thr8 > 0 || (f32_mask && p.D == 32) ? 2 : 3;
     // (beside mask and dropout at D = 128 whole launches of multiples of 256 have eight waves, half the items: bf16 fp32 mask, 10 heads,
     // S=4096, whole 90 us, split 213)
     const int whole_rows = p.D == 128 && waves == 4 && p.S % 256 == 0 ? 256 : 32 * waves;
