@@ -68,3 +68,27 @@ def test_four_and_eight_waves_agree(heads, causal, device):
         sums = parity.oracle_abs_sums(q[at], k[at], v[at], d_o[at], o=o[at], **kw)[1:]
         for name, got, want, total in zip(("dQ", "dK", "dV"), grads, ref, sums):
             parity.close(got[at], want, dtype, name, total)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("causal,heads,S", [(False, 1025, 64), (False, 513, 130), (False, 1025, 128), (False, 257, 512), (True, 513, 65), (True, 513, 128),
+                                            (True, 171, 321), (True, 129, 512), (True, 171, 384)])
+def test_launches_of_several_rounds(causal, heads, S, p, device):
+    """Just beyond the number of workgroups from which three of them share a CU, with a ring of three tiles: one to eight tiles, ragged ends,
+    first and last heads against the oracle."""
+    D, dtype, seed = 64, torch.bfloat16, 99
+    g = torch.Generator().manual_seed(heads + S)
+    q, k, v, d_o = [torch.randn(1, heads, S, D, generator=g).to(dtype) for _ in range(4)]
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    scale = 1.0 / math.sqrt(D)
+    o, lse = Attention._forward(tq, tk, tv, None, p, causal, scale, seed, 0)
+    grads = Attention._backward(tdo, tq, tk, tv, o, lse, None, scale, p, causal, seed, 0, False)[:3]
+    assert all(x.isfinite().all() for x in (o, *grads))
+    for h in [0] + ([heads - 1] if p == 0.0 else []):  # (decisions depend on the head's number: the oracle counts from 0)
+        at = (slice(0, 1), slice(h, h + 1))
+        kw = dict(mask=None, dropout_p=p, is_causal=causal, scale=scale, seed=seed, offset=0)
+        parity.close(o[at], parity.oracle_forward(q[at], k[at], v[at], **kw)[0], dtype, "O")
+        ref = parity.oracle_backward(q[at], k[at], v[at], d_o[at], o=o[at], **kw)[:3]
+        sums = parity.oracle_abs_sums(q[at], k[at], v[at], d_o[at], o=o[at], **kw)[1:]
+        for name, got, want, total in zip(("dQ", "dK", "dV"), grads, ref, sums):
+            parity.close(got[at], want, dtype, name, total)

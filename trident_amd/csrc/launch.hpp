@@ -52,5 +52,11 @@ int persistent_grid(int items);
 // as many again: the heaviest start first, and the light ones fill up behind them (bf16 with dropout, 288-384 workgroups,
 // S = 1025-2100: forward and dQ 0.85-0.91 of the time of 256-row ones; 384 at S = 300: 1.27).
 bool four_waves_fit_one_round(const KParams& p);
+// Whether forward and dQ at D = 64 without a mask run their 128-row workgroups three to a CU (in 168 registers, with a ring of three tiles)
+// instead of two: launches of several rounds. Time of three over that of two, or of the eight-wave kernels that ran before, by the number
+// of workgroups: up to two per CU forward 0.97-1.06, dQ 0.97-1.09; causal at 3.4 to 4 per CU forward 0.93-0.98 (16 heads of S = 8192: 1.03),
+// dQ 0.81-0.98, at 5.5 to 16 forward 0.88-0.92, dQ 0.88-0.93; not causal at 3.4 to 4 forward 0.96-1.09, dQ 0.98-1.06, from 5.5 on forward
+// 0.90-0.96, dQ 0.90-1.01.
+bool three_workgroups_per_cu(const KParams& p);
 
 }  // namespace tri

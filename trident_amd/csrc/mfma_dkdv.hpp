@@ -36,15 +36,17 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // row index to S - 1, query rows >= S get probability 0 (they would otherwise add the last row once more), keys >= S
 // are not stored.
 // SPLIT (with RAGGED): a workgroup streams one part of its item's row tiles (split.hpp).
+template <int D, int MASK, bool DROPOUT>
+constexpr bool kThree = D == 64 && MASK == kNoMask && !DROPOUT;
 template <typename T, int D, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, RAGGED && !(MASK != kNoMask && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
+__global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(MASK != kNoMask && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
     constexpr int NW = 4;
     constexpr int kKeys = 32 * NW;
     // (a ring of three, or two beside an fp32 mask, where it lets a second workgroup onto the CU beside the mask regions, whose tiles hide what
     // the shorter lead leaves of the loads' latency: launch_dkdv_dropout says what that gives)
-    constexpr int kStages = MASK != kNoMask && D == 64 && !(DROPOUT && RAGGED) ? (MASK == kMaskT ? 3 : 2) : 4;
+    constexpr int kStages = MASK != kNoMask && D == 64 && !(DROPOUT && RAGGED) ? (MASK == kMaskT ? 3 : 2) : kThree<D, MASK, DROPOUT> ? 3 : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes + 2 * kBN * 4;  // Q tile, dO tile, lse, delta
     constexpr int KK = D / 16;
@@ -216,8 +218,8 @@ __global__ __launch_bounds__(256, RAGGED && !(MASK != kNoMask && D == 64 && !DRO
 
     [[maybe_unused]] DropoutKeys drop;
     if constexpr (DROPOUT) drop.init(p, bh, key >> 2);
-    const int row_off0 = Tile::off(l32, h);
-    const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
+    int row_off0 = Tile::off(l32, h);
+    int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
     for (int j = t_begin; j < n_tiles; ++j) {
         {
@@ -254,6 +256,8 @@ __global__ __launch_bounds__(256, RAGGED && !(MASK != kNoMask && D == 64 && !DRO
         const float* sLse = reinterpret_cast<const float*>(sG + Tile::kBytes);
         const float* sDelta = sLse + kBN;
         const int r0 = j * kBN;
+        // (the fragments' offsets of the column blocks are made from these here, not kept in registers across the loop)
+        if constexpr (kThree<D, MASK, DROPOUT>) asm volatile("" : "+v"(row_off0), "+v"(tr_off0), "+v"(tr_off1));
         const bool diag = CAUSAL && r0 < wkey0 + 31;  // some row of the tile is above some key of the wave
 #pragma unroll 1
         for (int qb = 0; qb < 2; ++qb) {

@@ -6,8 +6,19 @@ namespace tri {
 namespace {
 
 // ---------------------------------------------------------------------------------- launch
+template <typename T, bool CAUSAL, bool RAGGED>
+int launch_dq_three(const KParams& p, hipStream_t stream) {  // (with delta)
+    const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, kNoMask, true, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, kNoMask, false, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
 template <typename T, int D, int NW, bool CAUSAL, int MASK>
 int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = false) {
+    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
+        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, false>(p, stream);
+    }
     const dim3 grid(p.B * p.H * (p.S / (32 * NW))), block(64 * NW);
     if constexpr (NW == 8 && D == 128 && MASK != kNoMask) {
         // with a mask gradient or dropout on top of a mask the 8-wave kernel does not fit its registers at D = 128 and
@@ -44,9 +55,9 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
 // whether the phased dQ kernel serves this problem (no mask, 256-row workgroups, D >= 64; with dropout at D = 128 it
 // fits its registers only under the causal mask, without boundary handling and with a fragment ring of 4). At D = 32 the
 // kernel above needs 112 registers, and four of its workgroups that share a CU measured 27 % faster than the phased pairs.
-// At D = 64 with S a multiple of 256 only launches that fill the chip with 256-row workgroups several times over: time of two unphased
-// workgroups of four waves per CU over that of the phased one, at half as many items of 256 rows as CUs 0.80-0.90, at as many 1.03-1.09,
-// beyond 1.00-1.09 (causal 0.78-0.84, 0.83-0.95, and 0.97-1.07 from twice as many on); with dropout 0.69-0.98.
+// At D = 64 with S a multiple of 256 only launches that fill the chip with 256-row workgroups, and not causal ones: time of
+// unphased workgroups of four waves, two or three to a CU, over that of the phased one, at half as many items of 256 rows as CUs 0.80-0.90, at
+// as many 1.03-1.09, beyond 0.90-1.06 (causal 0.78-0.84, 0.83-0.95 and 0.81-0.98); with dropout 0.69-0.98.
 // Lengths that are no multiple of 256: at D = 128 the phased kernel with boundary handling (against 4 unphased waves, bf16
 // causal, heads x S: 768 x 130 0.071 -> 0.044 ms, 768 x 450 0.216 -> 0.152, 136 x 1531 0.216 -> 0.145; 768 x 65 equal); at
 // D = 64 two 128-row workgroups share a CU, which is 5-30 % faster than the phased kernel up to S = 3000.
@@ -55,7 +66,7 @@ bool dq_is_phased(const KParams& p) {
     if (MASK != kNoMask) return false;
     if (D == 64) {
         const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256), cus = persistent_grid(1 << 20);
-        return p.S % 256 == 0 && p.thr8 <= 0 && (p.causal ? items > cus : 2 * items > cus);
+        return p.S % 256 == 0 && p.thr8 <= 0 && !p.causal && 2 * items > cus;
     }
     return D == 128 && (p.thr8 <= 0 || (p.causal && p.S % 256 == 0));
 }
@@ -71,6 +82,9 @@ bool dq_runs_four_waves(const KParams& p) {
 // any length (no mask, or a padded one), with boundary handling
 template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
+    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
+        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, true>(p, stream);
+    }
     const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
     if constexpr (MASK != kNoMask) {
         if constexpr (D <= 64) {
@@ -116,7 +130,7 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
         if (p.S % 256 != 0 && dq_runs_four_waves(p))
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
     }
-    if constexpr (MASK == kNoMask && D >= 64) {
+    if constexpr (MASK == kNoMask && (D == 128 || (D == 64 && !CAUSAL))) {
         if (dq_is_phased<D, MASK>(p)) {
             if constexpr (D == 128) {
                 if (p.S % 256 != 0) return launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);

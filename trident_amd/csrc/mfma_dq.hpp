@@ -42,16 +42,18 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from
 // key0; the first part stores delta. Parts beside a mask at D = 16 are held to 168 registers: at 169, with two workgroups per CU instead
 // of three, they took a quarter longer (bf16 key mask, 4 heads, S=10368, with the second launch: 77 -> 96 us).
+// THREE (D = 64, no mask, 4 waves): three workgroups to a CU instead of two (three_workgroups_per_cu).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool DMASK = false, bool DELTA = false,
-          bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 16 && SPLIT && MASK != kNoMask ? 3 : 2) void mfma_dq_kernel(const KParams p) {
+          bool SPLIT = false, bool THREE = false>
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE || D == 16 && SPLIT && MASK != kNoMask ? 3 : 2) void mfma_dq_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
+    static_assert(!THREE || (D == 64 && NW == 4 && MASK == 0 && !SPLIT), "three workgroups per CU");
     static_assert(!DELTA || MASK == 0 || (D <= 64 && !DMASK), "delta on the way: no mask, or a small head without a mask gradient");
     using Tile = SwzTile<D>;
     constexpr int kRows = 32 * NW;
-    constexpr int kStages = MASK == kMaskF32 && D == 64 && NW == 4 ? 3 : 4;
+    constexpr int kStages = THREE || (MASK == kMaskF32 && D == 64 && NW == 4) ? 3 : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes;  // K tile, V tile
     constexpr int KK = D / 16;
@@ -235,10 +237,12 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : D == 1
 
     [[maybe_unused]] DropoutRows drop;
     if constexpr (DROPOUT) drop.init(p, bh, qrow >> 2);
-    const int row_off0 = Tile::off(l32, h);
-    const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
+    int row_off0 = Tile::off(l32, h);
+    int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
     for (int j = 0; j < n_tiles; ++j) {
+        // (the fragments' offsets of the column blocks are made from these here, not kept in registers across the loop)
+        if constexpr (THREE) asm volatile("" : "+v"(row_off0), "+v"(tr_off0), "+v"(tr_off1));
         // tile j has landed (up to two younger tiles may still be in flight) and is visible to all
         // waves; every wave is done with tile j-1, whose slot takes the load of tile j+3
         {

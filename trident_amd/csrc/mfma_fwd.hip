@@ -5,6 +5,14 @@
 namespace tri {
 namespace {
 
+template <typename T, bool CAUSAL, bool RAGGED>
+int launch_fwd_three(const KParams& p, hipStream_t stream) {
+    const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, kNoMask, true, RAGGED, false, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, kNoMask, false, RAGGED, false, true>), grid, block, 0, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
 template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
     if constexpr (D == 128 && NW == 8 && MASK != kNoMask) {
@@ -12,6 +20,9 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
         if (p.thr8 > 0) return launch_fwd_ragged<T, D, 4, CAUSAL, MASK>(p, stream);
     }
     const int items = p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW));
+    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
+        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true>(p, stream);
+    }
     if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
         if (p.S % 128 == 0) {  // (causal only with dropout: fwd_runs_four_waves)
             if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), dim3(items), dim3(64 * NW), 0, stream, p);
@@ -32,14 +43,14 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
 
 template <typename T, int D, int NW, bool CAUSAL, int MASK>
 int launch_fwd_dropout(const KParams& p, hipStream_t stream) {
+    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
+        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, false>(p, stream);
+    }
     const int items = p.B * p.H * (p.S / (32 * NW));
     // (the kernel's kPersistent: one workgroup per CU walks the items)
     const dim3 grid(NW == 8 && MASK == kNoMask ? persistent_grid(items) : items), block(64 * NW);
-    if (p.thr8 > 0) {
-        if constexpr (!(D == 64 && NW == 8)) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
-    } else {
-        hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
-    }
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -66,27 +77,16 @@ bool fwd_runs_four_waves(const KParams& p) {
     return p.S > 128 && (whole ? !p.causal : p.S <= 512);
 }
 
-// D = 64, S a multiple of 256: eight waves in two opposite phases, one workgroup per CU, or two workgroups of four waves, whose starts and
-// ends pass behind one another's tiles and which leave less of the chip idle in the last round. Time of the four over that of the
-// eight: without a mask 0.82-0.86 at half as many items of 256 rows as CUs, 0.93-0.99 at as many, 0.99-1.03 beyond (causal 0.77-0.86, 0.88-0.91
-// and at twice as many 0.95-1.00, beyond 1.00-1.03); with dropout 0.70-0.99; beside 16-bit masks 0.90-1.01; beside fp32 ones, whose ring of three
-// lets two workgroups onto a CU, 0.88-0.96, length masks 0.84-1.00 (dense ones in whole rounds of S = 2048 1.04-1.06).
-bool fwd_runs_eight_waves(const KParams& p) {
-    const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256);
-    return p.mask == nullptr && p.thr8 <= 0 && items > (p.causal ? 2 : 1) * static_cast<int64_t>(persistent_grid(1 << 20));
-}
-
 template <typename T, int D>
 int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
-    // 8 waves (256 query rows) at D = 128 when the sequence allows it: two waves per SIMD out of phase. At D = 32 the vector ALU
-    // is the busy unit and a workgroup's phases are short: four independent 4-wave workgroups per CU (the kernel then
-    // fits 128 registers) measured 28 % faster than the 8-wave pairs.
+    // 8 waves (256 query rows) at D = 128 when the sequence allows it: two waves per SIMD out of phase. Up to D = 64 four waves everywhere,
+    // whose workgroups share a CU, so that starts and ends pass behind one another's tiles and less of the chip is idle in the last round. Time of
+    // the four over that of the eight at multiples of 256: D = 32 0.78; D = 64 without a mask 0.82-0.86 at half as many items of 256 rows as CUs,
+    // 0.93-0.99 at as many, 0.99-1.03 at twice as many (causal 0.77-0.86, 0.88-0.91 and 0.95-1.00), more than that: three_workgroups_per_cu; with
+    // dropout 0.70-0.99; beside 16-bit masks 0.90-1.01; beside fp32 ones, whose ring of three lets two workgroups onto a CU, 0.88-0.96, length
+    // masks 0.84-1.00 (dense ones in whole rounds of S = 2048 1.04-1.06).
     if constexpr (D == 128) {
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
-    }
-    if constexpr (D == 64) {
-        if (p.S % 256 == 0 && fwd_runs_eight_waves(p))
-            return p.causal ? launch_fwd_dropout<T, D, 8, true, kNoMask>(p, stream) : launch_fwd_dropout<T, D, 8, false, kNoMask>(p, stream);
     }
     // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
     // one workgroup per CU, so that four waves are one per SIMD. bf16 causal, heads x S: 768 x 130 0.057 -> 0.034 ms,

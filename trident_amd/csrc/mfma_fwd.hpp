@@ -36,16 +36,18 @@ enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
 // their row index to S - 1, the scores of keys >= S are set to -inf, and rows >= S are not stored. A wave without a
 // single row of its own only fetches its share of the tiles and meets the barriers.
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from key0.
-template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : 2) void mfma_fwd_kernel(const KParams p) {
+// THREE (D = 64, no mask, 4 waves): three workgroups to a CU instead of two (three_workgroups_per_cu).
+template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false, bool THREE = false>
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
+    static_assert(!THREE || (D == 64 && NW == 4 && MASK == 0 && !SPLIT), "three workgroups per CU");
     using Tile = SwzTile<D>;
     // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions, at D = 64 32 KiB of the 80 with which
-    // two workgroups of 4 waves share a CU. The ring then has
+    // two workgroups of 4 waves share a CU; three have 53 KiB each. The ring then has
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
     // phase before V of tile t, so with K(j + dist) and V(j + dist - 1) requested together every tile keeps the lead
     // it has in the ring of four, and both fit three slots. The first fragments of V wait for the barrier, though.
-    constexpr bool kLeadK = MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4));
+    constexpr bool kLeadK = THREE || (MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4)));
     constexpr int kStages = kLeadK ? 3 : 4;  // LDS ring depth
     constexpr int kLag = kLeadK ? 1 : 0;     // how many tiles the V requests trail the K requests
     constexpr int kBM = 32 * NW;

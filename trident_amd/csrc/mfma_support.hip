@@ -237,6 +237,11 @@ bool four_waves_fit_one_round(const KParams& p) {
     return persistent_grid(busy) == busy;
 }
 
+bool three_workgroups_per_cu(const KParams& p) {
+    const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
+    return p.D == 64 && p.mask == nullptr && items > (p.causal ? 2 : 4) * static_cast<int64_t>(persistent_grid(1 << 20));
+}
+
 int launch_delta(int dtype, const KParams& p, hipStream_t stream) {
     const bool vec = (dtype == TRI_ATTN_F16 || dtype == TRI_ATTN_BF16) && (p.D == 16 || p.D == 32 || p.D == 64 || p.D == 128) &&
                      aligned16(p.o) && aligned16(p.d_o) && strides8(p.os) && strides8(p.dos);
