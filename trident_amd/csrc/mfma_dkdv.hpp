@@ -226,7 +226,8 @@ __global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(M
             // with a staged mask, block j must have landed too: only tile j + kAhead - 1 was issued after it
             // (the kAhead first tiles after the first block)
             // (a block that is all zero was never requested: then the kAhead - 1 youngest tiles are what may be in flight)
-            const int younger = kMaskViaLds && j > t_begin && !mask_is_zero(j) ? min(1, max(0, n_tiles - (kAhead - 1) - j)) : min(kAhead - 1, n_tiles - 1 - j);
+            // (kAhead == 1: tile j itself was issued after its mask block, nothing may be in flight)
+            const int younger = kMaskViaLds && j > t_begin && !mask_is_zero(j) ? min(min(1, kAhead - 1), max(0, n_tiles - (kAhead - 1) - j)) : min(kAhead - 1, n_tiles - 1 - j);
             if (younger == 2) TRI_WAIT_VMCNT(2 * kLoadsPerTile);
             else if (younger == 1) TRI_WAIT_VMCNT(kLoadsPerTile);
             else TRI_WAIT_VMCNT(0);
