@@ -58,5 +58,8 @@ bool four_waves_fit_one_round(const KParams& p);
 // dQ 0.81-0.98, at 5.5 to 16 forward 0.88-0.92, dQ 0.88-0.93; not causal at 3.4 to 4 forward 0.96-1.09, dQ 0.98-1.06, from 5.5 on forward
 // 0.90-0.96, dQ 0.90-1.01.
 bool three_workgroups_per_cu(const KParams& p);
+// Whether the mask is one of keys (the same for every row) that is 0 or -inf, of the operand type and over few enough tiles for the kernels
+// that keep it as bits (KeyBits; at D = 128 without dropout).
+bool mask_is_key_bits(const KParams& p);
 
 }  // namespace tri

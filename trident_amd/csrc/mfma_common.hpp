@@ -302,7 +302,7 @@ __device__ __forceinline__ bool map_item(int bid, int grid, int round, int num_h
 
 template <int MASK>
 __device__ __forceinline__ void map_block_for(const KParams& p, int bid, int num_tiles, int order, int* bh, int* tile) {
-    if (MASK != 0 && p.ms[1] == 0 && p.H > 1) map_block_shared_mask(bid, p.B, p.H, num_tiles, bh, tile);
+    if ((MASK == 1 || MASK == 2) && p.ms[1] == 0 && p.H > 1) map_block_shared_mask(bid, p.B, p.H, num_tiles, bh, tile);
     else map_block(bid, p.B * p.H, num_tiles, order, bh, tile);
 }
 
@@ -328,6 +328,43 @@ __device__ __forceinline__ TileClasses tile_classes(const uint8_t* first, int64_
     r.active = __builtin_amdgcn_ballot_w64(lane < n && !all_ninf);
     return r;
 }
+
+// A mask of keys (the same for every row of a head) whose values are 0 or -inf, over up to 64 tiles: lane t keeps a bit per key of tile t (1:
+// visible), and the uniform masks say what the classes of a matrix's blocks say. A mask's row is read once, in 8 loads per wave, and no
+// tile has anything to stage: launches beside padding run as those without a mask, in their registers and LDS, and only a tile in which
+// some keys are visible and some are not selects. Kernel times, us, values staged in LDS -> so (forward, dQ, dK/dV; bf16, heads x S): D = 64 256 x
+// 1024 99, 119, 190 -> 83, 101, 153, 192 x 768 48, 58, 85 -> 40, 49, 69, with dropout 128 x 700 49, 50, 106 -> 46, 46, 71; D = 32 128 x 1024 36, 43, 68 ->
+// 30, 33, 43; D = 16 128 x 2048 96, 99, 172 -> 88, 88, 141; D = 128, whose dQ pass is the phased one so and computes delta, with the pre-pass 192 x
+// 777 512 -> 418 in all, 32 x 1300 215 -> 167, 192 x 384 161 -> 137.
+struct KeyBits {
+    uint32_t lo, hi;
+    TileClasses tiles;
+    // `row`: the values of tile 0's first key on (readable and finite up to the end of the last tile); keys: how many keys there are from there on
+    __device__ __forceinline__ void load(const void* row, int keys, int n, int lane) {
+        lo = hi = 0;
+        const int left = keys - lane * 64;  // (keys of this lane's tile that exist)
+        if (lane < n) {
+            const u32x4* const from = static_cast<const u32x4*>(row) + lane * 8;
+            u32x4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = from[i];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) {  // (of the two values only -inf has the topmost bit of its exponent)
+                const uint32_t two = ~v[i >> 2][i & 3];
+                uint32_t& word = i < 16 ? lo : hi;
+                word |= ((two >> 14 & 1) | (two >> 29 & 2)) << (2 * (i & 15));
+            }
+        }
+        const uint32_t real_lo = left >= 32 ? ~0u : left > 0 ? (1u << left) - 1 : 0u;
+        const uint32_t real_hi = left >= 64 ? ~0u : left > 32 ? (1u << (left - 32)) - 1 : 0u;
+        tiles.zero = __builtin_amdgcn_ballot_w64(lane < n && ((~lo & real_lo) | (~hi & real_hi)) == 0);
+        tiles.active = __builtin_amdgcn_ballot_w64(((lo & real_lo) | (hi & real_hi)) != 0);
+    }
+    // bits of key block kb (32 keys) of tile t, those of keys c_row(i, h) at c_row(i, 0)
+    __device__ __forceinline__ uint32_t block(int t, int kb, int h) const {
+        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(kb ? hi : lo), t)) >> (4 * h);
+    }
+};
 
 // ---------------------------------------------------------------- coalesced epilogue
 // A wave holds NB transposed C tiles: lane = output row (l32, two lanes per row), 16 registers per

@@ -83,6 +83,9 @@ template <typename T, int D>
 int launch_dkdv_variant(int dtype, const KParams& p, hipStream_t stream) {
     if (p.causal) return launch_dkdv_dropout<T, D, true, kNoMask>(p, stream);
     if (p.mask == nullptr) return launch_dkdv_dropout<T, D, false, kNoMask>(p, stream);
+    if constexpr (D < 128) {
+        if (mask_is_key_bits(p)) return launch_dkdv_dropout<T, D, false, kMaskKeys>(p, stream);
+    }
     if (p.mask_dtype == TRI_ATTN_F32) return launch_dkdv_dropout<T, D, false, kMaskF32>(p, stream);
     if (p.mask_dtype == dtype) return launch_dkdv_dropout<T, D, false, kMaskT>(p, stream);
     return TRI_ATTN_EDTYPE;

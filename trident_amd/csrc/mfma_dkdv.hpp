@@ -17,7 +17,7 @@ namespace {
 constexpr int kBM = 128;  // stationary rows per workgroup
 constexpr int kBN = 64;   // streamed rows per tile
 
-enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
+enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2, kMaskKeys = 3 };  // (kMaskKeys: of the operand type, see KeyBits)
 
 template <typename T, int MASK>
 __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
@@ -37,16 +37,17 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // are not stored.
 // SPLIT (with RAGGED): a workgroup streams one part of its item's row tiles (split.hpp).
 template <int D, int MASK, bool DROPOUT>
-constexpr bool kThree = D == 64 && MASK == kNoMask && !DROPOUT;
+constexpr bool kThree = D == 64 && (MASK == kNoMask || MASK == kMaskKeys) && !DROPOUT;
 template <typename T, int D, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(MASK != kNoMask && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
+__global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !((MASK == kMaskF32 || MASK == kMaskT) && D == 64 && !DROPOUT) ? 1 : 2) void mfma_dkdv_wide_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
     constexpr int NW = 4;
     constexpr int kKeys = 32 * NW;
     // (a ring of three, or two beside an fp32 mask, where it lets a second workgroup onto the CU beside the mask regions, whose tiles hide what
     // the shorter lead leaves of the loads' latency: launch_dkdv_dropout says what that gives)
-    constexpr int kStages = MASK != kNoMask && D == 64 && !(DROPOUT && RAGGED) ? (MASK == kMaskT ? 3 : 2) : kThree<D, MASK, DROPOUT> ? 3 : 4;
+    constexpr bool kMatrix = MASK == kMaskF32 || MASK == kMaskT;  // a mask whose values are read tile by tile
+    constexpr int kStages = kMatrix && D == 64 && !(DROPOUT && RAGGED) ? (MASK == kMaskT ? 3 : 2) : kThree<D, MASK, DROPOUT> ? 3 : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes + 2 * kBN * 4;  // Q tile, dO tile, lse, delta
     constexpr int KK = D / 16;
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(M
     // of the operand type) when it fits (D = 64). Plain loads would be tracked by the compiler, whose waits for them
     // also drain the LDS-direct tile loads issued in between (the counter completes in order), which makes the
     // tile prefetch synchronous. Geometry of a 64-row SwzTile<64> / SwzTile<32> (128- or 64-byte rows = 32 keys).
-    constexpr bool kMaskViaLds = MASK != kNoMask && D <= 64;
+    constexpr bool kMaskViaLds = kMatrix && D <= 64;
     constexpr int kMaskElt = MASK == kMaskF32 ? 4 : 2;
     using MaskTile = std::conditional_t<MASK == kMaskF32, SwzTile<64>, SwzTile<32>>;
     constexpr int kMaskLoads = MaskTile::kBlocks;
@@ -98,6 +99,12 @@ __global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(M
     }
     const float c = p.scale_log2;
     [[maybe_unused]] const float inv_scale = p.inv_scale;  // (a mask value joins its score before the scale: s + mask / scale)
+    // a mask of keys is one value per lane
+    bool hidden = false, some_hidden = false;
+    if constexpr (MASK == kMaskKeys) {
+        hidden = mask_at<T, kMaskT>(p.mask, b * p.ms[0] + hd * p.ms[1] + key_ld) != 0.f;
+        some_hidden = __builtin_amdgcn_ballot_w64(hidden) != 0;
+    }
     // Without dropout the subtraction in dS = P (dP - delta) is left to the matrix pipe: the dP accumulators start from
     // the rows' delta values (as they come from the tile: the accumulator's layout) and take the product with the V
     // fragments negated, which gives delta - dP; dS then comes out negated and the sign goes into dK's final scale.
@@ -264,14 +271,14 @@ __global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(M
         for (int qb = 0; qb < 2; ++qb) {
             const int rb = r0 + 32 * qb;
             if (CAUSAL && rb + 31 < wkey0) continue;  // whole block above the wave's keys
-            float mk[MASK != kNoMask ? 16 : 1];
-            const bool masked = MASK != kNoMask && !mask_is_zero(j);
+            float mk[kMatrix ? 16 : 1];
+            const bool masked = kMatrix && !mask_is_zero(j);
             if constexpr (kMaskViaLds) {
                 if (masked) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) mk[i] = qb ? mk2[16 + i] : mk2[i];  // static indices keep it in registers
                 }
-            } else if constexpr (MASK != kNoMask) {
+            } else if constexpr (kMatrix) {
                 if (masked) {
                     const int64_t mbase = b * p.ms[0] + hd * p.ms[1] + key_ld;
 #pragma unroll
@@ -307,6 +314,11 @@ __global__ __launch_bounds__(256, (kThree<D, MASK, DROPOUT>) ? 3 : RAGGED && !(M
                 asm volatile("");           // (a real branch: the other blocks skip the comparisons)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) s[i] = key <= rb + c_row(i, h) ? s[i] : -INFINITY;
+            }
+            if (MASK == kMaskKeys && some_hidden) {
+                asm volatile("");
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = hidden ? -INFINITY : s[i];
             }
             if (RAGGED && rb + 32 > p.S) {  // query rows that do not exist contribute nothing
 #pragma unroll

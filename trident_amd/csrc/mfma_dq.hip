@@ -6,18 +6,18 @@ namespace tri {
 namespace {
 
 // ---------------------------------------------------------------------------------- launch
-template <typename T, bool CAUSAL, bool RAGGED>
+template <typename T, bool CAUSAL, bool RAGGED, int MASK>
 int launch_dq_three(const KParams& p, hipStream_t stream) {  // (with delta)
     const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, kNoMask, true, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, kNoMask, false, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, MASK, true, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_dq_kernel<T, 64, 4, CAUSAL, MASK, false, RAGGED, false, true, false, true>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
 template <typename T, int D, int NW, bool CAUSAL, int MASK>
 int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = false) {
-    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
-        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, false>(p, stream);
+    if constexpr (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
+        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, false, MASK>(p, stream);
     }
     const dim3 grid(p.B * p.H * (p.S / (32 * NW))), block(64 * NW);
     if constexpr (NW == 8 && D == 128 && MASK != kNoMask) {
@@ -27,7 +27,7 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
         if (p.dmask != nullptr || p.thr8 > 0) return launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
         hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
     } else {
-        if constexpr (MASK != kNoMask) {
+        if constexpr (MASK == kMaskF32 || MASK == kMaskT) {
             if (p.dmask != nullptr) {
                 if (p.thr8 > 0) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, true>), grid, block, 0, stream, p);
                 else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, false, false, true>), grid, block, 0, stream, p);
@@ -63,6 +63,7 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
 // D = 64 two 128-row workgroups share a CU, which is 5-30 % faster than the phased kernel up to S = 3000.
 template <int D, int MASK>
 bool dq_is_phased(const KParams& p) {
+    if (MASK == kMaskKeys) return D == 128 && p.thr8 <= 0;
     if (MASK != kNoMask) return false;
     if (D == 64) {
         const int64_t items = static_cast<int64_t>(p.B) * p.H * (p.S / 256), cus = persistent_grid(1 << 20);
@@ -82,8 +83,8 @@ bool dq_runs_four_waves(const KParams& p) {
 // any length (no mask, or a padded one), with boundary handling
 template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
-    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
-        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, true>(p, stream);
+    if constexpr (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
+        if (with_delta && three_workgroups_per_cu(p)) return launch_dq_three<T, CAUSAL, true, MASK>(p, stream);
     }
     const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
     if constexpr (MASK != kNoMask) {
@@ -109,9 +110,14 @@ int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
     return static_cast<int>(hipGetLastError());
 }
 
-template <typename T, int D, bool CAUSAL, bool RAGGED>
+template <typename T, int D, bool CAUSAL, bool RAGGED, int MASK>
 int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
     const dim3 grid(p.B * p.H * ((p.S + 255) / 256)), block(512);
+    if constexpr (MASK == kMaskKeys) {
+        if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, RAGGED, false, true>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false, RAGGED, false, true>), grid, block, 0, stream, p);
+        return static_cast<int>(hipGetLastError());
+    }
     if constexpr (D == 128 && CAUSAL && !RAGGED) {
         if (p.thr8 > 0) {
             if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true, RAGGED>), grid, block, 0, stream, p);
@@ -130,14 +136,16 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
         if (p.S % 256 != 0 && dq_runs_four_waves(p))
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
     }
-    if constexpr (MASK == kNoMask && (D == 128 || (D == 64 && !CAUSAL))) {
+    if constexpr ((MASK == kNoMask || MASK == kMaskKeys) && (D == 128 || (D == 64 && !CAUSAL && MASK == kNoMask))) {
         if (dq_is_phased<D, MASK>(p)) {
             if constexpr (D == 128) {
-                if (p.S % 256 != 0) return launch_dq_phased<T, D, CAUSAL, true>(p, stream, with_delta);
+                if (p.S % 256 != 0) return launch_dq_phased<T, D, CAUSAL, true, MASK>(p, stream, with_delta);
             }
-            return launch_dq_phased<T, D, CAUSAL, false>(p, stream, with_delta);
+            return launch_dq_phased<T, D, CAUSAL, false, MASK>(p, stream, with_delta);
         }
     }
+    if constexpr (D == 128 && MASK == kMaskKeys) return TRI_ATTN_ESHAPE;  // (without dropout: mask_is_key_bits)
+    else {
     if (with_delta && MASK != kNoMask && (D > 64 || p.dmask != nullptr)) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
     // D = 128: 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows). Up to D = 64 always 4: several such workgroups
     // share a CU (time over that of 8 waves at multiples of 256: D = 32 0.92-1.00; D = 64 beside 16-bit masks 0.90-1.02, beside fp32 ones with a
@@ -151,12 +159,14 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     // a padded mask: four waves; at D = 128 with the whole register file (in 256 registers the kernel spills)
     if constexpr (MASK != kNoMask) return launch_dq_ragged<T, D, 4, CAUSAL, MASK>(p, stream, with_delta);
     return TRI_ATTN_ESHAPE;
+    }
 }
 
 template <typename T, int D>
 int launch_dq_variant(int dtype, const KParams& p, hipStream_t stream, bool with_delta) {
     if (p.causal) return launch_dq_dropout<T, D, true, kNoMask>(p, stream, with_delta);
     if (p.mask == nullptr) return launch_dq_dropout<T, D, false, kNoMask>(p, stream, with_delta);
+    if (mask_is_key_bits(p)) return launch_dq_dropout<T, D, false, kMaskKeys>(p, stream, with_delta);
     if (p.mask_dtype == TRI_ATTN_F32) return launch_dq_dropout<T, D, false, kMaskF32>(p, stream, with_delta);
     if (p.mask_dtype == dtype) return launch_dq_dropout<T, D, false, kMaskT>(p, stream, with_delta);
     return TRI_ATTN_EDTYPE;

@@ -17,7 +17,7 @@ namespace {
 
 constexpr int kBN = 64;   // streamed rows per tile
 
-enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
+enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2, kMaskKeys = 3 };  // (kMaskKeys: of the operand type, see KeyBits)
 
 template <typename T, int MASK>
 __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
@@ -49,7 +49,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
-    static_assert(!THREE || (D == 64 && NW == 4 && MASK == 0 && !SPLIT), "three workgroups per CU");
+    static_assert(!THREE || (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys) && !SPLIT), "three workgroups per CU");
+    constexpr bool kMatrix = MASK == kMaskF32 || MASK == kMaskT;  // a mask whose values are read tile by tile
     static_assert(!DELTA || MASK == 0 || (D <= 64 && !DMASK), "delta on the way: no mask, or a small head without a mask gradient");
     using Tile = SwzTile<D>;
     constexpr int kRows = 32 * NW;
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     // A mask block of a wave (32 rows x 64 keys) goes through a private LDS region (8 KiB fp32, 4 KiB for a mask of
     // the operand type) when it fits (D = 64): lanes own rows, so direct loads would touch 32 cache lines per
     // instruction, while LDS-direct loads fetch whole rows. Geometry of a 32-row SwzTile<128> / SwzTile<64>.
-    constexpr bool kMaskViaLds = MASK != kNoMask && D <= 64;  // (at D = 128 the 4 KiB regions of a 16-bit mask would fit, but the kernel then spills)
+    constexpr bool kMaskViaLds = kMatrix && D <= 64;  // (at D = 128 the 4 KiB regions of a 16-bit mask would fit, but the kernel then spills)
     constexpr int kMaskElt = MASK == kMaskF32 ? 4 : 2;
     using MaskTile = std::conditional_t<MASK == kMaskF32, SwzTile<128>, SwzTile<64>>;
     constexpr int kMaskBytes = 32 * MaskTile::kRowBytes;
@@ -136,7 +137,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     // With the classes of the mask's blocks at hand: key tiles behind the last one that is not masked out altogether
     // are not streamed, and tiles whose mask is all zero over the workgroup's rows are not read.
     uint64_t zero_tiles = 0;
-    if constexpr (MASK != kNoMask) {
+    [[maybe_unused]] KeyBits key_bits;
+    if constexpr (MASK == kMaskKeys) {  // (at most 64 tiles)
+        key_bits.load(static_cast<const T*>(p.mask) + b * p.ms[0] + hd * p.ms[1], p.S, n_tiles, lane);
+        zero_tiles = key_bits.tiles.zero;
+        n_tiles = key_bits.tiles.active ? 64 - __builtin_clzll(key_bits.tiles.active) : 1;
+        my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
+    } else if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
             const uint8_t* const classes = p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (q0 / 64) * p.mcs[2] + key0 / kBN;
             const int across = RAGGED ? min(kRows / 64, num_key_tiles - q0 / 64) : kRows / 64;
@@ -283,15 +290,15 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
         const bool diag = CAUSAL && t0 + kBN - 1 > wrow0;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-            float mk[MASK != kNoMask ? 16 : 1];
+            float mk[kMatrix ? 16 : 1];
             // (at D = 128 the registers do not hold a second form of the arithmetic: a tile whose mask is all zero adds zeros)
-            const bool masked = MASK != kNoMask && (D == 128 || !mask_is_zero(j));
+            const bool masked = kMatrix && (D == 128 || !mask_is_zero(j));
             if constexpr (kMaskViaLds) {
                 if (masked) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) mk[i] = mk2[16 * kb + i];
                 }
-            } else if constexpr (MASK != kNoMask) {
+            } else if constexpr (kMatrix) {
                 if (mask_is_zero(j)) {
 #pragma unroll
                     for (int i = 0; i < 16; ++i) mk[i] = 0.f;
@@ -325,6 +332,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
                 asm volatile("");                     // (a real branch: the other blocks skip the comparisons)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) st[i] = t0 + 32 * kb + c_row(i, h) <= qrow ? st[i] : -INFINITY;
+            }
+            if constexpr (MASK == kMaskKeys) {
+                if (!mask_is_zero(j)) {
+                    const uint32_t visible = key_bits.block(j, kb, h);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) st[i] = (visible >> c_row(i, 0) & 1) != 0 ? st[i] : -INFINITY;
+                }
             }
             if (RAGGED && !CAUSAL && t0 + 32 * kb + 32 > p.S) {  // keys that do not exist
                 int left = p.S - t0 - 32 * kb - 4 * h;
@@ -411,9 +425,11 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
 // (trident/kernel/softmax.py:180-238) disappears into the prologue that loads the dO rows anyway.
 // RAGGED: S is not a multiple of 256; rows and keys at or beyond S as in the kernel above (clamped loads, probability 0,
 // not stored), a wave without a single row of its own only fetches and meets the barriers.
-template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false, bool SPLIT = false>
+// KEYS: beside a mask of keys that is 0 or -inf (KeyBits).
+template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false, bool SPLIT = false, bool KEYS = false>
 __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p) {
     static_assert(!RAGGED || D == 128, "boundary handling: D = 128 only");
+    static_assert(!KEYS || !(CAUSAL || SPLIT), "a mask excludes the causal variant");
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     using Tile = SwzTile<D>;
     constexpr int NW = 8;
@@ -503,6 +519,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         }
     }
 
+    [[maybe_unused]] KeyBits key_bits;
+    if constexpr (KEYS) {  // (at most 64 tiles; those behind the last one with a visible key are not streamed)
+        key_bits.load(static_cast<const T*>(p.mask) + b * p.ms[0] + hd * p.ms[1], p.S, n_tiles, lane);
+        n_tiles = key_bits.tiles.active ? 64 - __builtin_clzll(key_bits.tiles.active) : 1;
+        my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
+    }
+
     // A wave fetches blocks wave, wave + NW, ... of the K tile and of the V tile: their rows are a
     // multiple of 16 apart, so one per-lane source offset serves all of them.
     const uint32_t koff = static_cast<uint32_t>(Tile::src_off(wave, lane, krow_bytes));
@@ -577,7 +600,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     // Without dropout the subtraction in dS = P (dP - delta) is left to the matrix pipe: the dP^T accumulators start from
     // delta and take the product with the dO rows negated (delta - dP^T); dS^T comes out negated and the sign goes into
     // the scale of the final store.
-    constexpr bool kDeltaInAcc = !DROPOUT && !RAGGED;  // (boundary handling leaves no registers for it)
+    constexpr bool kDeltaInAcc = !DROPOUT && !RAGGED && !KEYS;  // (boundary handling and a mask leave no registers for it)
     f32x16 dlt16;
     if constexpr (kDeltaInAcc) {
 #pragma unroll
@@ -662,6 +685,13 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         // causal comparison)
         auto softmax_backward = [&](auto on_diagonal, int kb) {
             const int first_key = key0 + t * kBN + 32 * kb;
+            if constexpr (KEYS) {
+                if (!((key_bits.tiles.zero >> t) & 1)) {
+                    const uint32_t visible = key_bits.block(t, kb, h);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) st[kb][i] = (visible >> c_row(i, 0) & 1) != 0 ? st[kb][i] : -INFINITY;
+                }
+            }
             if (RAGGED && !CAUSAL && first_key + 32 > p.S) {  // keys that do not exist (under the causal mask no existing row sees them)
                 asm volatile("");                        // (a real branch)
 #pragma unroll

@@ -5,23 +5,23 @@
 namespace tri {
 namespace {
 
-template <typename T, bool CAUSAL, bool RAGGED>
+template <typename T, bool CAUSAL, bool RAGGED, int MASK>
 int launch_fwd_three(const KParams& p, hipStream_t stream) {
     const dim3 grid(p.B * p.H * ((p.S + 127) / 128)), block(256);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, kNoMask, true, RAGGED, false, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, kNoMask, false, RAGGED, false, true>), grid, block, 0, stream, p);
+    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, MASK, true, RAGGED, false, true>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_fwd_kernel<T, 64, 4, CAUSAL, MASK, false, RAGGED, false, true>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
 template <typename T, int D, int NW, bool CAUSAL, int MASK = kNoMask>
 int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
-    if constexpr (D == 128 && NW == 8 && MASK != kNoMask) {
+    if constexpr (D == 128 && NW == 8 && MASK != kNoMask && MASK != kMaskKeys) {
         // (mask, dropout and boundary handling together need the whole register file: four waves)
         if (p.thr8 > 0) return launch_fwd_ragged<T, D, 4, CAUSAL, MASK>(p, stream);
     }
     const int items = p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW));
-    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
-        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true>(p, stream);
+    if constexpr (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
+        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true, MASK>(p, stream);
     }
     if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
         if (p.S % 128 == 0) {  // (causal only with dropout: fwd_runs_four_waves)
@@ -43,14 +43,17 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
 
 template <typename T, int D, int NW, bool CAUSAL, int MASK>
 int launch_fwd_dropout(const KParams& p, hipStream_t stream) {
-    if constexpr (D == 64 && NW == 4 && MASK == kNoMask) {
-        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, false>(p, stream);
+    if constexpr (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
+        if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, false, MASK>(p, stream);
     }
     const int items = p.B * p.H * (p.S / (32 * NW));
     // (the kernel's kPersistent: one workgroup per CU walks the items)
     const dim3 grid(NW == 8 && MASK == kNoMask ? persistent_grid(items) : items), block(64 * NW);
-    if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
+    if (p.thr8 > 0) {
+        if constexpr (!(D == 128 && MASK == kMaskKeys)) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
+    } else {
+        hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), grid, block, 0, stream, p);
+    }
     return static_cast<int>(hipGetLastError());
 }
 
@@ -86,6 +89,8 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     // dropout 0.70-0.99; beside 16-bit masks 0.90-1.01; beside fp32 ones, whose ring of three lets two workgroups onto a CU, 0.88-0.96, length
     // masks 0.84-1.00 (dense ones in whole rounds of S = 2048 1.04-1.06).
     if constexpr (D == 128) {
+        if (mask_is_key_bits(p))
+            return p.S % 256 == 0 ? launch_fwd_dropout<T, D, 8, false, kMaskKeys>(p, stream) : launch_fwd_ragged<T, D, 8, false, kMaskKeys>(p, stream);
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
     }
     // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
@@ -97,6 +102,10 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
             if (fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
             return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
         }
+    }
+    if constexpr (D < 128) {
+        if (mask_is_key_bits(p))
+            return p.S % 128 == 0 ? launch_fwd_dropout<T, D, 4, false, kMaskKeys>(p, stream) : launch_fwd_ragged<T, D, 4, false, kMaskKeys>(p, stream);
     }
     if (p.S % 128 == 0) return launch_fwd_variant<T, D, 4>(dtype, p, stream);
     if (p.mask != nullptr) {

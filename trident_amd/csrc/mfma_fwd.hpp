@@ -30,7 +30,7 @@ namespace {
 constexpr int kBN = 64;      // keys per tile
 constexpr float kTau = 8.f;  // lazy-rescale threshold, log2 domain
 
-enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
+enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2, kMaskKeys = 3 };  // (kMaskKeys: of the operand type, see KeyBits)
 
 // RAGGED (no mask, or a padded one): S is not a multiple of 32 NW. Query rows and keys at or beyond S do not exist: row and tile loads clamp
 // their row index to S - 1, the scores of keys >= S are set to -inf, and rows >= S are not stored. A wave without a
@@ -40,7 +40,8 @@ enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2 };
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false, bool THREE = false>
 __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
-    static_assert(!THREE || (D == 64 && NW == 4 && MASK == 0 && !SPLIT), "three workgroups per CU");
+    static_assert(!THREE || (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys) && !SPLIT), "three workgroups per CU");
+    constexpr bool kMatrix = MASK == kMaskF32 || MASK == kMaskT;  // a mask whose values are read tile by tile
     using Tile = SwzTile<D>;
     // An fp32 mask at D = 128 (8 waves, no dropout) needs 64 KiB of LDS for its staging regions, at D = 64 32 KiB of the 80 with which
     // two workgroups of 4 waves share a CU; three have 53 KiB each. The ring then has
@@ -66,13 +67,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     // operand fragments in flight (two of mask, dropout and boundary handling leave room for four only at D = 128)
     // (at D = 32 the O^T product has four steps, and the softmax phase may request fragments of tile j only: tile j + 1
     // becomes visible with the barrier behind it)
-    constexpr int kRing = (D <= 32 || (D == 128 && (MASK != kNoMask) + (RAGGED && NW == 8) + DROPOUT >= 2)) ? 4 : 6;
+    constexpr int kRing = (D <= 32 || (D == 128 && kMatrix + (RAGGED && NW == 8) + DROPOUT >= 2)) ? 4 : 6;
     static_assert(kRing <= kPvSteps, "the softmax phase requests fragments of the O^T product only");
     // A mask block of a wave (32 rows x 64 keys) goes through a private LDS region (8 KiB for an fp32 mask, 4 KiB
     // for one of the operand type) when it fits (D = 64): lanes own rows, so direct loads would touch 32 cache
     // lines per instruction, while LDS-direct loads fetch whole rows (256 or 128 bytes) and the swizzled tile is
     // read back 16 or 8 bytes at a time. The region has the geometry of a 32-row SwzTile<128> / SwzTile<64>.
-    constexpr bool kMaskViaLds = MASK != kNoMask && (D <= 64 || (NW == 8 && !DROPOUT));  // (D = 128: 4 KiB regions fit, 8 KiB ones do not; with dropout the registers for the staged values are not there)
+    constexpr bool kMaskViaLds = kMatrix && (D <= 64 || (NW == 8 && !DROPOUT));  // (D = 128: 4 KiB regions fit, 8 KiB ones do not; with dropout the registers for the staged values are not there)
     constexpr int kMaskElt = MASK == kMaskF32 ? 4 : 2;
     using MaskTile = std::conditional_t<MASK == kMaskF32, SwzTile<128>, SwzTile<64>>;
     constexpr int kMaskBytes = 32 * MaskTile::kRowBytes;
@@ -139,7 +140,13 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     // masked out altogether are not streamed at all, and tiles whose mask is all zero over the workgroup's rows are not
     // read (a key-padding or length mask is all zero but for one column of blocks).
     uint64_t zero_tiles = 0;
-    if constexpr (MASK != kNoMask) {
+    [[maybe_unused]] KeyBits key_bits;
+    if constexpr (MASK == kMaskKeys) {  // (at most 64 tiles)
+        key_bits.load(static_cast<const T*>(p.mask) + b * p.ms[0] + hd * p.ms[1], p.S, n_tiles, lane);
+        zero_tiles = key_bits.tiles.zero;
+        n_tiles = key_bits.tiles.active ? 64 - __builtin_clzll(key_bits.tiles.active) : 1;  // (as below)
+        my_tiles = RAGGED && wrow0 >= p.S ? 0 : n_tiles;
+    } else if constexpr (MASK != kNoMask) {
         if (p.mcls != nullptr && n_tiles <= 64) {
             const uint8_t* const classes = p.mcls + b * p.mcs[0] + hd * p.mcs[1] + (qt * kBM / 64) * p.mcs[2] + key0 / kBN;
             const int across = RAGGED ? min(kBM / 64, num_key_tiles - qt * kBM / 64) : kBM / 64;
@@ -159,7 +166,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     const float inv_scale = p.inv_scale;  // (a mask value joins its score before the scale: s + mask / scale)
     // ... except a padded one (RAGGED), which joins it behind the scale, in the log2 domain: mask / scale would take finite
     // values below about -3.4e38 * scale to -inf, and a row of nothing else to NaN. One multiplication per score more.
-    constexpr bool kMaskAfter = RAGGED && MASK != kNoMask;
+    constexpr bool kMaskAfter = RAGGED && kMatrix;
 
     char* mask_lds = smem + kStages * kStageBytes + wave * kMaskBytes;
     auto issue_mask = [&](int t) {  // mask block of tile t -> this wave's region (8 LDS-direct loads), unless it is all zero
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
         const int i = idx % kPerOperand;
         if (RAGGED && (t + 1) * kBN > keys) {  // the sequence ends inside this tile: clamped rows, offsets from the tile's first row
             int l = lane;
-            if constexpr (D == 128 && MASK != kNoMask) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
+            if constexpr (D == 128 && kMatrix) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
             const int last = keys - 1 - t * kBN;
             if (idx < kPerOperand)
                 lds_direct_load16(kbase + static_cast<int64_t>(t) * kBN * krow_bytes,
@@ -273,11 +280,11 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     auto v_frag = [&](const char* sV, int s) { return Tile::tr_frag(sV, tr_off0 ^ ((s % DB) << 6), tr_off1 ^ ((s % DB) << 6), s / DB); };
 
     f32x16 sc[2];  // scores of this lane: sc[kb][i] is key t0 + 32*kb + c_row(i,h)
-    float mk[MASK != kNoMask ? 32 : 1];
+    float mk[kMatrix ? 32 : 1];
 
     // additive mask values of this lane's row for tile t, straight from memory
     auto load_mask = [&](int t) {
-        if constexpr (MASK != kNoMask && !kMaskViaLds) {
+        if constexpr (kMatrix && !kMaskViaLds) {
             if (mask_is_zero(t)) return;  // (the tile then takes the arithmetic of a tile without a mask: mk is not read)
             const int64_t mrow = b * p.ms[0] + hd * p.ms[1] + static_cast<int64_t>(RAGGED ? min(qrow, p.S - 1) : qrow) * p.ms[2] + key0 + t * kBN;
 #pragma unroll
@@ -483,7 +490,16 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
             // divided by the scale: one multiply-add per score, none in a tile whose mask is all zero. (c_tile: what is left
             // to multiply by.)
             const float c_tile = kMaskAfter && !mask_is_zero(j) ? 1.f : c;
-            if constexpr (MASK != kNoMask) {
+            if constexpr (MASK == kMaskKeys) {
+                if (!mask_is_zero(j)) {
+#pragma unroll
+                    for (int kb = 0; kb < 2; ++kb) {
+                        const uint32_t visible = key_bits.block(j, kb, h);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) x[16 * kb + i] = (visible >> c_row(i, 0) & 1) != 0 ? x[16 * kb + i] : -INFINITY;
+                    }
+                }
+            } else if constexpr (MASK != kNoMask) {
                 if (!mask_is_zero(j)) {
 #pragma unroll
                     for (int e = 0; e < 32; ++e) x[e] = kMaskAfter ? fmaf(mk[e], kLog2e, x[e] * c) : fmaf(mk[e], inv_scale, x[e]);
@@ -635,7 +651,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     static_assert(kStages == 4 || kStages == 3, "the tile loop is unrolled over the ring's slots");
     // (a mask and dropout together at D = 128 have no registers to spare for four copies of the step: rolled, the slot
     // is a run-time value there and every fragment read adds it to its address)
-    constexpr bool kUnrolled = !(D == 128 && MASK != kNoMask && DROPOUT);
+    constexpr bool kUnrolled = !(D == 128 && kMatrix && DROPOUT);
     if constexpr (kUnrolled && kStages == 3) {
         for (int j = 0; j < my_tiles; j += 3) {
             tile_step(j, 0);

@@ -212,9 +212,11 @@ bool mfma_supported(int which, int dtype, const KParams& p) {
 // 521 -> 511, fp16 B=16 H=12 S=777 D=64, key padding, 254 -> 245); not at D = 128, whose masked kernels fill their registers
 // (a row of O is 32 more in the prologue), and not where the pass writes a mask gradient, whose variants would double.
 bool mfma_dq_fuses_delta(const KParams& p) {
-    if (p.mask != nullptr && (p.D > 64 || p.dmask != nullptr)) return false;
+    // (beside a mask of keys at D = 128 the phased kernel runs, in one piece)
+    const bool keys = p.D == 128 && mask_is_key_bits(p) && mfma_dq_workspace(p, false) == 0;
+    if (p.mask != nullptr && ((p.D > 64 && !keys) || p.dmask != nullptr)) return false;
     if (!aligned16(p.o) || !strides8(p.os)) return false;
-    const bool phased = p.mask == nullptr && (p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0);  // (as the launcher decides)
+    const bool phased = keys || p.mask == nullptr && (p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0);  // (as the launcher decides)
     return !phased || tile_offsets_fit(p.os);
 }
 
@@ -237,9 +239,14 @@ bool four_waves_fit_one_round(const KParams& p) {
     return persistent_grid(busy) == busy;
 }
 
+bool mask_is_key_bits(const KParams& p) {  // (of 16-bit problems: mfma_supported; a 16-bit mask is of their type)
+    return p.mask != nullptr && p.mask_binary && p.mask_padded && p.ms[2] == 0 && p.mask_dtype != TRI_ATTN_F32 && p.mcls != nullptr &&
+           p.dmask == nullptr && (p.D <= 64 || p.thr8 <= 0) && p.S <= 64 * 64;
+}
+
 bool three_workgroups_per_cu(const KParams& p) {
     const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
-    return p.D == 64 && p.mask == nullptr && items > (p.causal ? 2 : 4) * static_cast<int64_t>(persistent_grid(1 << 20));
+    return p.D == 64 && (p.mask == nullptr || mask_is_key_bits(p)) && items > (p.causal ? 2 : 4) * static_cast<int64_t>(persistent_grid(1 << 20));
 }
 
 int launch_delta(int dtype, const KParams& p, hipStream_t stream) {
