@@ -1,5 +1,5 @@
 """Head size 64 in workgroups of four waves: fp32 masks with a ring of three (forward, dQ) or two tiles (dK/dV), two workgroups on a CU,
-and the numbers of items from which launches without a mask take eight waves."""
+and the numbers of items from which launches without a mask take eight waves. Head size 128 in such workgroups."""
 import math
 
 import pytest
@@ -84,6 +84,30 @@ def test_launches_of_several_rounds(causal, heads, S, p, device):
     o, lse = Attention._forward(tq, tk, tv, None, p, causal, scale, seed, 0)
     grads = Attention._backward(tdo, tq, tk, tv, o, lse, None, scale, p, causal, seed, 0, False)[:3]
     assert all(x.isfinite().all() for x in (o, *grads))
+    for h in [0] + ([heads - 1] if p == 0.0 else []):  # (decisions depend on the head's number: the oracle counts from 0)
+        at = (slice(0, 1), slice(h, h + 1))
+        kw = dict(mask=None, dropout_p=p, is_causal=causal, scale=scale, seed=seed, offset=0)
+        parity.close(o[at], parity.oracle_forward(q[at], k[at], v[at], **kw)[0], dtype, "O")
+        ref = parity.oracle_backward(q[at], k[at], v[at], d_o[at], o=o[at], **kw)[:3]
+        sums = parity.oracle_abs_sums(q[at], k[at], v[at], d_o[at], o=o[at], **kw)[1:]
+        for name, got, want, total in zip(("dQ", "dK", "dV"), grads, ref, sums):
+            parity.close(got[at], want, dtype, name, total)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,S", [(2, 16), (3, 64), (9, 65), (5, 128), (4, 129), (128, 256), (129, 256), (64, 257), (171, 384), (65, 511), (64, 512),
+                                     (228, 320), (129, 512), (9, 1000), (84, 1016), (33, 1025), (103, 640)])
+def test_head_size_128_in_four_waves(heads, S, causal, p, device):
+    """Around the numbers of heads and rows at which workgroups of four waves (two to a CU, a ring of two tiles) take over from eight: the first
+    and last heads match the oracle."""
+    D, dtype, seed = 128, torch.bfloat16, 31
+    g = torch.Generator().manual_seed(heads + S)
+    q, k, v, d_o = [torch.randn(1, heads, S, D, generator=g).to(dtype) for _ in range(4)]
+    tq, tk, tv, tdo = [x.to(device) for x in (q, k, v, d_o)]
+    scale = 1.0 / math.sqrt(D)
+    o, lse = Attention._forward(tq, tk, tv, None, p, causal, scale, seed, 0)
+    grads = Attention._backward(tdo, tq, tk, tv, o, lse, None, scale, p, causal, seed, 0, False)[:3]
     for h in [0] + ([heads - 1] if p == 0.0 else []):  # (decisions depend on the head's number: the oracle counts from 0)
         at = (slice(0, 1), slice(h, h + 1))
         kw = dict(mask=None, dropout_p=p, is_causal=causal, scale=scale, seed=seed, offset=0)

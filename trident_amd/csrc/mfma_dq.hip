@@ -34,7 +34,7 @@ int launch_dq_waves(const KParams& p, hipStream_t stream, bool with_delta = fals
                 return static_cast<int>(hipGetLastError());
             }
         }
-        if constexpr (MASK == kNoMask && D == 128) {  // (without dropout: the phased kernel)
+        if constexpr (MASK == kNoMask && D == 128 && NW == 8) {  // (without dropout: the phased kernel)
             if (with_delta) hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true, false, false, true>), grid, block, 0, stream, p);
             else hipLaunchKernelGGL((mfma_dq_kernel<T, D, NW, CAUSAL, MASK, true>), grid, block, 0, stream, p);
         } else {
@@ -72,12 +72,28 @@ bool dq_is_phased(const KParams& p) {
     return D == 128 && (p.thr8 <= 0 || (p.causal && p.S % 256 == 0));
 }
 
-// D = 128 without a mask, S no multiple of 256: the unphased kernel in workgroups of four waves. One key tile (S <= 64) is over
-// before phases pay: time over that of the phased kernel 0.81-0.99 (with dropout, against eight unphased waves, 0.92-1.01).
-// With dropout also where all workgroups are on the chip at once: 0.79-0.89 (causal S = 384 1.05; as the forward).
+// D = 128 without a mask: workgroups of four waves (kPair), two to a CU, instead of one of eight, whose pairs of waves are phased where their
+// registers allow it. Four waves gain where 128 rows waste less than 256 (rows that do not exist, keys above the diagonal), where starts and
+// ends are a large part of the time, and where 256-row items leave CUs idle in the last round; per tile the phased kernel needs less (time of
+// four waves over its beyond these rules: without dropout 1.04-1.19, with it 1.00-1.10, causal 0.98-1.10). By the rules in turn:
+//   S <= 128            0.60-0.79 from 512 heads on, 0.89-1.02 up to 64
+//   without dropout, up to 512 rows
+//     up to a workgroup per CU              0.87-1.01 (causal S = 384, whose second item is light: 1.00-1.07, not taken)
+//     more than two per CU, causal          0.76-0.95
+//     more than two per CU, S in 257 .. 384 0.79-0.93
+//   with dropout
+//     up to a workgroup per CU              0.72-0.95
+//     not causal, fewer half rounds than eight waves take (each of their rounds is two)  0.66-0.90
+//     causal, up to 8/3 per CU              0.81-0.93; S <= 512, or S <= 1024 with a half-empty last item 0.69-0.90
 bool dq_runs_four_waves(const KParams& p) {
-    if (p.S <= 64) return true;
-    return p.thr8 > 0 && p.S > 128 && (!p.causal || p.S % 128 != 0 || p.S >= 640) && four_waves_fit_one_round(p);
+    const int64_t cus = persistent_grid(1 << 20), heads = static_cast<int64_t>(p.B) * p.H;
+    const int64_t items = heads * ((p.S + 127) / 128), items256 = heads * ((p.S + 255) / 256);
+    const bool half_empty = (p.S - 1) % 256 < 128;
+    if (p.S <= 128) return true;
+    if (p.thr8 <= 0) return p.S <= 512 && (items <= cus ? !p.causal || p.S % 256 != 128 : items > 2 * cus && (p.causal || half_empty));
+    if (items <= cus) return true;
+    if (p.causal) return 3 * items <= 8 * cus || p.S <= (half_empty ? 1024 : 512);
+    return (items + cus - 1) / cus < 2 * ((items256 + cus - 1) / cus);
 }
 
 // any length (no mask, or a padded one), with boundary handling
@@ -133,7 +149,7 @@ int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     if constexpr (D == 128 && MASK == kNoMask) {
-        if (p.S % 256 != 0 && dq_runs_four_waves(p))
+        if (dq_runs_four_waves(p))
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
     }
     if constexpr ((MASK == kNoMask || MASK == kMaskKeys) && (D == 128 || (D == 64 && !CAUSAL && MASK == kNoMask))) {
@@ -150,7 +166,7 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     // D = 128: 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows). Up to D = 64 always 4: several such workgroups
     // share a CU (time over that of 8 waves at multiples of 256: D = 32 0.92-1.00; D = 64 beside 16-bit masks 0.90-1.02, beside fp32 ones with a
     // ring of three 0.78-1.05, in most cases 0.95-0.98)
-    if constexpr (D == 128) {
+    if constexpr (D == 128 && !CAUSAL) {  // (causal: the phased kernel)
         if (p.S % 256 == 0) return launch_dq_waves<T, D, 8, CAUSAL, MASK>(p, stream, with_delta);
     }
     if constexpr (D == 128 && MASK == kNoMask) return launch_dq_ragged<T, D, 8, CAUSAL>(p, stream, with_delta);  // (dropout)

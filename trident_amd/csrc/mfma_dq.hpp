@@ -28,8 +28,8 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // ------------------------------------------------------------------------------------ dQ
 // A workgroup of NW waves owns 32*NW query rows, one wave 32 of them with its Q and dO rows in
 // registers (B operands) and dQ^T in fp32 accumulators; two waves per SIMD. K and V stream as
-// 64-key swizzled LDS tiles in a ring of 4, filled by LDS-direct loads three tiles ahead (no
-// staging registers, no ds_write). Per 32-key block: S^T = K Q^T and dP^T = V dO^T from row
+// 64-key swizzled LDS tiles in a ring of 4 (3, 2: kStages), filled by LDS-direct loads three (two, one)
+// tiles ahead (no staging registers, no ds_write). Per 32-key block: S^T = K Q^T and dP^T = V dO^T from row
 // fragments, dS^T = P^T (dP^T - delta) on the vector ALU, dQ^T += K^T dS^T with K^T read through
 // transposed LDS reads of the same K tile.
 // RAGGED (no mask, or a padded one; no mask gradient): S is not a multiple of 32 NW. Rows and keys at or beyond S do not exist: loads clamp
@@ -45,7 +45,7 @@ __device__ __forceinline__ float mask_at(const void* mask, int64_t off) {
 // THREE (D = 64, no mask, 4 waves): three workgroups to a CU instead of two (three_workgroups_per_cu).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool DMASK = false, bool DELTA = false,
           bool SPLIT = false, bool THREE = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE || D == 16 && SPLIT && MASK != kNoMask ? 3 : 2) void mfma_dq_kernel(const KParams p) {
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != kNoMask || SPLIT) ? 1 : THREE || D == 16 && SPLIT && MASK != kNoMask ? 3 : 2) void mfma_dq_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!RAGGED || !DMASK, "ragged lengths: no mask gradient");
     static_assert(!DMASK || MASK != 0, "a mask gradient needs a mask");
@@ -54,7 +54,11 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     static_assert(!DELTA || MASK == 0 || (D <= 64 && !DMASK), "delta on the way: no mask, or a small head without a mask gradient");
     using Tile = SwzTile<D>;
     constexpr int kRows = 32 * NW;
-    constexpr int kStages = THREE || (MASK == kMaskF32 && D == 64 && NW == 4) ? 3 : 4;
+    // Without a mask the workgroups of four waves at D = 128 run two to a CU: a ring of two tiles in half of the LDS, and half of the registers.
+    // One alone, with a ring of four and all registers, leaves a wave per SIMD (time of the two over its: 0.72-0.78 at S <= 128; causal with
+    // dropout 40 heads x 1000 48.7 -> 40.4 us).
+    constexpr bool kPair = D == 128 && NW == 4 && MASK == kNoMask && !SPLIT;
+    constexpr int kStages = kPair ? 2 : THREE || (MASK == kMaskF32 && D == 64 && NW == 4) ? 3 : 4;
     constexpr int kAhead = kStages - 1;  // tile j + kAhead is requested in tile j, into the slot of tile j - 1
     constexpr int kStageBytes = 2 * Tile::kBytes;  // K tile, V tile
     constexpr int KK = D / 16;
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
             const char* tile_src = is_v ? vbase + static_cast<int64_t>(t) * kBN * vrow_bytes
                                         : kbase + static_cast<int64_t>(t) * kBN * krow_bytes;
             // the sequence ends inside this tile (at D = 128 every tile takes the clamped form: no registers for kept offsets)
-            if (RAGGED && (D == 128 || (t + 1) * kBN > keys)) {
+            if (RAGGED && ((D == 128 && !kPair) || (t + 1) * kBN > keys)) {
                 int l = lane;
                 asm volatile("" : "+v"(l));
                 lds_direct_load16(tile_src, Tile::src_off_clamped(is_v ? blk - Tile::kBlocks : blk, l, is_v ? vrow_bytes : krow_bytes,
@@ -206,7 +210,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
         issue_mask(0);
         issue_tile(0);
     }
-    if (1 < n_tiles) issue_tile(1);
+    if (kAhead > 1 && 1 < n_tiles) issue_tile(1);
     if (kAhead > 2 && 2 < n_tiles) issue_tile(2);
     // (the row fragments were requested before the tiles, so both latencies overlap)
 #pragma unroll
@@ -249,9 +253,9 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
 
     for (int j = 0; j < n_tiles; ++j) {
         // (the fragments' offsets of the column blocks are made from these here, not kept in registers across the loop)
-        if constexpr (THREE) asm volatile("" : "+v"(row_off0), "+v"(tr_off0), "+v"(tr_off1));
-        // tile j has landed (up to two younger tiles may still be in flight) and is visible to all
-        // waves; every wave is done with tile j-1, whose slot takes the load of tile j+3
+        if constexpr (THREE || kPair) asm volatile("" : "+v"(row_off0), "+v"(tr_off0), "+v"(tr_off1));
+        // tile j has landed (up to kAhead - 1 younger tiles may still be in flight) and is visible to all
+        // waves; every wave is done with tile j-1, whose slot takes the load of tile j + kAhead
         {
             // with a staged mask, block j must have landed too: only tile j + kAhead - 1 was issued after it
             // (the kAhead first tiles after the first block)
