@@ -24,9 +24,9 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
         if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true, MASK>(p, stream);
     }
     if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
-        if (p.S % 128 == 0) {
+        if (p.S % 128 == 0) {  // (causal only with dropout: fwd_runs_four_waves)
             if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), dim3(items), dim3(64 * NW), 0, stream, p);
-            else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
+            else if constexpr (!CAUSAL) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
@@ -91,7 +91,6 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     if constexpr (D == 128) {
         if (mask_is_key_bits(p))
             return p.S % 256 == 0 ? launch_fwd_dropout<T, D, 8, false, kMaskKeys>(p, stream) : launch_fwd_ragged<T, D, 8, false, kMaskKeys>(p, stream);
-        if (p.mask == nullptr && fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
     }
     // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
@@ -100,6 +99,7 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     // that leave CUs idle either way are another matter (above).
     if constexpr (D == 128) {
         if (p.mask == nullptr) {
+            if (fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
             return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
         }
     }
