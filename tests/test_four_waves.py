@@ -97,7 +97,8 @@ def test_launches_of_several_rounds(causal, heads, S, p, device):
 @pytest.mark.parametrize("p", [0.0, 0.1])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("heads,S", [(2, 16), (3, 64), (9, 65), (5, 128), (4, 129), (128, 256), (129, 256), (64, 257), (171, 384), (65, 511), (64, 512),
-                                     (228, 320), (129, 512), (9, 1000), (84, 1016), (33, 1025), (103, 640)])
+                                     (228, 320), (129, 512), (9, 1000), (84, 1016), (33, 1025), (103, 640), (23, 2048), (40, 1281), (129, 777),
+                                     (52, 2049), (257, 512)])
 def test_head_size_128_in_four_waves(heads, S, causal, p, device):
     """Around the numbers of heads and rows at which workgroups of four waves (two to a CU, a ring of two tiles) take over from eight: the first
     and last heads match the oracle."""

@@ -48,10 +48,6 @@ enum MaskClass { kMaskZero = 0, kMaskNegInf = 1, kMaskMixed = 2 };
 // Number of workgroups for a kernel whose workgroups are persistent (one per CU, each walking several of
 // the `items`): min(items, CUs of the current device).
 int persistent_grid(int items);
-// Whether workgroups of 128 rows are all on the chip at once, one per CU. Causal ones from S = 1024 on also where they are half
-// as many again: the heaviest start first, and the light ones fill up behind them (bf16 with dropout, 288-384 workgroups,
-// S = 1025-2100: forward and dQ 0.85-0.91 of the time of 256-row ones; 384 at S = 300: 1.27).
-bool four_waves_fit_one_round(const KParams& p);
 // Whether forward and dQ at D = 64 without a mask run their 128-row workgroups three to a CU (in 168 registers, with a ring of three tiles)
 // instead of two: launches of several rounds. Time of three over that of two, or of the eight-wave kernels that ran before, by the number
 // of workgroups: up to two per CU forward 0.97-1.06, dQ 0.97-1.09; causal at 3.4 to 4 per CU forward 0.93-0.98 (16 heads of S = 8192: 1.03),

@@ -24,9 +24,9 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
         if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true, MASK>(p, stream);
     }
     if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
-        if (p.S % 128 == 0) {  // (causal only with dropout: fwd_runs_four_waves)
+        if (p.S % 128 == 0) {
             if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), dim3(items), dim3(64 * NW), 0, stream, p);
-            else if constexpr (!CAUSAL) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
+            else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
@@ -59,7 +59,7 @@ int launch_fwd_dropout(const KParams& p, hipStream_t stream) {
 
 template <typename T, int D, int NW>
 int launch_fwd_variant(int dtype, const KParams& p, hipStream_t stream) {
-    if constexpr (!(D == 128 && NW == 4)) {  // (without a mask D = 128 never runs four waves: launch_fwd_waves)
+    if constexpr (!(D == 128 && NW == 4)) {  // (without a mask: launch_fwd_ragged)
         if (p.causal) return launch_fwd_dropout<T, D, NW, true, kNoMask>(p, stream);
         if (p.mask == nullptr) return launch_fwd_dropout<T, D, NW, false, kNoMask>(p, stream);
     }
@@ -68,21 +68,41 @@ int launch_fwd_variant(int dtype, const KParams& p, hipStream_t stream) {
     return TRI_ATTN_EDTYPE;
 }
 
-// D = 128 without a mask, S no multiple of 256: 128-row workgroups of four waves where they are all on the chip at once, which
-// then is a matter of one workgroup's time. bf16, time of the four waves over that of the eight: with dropout 0.78-0.98
-// (causal 0.79-0.97, but 1.03 at S = 384, whose last 256 rows are half empty for the eight), without 0.92-0.98 at S = 129 .. 500
-// and from 640 on 1.00-1.12 with boundary handling, 0.88-0.94 at multiples of 128, which need none; causal 0.86-1.00 up to
-// S = 500, 1.02-1.19 beyond and at multiples of 128; S <= 128 without dropout 1.00-1.05.
+// D = 128 without a mask: workgroups of four waves (kPair), two to a CU, instead of one of eight whose waves run in opposite phases. Per tile
+// the eight need up to 9 % less time (not causal, without dropout); four waves gain where 128 rows waste less than 256 (rows that do not exist, keys
+// above the diagonal), where starts and ends are a large part of the time, and where 256-row items leave CUs idle in the last round. Beside dropout
+// two independent workgroups overlap the generator with the other one's MFMAs better than the phases do. Time of four waves over that of eight, bf16,
+// 0.4 to 24 workgroups per CU (a half round: of workgroups of four waves; a round of the eight is two):
+//   S <= 128                                      0.56-0.88
+//   up to a workgroup per CU                      0.68-0.90
+//   causal with dropout                           0.54-1.03 (from 4096 rows on, in whole rounds of the eight, 0.91-1.03; 16384 rows in such 0.98-1.02)
+//   causal, up to 1024 rows                       0.64-1.02; 3 to 4 per CU without a half-empty last item 0.88-1.14; beyond 16 or 10 per CU, out of
+//                                                 the caches, 0.91-1.14 (a head's items, heaviest first, read its keys far apart in time)
+//   causal, longer                                up to 3 per CU 0.70-1.02; up to 5 where the eight's last round is not full 0.82-1.03, else 0.96-1.18
+//   not causal with dropout, fewer half rounds    0.53-0.92; else up to 512 rows 0.78-1.00, up to 1024 and from 4 per CU on 0.77-0.99, others 0.93-1.09
+//   not causal, up to 512 rows                    fewer half rounds 0.64-1.00; more than four per CU 0.75-0.99; else 0.89-1.15
+//   not causal, longer, three quarters of the half rounds  0.61-1.08 (0.89-0.98 in most; 1000 rows of a number of heads the XCDs don't share evenly
+//                                                 1.04-1.08, not taken); up to 800 rows from 8 per CU on, fewer half rounds 0.83-0.97; else 0.91-1.17
 bool fwd_runs_four_waves(const KParams& p) {
-    if (!four_waves_fit_one_round(p)) return false;
-    const bool whole = p.S % 128 == 0;
-    if (p.thr8 > 0) return !p.causal || !whole || p.S >= 640;
-    return p.S > 128 && (whole ? !p.causal : p.S <= 512);
+    const int64_t cus = persistent_grid(1 << 20), heads = static_cast<int64_t>(p.B) * p.H;
+    const int64_t items = heads * ((p.S + 127) / 128), items256 = heads * ((p.S + 255) / 256);
+    const int64_t halves = (items + cus - 1) / cus, rounds256 = (items256 + cus - 1) / cus;
+    const bool half_empty = (p.S - 1) % 256 < 128;
+    if (p.S <= 128 || items <= cus) return true;
+    if (p.causal && p.thr8 > 0) return p.S <= 8192 || items <= 3 * cus;
+    if (p.causal) {
+        if (p.S <= 1024) return items <= (p.S <= 800 ? 16 : 10) * cus && (half_empty || p.S < 256 || items <= 3 * cus || items > 4 * cus);
+        return items <= 3 * cus || (items <= 5 * cus && 16 * items256 <= 15 * rounds256 * cus);
+    }
+    if (p.thr8 > 0) return p.S <= 512 || halves < 2 * rounds256 || (p.S <= 1024 && items > 4 * cus);
+    if (p.S <= 512) return halves < 2 * rounds256 || items > 4 * cus;
+    if (4 * halves <= 6 * rounds256) return half_empty || p.S > 1024 || heads % 8 == 0;
+    return p.S <= 800 && items > 8 * cus && halves < 2 * rounds256;
 }
 
 template <typename T, int D>
 int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
-    // 8 waves (256 query rows) at D = 128 when the sequence allows it: two waves per SIMD out of phase. Up to D = 64 four waves everywhere,
+    // 8 waves (256 query rows) at D = 128 where the sequence allows it (without a mask as above): two waves per SIMD out of phase. Up to D = 64 four waves everywhere,
     // whose workgroups share a CU, so that starts and ends pass behind one another's tiles and less of the chip is idle in the last round. Time of
     // the four over that of the eight at multiples of 256: D = 32 0.78; D = 64 without a mask 0.82-0.86 at half as many items of 256 rows as CUs,
     // 0.93-0.99 at as many, 0.99-1.03 at twice as many (causal 0.77-0.86, 0.88-0.91 and 0.95-1.00), more than that: three_workgroups_per_cu; with
@@ -91,17 +111,9 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     if constexpr (D == 128) {
         if (mask_is_key_bits(p))
             return p.S % 256 == 0 ? launch_fwd_dropout<T, D, 8, false, kMaskKeys>(p, stream) : launch_fwd_ragged<T, D, 8, false, kMaskKeys>(p, stream);
+        if (p.mask == nullptr && fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
-    }
-    // Without a mask D = 128 keeps the 8 waves at every other length too, with boundary handling: its ring leaves room for
-    // one workgroup per CU, so that four waves are one per SIMD. bf16 causal, heads x S: 768 x 130 0.057 -> 0.034 ms,
-    // 768 x 450 0.168 -> 0.110, 136 x 1531 0.170 -> 0.109, 32 x 3000 0.141 -> 0.084; 768 x 65 0.026 -> 0.022. Launches
-    // that leave CUs idle either way are another matter (above).
-    if constexpr (D == 128) {
-        if (p.mask == nullptr) {
-            if (fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
-            return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
-        }
+        if (p.mask == nullptr) return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);
     }
     if constexpr (D < 128) {
         if (mask_is_key_bits(p))

@@ -38,7 +38,7 @@ enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2, kMaskKeys = 3 };  // (kMa
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from key0.
 // THREE (D = 64, no mask, 4 waves): three workgroups to a CU instead of two (three_workgroups_per_cu).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false, bool THREE = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != kNoMask || SPLIT) ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!THREE || (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys) && !SPLIT), "three workgroups per CU");
     constexpr bool kMatrix = MASK == kMaskF32 || MASK == kMaskT;  // a mask whose values are read tile by tile
@@ -48,8 +48,14 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
     // phase before V of tile t, so with K(j + dist) and V(j + dist - 1) requested together every tile keeps the lead
     // it has in the ring of four, and both fit three slots. The first fragments of V wait for the barrier, though.
-    constexpr bool kLeadK = THREE || (MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4)));
-    constexpr int kStages = kLeadK ? 3 : 4;  // LDS ring depth
+    // Without a mask the workgroups of four waves at D = 128 run two to a CU: two slots per operand in 64 KiB, half of the registers. Tile
+    // j's matrix phase, behind a barrier that every wave meets once it is done with K of tile j and V of tile j - 1, requests K of tile j + 2
+    // and V of tile j + 1 into their slots, and the barrier of tile j + 1 awaits both. A workgroup alone on its CU (eight waves and a ring of four,
+    // or four waves) leaves the CU to its start, its end and its barriers; two hide one another's. bf16, us, eight waves -> two times four, heads x S:
+    // 1024 x 128 32.9 -> 24.1, causal 40 x 1024 28.0 -> 24.1; with dropout 1024 x 300 130 -> 102, causal 32 x 2048 76.8 -> 56.3, 40 x 4096 243 -> 213.
+    constexpr bool kPair = D == 128 && NW == 4 && MASK == kNoMask && !SPLIT;
+    constexpr bool kLeadK = THREE || kPair || (MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4)));
+    constexpr int kStages = kPair ? 2 : kLeadK ? 3 : 4;  // LDS ring depth
     constexpr int kLag = kLeadK ? 1 : 0;     // how many tiles the V requests trail the K requests
     constexpr int kBM = 32 * NW;
     constexpr int kKBytes = Tile::kBytes;
@@ -444,7 +450,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     l = 0.f;
     // tile 0 has landed and is visible to all waves (a later item's requests are older than the stores of the
     // item before it: everything is awaited)
-    if (!first_item || kLeadK) TRI_WAIT_VMCNT(0);  // (the K-leading ring requests in another order: it awaits everything)
+    if (kPair && n_tiles > 1) TRI_WAIT_VMCNT(2 * kPerOperand);  // (K of tile 1 and V of tile 0 follow: 2 kPerOperand loads)
+    else if (!first_item || kLeadK) TRI_WAIT_VMCNT(0);  // (the K-leading ring requests in another order: it awaits everything)
     else if (n_first == 3) TRI_WAIT_VMCNT(2 * kBlocksPerWave);
     else if (n_first == 2) TRI_WAIT_VMCNT(kBlocksPerWave);
     else TRI_WAIT_VMCNT(0);
@@ -475,7 +482,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
         // slot of tile j+dist: every wave is done with the tile it held (two barriers ago at the latest)
         const bool issued = j + dist < n_tiles;            // the K tile requested in this step exists
         const bool issued_v = j + dist - kLag < n_tiles;   // ... its V tile (the same tile, or the one before it)
-        if (issued_v) issue_slice(j + dist, 0, issued, issued_v);
+        if (!kPair && issued_v) issue_slice(j + dist, 0, issued, issued_v);
         const int t0 = key0 + j * kBN;
         constexpr bool active = true;
 
@@ -556,7 +563,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
             // exponentials in four groups of eight keys (one B operand each); the remaining loads of the
             // next tile and the first fragment reads of the matrix phase (tile j has been visible since
             // the previous barrier) are issued between the groups, so that none of them queues
-            if (issued_v) issue_slice(j + dist, 1, issued, issued_v);
+            if (!kPair && issued_v) issue_slice(j + dist, 1, issued, issued_v);
             constexpr int kNow = kDefer ? 2 : 4;  // groups whose exponentials are taken here
 #pragma unroll
             for (int ks = 0; ks < kNow; ++ks) {
@@ -566,7 +573,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
                     if constexpr (kVectorSum && !DROPOUT) l += x[e];
                 }
                 if constexpr (!DROPOUT) pb[ks] = pack8<T>(&x[8 * ks]);
-                if (ks < 2 && issued_v) issue_slice(j + dist, 2 + ks, issued, issued_v);
+                if (ks < 2 && !kPair && issued_v) issue_slice(j + dist, 2 + ks, issued, issued_v);
                 if (ks < 2 && !kLeadK) {
 #pragma unroll
                     for (int r = kRing / 2 * ks; r < kRing / 2 * (ks + 1); ++r) ring[r] = frag(Yes{}, st, r);
@@ -618,7 +625,8 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
         // after the barrier it is visible to every wave, and the partner group changes phase. The
         // fragment reads stay in flight across the barrier: nothing overwrites their slot before the
         // barrier after next.
-        wait_loads(kMaskViaLds && with_s && !mask_is_zero(j + 1), issued, issued_v);
+        if constexpr (kPair) TRI_WAIT_VMCNT(0);  // (K of tile j + 1, V of tile j)
+        else wait_loads(kMaskViaLds && with_s && !mask_is_zero(j + 1), issued, issued_v);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
@@ -635,6 +643,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
                 for (int r = 0; r < kRing; ++r) ring[r] = frag(Yes{}, st, r);
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if (kPair && issued_v) issue_tile(j + dist, issued, issued_v);
             // the few instructions of this phase go first, so that the matrix pipe never waits for an
             // issue slot behind the partner's vector work
             __builtin_amdgcn_s_setprio(2);
@@ -648,11 +657,16 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    static_assert(kStages == 4 || kStages == 3, "the tile loop is unrolled over the ring's slots");
+    static_assert(kStages >= 2 && kStages <= 4, "the tile loop is unrolled over the ring's slots");
     // (a mask and dropout together at D = 128 have no registers to spare for four copies of the step: rolled, the slot
     // is a run-time value there and every fragment read adds it to its address)
     constexpr bool kUnrolled = !(D == 128 && kMatrix && DROPOUT);
-    if constexpr (kUnrolled && kStages == 3) {
+    if constexpr (kUnrolled && kStages == 2) {
+        for (int j = 0; j < my_tiles; j += 2) {
+            tile_step(j, 0);
+            if (j + 1 < my_tiles) tile_step(j + 1, 1);
+        }
+    } else if constexpr (kUnrolled && kStages == 3) {
         for (int j = 0; j < my_tiles; j += 3) {
             tile_step(j, 0);
             if (j + 1 < my_tiles) tile_step(j + 1, 1);
@@ -670,9 +684,11 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED ? 1 : THREE 
     }
     for (int j = my_tiles; j < n_tiles; ++j) {
         const bool issued = j + dist < n_tiles, issued_v = j + dist - kLag < n_tiles;
-        if (issued_v) issue_tile(j + dist, issued, issued_v);
-        wait_loads(false, issued, issued_v);
+        if (!kPair && issued_v) issue_tile(j + dist, issued, issued_v);
+        if constexpr (kPair) TRI_WAIT_VMCNT(0);
+        else wait_loads(false, issued, issued_v);
         lds_barrier();
+        if (kPair && issued_v) issue_tile(j + dist, issued, issued_v);
         if constexpr (kPingPong) lds_barrier();
     }
     if (kPingPong && group == 0) lds_barrier();  // group 1 is still in its last matrix phase

@@ -232,13 +232,6 @@ int persistent_grid(int items) {
     return items < n ? items : n;
 }
 
-bool four_waves_fit_one_round(const KParams& p) {
-    const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
-    if (items > 1 << 20) return false;
-    const int busy = static_cast<int>(p.causal && p.S >= 1024 ? (2 * items + 2) / 3 : items);
-    return persistent_grid(busy) == busy;
-}
-
 bool mask_is_key_bits(const KParams& p) {  // (of 16-bit problems: mfma_supported; a 16-bit mask is of their type)
     return p.mask != nullptr && p.mask_binary && p.mask_padded && p.ms[2] == 0 && p.mask_dtype != TRI_ATTN_F32 && p.mcls != nullptr &&
            p.dmask == nullptr && (p.D <= 64 || p.thr8 <= 0) && p.S <= 64 * 64;
