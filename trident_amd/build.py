@@ -45,13 +45,13 @@ FLAGS = [
 BASELINE_KERNELS = {
     "mfma_fwd_kernel<_Float16, 64, 4, false, 0, false, false, false, false>": "C2 fwd",
     "mfma_fwd_kernel<__bf16, 128, 8, true, 0, false, false, false, false>": "C3 fwd",
-    "mfma_dq_phased_kernel<__bf16, 128, true, false, true, false, false, false>": "C3 dQ + delta",
+    "mfma_dq_phased_kernel<__bf16, 128, true, false, true, false, false, false, 8>": "C3 dQ + delta",
     "mfma_dkdv_phased_kernel<__bf16, 128, true, false, 0, false, false>": "C3 dK/dV",
     "mfma_fwd_kernel<__bf16, 64, 4, false, 1, false, false, false, false>": "C4 fwd",
     "mfma_dkdv_wide_kernel<__bf16, 64, false, 1, false, false, false>": "C4 dK/dV",
     "mfma_dq_kernel<__bf16, 64, 4, false, 1, false, false, false, true, false, false>": "C4 dQ + delta",
     "mfma_fwd_kernel<__bf16, 128, 8, true, 0, true, false, false, false>": "C5 fwd",
-    "mfma_dq_phased_kernel<__bf16, 128, true, true, true, false, false, false>": "C5 dQ + delta",
+    "mfma_dq_phased_kernel<__bf16, 128, true, true, true, false, false, false, 8>": "C5 dQ + delta",
     "mfma_dkdv_phased_kernel<__bf16, 128, true, true, 0, false, false>": "C5 dK/dV",
     "mfma32_fwd_kernel<float, 32, false>": "C1 fwd",
 }

@@ -72,28 +72,46 @@ bool dq_is_phased(const KParams& p) {
     return D == 128 && (p.thr8 <= 0 || (p.causal && p.S % 256 == 0));
 }
 
-// D = 128 without a mask: workgroups of four waves (kPair), two to a CU, instead of one of eight, whose pairs of waves are phased where their
+// D = 128 without a mask: workgroups of four waves, two to a CU, instead of one of eight, whose pairs of waves are phased where their
 // registers allow it. Four waves gain where 128 rows waste less than 256 (rows that do not exist, keys above the diagonal), where starts and
-// ends are a large part of the time, and where 256-row items leave CUs idle in the last round; per tile the phased kernel needs less (time of
-// four waves over its beyond these rules: without dropout 1.04-1.19, with it 1.00-1.10, causal 0.98-1.10). By the rules in turn:
-//   S <= 128            0.60-0.79 from 512 heads on, 0.89-1.02 up to 64
-//   without dropout, up to 512 rows
-//     up to a workgroup per CU              0.87-1.01 (causal S = 384, whose second item is light: 1.00-1.07, not taken)
-//     more than two per CU, causal          0.76-0.95
-//     more than two per CU, S in 257 .. 384 0.79-0.93
-//   with dropout
-//     up to a workgroup per CU              0.72-0.95
-//     not causal, fewer half rounds than eight waves take (each of their rounds is two)  0.66-0.90
-//     causal, up to 8/3 per CU              0.81-0.93; S <= 512, or S <= 1024 with a half-empty last item 0.69-0.90
+// ends are a large part of the time, and where 256-row items leave CUs idle in the last round; per tile the eight phased waves need less. Time of
+// four waves over that of eight, bf16, 0.5 to 24 workgroups per CU (a half round: of workgroups of four waves; a round of the eight is two):
+//   S <= 128                                  0.58-0.95
+//   up to a workgroup per CU                  0.72-0.98 (causal 384 rows, whose second item is light, 0.92-1.01)
+//   causal with dropout, up to 1024 rows      0.67-1.03; longer: up to 8/3 per CU 0.81-0.91, 4 to 16 up to 4096 rows 0.86-1.01; else 0.94-1.11
+//   causal, up to 800 rows, up to 16 per CU   0.68-1.02, but one to two per CU at 257 to 384 rows 0.95-1.08, three to four
+//                                             at more without a half-empty last item 0.96-1.09; beyond 16 1.01-1.12, out of the caches
+//   causal, longer, up to 3/2 per CU          0.90-1.01; else 0.96-1.17
+//   not causal with dropout                   fewer half rounds 0.58-0.98; up to 800 rows from two per CU on 0.62-0.97, up to 2048 from four on
+//                                             0.89-1.00; else 0.95-1.09
+//   not causal, up to 512 rows, above two per CU  0.69-0.97; one to two 1.00-1.07
+//   not causal, up to 800 rows, half-empty last item, eight waves in more than a round  0.67-1.03
+//   not causal, longer, three quarters of the half rounds  0.92-1.02; else 0.96-1.20
 bool dq_runs_four_waves(const KParams& p) {
     const int64_t cus = persistent_grid(1 << 20), heads = static_cast<int64_t>(p.B) * p.H;
     const int64_t items = heads * ((p.S + 127) / 128), items256 = heads * ((p.S + 255) / 256);
+    const int64_t halves = (items + cus - 1) / cus, rounds256 = (items256 + cus - 1) / cus;
     const bool half_empty = (p.S - 1) % 256 < 128;
-    if (p.S <= 128) return true;
-    if (p.thr8 <= 0) return p.S <= 512 && (items <= cus ? !p.causal || p.S % 256 != 128 : items > 2 * cus && (p.causal || half_empty));
-    if (items <= cus) return true;
-    if (p.causal) return 3 * items <= 8 * cus || p.S <= (half_empty ? 1024 : 512);
-    return (items + cus - 1) / cus < 2 * ((items256 + cus - 1) / cus);
+    if (p.S <= 128 || items <= cus) return true;
+    if (p.causal && p.thr8 > 0) return p.S <= 1024 || 3 * items <= 8 * cus || (p.S <= 4096 && items > 4 * cus && items <= 16 * cus);
+    if (p.causal) {
+        if (p.S > 800) return 2 * items <= 3 * cus;
+        if (p.S > 256 && items > (p.S <= 384 ? 1 : 3) * cus && items <= (p.S <= 384 ? 2 : 4) * cus) return p.S > 384 && half_empty;
+        return items <= 16 * cus;
+    }
+    if (p.thr8 > 0) return halves < 2 * rounds256 || (p.S <= 800 && items > 2 * cus) || (p.S <= 2048 && items > 4 * cus);
+    if (p.S <= 512) return items > 2 * cus;
+    if (p.S <= 800 && half_empty) return items256 > cus;
+    return 4 * halves <= 6 * rounds256;
+}
+
+// ... and whether those four run phases (mfma_dq_phased_kernel, whose rows come through LDS) or not (kPair): a few tiles are over before that
+// pays. Time of the phased over the unphased ones: S <= 128 0.83-1.10; up to a workgroup per CU 0.84-1.06; else up to 384 rows 0.93-1.13, with
+// dropout up to 800 rows 0.95-1.13, beyond 0.91-1.05.
+bool dq_four_waves_phased(const KParams& p) {
+    if (p.S <= 128) return false;
+    const int64_t items = static_cast<int64_t>(p.B) * p.H * ((p.S + 127) / 128);
+    return p.S > (p.thr8 > 0 ? 800 : 384) || items <= persistent_grid(1 << 20);
 }
 
 // any length (no mask, or a padded one), with boundary handling
@@ -126,31 +144,30 @@ int launch_dq_ragged(const KParams& p, hipStream_t stream, bool with_delta) {
     return static_cast<int>(hipGetLastError());
 }
 
-template <typename T, int D, bool CAUSAL, bool RAGGED, int MASK>
+template <typename T, int D, bool CAUSAL, bool RAGGED, int MASK, int NW = 8>
 int launch_dq_phased(const KParams& p, hipStream_t stream, bool with_delta) {
-    const dim3 grid(p.B * p.H * ((p.S + 255) / 256)), block(512);
-    if constexpr (MASK == kMaskKeys) {
-        if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, RAGGED, false, true>), grid, block, 0, stream, p);
-        else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false, RAGGED, false, true>), grid, block, 0, stream, p);
-        return static_cast<int>(hipGetLastError());
-    }
-    if constexpr (D == 128 && CAUSAL && !RAGGED) {
+    const dim3 grid(p.B * p.H * ((p.S + 32 * NW - 1) / (32 * NW))), block(64 * NW);
+    constexpr bool kKeys = MASK == kMaskKeys;
+    if constexpr (NW == 4 || (D == 128 && CAUSAL && !RAGGED)) {
         if (p.thr8 > 0) {
-            if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true, RAGGED>), grid, block, 0, stream, p);
-            else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, false, RAGGED>), grid, block, 0, stream, p);
+            if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, true, RAGGED, false, kKeys, NW>), grid, block, 0, stream, p);
+            else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, true, false, RAGGED, false, kKeys, NW>), grid, block, 0, stream, p);
             return static_cast<int>(hipGetLastError());
         }
     }
-    if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, RAGGED>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false, RAGGED>), grid, block, 0, stream, p);
+    if (with_delta) hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, true, RAGGED, false, kKeys, NW>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((mfma_dq_phased_kernel<T, D, CAUSAL, false, false, RAGGED, false, kKeys, NW>), grid, block, 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
 template <typename T, int D, bool CAUSAL, int MASK>
 int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
     if constexpr (D == 128 && MASK == kNoMask) {
-        if (dq_runs_four_waves(p))
+        if (dq_runs_four_waves(p)) {
+            if (dq_four_waves_phased(p))
+                return p.S % 128 == 0 ? launch_dq_phased<T, D, CAUSAL, false, MASK, 4>(p, stream, with_delta) : launch_dq_phased<T, D, CAUSAL, true, MASK, 4>(p, stream, with_delta);
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
+        }
     }
     if constexpr ((MASK == kNoMask || MASK == kMaskKeys) && (D == 128 || (D == 64 && !CAUSAL && MASK == kNoMask))) {
         if (dq_is_phased<D, MASK>(p)) {

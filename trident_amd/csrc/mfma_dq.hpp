@@ -416,7 +416,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != 
     }
 }
 
-// ------------------------------------------------------------------ dQ, phased (8 waves, no mask)
+// ------------------------------------------------------------------ dQ, phased (no mask, or one of keys)
 // Same data flow and tile ring as above, restructured so that the two waves of a SIMD (w and w+4)
 // never do the same kind of work at once. Per 64-key tile a wave runs a vector phase (P and dS of the
 // tile from its S^T and dP^T, packed as B operands) and a matrix phase (dQ^T += K^T dS^T of this
@@ -430,16 +430,25 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != 
 // RAGGED: S is not a multiple of 256; rows and keys at or beyond S as in the kernel above (clamped loads, probability 0,
 // not stored), a wave without a single row of its own only fetches and meets the barriers.
 // KEYS: beside a mask of keys that is 0 or -inf (KeyBits).
-template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false, bool SPLIT = false, bool KEYS = false>
-__global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p) {
+// NW = 4 (D = 128): workgroups of 128 rows, two to a CU, whose waves share a SIMD without any order between them. 80 KiB of LDS hold three K
+// tiles and two V tiles: a tile's matrix phase, behind a barrier that every wave meets once it is done with the phase before (K of tiles t - 1
+// and t, V of tile t), requests K and V of tile t + 2 into the slots of K of tile t - 1 and V of tile t; the next tile's barrier awaits them.
+// bf16, us, eight waves -> these, heads x S: 16 x 1024 31.4 -> 26.5, 640 x 256 60.6 -> 51.7 (unphased four), 72 x 777 61.3 -> 43.0, causal 104 x 640
+// 37.4 -> 30.1; with dropout 16 x 2048 95.8 -> 65.6, 40 x 4096 588 -> 502, causal 64 x 4096 463 -> 425.
+template <typename T, int D, bool CAUSAL, bool DROPOUT, bool DELTA, bool RAGGED = false, bool SPLIT = false, bool KEYS = false, int NW = 8>
+__global__ __launch_bounds__(64 * NW, 2) void mfma_dq_phased_kernel(const KParams p) {
     static_assert(!RAGGED || D == 128, "boundary handling: D = 128 only");
     static_assert(!KEYS || !(CAUSAL || SPLIT), "a mask excludes the causal variant");
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
+    static_assert(NW == 8 || (NW == 4 && D == 128 && !SPLIT), "eight waves, or four at D = 128");
     using Tile = SwzTile<D>;
-    constexpr int NW = 8;
+    constexpr bool kPair = NW == 4;
     constexpr int kRows = 32 * NW;
     constexpr int kStages = 4;
     constexpr int kStageBytes = 2 * Tile::kBytes;  // K tile, V tile
+    // byte offsets of K and V of tile t (-1 is never read)
+    auto k_slot = [](int t) { return kPair ? static_cast<int>(static_cast<unsigned>(t + 3) % 3) * Tile::kBytes : ((t + kStages) % kStages) * kStageBytes; };
+    auto v_slot = [](int t) { return kPair ? (3 + (t & 1)) * Tile::kBytes : ((t + kStages) % kStages) * kStageBytes + Tile::kBytes; };
     constexpr int KK = D / 16;
     constexpr int DB = D / 32;
     constexpr int kBlocksPerWave = 2 * Tile::kBlocks / NW;
@@ -459,8 +468,12 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     // for a single plain load).
     constexpr int kWaveRowBytes = 32 * Tile::kRowBytes;  // a wave's rows of one operand
     constexpr int kRowLoads = kWaveRowBytes / 1024;      // LDS-direct loads per wave and operand
-    __shared__ __attribute__((aligned(1024))) char smem[kStageBytes + 2 * NW * kWaveRowBytes];
-    static_assert(kStageBytes + 2 * NW * kWaveRowBytes >= kStages * kStageBytes, "the ring lies inside");
+    // (four waves: the Q rows in the place of K of tiles 1 and 2, the dO rows in that of the V tiles)
+    constexpr int kStaging = kPair ? Tile::kBytes : kStageBytes;
+    constexpr int kRingBytes = kPair ? 5 * Tile::kBytes : kStages * kStageBytes;
+    __shared__ __attribute__((aligned(1024))) char smem[kStaging + 2 * NW * kWaveRowBytes];
+    static_assert(kStaging + 2 * NW * kWaveRowBytes >= kRingBytes, "the ring lies inside");
+    static_assert(!kPair || kStaging + NW * kWaveRowBytes == 3 * Tile::kBytes, "the V tiles take the place of the dO rows");
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -496,7 +509,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     float lse = p.lse[static_cast<int64_t>(bh) * p.S + qrow_ld];
     float dlt = 0.f;
     if constexpr (!DELTA) dlt = p.delta[static_cast<int64_t>(bh) * p.S + qrow_ld];
-    char* q_stage = smem + kStageBytes + wave * kWaveRowBytes;
+    char* q_stage = smem + kStaging + wave * kWaveRowBytes;
     char* g_stage = q_stage + NW * kWaveRowBytes;
 #pragma unroll
     for (int blk = 0; blk < kRowLoads; ++blk)
@@ -534,8 +547,41 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     // multiple of 16 apart, so one per-lane source offset serves all of them.
     const uint32_t koff = static_cast<uint32_t>(Tile::src_off(wave, lane, krow_bytes));
     const uint32_t voff = static_cast<uint32_t>(Tile::src_off(wave, lane, vrow_bytes));
+    auto issue_k = [&](int t) {  // (four waves)
+        char* stage = smem + k_slot(t) + wave * 1024;
+        const bool partial = RAGGED && (t + 1) * kBN > keys;
+        int l = lane;
+        if constexpr (kPair) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
+#pragma unroll
+        for (int i = 0; i < kPerOperand; ++i) {
+            if (partial)
+                lds_direct_load16(kbase + static_cast<int64_t>(t) * kBN * krow_bytes,
+                                  Tile::src_off_clamped(wave + i * NW, l, krow_bytes, keys - 1 - t * kBN), stage + i * NW * 1024);
+            else
+                lds_direct_load16(kbase + (static_cast<int64_t>(t) * kBN + i * kRowStep) * krow_bytes, koff, stage + i * NW * 1024);
+        }
+    };
+    auto issue_v = [&](int t) {
+        char* stage = smem + v_slot(t) + wave * 1024;
+        const bool partial = RAGGED && (t + 1) * kBN > keys;
+        int l = lane;
+        if constexpr (kPair) asm volatile("" : "+v"(l));  // (offsets made here, not kept in registers across the loop)
+#pragma unroll
+        for (int i = 0; i < kPerOperand; ++i) {
+            if (partial)
+                lds_direct_load16(vbase + static_cast<int64_t>(t) * kBN * vrow_bytes,
+                                  Tile::src_off_clamped(wave + i * NW, l, vrow_bytes, keys - 1 - t * kBN), stage + i * NW * 1024);
+            else
+                lds_direct_load16(vbase + (static_cast<int64_t>(t) * kBN + i * kRowStep) * vrow_bytes, voff, stage + i * NW * 1024);
+        }
+    };
     auto issue_tile = [&](int t) {
-        char* stage = smem + (t % kStages) * kStageBytes + wave * 1024;
+        if constexpr (kPair) {
+            issue_k(t);
+            issue_v(t);
+            return;
+        }
+        char* stage = smem + k_slot(t) + wave * 1024;
         if (RAGGED && (t + 1) * kBN > keys) {  // the sequence ends inside this tile
             const int last = keys - 1 - t * kBN;
 #pragma unroll
@@ -566,16 +612,22 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
             return;
         }
     }
-    issue_tile(0);
+    if constexpr (kPair) issue_k(0);
+    else issue_tile(0);
 
-    const int row_off0 = Tile::off(l32, h);
-    TRI_WAIT_VMCNT(kBlocksPerWave);  // this wave's Q and dO rows have landed (tile 0 may be on its way)
+    int row_off0 = Tile::off(l32, h);
+    TRI_WAIT_VMCNT(kPair ? kPerOperand : kBlocksPerWave);  // this wave's Q and dO rows have landed (tile 0 may be on its way)
     asm volatile("" ::: "memory");
     u32x4 qf[KK], gf[KK];
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
         qf[kk] = lds_read16(q_stage, row_off0 ^ (kk << 5));
         gf[kk] = lds_read16(g_stage, row_off0 ^ (kk << 5));
+    }
+    if constexpr (kPair) {  // every wave has its rows in registers: the V tiles can follow
+        lds_barrier();
+        issue_v(0);
+        if (n_tiles > 1) issue_v(1);
     }
     if constexpr (DELTA) {
         // the O rows follow into the place of the Q rows; this lane holds half of its row (the other half is
@@ -617,17 +669,17 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     }
     [[maybe_unused]] DropoutRows drop;
     if constexpr (DROPOUT) drop.init(p, bh, qrow >> 2);
-    const int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
+    int tr_off0 = Tile::tr_off(0, 0, lane), tr_off1 = Tile::tr_off(0, 1, lane);
 
     // fragment n of the matrix phase of tile t: n < kDqSteps: K^T of tile t (column block n % DB, K-step
     // n / DB); then the K rows (key block 0, 1) and the V rows (key block 0, 1) of tile t + 1
     auto frag = [&](int t, int n) {
         if (n < kDqSteps) {
-            const char* sK = smem + ((t + kStages) % kStages) * kStageBytes;
+            const char* sK = smem + k_slot(t);
             return Tile::tr_frag(sK, tr_off0 ^ ((n % DB) << 6), tr_off1 ^ ((n % DB) << 6), n / DB);
         }
         const int m = n - kDqSteps;
-        const char* sT = smem + ((t + 1) % kStages) * kStageBytes + (m < 2 * KK ? 0 : Tile::kBytes);
+        const char* sT = smem + (m < 2 * KK ? k_slot(t + 1) : v_slot(t + 1));
         return lds_read16(sT, (row_off0 ^ ((m % KK) << 5)) + 32 * ((m / KK) & 1) * Tile::kRowBytes);
     };
     f32x16 st[2], dpt[2];  // S^T and dP^T of the current tile (two key blocks)
@@ -667,8 +719,12 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     settle(lse);
     if constexpr (!DELTA) settle(dlt);
     lds_barrier();
-    if (n_first > 1) issue_tile(1);
-    if (n_first > 2) issue_tile(2);
+    if constexpr (kPair) {
+        if (n_first > 1) issue_k(1);
+    } else {
+        if (n_first > 1) issue_tile(1);
+        if (n_first > 2) issue_tile(2);
+    }
     if (group == 1) {
         // group 1 starts one phase late; group 0 reads tile 1 in its first matrix phase
         if (n_first == 3) TRI_WAIT_VMCNT(kBlocksPerWave);
@@ -684,7 +740,9 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
 
     for (int t = 0; t < my_tiles; ++t) {
         const bool issued = t + dist < n_tiles;
-        if (issued) issue_tile(t + dist);
+        // (the fragments' offsets of the column blocks are made from these here, not kept in registers across the loop)
+        if constexpr (kPair) asm volatile("" : "+v"(row_off0), "+v"(tr_off0), "+v"(tr_off1));
+        if (!kPair && issued) issue_tile(t + dist);
         // ---- vector phase: P and dS of the tile (only 32-key blocks that cross the diagonal pay for the
         // causal comparison)
         auto softmax_backward = [&](auto on_diagonal, int kb) {
@@ -735,29 +793,36 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
         for (int r = 0; r < kRing; ++r) ring[r] = frag(t, r);
         // tile t + dist - 1 has landed (the newest one may still be in flight); after the barrier it is
         // visible to every wave, and the partner group changes phase
-        wait_tile(issued);
+        wait_tile(!kPair && issued);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+        if (kPair && issued) issue_tile(t + dist);
         // ---- matrix phase (a wave's last tile has no successor to score; the dropout variant runs the S^T /
         // dP^T steps all the same, on whatever the next slot holds: leaving them out costs it registers it does
         // not have, and the result is never used)
         __builtin_amdgcn_s_setprio(2);
         matrix_phase(Yes{}, t, DROPOUT || t + 1 < my_tiles);
         __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
-        lds_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!kPair) {
+            __builtin_amdgcn_sched_barrier(0);
+            lds_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     // afterwards a wave only keeps fetching its share of the remaining tiles and meeting the barriers
     for (int t = my_tiles; t < n_tiles; ++t) {
         const bool issued = t + dist < n_tiles;
-        if (issued) issue_tile(t + dist);
-        wait_tile(issued);
+        if (!kPair && issued) issue_tile(t + dist);
+        wait_tile(!kPair && issued);
         lds_barrier();
-        lds_barrier();
+        if constexpr (kPair) {
+            if (issued) issue_tile(t + dist);
+        } else {
+            lds_barrier();
+        }
     }
-    if (group == 0) lds_barrier();  // group 1 is still in its last matrix phase
+    if (!kPair && group == 0) lds_barrier();  // group 1 is still in its last matrix phase
 
     if constexpr (SPLIT) {
         if (part.count > 1) {
@@ -771,7 +836,7 @@ __global__ __launch_bounds__(512, 2) void mfma_dq_phased_kernel(const KParams p)
     lds_barrier();
     {
         using Store = RowBlockStore<T, DB>;
-        static_assert(NW * Store::kPatchBytes <= kStages * kStageBytes, "patches must fit into the ring");
+        static_assert(NW * Store::kPatchBytes <= kRingBytes, "patches must fit into the ring");
         char* out0 = static_cast<char*>(p.dq) + (b * p.dqs[0] + hd * p.dqs[1] + static_cast<int64_t>(wrow0) * p.dqs[2]) * 2;
         const float sc = kDeltaInAcc ? -p.scale : p.scale;
         // the lane index taken afresh: the epilogue's per-lane offsets are then computed here instead of being

@@ -216,7 +216,7 @@ bool mfma_dq_fuses_delta(const KParams& p) {
     const bool keys = p.D == 128 && mask_is_key_bits(p) && mfma_dq_workspace(p, false) == 0;
     if (p.mask != nullptr && ((p.D > 64 && !keys) || p.dmask != nullptr)) return false;
     if (!aligned16(p.o) || !strides8(p.os)) return false;
-    const bool phased = keys || p.mask == nullptr && (p.D == 128 ? p.thr8 <= 0 || (p.causal && p.S % 256 == 0) : p.D == 64 && p.S % 256 == 0);  // (as the launcher decides)
+    const bool phased = keys || p.mask == nullptr && (p.D == 128 || (p.D == 64 && p.S % 256 == 0));  // (as the launcher may decide)
     return !phased || tile_offsets_fit(p.os);
 }
 
