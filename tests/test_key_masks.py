@@ -59,8 +59,10 @@ def test_bits_against_the_oracle(S, p, D, dtype, device):
 
 
 @pytest.mark.parametrize("form", ["batch", "head", "one", "strided"])
-@pytest.mark.parametrize("heads,S,D", [(2, 4096, 64), (2, 4097, 64), (40, 640, 64), (40, 333, 128), (3, 2048, 128), (64, 200, 32)])
-def test_bits_against_the_additive_mask(heads, S, D, form, device):
+@pytest.mark.parametrize("heads,S,D,p", [(2, 4096, 64, 0.0), (2, 4097, 64, 0.0), (40, 640, 64, 0.0), (40, 333, 128, 0.0), (3, 2048, 128, 0.0),
+                                         (64, 200, 32, 0.0), (24, 512, 128, 0.0), (1, 40, 128, 0.2), (40, 333, 128, 0.2), (24, 512, 128, 0.2),
+                                         (3, 2048, 128, 0.2), (30, 130, 128, 0.2)])
+def test_bits_against_the_additive_mask(heads, S, D, p, form, device):
     """Forms of a mask of keys: per batch, per head, one for all, every other entry of a wider tensor; the last length of the bits and the
     first behind it; launches of many heads, three workgroups to a CU, and of few, split."""
     B, dtype = 5, torch.bfloat16
@@ -70,9 +72,9 @@ def test_bits_against_the_additive_mask(heads, S, D, form, device):
     mask = {"batch": visible[:, None, None, :], "one": visible[0][None, None, None, :],
             "head": torch.stack([visible.roll(h, 0) for h in range(heads)], 1)[:, :, None, :],
             "strided": torch.stack([visible, ~visible], -1).flatten(1)[:, None, None, ::2]}[form]
-    got = _step(q, k, v, d_o, mask, 0.0, device)
+    got = _step(q, k, v, d_o, mask, p, device)
     additive = torch.zeros(mask.shape).masked_fill(~mask, -math.inf).to(dtype).expand(mask.shape[0], mask.shape[1], S, S)
-    want = _step(q, k, v, d_o, additive, 0.0, device)
+    want = _step(q, k, v, d_o, additive, p, device)
     for name, a, b in zip(("O", "dQ", "dK", "dV"), got, want):
         # both round P, dS and the result to bf16: the difference of two roundings of terms whose sum is of order 1
         error = (a.float() - b.float()).norm() / b.float().norm()

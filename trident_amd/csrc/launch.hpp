@@ -55,7 +55,7 @@ int persistent_grid(int items);
 // 0.90-0.96, dQ 0.90-1.01.
 bool three_workgroups_per_cu(const KParams& p);
 // Whether the mask is one of keys (the same for every row) that is 0 or -inf, of the operand type and over few enough tiles for the kernels
-// that keep it as bits (KeyBits; at D = 128 without dropout).
+// that keep it as bits (KeyBits).
 bool mask_is_key_bits(const KParams& p);
 
 }  // namespace tri

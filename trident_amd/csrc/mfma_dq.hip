@@ -92,6 +92,8 @@ bool dq_runs_four_waves(const KParams& p) {
     const int64_t items = heads * ((p.S + 127) / 128), items256 = heads * ((p.S + 255) / 256);
     const int64_t halves = (items + cus - 1) / cus, rounds256 = (items256 + cus - 1) / cus;
     const bool half_empty = (p.S - 1) % 256 < 128;
+    // (long rows with boundary handling, without dropout: 1.02-1.05 but where the eight need half as many half rounds more, 0.81)
+    if (p.S > 1024 && p.S % 128 != 0 && p.thr8 <= 0) return !p.causal && items > cus && 3 * halves <= 4 * rounds256;
     if (p.S <= 128 || items <= cus) return true;
     if (p.causal && p.thr8 > 0) return p.S <= 1024 || 3 * items <= 8 * cus || (p.S <= 4096 && items > 4 * cus && items <= 16 * cus);
     if (p.causal) {
@@ -169,6 +171,12 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
             return p.S % 128 == 0 ? launch_dq_waves<T, D, 4, CAUSAL, MASK>(p, stream, with_delta) : launch_dq_ragged<T, D, 4, CAUSAL>(p, stream, with_delta);
         }
     }
+    if constexpr (D == 128 && MASK == kMaskKeys) {
+        // Four phased waves, with dropout always (training step on a padded batch against the kernels that read the mask's values and had a CU
+        // for four waves: 0.70-0.89, one item per CU 0.83-1.01); without it as without a mask (0.57-1.02), but not at 385 to 512 rows (1.05-1.07)
+        if (p.thr8 > 0 || (dq_runs_four_waves(p) && (p.S <= 384 || p.S > 512)))
+            return p.S % 128 == 0 ? launch_dq_phased<T, D, CAUSAL, false, MASK, 4>(p, stream, with_delta) : launch_dq_phased<T, D, CAUSAL, true, MASK, 4>(p, stream, with_delta);
+    }
     if constexpr ((MASK == kNoMask || MASK == kMaskKeys) && (D == 128 || (D == 64 && !CAUSAL && MASK == kNoMask))) {
         if (dq_is_phased<D, MASK>(p)) {
             if constexpr (D == 128) {
@@ -177,7 +185,7 @@ int launch_dq_dropout(const KParams& p, hipStream_t stream, bool with_delta) {
             return launch_dq_phased<T, D, CAUSAL, false, MASK>(p, stream, with_delta);
         }
     }
-    if constexpr (D == 128 && MASK == kMaskKeys) return TRI_ATTN_ESHAPE;  // (without dropout: mask_is_key_bits)
+    if constexpr (D == 128 && MASK == kMaskKeys) return TRI_ATTN_ESHAPE;  // (never: the two above take every such problem)
     else {
     if (with_delta && MASK != kNoMask && (D > 64 || p.dmask != nullptr)) return TRI_ATTN_ESHAPE;  // (callers ask mfma_dq_fuses_delta first)
     // D = 128: 8 waves (256 query rows) when the sequence allows it, else 4 waves (128 rows). Up to D = 64 always 4: several such workgroups

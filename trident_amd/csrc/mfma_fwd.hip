@@ -23,7 +23,7 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
     if constexpr (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
         if (three_workgroups_per_cu(p)) return launch_fwd_three<T, CAUSAL, true, MASK>(p, stream);
     }
-    if constexpr (D == 128 && NW == 4 && MASK == kNoMask) {
+    if constexpr (D == 128 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys)) {
         if (p.S % 128 == 0) {
             if (p.thr8 > 0) hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true>), dim3(items), dim3(64 * NW), 0, stream, p);
             else hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false>), dim3(items), dim3(64 * NW), 0, stream, p);
@@ -35,7 +35,7 @@ int launch_fwd_ragged(const KParams& p, hipStream_t stream) {
     if (p.thr8 > 0) {
         if constexpr (!(D == 128 && NW == 8 && MASK != kNoMask))
             hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, true, true>), grid, block, 0, stream, p);
-    } else if constexpr (!(D == 128 && NW == 4 && MASK != kNoMask)) {
+    } else if constexpr (!(D == 128 && NW == 4 && MASK != kNoMask && MASK != kMaskKeys)) {
         hipLaunchKernelGGL((mfma_fwd_kernel<T, D, NW, CAUSAL, MASK, false, true>), grid, block, 0, stream, p);
     }
     return static_cast<int>(hipGetLastError());
@@ -109,8 +109,10 @@ int launch_fwd_waves(int dtype, const KParams& p, hipStream_t stream) {
     // dropout 0.70-0.99; beside 16-bit masks 0.90-1.01; beside fp32 ones, whose ring of three lets two workgroups onto a CU, 0.88-0.96, length
     // masks 0.84-1.00 (dense ones in whole rounds of S = 2048 1.04-1.06).
     if constexpr (D == 128) {
-        if (mask_is_key_bits(p))
+        if (mask_is_key_bits(p)) {  // (with dropout always four waves: two workgroups to a CU against one of four waves that read the mask's values)
+            if (p.thr8 > 0 || fwd_runs_four_waves(p)) return launch_fwd_ragged<T, D, 4, false, kMaskKeys>(p, stream);
             return p.S % 256 == 0 ? launch_fwd_dropout<T, D, 8, false, kMaskKeys>(p, stream) : launch_fwd_ragged<T, D, 8, false, kMaskKeys>(p, stream);
+        }
         if (p.mask == nullptr && fwd_runs_four_waves(p)) return p.causal ? launch_fwd_ragged<T, D, 4, true>(p, stream) : launch_fwd_ragged<T, D, 4, false>(p, stream);
         if (p.S % 256 == 0) return launch_fwd_variant<T, D, 8>(dtype, p, stream);
         if (p.mask == nullptr) return p.causal ? launch_fwd_ragged<T, D, 8, true>(p, stream) : launch_fwd_ragged<T, D, 8, false>(p, stream);

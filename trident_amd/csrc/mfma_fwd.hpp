@@ -38,7 +38,7 @@ enum MaskKind { kNoMask = 0, kMaskF32 = 1, kMaskT = 2, kMaskKeys = 3 };  // (kMa
 // SPLIT (with RAGGED): a workgroup streams one part of its item's tiles (split.hpp). Tiles count from the part's first one, keys from key0.
 // THREE (D = 64, no mask, 4 waves): three workgroups to a CU instead of two (three_workgroups_per_cu).
 template <typename T, int D, int NW, bool CAUSAL, int MASK, bool DROPOUT, bool RAGGED = false, bool SPLIT = false, bool THREE = false>
-__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != kNoMask || SPLIT) ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
+__global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK == kMaskF32 || MASK == kMaskT || SPLIT) ? 1 : THREE ? 3 : 2) void mfma_fwd_kernel(const KParams p) {
     static_assert(RAGGED || !SPLIT, "parts have boundary handling");
     static_assert(!THREE || (D == 64 && NW == 4 && (MASK == kNoMask || MASK == kMaskKeys) && !SPLIT), "three workgroups per CU");
     constexpr bool kMatrix = MASK == kMaskF32 || MASK == kMaskT;  // a mask whose values are read tile by tile
@@ -48,12 +48,12 @@ __global__ __launch_bounds__(NW * 64, D == 128 && NW == 4 && RAGGED && (MASK != 
     // three slots per operand and the K tiles run one tile ahead of the V tiles: K of tile t is last read one matrix
     // phase before V of tile t, so with K(j + dist) and V(j + dist - 1) requested together every tile keeps the lead
     // it has in the ring of four, and both fit three slots. The first fragments of V wait for the barrier, though.
-    // Without a mask the workgroups of four waves at D = 128 run two to a CU: two slots per operand in 64 KiB, half of the registers. Tile
+    // Without a mask or beside one of keys the workgroups of four waves at D = 128 run two to a CU: two slots per operand in 64 KiB, half of the registers. Tile
     // j's matrix phase, behind a barrier that every wave meets once it is done with K of tile j and V of tile j - 1, requests K of tile j + 2
     // and V of tile j + 1 into their slots, and the barrier of tile j + 1 awaits both. A workgroup alone on its CU (eight waves and a ring of four,
     // or four waves) leaves the CU to its start, its end and its barriers; two hide one another's. bf16, us, eight waves -> two times four, heads x S:
     // 1024 x 128 32.9 -> 24.1, causal 40 x 1024 28.0 -> 24.1; with dropout 1024 x 300 130 -> 102, causal 32 x 2048 76.8 -> 56.3, 40 x 4096 243 -> 213.
-    constexpr bool kPair = D == 128 && NW == 4 && MASK == kNoMask && !SPLIT;
+    constexpr bool kPair = D == 128 && NW == 4 && !kMatrix && !SPLIT;
     constexpr bool kLeadK = THREE || kPair || (MASK == 1 && ((D == 128 && NW == 8 && !DROPOUT) || (D == 64 && NW == 4)));
     constexpr int kStages = kPair ? 2 : kLeadK ? 3 : 4;  // LDS ring depth
     constexpr int kLag = kLeadK ? 1 : 0;     // how many tiles the V requests trail the K requests

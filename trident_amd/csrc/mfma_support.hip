@@ -234,7 +234,7 @@ int persistent_grid(int items) {
 
 bool mask_is_key_bits(const KParams& p) {  // (of 16-bit problems: mfma_supported; a 16-bit mask is of their type)
     return p.mask != nullptr && p.mask_binary && p.mask_padded && p.ms[2] == 0 && p.mask_dtype != TRI_ATTN_F32 && p.mcls != nullptr &&
-           p.dmask == nullptr && (p.D <= 64 || p.thr8 <= 0) && p.S <= 64 * 64;
+           p.dmask == nullptr && p.S <= 64 * 64;
 }
 
 bool three_workgroups_per_cu(const KParams& p) {
